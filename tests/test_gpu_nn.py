@@ -240,6 +240,16 @@ def test_batch_norm(rt, shape, mode):
         gpu_op.bn_backward(gx, gdy, gdx, mode, mean_p, var_p, lst, rt.cudnn, rt.stream)
 
 
+# more rows than the register kernels hold: fewest rows, one and two narrow column blocks, one to four tiles of
+# 256 rows, whole and ragged; the wide column blocks (16 384 columns and more on 256 units), whole and ragged
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(129, 1, 1), (1000, 1, 10), (256, 1, 16), (257, 1, 17), (129, 1, 16384), (130, 4, 64, 65)], ids=str)
+def test_batch_norm_with_rows_walked_in_tiles(rt, shape):
+    test_batch_norm(rt, shape, "pre_activation")
+    if len(shape) == 4:
+        test_fused_batch_norm_relu_equals_the_two_ops(rt, shape)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["pre_activation", "spatial"])
 def test_batch_norm_with_mean_far_from_zero(rt, mode):
