@@ -97,13 +97,24 @@ __global__ __launch_bounds__(kThreads) void midsum_kernel(const float *__restric
   if (threadIdx.x == 0) out[(int64_t)blockIdx.y * B + b] = total;
 }
 
-// out[j] = sum_chunk partial[chunk*B + j], chunks added in index order
+// out[j] = sum_chunk partial[chunk*B + j], chunks added in index order.  Bound by the loads' latency (a few
+// KB from the L2): sixteen of them are in flight before the first addition.  One at a time, the 84 to 250
+// chunks of a narrow bias gradient at batch 1000 took 27 us on average.
 __global__ __launch_bounds__(kThreads) void finalsum_kernel(const float *__restrict__ partial,
                                                            float *__restrict__ out, int B, int chunks) {
+  constexpr int DEPTH = 16;
   const int j = blockIdx.x * kThreads + threadIdx.x;
   if (j >= B) return;
   float s = 0.f;
-  for (int c = 0; c < chunks; ++c) s += partial[(int64_t)c * B + j];
+  int c = 0;
+  for (; c + DEPTH <= chunks; c += DEPTH) {
+    float v[DEPTH];
+#pragma unroll
+    for (int e = 0; e < DEPTH; ++e) v[e] = partial[(int64_t)(c + e) * B + j];
+#pragma unroll
+    for (int e = 0; e < DEPTH; ++e) s += v[e];
+  }
+  for (; c < chunks; ++c) s += partial[(int64_t)c * B + j];
   out[j] = s;
 }
 
