@@ -86,6 +86,33 @@ def test_conv_forward_and_gradients(rt, case):
     _check_conv_case(rt, case)
 
 
+# grad-data of strided filters by phases: u*v = 2, 3 and 4, a phase without taps (filter smaller than the stride
+# one way), a phase without pixels (one input row), rows and columns that no tap reaches (rows past the last window),
+# padding larger than a phase's offset, both filter loaders (channels a multiple of 4 or not), every tile shape
+PHASE_CASES = [
+    (2, 5, 9, 11, 7, 3, 3, "SAME", 2, 1),
+    (2, 8, 9, 11, 7, 2, 5, "VALID", 1, 2),
+    (3, 6, 10, 8, 9, 3, 4, "VALID", 1, 3),
+    (2, 4, 13, 9, 3, 3, 1, "VALID", 4, 1),
+    (2, 12, 8, 8, 6, 2, 1, "VALID", 2, 2),
+    (2, 12, 8, 7, 6, 1, 3, "VALID", 2, 2),
+    (5, 3, 1, 9, 4, 1, 3, "VALID", 2, 2),
+    (2, 8, 12, 14, 10, 5, 5, "SAME", 2, 2),
+    (1, 70, 31, 29, 20, 7, 7, "SAME", 2, 2),
+    (4, 130, 56, 56, 33, 3, 3, "SAME", 2, 2),
+    (16, 128, 57, 55, 64, 3, 3, "VALID", 2, 2),
+]
+
+
+@pytest.mark.parametrize("case", PHASE_CASES, ids=lambda c: "x".join(str(v) for v in c))
+def test_strided_grad_data_by_phases(rt, case):
+    from tinyflow_amd import gpu_op
+    N, C, H, W, K, R, S, padding, u, v = case
+    _, lst = gpu_op.convolution_2d_forward_get_out_shape((N, C, H, W), (K, C, R, S), "NCHW", padding, u, v)
+    assert "dgrad_phases" in _describe(lst, 1)
+    _check_conv_case(rt, case)
+
+
 # 3x3 / stride-1 shapes for the Winograd form (forced on: the planner would pick the
 # direct form for most of these small sizes).  (.., expect forward, expect grad-data)
 WINOGRAD_CASES = [

@@ -43,7 +43,7 @@ __device__ inline float buf_load(__amdgpu_buffer_rsrc_t r, uint32_t byte_off) {
 // exact for n < 2^31.
 struct FastDiv {
   uint32_t d, mul, shift;
-  FastDiv() : d(1), mul(0), shift(0) {}
+  __host__ __device__ FastDiv() : d(1), mul(0), shift(0) {}
   explicit FastDiv(uint32_t div) : d(div ? div : 1) {
     div = d;
     uint32_t l = 0;
@@ -357,6 +357,17 @@ __device__ inline int xcd_contiguous(int id, int n) {
   return id < (per_xcd << 3) ? (id & 7) * per_xcd + (id >> 3) : id;
 }
 
+// Reduction length of this workgroup's problem: the launch's, unless the problems on
+// blockIdx.y differ in it and their B loader knows (it defines problem_k_extent()).
+template <class L, class = void>
+struct ProblemExtent {
+  static __device__ inline int of(const L &, int k_extent) { return k_extent; }
+};
+template <class L>
+struct ProblemExtent<L, std::void_t<decltype(&L::problem_k_extent)>> {
+  static __device__ inline int of(const L &loader, int) { return loader.problem_k_extent(); }
+};
+
 // ---- the kernel ----------------------------------------------------------------------
 // Work decomposition: gridDim.x = tiles_m * tiles_n * splits (plus, with a fold, the
 // pieces of the folded tiles behind the plain workgroups).  Hardware hands
@@ -415,7 +426,8 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(const ALoader al, const B
     k_begin = piece * fold.k_per_piece;
     k_end = k_begin + fold.k_per_piece;
   }
-  if (k_end > k_extent) k_end = k_extent;
+  const int own_extent = ProblemExtent<BLoader>::of(bl, k_extent);
+  if (k_end > own_extent) k_end = own_extent;
   const int tm = tile % tiles_m, tn = tile / tiles_m;
   const int m0 = tm * BM, n0 = tn * BN;
 
