@@ -308,6 +308,36 @@ def test_fused_update_is_bit_identical_to_per_variable_updates():
             assert a.tobytes() == b.tobytes()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [7, 64])
+def test_fused_adam_update_is_bit_identical_to_per_variable_updates(batch):
+    """One multi-tensor launch against two calls per variable: losses, parameters and moments over
+    three steps.  LeNet-5 has tensors shorter than a vector, of no multiple of four elements and of
+    more than one piece of the run table."""
+    from tinyflow_amd import models
+    from tinyflow_amd.TrainExecuteAdam import TrainExecutor
+    runs = []
+    for fused in (False, True):
+        rng = np.random.RandomState(22)
+        model = models.lenet5(rng, batch=batch, head="softmax_xent")
+        X, y = models.synthetic_batch(rng, model.input_shape, model.n_class, "normal")
+        ex = TrainExecutor(model.loss, 0.01)
+        ex.fused_update = fused
+        ex.init_Variable(dict(model.variables))
+        steps = []
+        for _ in range(3):
+            out = list(ex.run({model.X: X, model.y_: y}))
+            for v in ex.Variable_node_list:
+                out += ex.moments_of(v)
+            steps.append([o.asnumpy() for o in out])
+        assert (ex._fused_sgd is not None) == fused
+        runs.append(steps)
+        ex.close()
+    for a_step, b_step in zip(*runs):
+        for a, b in zip(a_step, b_step):
+            assert a.tobytes() == b.tobytes()
+
+
 @pytest.mark.parametrize("config", ["mlp", "lenet5"])
 def test_adam_executor_matches_oracle(config):
     """Three Adam steps (the reference's TrainExecuteAdam flow): loss, gradients, both

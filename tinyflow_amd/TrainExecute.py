@@ -20,6 +20,8 @@ from . import gpu_op, ndarray
 class TrainExecutor(object):
     """Runs forward + backward + SGD update for one loss node."""
 
+    _update_op = ad.SgdOp   # the update nodes that one multi-tensor call can apply together
+
     def __init__(self, targetloss, learning_rate, ctx=ndarray.gpu(0), fuse_bn_relu=False, fused_update=True):
         """``fuse_bn_relu`` (no counterpart in the reference): evaluate every batch
         norm whose only reader is a ReLU together with that ReLU, forward and
@@ -27,7 +29,7 @@ class TrainExecutor(object):
         batch-norm output and the ReLU's input gradient are then never materialised
         (``value_of`` does not know them).
 
-        ``fused_update``: apply all SGD updates of a step with one call of the
+        ``fused_update``: apply all updates of a step with one call of the
         multi-tensor entry point (``sgd_compute_o``, reference gpu_op.py:939-945) behind
         the last node of the step instead of one ``sgd_update`` per variable.  Every
         update still comes after the last reader of its parameter, which is all
@@ -57,6 +59,9 @@ class TrainExecutor(object):
         """One in-place update node per variable, in ``Variable_node_list`` order."""
         return getcomputelist(self.Variable_node_list, self.Variable_node_grad_list, self.learning_rate)
 
+    def _fuse_updates(self, updates):
+        return _FusedSgd(updates)
+
     def infer_shape(self, feed_shapes):
         """Shapes of every node from the shapes of the fed nodes."""
         self.node_to_shape_map = dict(feed_shapes)
@@ -83,7 +88,7 @@ class TrainExecutor(object):
         self.infer_shape({node: np.shape(value) for node, value in feed_dict.items()})
         plan = []
         fused = {}
-        fused_sgd = []   # (parameter array, gradient array, learning rate) of the updates applied in one call
+        fused_updates = []   # (update node, its input arrays) of the updates applied in one call
         if self.fuse_bn_relu:
             fused.update(find_bn_relu_pairs(self.topo_order, {self.targetloss}))
             fused.update(find_add_relu_pairs(self.topo_order, {self.targetloss}, self.node_to_shape_map))
@@ -115,8 +120,8 @@ class TrainExecutor(object):
             assert node.isw not in (1, 2), "no value fed for %s" % node.name
             input_vals = [self.node_to_arr_map.get(i) if i in unread_zeros else self.node_to_arr_map[i]
                           for i in node.inputs]
-            if node.issgd and self.fused_update and isinstance(node.op, ad.SgdOp):
-                fused_sgd.append((input_vals[0], input_vals[1], node.learning_rate))
+            if node.issgd and self.fused_update and isinstance(node.op, self._update_op):
+                fused_updates.append((node, input_vals))
                 continue
             if node.issgd:
                 node_val = None  # updates its parameter in place
@@ -130,8 +135,8 @@ class TrainExecutor(object):
         if self._fused_sgd is not None:
             self._fused_sgd.close()
             self._fused_sgd = None
-        if fused_sgd:
-            self._fused_sgd = _FusedSgd(fused_sgd)
+        if fused_updates:
+            self._fused_sgd = self._fuse_updates(fused_updates)
         self.isfirstrun = 1
 
     def run(self, feed_dict, Accuracy_node=None, convert_to_numpy_ret_vals=False):
@@ -186,38 +191,47 @@ class TrainExecutor(object):
             pass
 
 
-class _FusedSgd(object):
-    """All SGD updates of a step as one launch: the pointer tables and the index ->
-    (tensor, offset) tables of ``sgd_compute_o`` (reference gpu_op.py:887-945), built
-    once for the step's parameter and gradient arrays, which keep their storage from
+class FusedUpdate(object):
+    """All parameter updates of a step as one launch: the pointer tables and the index ->
+    (tensor, offset) tables of ``sgd_compute_o`` / ``adam_compute_o`` (reference
+    gpu_op.py:887-945), built once for the step's arrays, which keep their storage from
     step to step.  The call has no stream argument: it runs on the default stream,
-    which is ordered behind the executor's stream and in front of its next launch."""
+    which is ordered behind the executor's stream and in front of its next launch.
+
+    ``updates``: pairs of an update node and its input arrays, parameter first."""
 
     def __init__(self, updates):
-        rates = set(lr for _, _, lr in updates)
+        rates = set(node.learning_rate for node, _ in updates)
         assert len(rates) == 1, "one learning rate per step"
         self.learning_rate = rates.pop()
-        self.arrays = [(w, g) for w, g, _ in updates]   # keeps the storage alive
-        sizes = [int(np.prod(w.shape)) for w, _ in self.arrays]
-        for (w, g), n in zip(self.arrays, sizes):
-            assert int(np.prod(g.shape)) == n, "gradient and parameter sizes differ"
+        self.arrays = [arrays for _, arrays in updates]   # keeps the storage alive
+        sizes = [int(np.prod(arrays[0].shape)) for arrays in self.arrays]
+        for arrays, n in zip(self.arrays, sizes):
+            assert all(int(np.prod(a.shape)) == n for a in arrays), "gradient and parameter sizes differ"
         assert sum(sizes) < 2 ** 31
         # whole tensors end to end: the tables are built from the sizes, not from
         # per-parameter (tensor, offset) arrays
         self.tables, self.count = gpu_op.get_tensor_runs_cuda_pointer(sizes)
-        self.pointers = gpu_op.get_n2_cuda_pointer([w.handle.contents.data for w, _ in self.arrays],
-                                                   [g.handle.contents.data for _, g in self.arrays], len(sizes))
-
-    def apply(self):
-        gpu_op.sgd_compute_o(self.pointers, self.tables, self.count, self.learning_rate)
+        columns = [[a.handle.contents.data for a in column] for column in zip(*self.arrays)]
+        self.n_tables = len(columns)
+        self.pointers = self._pointer_tables(columns, len(sizes))
 
     def close(self):
         """Gives the device tables back (waits for the last update that reads them)."""
         if self.tables is not None:
             gpu_op.free_index_cuda_pointer(self.tables)
-            gpu_op.free_n_cuda_pointer(self.pointers, 2)
+            gpu_op.free_n_cuda_pointer(self.pointers, self.n_tables)
             self.tables = self.pointers = None
             self.arrays = []
+
+
+class _FusedSgd(FusedUpdate):
+    @staticmethod
+    def _pointer_tables(columns, n):
+        return gpu_op.get_n2_cuda_pointer(*columns, n)
+
+    def apply(self):
+        gpu_op.sgd_compute_o(self.pointers, self.tables, self.count, self.learning_rate)
 
 
 def find_bn_relu_pairs(topo_order, outputs):

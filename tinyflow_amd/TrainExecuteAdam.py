@@ -11,12 +11,14 @@ step t (counted from 1) corrects with 1 - b1^t and 1 - b2^t.
 import numpy as np
 
 from . import autodiff as ad
-from . import ndarray
+from . import gpu_op, ndarray
 from . import TrainExecute as _sgd
 
 
 class TrainExecutor(_sgd.TrainExecutor):
     """Runs forward + backward + Adam update for one loss node."""
+
+    _update_op = ad.AdamOp
 
     def __init__(self, targetloss, learning_rate=0.001, ctx=ndarray.gpu(0), fuse_bn_relu=False):
         self.b1 = 0.9
@@ -33,6 +35,9 @@ class TrainExecutor(_sgd.TrainExecutor):
             self.Variable_node_list, self.Variable_node_grad_list, self.b1, self.b2, self.b1t, self.b2t, self.e,
             self.learning_rate)
         return nodes
+
+    def _fuse_updates(self, updates):
+        return _FusedAdam(updates)
 
     def init_Variable(self, feed_dict):
         """Initial values (numpy) of the trainable variables; the moments start at zero."""
@@ -54,6 +59,26 @@ class TrainExecutor(_sgd.TrainExecutor):
         """Device arrays (m, v) of a trainable variable."""
         m, v = self.Variable_node_to_mv[variable]
         return self.node_to_arr_map[m], self.node_to_arr_map[v]
+
+
+class _FusedAdam(_sgd.FusedUpdate):
+    """One launch that reads and writes each parameter and moment once (28 bytes per
+    parameter), where the two calls of an ``adam_op`` move 36 and every variable costs two
+    launches: VGG-16 at batch 6, 96 pixels 0.40 ms in 38 launches.  The same arithmetic per
+    element."""
+
+    def __init__(self, updates):
+        _sgd.FusedUpdate.__init__(self, updates)
+        self.node = updates[0][0]   # b1, b2, e and the shared powers are the executor's for every variable
+
+    @staticmethod
+    def _pointer_tables(columns, n):
+        return gpu_op.get_n4_cuda_pointer(*columns, n)
+
+    def apply(self):
+        node = self.node
+        gpu_op.adam_compute_o(self.pointers, self.tables, self.count, node.b1, node.b2, node.b1t[0], node.b2t[0],
+                              node.e, node.learning_rate)
 
 
 def getcomputelist(Variable_node_list, Variable_node_grad_list, b1, b2, b1t, b2t, e, learning_rate):
