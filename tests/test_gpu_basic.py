@@ -188,6 +188,23 @@ def test_matmul(rt, sa, ta, sb, tb):
     np.testing.assert_allclose(c.asnumpy(), ref, rtol=1e-5, atol=1e-4)
 
 
+# the 32-row tile (at most 32 rows, weights of 2^20 elements or more): one row, a full and a short tile, all four
+# transpose cases, columns and reductions that end inside a tile, splits summed in the kernel and by the separate pass;
+# one row too many and extents without 16-byte loads take the 64-row tile
+@pytest.mark.parametrize("sa,ta,sb,tb", [
+    ((1, 1024), False, (1024, 1024), False),
+    ((32, 4096), False, (4096, 260), False),
+    ((31, 1028), False, (1100, 1028), True),
+    ((1028, 12), True, (1028, 1036), False),
+    ((1028, 32), True, (1100, 1028), True),
+    ((7, 36), False, (36, 40000), False),
+    ((33, 1024), False, (1024, 1024), False),
+    ((5, 1025), False, (1025, 1027), False),
+], ids=str)
+def test_matmul_of_few_rows_with_large_weights(rt, sa, ta, sb, tb):
+    test_matmul(rt, sa, ta, sb, tb)
+
+
 def test_matmul_reference_integer_case(rt):
     """3x2 . 2x3 integer matrices and their gradients with a ones upstream
     (reference tests/autodiff_test.py:188-208)."""

@@ -380,9 +380,11 @@ template <int BM, int BN, int BK, class ALoader, class BLoader, class Epilogue>
 __global__ __launch_bounds__(THREADS) void gemm_kernel(const ALoader al, const BLoader bl, const Epilogue ep,
                                                       int k_extent, int k_per_split, int tiles_m, int tiles_n,
                                                       const Fold fold) {
-  constexpr int WM = BM / 2, WN = BN / 2;  // wave tile
+  // four waves, 2 x 2 over the tile, or side by side over a tile that is one MFMA high
+  constexpr int WAVES_M = BM == 32 ? 1 : 2;
+  constexpr int WM = BM / WAVES_M, WN = BN / (4 / WAVES_M);  // wave tile
   constexpr int TM = WM / 32, TN = WN / 32;
-  static_assert(TM >= 1 && TN >= 1, "tile too small for a 2x2 wave grid");
+  static_assert(TM >= 1 && TN >= 1, "tile too small for the wave grid");
   // LDS planes.  An operand whose loader fetches along the reduction (kKContig) is kept
   // as [m][k]: its vectors go to LDS untransposed, and a lane fetches the four
   // reduction elements of four consecutive MFMAs with one 16-byte read.  For that the
@@ -402,7 +404,7 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(const ALoader al, const B
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % WAVES_M, wn = wave / WAVES_M;
 
   // which tile, and which part of the reduction (all of this is scalar arithmetic)
   const int tiles = tiles_m * tiles_n;

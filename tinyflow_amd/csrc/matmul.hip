@@ -79,14 +79,19 @@ void launch(const AL &al, const BL &bl, const StoreRowMajor &ep, int K, const Ge
                      al, bl, ep, K, g.k_per_split, g.tiles_m, g.tiles_n, g.fold());
 }
 
+constexpr int64_t kFlatMinWeights = 1 << 20;  // elements: 4 MiB
+
+// 16-byte loads when both operands allow them (alignment, leading dimension and
+// the extent along each operand's contiguous direction multiples of 4)
+bool vec_operands(const float *A, bool tA, int lda, const float *B, bool tB, int ldb, int M, int N, int K) {
+  return vec4_ok(A, lda, tA ? M : K) && vec4_ok(B, ldb, tB ? K : N);
+}
+
 template <int BM, int BN, int BK>
 void dispatch(const float *A, bool tA, int lda, uint32_t a_bytes, const float *B, bool tB, int ldb,
               uint32_t b_bytes, const StoreRowMajor &ep, int M, int N, int K, const Geometry &g, hipStream_t s) {
-  // 16-byte loads when both operands allow them (alignment, leading dimension and
-  // the extent along each operand's contiguous direction multiples of 4)
-  const bool vec = vec4_ok(A, lda, tA ? M : K) && vec4_ok(B, ldb, tB ? K : N);
   const FastDiv whole(ONE_SEGMENT);
-  if (vec) {
+  if (BM == 32 || vec_operands(A, tA, lda, B, tB, ldb, M, N, K)) {  // the caller takes the 32-row tile only with both
     if (!tA && !tB) {
       Across4<BM, BK> al{A, a_bytes, lda, M, K, whole, 0};
       Along4<BN, BK> bl{B, b_bytes, ldb, N, K, whole, 0};
@@ -106,22 +111,24 @@ void dispatch(const float *A, bool tA, int lda, uint32_t a_bytes, const float *B
     }
     return;
   }
-  if (!tA && !tB) {
-    PlainAcross<BM, BK> al{A, a_bytes, lda, M, K};
-    PlainAlong<BN, BK> bl{B, b_bytes, ldb, N, K};
-    launch<BM, BN, BK>(al, bl, ep, K, g, s);
-  } else if (tA && !tB) {
-    PlainAlong<BM, BK> al{A, a_bytes, lda, M, K};
-    PlainAlong<BN, BK> bl{B, b_bytes, ldb, N, K};
-    launch<BM, BN, BK>(al, bl, ep, K, g, s);
-  } else if (!tA && tB) {
-    PlainAcross<BM, BK> al{A, a_bytes, lda, M, K};
-    PlainAcross<BN, BK> bl{B, b_bytes, ldb, N, K};
-    launch<BM, BN, BK>(al, bl, ep, K, g, s);
-  } else {
-    PlainAlong<BM, BK> al{A, a_bytes, lda, M, K};
-    PlainAcross<BN, BK> bl{B, b_bytes, ldb, N, K};
-    launch<BM, BN, BK>(al, bl, ep, K, g, s);
+  if constexpr (BM != 32) {
+    if (!tA && !tB) {
+      PlainAcross<BM, BK> al{A, a_bytes, lda, M, K};
+      PlainAlong<BN, BK> bl{B, b_bytes, ldb, N, K};
+      launch<BM, BN, BK>(al, bl, ep, K, g, s);
+    } else if (tA && !tB) {
+      PlainAlong<BM, BK> al{A, a_bytes, lda, M, K};
+      PlainAlong<BN, BK> bl{B, b_bytes, ldb, N, K};
+      launch<BM, BN, BK>(al, bl, ep, K, g, s);
+    } else if (!tA && tB) {
+      PlainAcross<BM, BK> al{A, a_bytes, lda, M, K};
+      PlainAcross<BN, BK> bl{B, b_bytes, ldb, N, K};
+      launch<BM, BN, BK>(al, bl, ep, K, g, s);
+    } else {
+      PlainAlong<BM, BK> al{A, a_bytes, lda, M, K};
+      PlainAcross<BN, BK> bl{B, b_bytes, ldb, N, K};
+      launch<BM, BN, BK>(al, bl, ep, K, g, s);
+    }
   }
 }
 
@@ -175,9 +182,18 @@ extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, co
 
   const int lda = (int)matA->shape[1], ldb = (int)matB->shape[1];
   const bool big = M > 64 && N > 64 && cdiv(M, 128) * cdiv(N, 128) >= num_cus();
-  const int bm = big ? 128 : 64, bn = big ? 128 : 64;
+  // At most 32 rows: a tile of one MFMA's height.  On the 64-row tile half of the matrix instructions work on
+  // padding, which for weights that come from memory costs as much as reading them, and a stage brings in half
+  // as many bytes of them: (32 x 25088)(25088 x 4096) 131 -> 70 us (5.9 TB/s) and the product with the transposed
+  // weights 149 -> 94; 6 x 4608 x 4096 27 -> 18 and 33 -> 22.  Reductions are split down to 128 there: 32 x 2048 x
+  // 1000 takes 11.5 on the 64-row tile, 12.0 split down to 256, 9.3 so; at 2^20 weights 11.6 against 8.7.  Smaller
+  // weights stay with the 64-row tile: their time is the launch's.
+  const bool flat = M <= 32 && N * K >= kFlatMinWeights &&
+                    vec_operands((const float *)matA->data, transposeA, lda, (const float *)matB->data, transposeB, ldb,
+                                 (int)M, (int)N, (int)K);
+  const int bm = big ? 128 : flat ? 32 : 64, bn = big || flat ? 128 : 64;
   const int tiles = cdiv(M, bm) * cdiv(N, bn);
-  const int splits = choose_splits(tiles, (int)K, 256);
+  const int splits = choose_splits(tiles, (int)K, flat ? 128 : 256);
   Geometry g = make_geometry((int)M, (int)N, (int)K, bm, bn, splits);
   plan_fold(g, (int)K, big ? 16 : 32, 1);
   FoldBuffers fb;
@@ -200,6 +216,9 @@ extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, co
   if (big)
     dispatch<128, 128, 16>((const float *)matA->data, transposeA, lda, (uint32_t)a_bytes, (const float *)matB->data,
                        transposeB, ldb, (uint32_t)b_bytes, ep, (int)M, (int)N, (int)K, g, s);
+  else if (flat)
+    dispatch<32, 128, 32>((const float *)matA->data, transposeA, lda, (uint32_t)a_bytes, (const float *)matB->data,
+                          transposeB, ldb, (uint32_t)b_bytes, ep, (int)M, (int)N, (int)K, g, s);
   else
     dispatch<64, 64, 32>((const float *)matA->data, transposeA, lda, (uint32_t)a_bytes, (const float *)matB->data,
                      transposeB, ldb, (uint32_t)b_bytes, ep, (int)M, (int)N, (int)K, g, s);
