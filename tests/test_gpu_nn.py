@@ -82,6 +82,23 @@ def test_pooling(rt, case, ties):
                                    rtol=1e-5)
 
 
+# planes at the edges of the workgroup sizes of the plane kernels (64, 256 and 1024 lanes, sixteen elements and four
+# windows each): full, one row more, no multiple of four elements, few lanes' worth
+@pytest.mark.parametrize("case", [
+    ((5, 3, 32, 32), "max", 0, 0, 2, 2, 2, 2),
+    ((5, 3, 34, 32), "max", 0, 0, 2, 2, 2, 2),
+    ((5, 3, 31, 33), "max", 1, 1, 2, 2, 3, 3),
+    ((2, 3, 64, 64), "max", 1, 1, 2, 2, 3, 3),
+    ((2, 3, 66, 64), "max", 0, 0, 2, 2, 2, 2),
+    ((2, 3, 63, 65), "max", 1, 1, 2, 2, 3, 3),
+    ((1000, 16, 10, 10), "max", 0, 0, 2, 2, 2, 2),
+    ((3, 5, 3, 3), "max", 1, 1, 2, 2, 3, 3),
+], ids=str)
+def test_pooling_at_the_edges_of_the_workgroup_sizes(rt, case):
+    for ties in (False, True):
+        test_pooling(rt, case, ties)
+
+
 def test_max_pool_routing_is_first_maximum(rt):
     """All-equal window: the gradient goes to the first position in row-major order."""
     from tinyflow_amd import gpu_op, ndarray
