@@ -20,57 +20,64 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// out[i] = sum_s partial[s * count + i], with the splits dealt round-robin to SG lane groups
-// of a workgroup so that a small output with many splits still has enough loads in flight
-// (a lane that adds them all waits for memory once per four splits: the 150 filter words of a
-// 1 -> 6 channel 5x5 layer with 500 splits took 95 us that way and take 5 us with 16 groups).
-// Group g adds splits g, g+SG, ... in that order, then group 0 adds the SG group sums in index
-// order: the order of additions depends on (splits, SG) only, never on timing.  T is four
-// consecutive floats where count and alignment allow it, else one.
-template <int SG, class T>
-__global__ __launch_bounds__(256) void split_sum_kernel(const T *__restrict__ partial, T *__restrict__ out,
-                                                       int64_t count, int splits) {
+// out[i] = sum_s partial[s * count + i] for 16-byte aligned data with count % 4 == 0, with the
+// splits dealt round-robin to SG lane groups of a workgroup so that a small output with
+// many splits still has enough loads in flight.  Group g adds splits g, g+SG,
+// ... in that order, then group 0 adds the SG group sums in index order: the
+// order of additions depends on (splits, SG) only, never on timing.
+template <int SG>
+__global__ __launch_bounds__(256) void split_sum_vec_kernel(const f32x4 *__restrict__ partial,
+                                                           f32x4 *__restrict__ out, int64_t count4, int splits) {
   constexpr int COLS = 256 / SG;
-  __shared__ T part[SG][COLS];
+  __shared__ f32x4 part[SG][COLS];
   const int col = threadIdx.x % COLS, g = threadIdx.x / COLS;
   const int64_t i = (int64_t)blockIdx.x * COLS + col;
-  T acc = {};
-  if (i < count) {
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  if (i < count4) {
     int k = g;
     for (; k + 3 * SG < splits; k += 4 * SG) {
-      const T v0 = __builtin_nontemporal_load(partial + (int64_t)k * count + i);
-      const T v1 = __builtin_nontemporal_load(partial + (int64_t)(k + SG) * count + i);
-      const T v2 = __builtin_nontemporal_load(partial + (int64_t)(k + 2 * SG) * count + i);
-      const T v3 = __builtin_nontemporal_load(partial + (int64_t)(k + 3 * SG) * count + i);
+      const f32x4 v0 = __builtin_nontemporal_load(partial + (int64_t)k * count4 + i);
+      const f32x4 v1 = __builtin_nontemporal_load(partial + (int64_t)(k + SG) * count4 + i);
+      const f32x4 v2 = __builtin_nontemporal_load(partial + (int64_t)(k + 2 * SG) * count4 + i);
+      const f32x4 v3 = __builtin_nontemporal_load(partial + (int64_t)(k + 3 * SG) * count4 + i);
       acc = (((acc + v0) + v1) + v2) + v3;
     }
-    for (; k < splits; k += SG) acc += __builtin_nontemporal_load(partial + (int64_t)k * count + i);
+    for (; k < splits; k += SG) acc += __builtin_nontemporal_load(partial + (int64_t)k * count4 + i);
   }
   if (SG == 1) {
-    if (i < count) out[i] = acc;
+    if (i < count4) out[i] = acc;
     return;
   }
   part[g][col] = acc;
   __syncthreads();
-  if (g == 0 && i < count) {
-    T total = part[0][col];
+  if (g == 0 && i < count4) {
+    f32x4 total = part[0][col];
 #pragma unroll
     for (int j = 1; j < SG; ++j) total += part[j][col];
     out[i] = total;
   }
 }
 
-template <class T>
-void launch_split_sum_of(const T *partial, T *out, int64_t count, int splits, hipStream_t s) {
-  // enough lane groups that about 64 K lanes are busy, as long as each group
-  // still has a few splits to add
-  int sg = 1;
-  while (sg < 16 && count * sg < 65536 && splits >= 8 * sg) sg *= 4;
-  const unsigned blocks = (unsigned)((count + 256 / sg - 1) / (256 / sg));
-  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, partial, out, count, splits); };
-  if (sg == 1) go(split_sum_kernel<1, T>);
-  else if (sg == 4) go(split_sum_kernel<4, T>);
-  else go(split_sum_kernel<16, T>);
+// Any other output: one lane per element, splits added in index order.  Bound by the loads' latency, so
+// thirty-two are in flight before the first addition, in workgroups of one wave that spread over the CUs: one load at
+// a time, the 150 filter words of a 1 -> 6 channel 5x5 layer with 500 splits took 95 us.
+__global__ __launch_bounds__(64) void split_sum_ordered_kernel(const float *__restrict__ partial,
+                                                              float *__restrict__ out, int64_t count, int splits) {
+  constexpr int DEPTH = 32;
+  const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  if (i >= count) return;
+  float s = partial[i];
+  int k = 1;
+  for (; k + DEPTH <= splits; k += DEPTH) {
+    float v[DEPTH];
+#pragma unroll
+    for (int e = 0; e < DEPTH; ++e) v[e] = __builtin_nontemporal_load(partial + (int64_t)(k + e) * count + i);
+#pragma unroll
+    for (int e = 0; e < DEPTH; ++e) s += v[e];
+  }
+#pragma unroll 4
+  for (; k < splits; ++k) s += __builtin_nontemporal_load(partial + (int64_t)k * count + i);
+  out[i] = s;
 }
 
 template <int BM, int BN, int BK, class AL, class BL>
@@ -138,10 +145,22 @@ namespace tf {
 
 int launch_split_sum(const float *partial, float *out, int64_t count, int splits, hipStream_t s) {
   const bool vec = count % 4 == 0 && ((reinterpret_cast<uintptr_t>(partial) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
-  if (vec)
-    launch_split_sum_of(reinterpret_cast<const f32x4 *>(partial), reinterpret_cast<f32x4 *>(out), count / 4, splits, s);
-  else
-    launch_split_sum_of(partial, out, count, splits, s);
+  if (vec) {
+    const int64_t count4 = count / 4;
+    const f32x4 *p4 = reinterpret_cast<const f32x4 *>(partial);
+    f32x4 *o4 = reinterpret_cast<f32x4 *>(out);
+    // enough lane groups that about 64 K lanes are busy, as long as each group
+    // still has a few splits to add
+    int sg = 1;
+    while (sg < 16 && count4 * sg < 65536 && splits >= 8 * sg) sg *= 4;
+    const unsigned blocks = (unsigned)((count4 + 256 / sg - 1) / (256 / sg));
+    if (sg == 1) hipLaunchKernelGGL(split_sum_vec_kernel<1>, dim3(blocks), dim3(256), 0, s, p4, o4, count4, splits);
+    else if (sg == 4) hipLaunchKernelGGL(split_sum_vec_kernel<4>, dim3(blocks), dim3(256), 0, s, p4, o4, count4, splits);
+    else hipLaunchKernelGGL(split_sum_vec_kernel<16>, dim3(blocks), dim3(256), 0, s, p4, o4, count4, splits);
+  } else {
+    const unsigned blocks = (unsigned)((count + 63) / 64);
+    hipLaunchKernelGGL(split_sum_ordered_kernel, dim3(blocks), dim3(64), 0, s, partial, out, count, splits);
+  }
   return 0;
 }
 
