@@ -208,6 +208,13 @@ int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA,
                         const DLArrayHandle matB, bool transposeB,
                         DLArrayHandle matC, void **handle, void **stream);
 
+/* No counterpart in the reference: introspection for tests, needs no GPU.  The tile (rows, columns) that
+ * an M x K by K x N product is launched on when both operands do or do not allow 16-byte loads (`vec`), the
+ * number of pieces that its reduction is cut into, and the first tile whose pieces are summed in the kernel
+ * (-1: in none). */
+int DLGpuMatrixMultiplyDescribe(int M, int N, int K, bool vec, int *tile_rows, int *tile_cols,
+                                int *pieces, int *first_folded_tile);
+
 /* ---------------------------------------------------------- reduce (bias) */
 
 /* Describe a sum-reduction from input_shapes to output_shapes (same rank;

@@ -4,6 +4,8 @@ Cases and tolerances follow the reference's own unit tests
 (tests/test_gpu_op.py:5-182): exact for set/broadcast/relu masks, rtol 1e-5 for
 sums, softmax and matmul at the reference's shapes.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -188,9 +190,9 @@ def test_matmul(rt, sa, ta, sb, tb):
     np.testing.assert_allclose(c.asnumpy(), ref, rtol=1e-5, atol=1e-4)
 
 
-# the 32-row tile (at most 32 rows, weights of 2^20 elements or more): one row, a full and a short tile, all four
-# transpose cases, columns and reductions that end inside a tile, splits summed in the kernel and by the separate pass;
-# one row too many and extents without 16-byte loads take the 64-row tile
+# products of few rows around the conditions of the 32-row tile: one row, a full and a short tile, all four transpose
+# cases, columns and reductions that end inside a tile; weights too small for it, one row too many and extents
+# without 16-byte loads take the 64-row tile
 @pytest.mark.parametrize("sa,ta,sb,tb", [
     ((1, 1024), False, (1024, 1024), False),
     ((32, 4096), False, (4096, 260), False),
@@ -200,9 +202,52 @@ def test_matmul(rt, sa, ta, sb, tb):
     ((7, 36), False, (36, 40000), False),
     ((33, 1024), False, (1024, 1024), False),
     ((5, 1025), False, (1025, 1027), False),
+    ((1, 4100), False, (4100, 1100), False),
+    ((33, 4100), False, (4100, 1100), False),
+    ((5, 4101), False, (4101, 1100), False),
 ], ids=str)
 def test_matmul_of_few_rows_with_large_weights(rt, sa, ta, sb, tb):
     test_matmul(rt, sa, ta, sb, tb)
+
+
+# the 32-row tile with the reduction whole, cut in pieces that a separate pass sums, cut in pieces that the kernel sums,
+# and cut only in the tiles past the last full round; (rows, K, N, transposes, pieces, first tile summed in the kernel)
+@pytest.mark.parametrize("m,k,n,ta,tb,pieces,first_folded", [
+    (32, 132, 33284, False, False, 1, -1),
+    (32, 4612, 1000, False, False, 17, -1),
+    (7, 4612, 1000, False, True, 17, -1),
+    (32, 1028, 8196, False, False, 4, 0),
+    (12, 1028, 8196, True, False, 4, 0),
+    (31, 700, 9000, False, True, 2, 0),
+    (4, 700, 9000, True, True, 2, 0),
+    (8, 256, 33284, False, False, 4, 256),
+    (32, 256, 33284, False, True, 4, 256),
+], ids=str)
+def test_matmul_rows_do_not_depend_on_the_row_tile(rt, m, k, n, ta, tb, pieces, first_folded):
+    """A product of at most 32 rows and large weights runs on a tile of its own; its rows are bit for bit those of the
+    36-row product with the same first rows, which runs on the 64 x 64 tile: the same pieces of the reduction, summed in
+    the same order."""
+    from tinyflow_amd import gpu_op
+    from tinyflow_amd._base import _LIB
+
+    def tile_of(rows):
+        plan = [ctypes.c_int() for _ in range(4)]
+        assert _LIB.DLGpuMatrixMultiplyDescribe(rows, n, k, True, *[ctypes.byref(v) for v in plan]) == 0
+        return tuple(v.value for v in plan)
+    assert tile_of(m) == (32, 128, pieces, first_folded)
+    assert tile_of(36) == (64, 64, pieces, max(-1, 2 * first_folded))
+    rng = np.random.RandomState(16)
+    a = rng.uniform(-1, 1, (36, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (n, k) if tb else (k, n)).astype(np.float32)
+    gb = _gpu(b, rt)
+    rows = []
+    for part in (a[:m], a):
+        c = _empty((len(part), n), rt)
+        gpu_op.matrix_multiply(_gpu(np.ascontiguousarray(part.T) if ta else part, rt), ta, gb, tb, c, rt.cublas, rt.stream)
+        rows.append(c.asnumpy())
+    assert rows[0].tobytes() == rows[1][:m].tobytes()
+    ref = O.matmul(a[:m].astype(np.float64), False, b.astype(np.float64), tb)
+    np.testing.assert_allclose(rows[0], ref, rtol=1e-5, atol=1e-4)
 
 
 def test_matmul_reference_integer_case(rt):

@@ -86,7 +86,7 @@ void launch(const AL &al, const BL &bl, const StoreRowMajor &ep, int K, const Ge
                      al, bl, ep, K, g.k_per_split, g.tiles_m, g.tiles_n, g.fold());
 }
 
-constexpr int64_t kFlatMinWeights = 1 << 20;  // elements: 4 MiB
+constexpr int64_t kFlatMinWeights = (1 << 22) + 1;  // elements: more than 16 MiB
 
 // 16-byte loads when both operands allow them (alignment, leading dimension and
 // the extent along each operand's contiguous direction multiples of 4)
@@ -177,6 +177,51 @@ int choose_splits(int tiles, int K, int min_k) {
 
 }  // namespace tf
 
+namespace {
+
+struct Plan {
+  int tile, splits;  // square tile that the reduction is planned for, k-splits asked for
+  Geometry g;        // of that tile
+  bool flat;         // launched on 32 x 128 tiles
+};
+
+// Two 64 x 64 tiles of at most 32 rows side by side are one 32 x 128 tile, with as many floats to fold.  Every
+// output element keeps the pieces of the reduction that it has on the 64 x 64 tiles and the order in which they
+// are summed, so the tile does not show in the bits of the result.
+void to_flat_tiles(Geometry &g, int N) {
+  g.tiles_n = cdiv(N, 128);
+  g.fold_first_tile /= 2;
+}
+
+Plan plan_product(int M, int N, int K, bool vec) {
+  Plan p;
+  p.tile = M > 64 && N > 64 && cdiv(M, 128) * cdiv(N, 128) >= num_cus() ? 128 : 64;
+  p.splits = choose_splits(cdiv(M, p.tile) * cdiv(N, p.tile), K, 256);
+  p.g = make_geometry(M, N, K, p.tile, p.tile, p.splits);
+  plan_fold(p.g, K, p.tile == 128 ? 16 : 32, 1);
+  // At most 32 rows: a tile of one MFMA's height.  On the 64-row tile half of the matrix instructions work on
+  // padding, which for weights that come from memory costs as much as reading them.  64-row against 32-row tile, us:
+  // 32 x 25088 x 4096 124 / 92 (4.5 TB/s), 32 x 4096 x 25088 with transposed weights 143 / 98, 6 x 4608 x 4096
+  // 27 / 20, 6 x 3200 x 2048 16.2 / 12.5; but 32 x 2048 x 2048, 2^22 weights, 11.7 / 12.0, and smaller ones likewise:
+  // their time is the launch's and the sum of the splits.
+  p.flat = M <= 32 && vec && (int64_t)N * K >= kFlatMinWeights && p.g.fold_first_tile % 2 == 0;
+  return p;
+}
+
+}  // namespace
+
+extern "C" int DLGpuMatrixMultiplyDescribe(int M, int N, int K, bool vec, int *tile_rows, int *tile_cols, int *pieces,
+                                           int *first_folded_tile) {
+  TF_REQUIRE(M > 0 && N > 0 && K > 0 && tile_rows && tile_cols && pieces && first_folded_tile, "bad arguments");
+  Plan p = plan_product(M, N, K, vec);
+  if (p.flat) to_flat_tiles(p.g, N);
+  *tile_rows = p.flat ? 32 : p.tile;
+  *tile_cols = p.flat ? 128 : p.tile;
+  *pieces = p.g.fold_pieces > 1 ? p.g.fold_pieces : p.g.splits;
+  *first_folded_tile = p.g.fold_pieces > 1 ? p.g.fold_first_tile : -1;
+  return 0;
+}
+
 extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, const DLArrayHandle matB,
                                    bool transposeB, DLArrayHandle matC, void **handle, void **stream) {
   announce_write(matC);
@@ -200,25 +245,14 @@ extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, co
   if (K == 0) return DLGpuArraySet(matC, 0.f, stream);
 
   const int lda = (int)matA->shape[1], ldb = (int)matB->shape[1];
-  const bool big = M > 64 && N > 64 && cdiv(M, 128) * cdiv(N, 128) >= num_cus();
-  // At most 32 rows: a tile of one MFMA's height.  On the 64-row tile half of the matrix instructions work on
-  // padding, which for weights that come from memory costs as much as reading them, and a stage brings in half
-  // as many bytes of them: (32 x 25088)(25088 x 4096) 131 -> 70 us (5.9 TB/s) and the product with the transposed
-  // weights 149 -> 94; 6 x 4608 x 4096 27 -> 18 and 33 -> 22.  Reductions are split down to 128 there: 32 x 2048 x
-  // 1000 takes 11.5 on the 64-row tile, 12.0 split down to 256, 9.3 so; at 2^20 weights 11.6 against 8.7.  Smaller
-  // weights stay with the 64-row tile: their time is the launch's.
-  const bool flat = M <= 32 && N * K >= kFlatMinWeights &&
-                    vec_operands((const float *)matA->data, transposeA, lda, (const float *)matB->data, transposeB, ldb,
-                                 (int)M, (int)N, (int)K);
-  const int bm = big ? 128 : flat ? 32 : 64, bn = big || flat ? 128 : 64;
-  const int tiles = cdiv(M, bm) * cdiv(N, bn);
-  const int splits = choose_splits(tiles, (int)K, flat ? 128 : 256);
-  Geometry g = make_geometry((int)M, (int)N, (int)K, bm, bn, splits);
-  plan_fold(g, (int)K, big ? 16 : 32, 1);
+  const Plan plan = plan_product((int)M, (int)N, (int)K,
+                                 vec_operands((const float *)matA->data, transposeA, lda, (const float *)matB->data,
+                                              transposeB, ldb, (int)M, (int)N, (int)K));
+  Geometry g = plan.g;
   FoldBuffers fb;
-  if (acquire_fold(g, bm, bn, 1, s, fb) != 0) {  // no scratch (this entry point cannot report it): no fold
+  if (acquire_fold(g, plan.tile, plan.tile, 1, s, fb) != 0) {  // no scratch (this entry point cannot report it): no fold
     release_fold(fb);
-    g = make_geometry((int)M, (int)N, (int)K, bm, bn, splits);
+    g = make_geometry((int)M, (int)N, (int)K, plan.tile, plan.tile, plan.splits);
   }
 
   float *dst = (float *)matC->data;
@@ -226,16 +260,17 @@ extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, co
   if (g.splits > 1) {
     partial = (float *)device_alloc((size_t)g.splits * M * N * sizeof(float));
     if (!partial) {  // no scratch: fall back to one pass over the whole reduction
-      g = make_geometry((int)M, (int)N, (int)K, bm, bn, 1);
+      g = make_geometry((int)M, (int)N, (int)K, plan.tile, plan.tile, 1);
     } else {
       dst = partial;
     }
   }
+  if (plan.flat) to_flat_tiles(g, (int)N);
   StoreRowMajor ep{dst, (int)N, (int)M, (int)N, M * N};
-  if (big)
+  if (plan.tile == 128)
     dispatch<128, 128, 16>((const float *)matA->data, transposeA, lda, (uint32_t)a_bytes, (const float *)matB->data,
                        transposeB, ldb, (uint32_t)b_bytes, ep, (int)M, (int)N, (int)K, g, s);
-  else if (flat)
+  else if (plan.flat)
     dispatch<32, 128, 32>((const float *)matA->data, transposeA, lda, (uint32_t)a_bytes, (const float *)matB->data,
                           transposeB, ldb, (uint32_t)b_bytes, ep, (int)M, (int)N, (int)K, g, s);
   else
