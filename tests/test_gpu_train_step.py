@@ -29,6 +29,8 @@ shallow network, which contains every structural element (stem, pool, projection
 blocks of stride 1 and 2, an identity block, average pool, classifier), is checked
 at the plain 1e-3 bound.
 """
+import gc
+
 import numpy as np
 import pytest
 
@@ -336,6 +338,55 @@ def test_fused_adam_update_is_bit_identical_to_per_variable_updates(batch):
     for a_step, b_step in zip(*runs):
         for a, b in zip(a_step, b_step):
             assert a.tobytes() == b.tobytes()
+
+
+def _three_lenet_steps(executor, steps=3, before_step=None):
+    """Every array of ``steps`` steps of LeNet-5 at batch 7: loss, parameters and, for Adam, moments."""
+    from tinyflow_amd import models
+    rng = np.random.RandomState(22)
+    model = models.lenet5(rng, batch=7, head="softmax_xent")
+    X, y = models.synthetic_batch(rng, model.input_shape, model.n_class, "normal")
+    ex = executor(model.loss)
+    ex.init_Variable(dict(model.variables))
+    values = []
+    for step in range(steps):
+        if before_step is not None:
+            before_step(ex, step)
+        out = list(ex.run({model.X: X, model.y_: y}))
+        if hasattr(ex, "moments_of"):
+            for v in ex.Variable_node_list:
+                out += ex.moments_of(v)
+        values.append([o.asnumpy().tobytes() for o in out])
+    return ex, values
+
+
+@pytest.mark.parametrize("optimizer", ["sgd", "adam"])
+@pytest.mark.parametrize("obstacle", ["too many parameters", "no room for the tables"])
+def test_updates_that_one_call_cannot_take_run_per_variable(monkeypatch, optimizer, obstacle):
+    """More parameters than the tables of the multi-tensor call can address (the limit is lowered here), or no
+    device memory for them: the step runs all the same and gives the same bits."""
+    from tinyflow_amd import TrainExecute, TrainExecuteAdam, gpu_op
+    module = TrainExecute if optimizer == "sgd" else TrainExecuteAdam
+    ex, want = _three_lenet_steps(lambda loss: module.TrainExecutor(loss, 0.01))
+    assert ex._fused_sgd is not None
+    ex.close()
+    del ex
+    gc.collect()
+    used = gpu_op.device_memory_stats()[1]
+    if obstacle == "too many parameters":
+        monkeypatch.setattr(TrainExecute.FusedUpdate, "max_parameters", 10000)
+    else:
+        def refuse(*args):
+            raise RuntimeError("no memory")
+        monkeypatch.setattr(gpu_op, "get_n2_cuda_pointer", refuse)
+        monkeypatch.setattr(gpu_op, "get_n4_cuda_pointer", refuse)
+    ex, got = _three_lenet_steps(lambda loss: module.TrainExecutor(loss, 0.01))
+    assert ex._fused_sgd is None
+    assert got == want
+    ex.close()
+    del ex
+    gc.collect()
+    assert gpu_op.device_memory_stats()[1] == used   # nothing of the refused tables is left
 
 
 @pytest.mark.parametrize("config", ["mlp", "lenet5"])

@@ -33,10 +33,12 @@ class TrainExecutor(object):
         multi-tensor entry point (``sgd_compute_o``, reference gpu_op.py:939-945) behind
         the last node of the step instead of one ``sgd_update`` per variable.  Every
         update still comes after the last reader of its parameter, which is all
-        ``swapsgd`` asks for, and the arithmetic per element is the same."""
+        ``swapsgd`` asks for, and the arithmetic per element is the same.  2**31
+        parameters or more, which the entry point's tables cannot address, and a device
+        without room for the tables get the calls per variable."""
         self.fuse_bn_relu = fuse_bn_relu
         self.fused_update = fused_update
-        self._fused_sgd = None
+        self._fused_sgd = None   # the step's one-call update, of whichever optimizer
         self.fused_pairs = 0
         self.targetloss = targetloss
         self.learning_rate = learning_rate
@@ -136,7 +138,12 @@ class TrainExecutor(object):
             self._fused_sgd.close()
             self._fused_sgd = None
         if fused_updates:
-            self._fused_sgd = self._fuse_updates(fused_updates)
+            try:
+                self._fused_sgd = self._fuse_updates(fused_updates) if FusedUpdate.fits(fused_updates) else None
+            except RuntimeError:   # no device memory for the tables: the calls per variable need none
+                self._fused_sgd = None
+            if self._fused_sgd is None:
+                plan += [(node.op.compute, node, input_vals, None) for node, input_vals in fused_updates]
         self.isfirstrun = 1
 
     def run(self, feed_dict, Accuracy_node=None, convert_to_numpy_ret_vals=False):
@@ -200,6 +207,8 @@ class FusedUpdate(object):
 
     ``updates``: pairs of an update node and its input arrays, parameter first."""
 
+    max_parameters = 2 ** 31 - 1   # the tables count in 32 bits
+
     def __init__(self, updates):
         rates = set(node.learning_rate for node, _ in updates)
         assert len(rates) == 1, "one learning rate per step"
@@ -208,13 +217,21 @@ class FusedUpdate(object):
         sizes = [int(np.prod(arrays[0].shape)) for arrays in self.arrays]
         for arrays, n in zip(self.arrays, sizes):
             assert all(int(np.prod(a.shape)) == n for a in arrays), "gradient and parameter sizes differ"
-        assert sum(sizes) < 2 ** 31
         # whole tensors end to end: the tables are built from the sizes, not from
         # per-parameter (tensor, offset) arrays
         self.tables, self.count = gpu_op.get_tensor_runs_cuda_pointer(sizes)
         columns = [[a.handle.contents.data for a in column] for column in zip(*self.arrays)]
         self.n_tables = len(columns)
-        self.pointers = self._pointer_tables(columns, len(sizes))
+        try:
+            self.pointers = self._pointer_tables(columns, len(sizes))
+        except RuntimeError:
+            gpu_op.free_index_cuda_pointer(self.tables)
+            raise
+
+    @classmethod
+    def fits(cls, updates):
+        """Whether the tables can address the parameters of these updates."""
+        return sum(int(np.prod(arrays[0].shape)) for _, arrays in updates) <= cls.max_parameters
 
     def close(self):
         """Gives the device tables back (waits for the last update that reads them)."""
