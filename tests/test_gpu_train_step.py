@@ -389,6 +389,31 @@ def test_updates_that_one_call_cannot_take_run_per_variable(monkeypatch, optimiz
     assert gpu_op.device_memory_stats()[1] == used   # nothing of the refused tables is left
 
 
+@pytest.mark.parametrize("first_step", [0, 2])
+def test_adam_rates_of_single_variables_count(first_step):
+    """The update nodes hold the learning rate, and a caller may give one of them another one, before the first step
+    or between two: the same bits as with one update call per variable."""
+    from tinyflow_amd.TrainExecuteAdam import TrainExecutor
+
+    def slow_down(ex, step):
+        if step == first_step:
+            ex.eval_node_list[1].learning_rate = 0.001
+    runs = []
+    for fused in (False, True):
+        def executor(loss):
+            ex = TrainExecutor(loss, 0.01)
+            ex.fused_update = fused
+            return ex
+        ex, values = _three_lenet_steps(executor, 4, slow_down)
+        assert (ex._fused_sgd is not None) == fused
+        ex.close()
+        runs.append(values)
+    assert runs[0] == runs[1]
+    ex, one_rate = _three_lenet_steps(lambda loss: TrainExecutor(loss, 0.01), 4)
+    ex.close()
+    assert runs[0] != one_rate
+
+
 @pytest.mark.parametrize("config", ["mlp", "lenet5"])
 def test_adam_executor_matches_oracle(config):
     """Three Adam steps (the reference's TrainExecuteAdam flow): loss, gradients, both

@@ -161,7 +161,7 @@ class TrainExecutor(object):
             if wanted:
                 raise MemoryError("%s: %d bytes of device scratch could not be allocated" % (node.name, wanted))
         if self._fused_sgd is not None:
-            self._fused_sgd.apply()
+            self._fused_sgd.apply(*handles)
         result = [self.node_to_arr_map[self.targetloss]]
         result += [self.node_to_arr_map[v] for v in reversed(self.Variable_node_list)]
         if Accuracy_node is not None:
@@ -210,9 +210,6 @@ class FusedUpdate(object):
     max_parameters = 2 ** 31 - 1   # the tables count in 32 bits
 
     def __init__(self, updates):
-        rates = set(node.learning_rate for node, _ in updates)
-        assert len(rates) == 1, "one learning rate per step"
-        self.learning_rate = rates.pop()
         self.arrays = [arrays for _, arrays in updates]   # keeps the storage alive
         sizes = [int(np.prod(arrays[0].shape)) for arrays in self.arrays]
         for arrays, n in zip(self.arrays, sizes):
@@ -243,11 +240,17 @@ class FusedUpdate(object):
 
 
 class _FusedSgd(FusedUpdate):
+    def __init__(self, updates):
+        rates = set(node.learning_rate for node, _ in updates)
+        assert len(rates) == 1, "one learning rate per step"
+        self.learning_rate = rates.pop()
+        FusedUpdate.__init__(self, updates)
+
     @staticmethod
     def _pointer_tables(columns, n):
         return gpu_op.get_n2_cuda_pointer(*columns, n)
 
-    def apply(self):
+    def apply(self, cudnnHandle, cublasHandle, cudaStream):
         gpu_op.sgd_compute_o(self.pointers, self.tables, self.count, self.learning_rate)
 
 

@@ -69,14 +69,20 @@ class _FusedAdam(_sgd.FusedUpdate):
 
     def __init__(self, updates):
         _sgd.FusedUpdate.__init__(self, updates)
-        self.node = updates[0][0]   # b1, b2, e and the shared powers are the executor's for every variable
+        self.nodes = [node for node, _ in updates]
 
     @staticmethod
     def _pointer_tables(columns, n):
         return gpu_op.get_n4_cuda_pointer(*columns, n)
 
-    def apply(self):
-        node = self.node
+    def apply(self, cudnnHandle, cublasHandle, cudaStream):
+        node = self.nodes[0]
+        # the executor gives every node the same numbers, but they are the nodes' and a caller may change them
+        # between steps
+        if len(set((n.b1, n.b2, n.b1t[0], n.b2t[0], n.e, n.learning_rate) for n in self.nodes)) != 1:
+            for n, arrays in zip(self.nodes, self.arrays):
+                n.op.compute(n, arrays, None, cudnnHandle, cublasHandle, cudaStream)
+            return
         gpu_op.adam_compute_o(self.pointers, self.tables, self.count, node.b1, node.b2, node.b1t[0], node.b2t[0],
                               node.e, node.learning_rate)
 
