@@ -323,8 +323,7 @@ def test_fused_adam_update_is_bit_identical_to_per_variable_updates(batch):
         rng = np.random.RandomState(22)
         model = models.lenet5(rng, batch=batch, head="softmax_xent")
         X, y = models.synthetic_batch(rng, model.input_shape, model.n_class, "normal")
-        ex = TrainExecutor(model.loss, 0.01)
-        ex.fused_update = fused
+        ex = TrainExecutor(model.loss, 0.01, fused_update=fused)
         ex.init_Variable(dict(model.variables))
         steps = []
         for _ in range(3):
@@ -400,11 +399,7 @@ def test_adam_rates_of_single_variables_count(first_step):
             ex.eval_node_list[1].learning_rate = 0.001
     runs = []
     for fused in (False, True):
-        def executor(loss):
-            ex = TrainExecutor(loss, 0.01)
-            ex.fused_update = fused
-            return ex
-        ex, values = _three_lenet_steps(executor, 4, slow_down)
+        ex, values = _three_lenet_steps(lambda loss: TrainExecutor(loss, 0.01, fused_update=fused), 4, slow_down)
         assert (ex._fused_sgd is not None) == fused
         ex.close()
         runs.append(values)

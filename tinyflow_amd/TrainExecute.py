@@ -30,8 +30,8 @@ class TrainExecutor(object):
         (``value_of`` does not know them).
 
         ``fused_update``: apply all updates of a step with one call of the
-        multi-tensor entry point (``sgd_compute_o``, reference gpu_op.py:939-945) behind
-        the last node of the step instead of one ``sgd_update`` per variable.  Every
+        multi-tensor entry point (``sgd_compute_o``, reference gpu_op.py:939-945, or its
+        Adam counterpart) behind the last node of the step instead of calls per variable.  Every
         update still comes after the last reader of its parameter, which is all
         ``swapsgd`` asks for, and the arithmetic per element is the same.  2**31
         parameters or more, which the entry point's tables cannot address, and a device

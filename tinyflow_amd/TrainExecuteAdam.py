@@ -20,7 +20,8 @@ class TrainExecutor(_sgd.TrainExecutor):
 
     _update_op = ad.AdamOp
 
-    def __init__(self, targetloss, learning_rate=0.001, ctx=ndarray.gpu(0), fuse_bn_relu=False):
+    def __init__(self, targetloss, learning_rate=0.001, ctx=ndarray.gpu(0), fuse_bn_relu=False,
+                 fused_update=True):
         self.b1 = 0.9
         self.b2 = 0.999
         self.e = 0.00000001
@@ -28,7 +29,7 @@ class TrainExecutor(_sgd.TrainExecutor):
         self.b2t = [0.999]
         self.mv = []
         self.Variable_node_to_mv = {}
-        _sgd.TrainExecutor.__init__(self, targetloss, learning_rate, ctx, fuse_bn_relu)
+        _sgd.TrainExecutor.__init__(self, targetloss, learning_rate, ctx, fuse_bn_relu, fused_update)
 
     def _update_nodes(self):
         nodes, self.mv, self.Variable_node_to_mv = getcomputelist(
