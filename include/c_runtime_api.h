@@ -417,6 +417,13 @@ int DLGpuAdam_o(void ****n4list, const void ***indexlist, const int count,
                 const float b1, const float b2, const float b1t, const float b2t,
                 const float e, const float learning_rate);
 
+/* No counterpart in the reference, whose fused update runs on the default stream: DLGpuAdam_o on `stream`.
+ * `written` are the arrays behind the first three pointer tables (parameters and moments), so that what
+ * the library derived from other arrays stays valid. */
+int DLGpuAdam_o_onStream(void ****n4list, const void ***indexlist, int count, float b1, float b2, float b1t,
+                         float b2t, float e, float learning_rate, const DLArrayHandle *written,
+                         int n_written, void **stream);
+
 /* No counterpart in the reference, which allocates the tables above with cudaMalloc
  * and never gives them back (gpu_op.cu:4628-4700): release calls for the index tables
  * and for the 2 or 4 pointer tables (device blocks and host cell; the cell is set to

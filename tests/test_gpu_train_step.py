@@ -29,6 +29,7 @@ shallow network, which contains every structural element (stem, pool, projection
 blocks of stride 1 and 2, an identity block, average pool, classifier), is checked
 at the plain 1e-3 bound.
 """
+import ctypes
 import gc
 
 import numpy as np
@@ -407,6 +408,70 @@ def test_adam_rates_of_single_variables_count(first_step):
     ex, one_rate = _three_lenet_steps(lambda loss: TrainExecutor(loss, 0.01), 4)
     ex.close()
     assert runs[0] != one_rate
+
+
+def test_adam_update_leaves_what_is_kept_for_other_arrays(rt, monkeypatch):
+    """The transformed input that a convolution keeps from its forward call for its grad-filter call outlives an Adam
+    step of another program, which writes neither the input nor the filter; a step that writes the input drops it."""
+    from tinyflow_amd import _base, gpu_op, ndarray
+    from tinyflow_amd.TrainExecuteAdam import TrainExecutor, _FusedAdam
+    monkeypatch.setenv("TINYFLOW_WINOGRAD", "4")
+
+    def taken():
+        count = ctypes.c_longlong()
+        assert _base._LIB.DLGpuKeptByproductCounts(None, ctypes.byref(count), None) == 0
+        return count.value
+    rng = np.random.RandomState(4)
+    x_shape, w_shape = (4, 64, 28, 28), (64, 64, 3, 3)
+    y_shape, desc = gpu_op.convolution_2d_forward_get_out_shape(x_shape, w_shape, "NCHW", "SAME", 1, 1)
+    x, w, dy = (ndarray.array(rng.normal(0, 1, s).astype(np.float32), rt.ctx) for s in (x_shape, w_shape, y_shape))
+    y, dw, m, v = (ndarray.array(np.zeros(s, np.float32), rt.ctx) for s in (y_shape, w_shape, x_shape, x_shape))
+    grad = ndarray.array(np.ones(x_shape, np.float32), rt.ctx)
+
+    def forward():
+        assert gpu_op.convolution_2d_forward(x, w, y, desc, rt.cudnn, rt.stream) == 0
+
+    def grad_filter():
+        before = taken()
+        assert gpu_op.convolution_backward_filter(x, dy, w, dw, desc, rt.cudnn, rt.stream) == 0
+        return taken() - before
+    grad_filter()   # a forward call keeps its transform once a grad-filter call has asked for one
+    forward()
+    assert grad_filter() == 1
+    forward()
+    ex, _ = _three_lenet_steps(lambda loss: TrainExecutor(loss, 0.01), 1)
+    assert grad_filter() == 1
+    node = ex._fused_sgd.nodes[0]
+    update = _FusedAdam([(node, [x, m, v, grad])])
+    forward()
+    update.apply(rt.cudnn, rt.cublas, rt.stream)
+    assert grad_filter() == 0
+    update.close()
+    ex.close()
+
+
+def test_adam_update_does_not_wait_for_other_streams(rt):
+    """A step's update runs on its own stream: it is done while an older, longer piece of work on another stream is
+    still running."""
+    import torch
+    from tinyflow_amd import gpu_op, ndarray
+    from tinyflow_amd.TrainExecuteAdam import TrainExecutor
+    ex, _ = _three_lenet_steps(lambda loss: TrainExecutor(loss, 0.01), 2)
+    n = 4096
+    a, b, c = (ndarray.array(np.ones((n, n), np.float32), rt.ctx) for _ in range(3))
+    gpu_op.matrix_multiply(a, False, b, False, c, rt.cublas, rt.stream)
+    torch.cuda.synchronize()
+    other, own = (torch.cuda.ExternalStream(ctypes.cast(cell.contents, ctypes.c_void_p).value)
+                  for cell in (rt.stream, ex.cudaStream))
+    for _ in range(60):   # about 60 ms
+        gpu_op.matrix_multiply(a, False, b, False, c, rt.cublas, rt.stream)
+    other_done, own_done = torch.cuda.Event(), torch.cuda.Event()
+    other_done.record(other)
+    ex._fused_sgd.apply(ex.cudnnHandle, ex.cublasHandle, ex.cudaStream)
+    own_done.record(own)
+    own_done.synchronize()
+    assert not other_done.query()
+    ex.close()
 
 
 @pytest.mark.parametrize("config", ["mlp", "lenet5"])

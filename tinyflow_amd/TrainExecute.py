@@ -202,8 +202,7 @@ class FusedUpdate(object):
     """All parameter updates of a step as one launch: the pointer tables and the index ->
     (tensor, offset) tables of ``sgd_compute_o`` / ``adam_compute_o`` (reference
     gpu_op.py:887-945), built once for the step's arrays, which keep their storage from
-    step to step.  The call has no stream argument: it runs on the default stream,
-    which is ordered behind the executor's stream and in front of its next launch.
+    step to step.
 
     ``updates``: pairs of an update node and its input arrays, parameter first."""
 
@@ -240,6 +239,9 @@ class FusedUpdate(object):
 
 
 class _FusedSgd(FusedUpdate):
+    """The call has no stream argument: it runs on the default stream, which is ordered behind
+    the executor's stream and in front of its next launch."""
+
     def __init__(self, updates):
         rates = set(node.learning_rate for node, _ in updates)
         assert len(rates) == 1, "one learning rate per step"

@@ -11,7 +11,7 @@ step t (counted from 1) corrects with 1 - b1^t and 1 - b2^t.
 import numpy as np
 
 from . import autodiff as ad
-from . import gpu_op, ndarray
+from . import _base, gpu_op, ndarray
 from . import TrainExecute as _sgd
 
 
@@ -71,6 +71,7 @@ class _FusedAdam(_sgd.FusedUpdate):
     def __init__(self, updates):
         _sgd.FusedUpdate.__init__(self, updates)
         self.nodes = [node for node, _ in updates]
+        self.written = _base.c_array(ndarray.DLArrayHandle, [a.handle for arrays in self.arrays for a in arrays[:3]])
 
     @staticmethod
     def _pointer_tables(columns, n):
@@ -84,8 +85,8 @@ class _FusedAdam(_sgd.FusedUpdate):
             for n, arrays in zip(self.nodes, self.arrays):
                 n.op.compute(n, arrays, None, cudnnHandle, cublasHandle, cudaStream)
             return
-        gpu_op.adam_compute_o(self.pointers, self.tables, self.count, node.b1, node.b2, node.b1t[0], node.b2t[0],
-                              node.e, node.learning_rate)
+        gpu_op.adam_compute_o_on_stream(self.pointers, self.tables, self.count, node.b1, node.b2, node.b1t[0],
+                                        node.b2t[0], node.e, node.learning_rate, self.written, cudaStream)
 
 
 def getcomputelist(Variable_node_list, Variable_node_grad_list, b1, b2, b1t, b2t, e, learning_rate):

@@ -499,13 +499,20 @@ extern "C" int DLGpuGetTensorRunsCudaPointer(const int64_t *sizes, int n_tensors
   return index_cell(result, d_number, d_prefix);
 }
 
+// The last fused update may still read its tables: waits for the one stream that runs kernels or, where there are
+// several or none known here, for the device.
+static hipError_t wait_for_updates() {
+  const hipStream_t s = streamless_launch_stream();
+  return s ? hipStreamSynchronize(s) : hipDeviceSynchronize();
+}
+
 // No counterpart in the reference (which never releases these tables): gives back the
 // device blocks and the host cell of DLGpuGetIndextoVaribaleNumberCudaPointer /
 // DLGpuGetTensorRunsCudaPointer.  The caller must not use `indexlist` afterwards.
 extern "C" int DLGpuFreeIndexCudaPointer(void ***indexlist) {
   TF_REQUIRE(indexlist, "bad arguments");
   if (!*indexlist) return 0;
-  TF_HIP(hipStreamSynchronize(streamless_launch_stream()));  // the last fused update may still read them
+  TF_HIP(wait_for_updates());
   RunPiece *pieces = nullptr;
   {
     std::lock_guard<std::mutex> g(run_mu);
@@ -563,7 +570,7 @@ extern "C" int DLGpuGetN4CudaPointer(void **output, void **m, void **v, void **g
 extern "C" int DLGpuFreeNCudaPointer(void ****list, int n_tables) {
   TF_REQUIRE(list && (n_tables == 2 || n_tables == 4), "bad arguments");
   if (!*list) return 0;
-  TF_HIP(hipStreamSynchronize(streamless_launch_stream()));  // the last fused update may still read them
+  TF_HIP(wait_for_updates());
   for (int i = 0; i < n_tables; ++i)
     if ((*list)[i]) device_free((*list)[i]);
   free(*list);
@@ -571,29 +578,44 @@ extern "C" int DLGpuFreeNCudaPointer(void ****list, int n_tables) {
   return 0;
 }
 
+namespace {
+int launch_multi_adam(void ****n4list, const void ***indexlist, int count, const MultiAdam &adam, hipStream_t s,
+                      const char *what) {
+  TF_REQUIRE(n4list && *n4list && indexlist && *indexlist && count >= 0, "bad arguments");
+  if (count == 0) return 0;
+  RunTable runs;
+  const int found = find_run_table((*indexlist)[0], count, runs);
+  TF_REQUIRE(found >= 0, "count %d is not the count the index tables were built for", count);
+  if (found)
+    hipLaunchKernelGGL((multi_tensor_kernel<4, MultiAdam>), dim3(runs.n_pieces), dim3(kThreads), 0, s, adam,
+                       (float *const *)((*n4list)[0]), (float *const *)((*n4list)[1]),
+                       (float *const *)((*n4list)[2]), (float *const *)((*n4list)[3]),
+                       (const RunPiece *)runs.pieces);
+  else
+    hipLaunchKernelGGL(adam_multi_kernel, dim3(grid_for(count)), dim3(kThreads), 0, s, (float **)((*n4list)[0]),
+                       (float **)((*n4list)[1]), (float **)((*n4list)[2]), (float **)((*n4list)[3]),
+                       (const int *)((*indexlist)[0]), (const int *)((*indexlist)[1]), adam.b1, adam.b2, adam.b1t,
+                       adam.b2t, adam.e, adam.lr, count);
+  return finish(s, what);
+}
+}  // namespace
+
 extern "C" int DLGpuAdam_o(void ****n4list, const void ***indexlist, const int count, const float b1,
                            const float b2, const float b1t, const float b2t, const float e,
                            const float learning_rate) {
   note_write_everything();  // the pointer tables name the written tensors, not their sizes
-  TF_REQUIRE(n4list && *n4list && indexlist && *indexlist && count >= 0, "bad arguments");
-  if (count == 0) return 0;
   // no stream argument: ordered against all streams that run kernels
-  hipStream_t s = streamless_launch_stream();
-  RunTable runs;
-  const int found = find_run_table((*indexlist)[0], count, runs);
-  TF_REQUIRE(found >= 0, "count %d is not the count the index tables were built for", count);
-  if (found) {
-    hipLaunchKernelGGL((multi_tensor_kernel<4, MultiAdam>), dim3(runs.n_pieces), dim3(kThreads), 0, s,
-                       MultiAdam{b1, b2, b1t, b2t, e, learning_rate}, (float *const *)((*n4list)[0]),
-                       (float *const *)((*n4list)[1]), (float *const *)((*n4list)[2]),
-                       (float *const *)((*n4list)[3]), (const RunPiece *)runs.pieces);
-    return finish(s, "DLGpuAdam_o");
-  }
-  hipLaunchKernelGGL(adam_multi_kernel, dim3(grid_for(count)), dim3(kThreads), 0, s,
-                     (float **)((*n4list)[0]), (float **)((*n4list)[1]), (float **)((*n4list)[2]),
-                     (float **)((*n4list)[3]), (const int *)((*indexlist)[0]), (const int *)((*indexlist)[1]), b1,
-                     b2, b1t, b2t, e, learning_rate, count);
-  return finish(s, "DLGpuAdam_o");
+  return launch_multi_adam(n4list, indexlist, count, MultiAdam{b1, b2, b1t, b2t, e, learning_rate},
+                           streamless_launch_stream(), "DLGpuAdam_o");
+}
+
+extern "C" int DLGpuAdam_o_onStream(void ****n4list, const void ***indexlist, int count, float b1, float b2, float b1t,
+                                    float b2t, float e, float learning_rate, const DLArrayHandle *written,
+                                    int n_written, void **stream) {
+  TF_REQUIRE(n_written >= 0 && (written || n_written == 0), "bad arguments");
+  for (int i = 0; i < n_written; ++i) announce_write(written[i]);
+  return launch_multi_adam(n4list, indexlist, count, MultiAdam{b1, b2, b1t, b2t, e, learning_rate}, stream_of(stream),
+                           "DLGpuAdam_o_onStream");
 }
 
 extern "C" int DLGpuSgd_o(void ****n2list, const void ***indexlist, const int count,

@@ -457,6 +457,15 @@ def adam_compute_o(n4list, indexinfolist, count, b1, b2, b1t, b2t, e, learning_r
                                 ctypes.c_float(e), ctypes.c_float(learning_rate)))
 
 
+def adam_compute_o_on_stream(n4list, indexinfolist, count, b1, b2, b1t, b2t, e, learning_rate, written, cudaStream):
+    """``adam_compute_o`` on ``cudaStream`` instead of the default stream (no counterpart in the
+    reference); ``written``: a ``c_array`` of the handles of the parameters and moments."""
+    check_call(_LIB.DLGpuAdam_o_onStream(n4list, indexinfolist, ctypes.c_int(count), ctypes.c_float(b1),
+                                         ctypes.c_float(b2), ctypes.c_float(b1t), ctypes.c_float(b2t),
+                                         ctypes.c_float(e), ctypes.c_float(learning_rate), written,
+                                         ctypes.c_int(len(written)), cudaStream))
+
+
 def getInt(intp):
     return _LIB.getInt(intp)
 
