@@ -267,6 +267,37 @@ def test_batch_norm_with_rows_walked_in_tiles(rt, shape):
         test_fused_batch_norm_relu_equals_the_two_ops(rt, shape)
 
 
+# more columns than the register kernels address, with rows on either side of the tiled forward form, and columns enough
+# for the backward form of one lane per column; the last columns do not fill a workgroup
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,columns", [(2, 2 ** 25 + 3), (12, 2 ** 25 + 3), (130, 393216 + 7)])
+def test_batch_norm_of_very_many_columns(rt, rows, columns):
+    """Columns are independent: the first, the last and some in between against the oracle."""
+    from tinyflow_amd import gpu_op, ndarray
+    rng = np.random.RandomState(37)
+    shape, mode = (rows, columns, 1, 1), "pre_activation"
+    # a prime number of values, repeated: no two of the columns compared are alike
+    x = np.resize(rng.normal(1, 2, 1000003).astype(np.float32), shape)
+    dy = np.resize(rng.normal(0, 1, 999983).astype(np.float32), shape)
+    picked = np.r_[0:300, 300:columns - 300:99991, columns - 300:columns]
+    mean_p, var_p, lst = gpu_op.bn_get_cudnnlist(shape, "NCHW", mode)
+    gx, gdy = _gpu(x, rt), _gpu(dy, rt)
+    gy, gdx = ndarray.empty(shape, rt.ctx), ndarray.empty(shape, rt.ctx)
+    assert gpu_op.bn_forward(gx, gy, mode, 0, mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+    assert gpu_op.bn_backward(gx, gdy, gdx, mode, mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+    x, dy = x[:, picked], dy[:, picked]
+    y, dx = gy.asnumpy()[:, picked], gdx.asnumpy()[:, picked]
+    x64, dy64 = x.astype(np.float64), dy.astype(np.float64)
+    y_ref, mean, istd = O.batch_norm_forward(x64, mode)
+    dx_ref = O.batch_norm_backward(x64, dy64, mode, mean, istd)
+    y32, mean32, istd32 = O.batch_norm_forward(x, mode)
+    dx32 = O.batch_norm_backward(x, dy, mode, mean32, istd32)
+    parity.compare(y, y_ref, y32, "batch norm forward, wide", "bn fwd %s" % (shape,), K_BN)
+    parity.compare(dx, dx_ref, dx32, "batch norm backward, wide", "bn bwd %s" % (shape,), K_BN)
+    if rows > 128:
+        test_fused_batch_norm_relu_equals_the_two_ops(rt, shape)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["pre_activation", "spatial"])
 def test_batch_norm_with_mean_far_from_zero(rt, mode):

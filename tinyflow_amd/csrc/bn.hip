@@ -78,13 +78,46 @@ __global__ __launch_bounds__(kThreads) void bn_pa_forward_kernel(const float *__
   }
 }
 
+// One lane per column, three sweeps over it, for few rows of more columns than the register kernels address: lanes
+// enough and no chain worth mentioning, so nothing but the bytes counts, where a tile of 64 rows would be mostly
+// padding.  67 M columns of 2 rows 578 us against 1926 in tiles, 34 M of 8 rows 950 against 1177; 16 rows 1947
+// against 1643, and the tiles are faster from there on.
+constexpr int kFewRows = 12;
+
+template <bool RELU>
+__global__ __launch_bounds__(kThreads) void bn_pa_forward_stream_kernel(const float *__restrict__ x,
+                                                                       float *__restrict__ y,
+                                                                       float *__restrict__ save_mean,
+                                                                       float *__restrict__ save_istd, int N,
+                                                                       int64_t L) {
+  const int64_t l = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (l >= L) return;
+  float s = 0.f;
+  for (int n = 0; n < N; ++n) s += x[(int64_t)n * L + l];
+  const float mean = s / (float)N;
+  float q = 0.f;
+  for (int n = 0; n < N; ++n) {
+    const float dlt = x[(int64_t)n * L + l] - mean;
+    q += dlt * dlt;
+  }
+  const float istd = 1.0f / sqrtf(q / (float)N + kEps);
+  save_mean[l] = mean;
+  save_istd[l] = istd;
+  for (int n = 0; n < N; ++n) {
+    const float out = (x[(int64_t)n * L + l] - mean) * istd;
+    y[(int64_t)n * L + l] = (RELU && out < 0.f) ? 0.f : out;
+  }
+}
+
 // More rows than registers: a workgroup owns COLS columns and walks them three times (the second
 // and third walk hit the cache) in tiles of 4096 elements.  All lanes fetch a tile and put it into
 // LDS, then lane c adds column c from there in row order while the fetch of the next tile is in
 // flight.  What bounds a narrow tensor is the chain of additions in a column, and the order stays
 // that chain's; taken straight from memory, each link waited for a load: the ten logits of a
-// batch of 1000 took 290 us forward and 250 us backward, now 29 and 27.  COLS is 64 (a 256-byte line per row)
-// where that gives every CU a workgroup, else 16.  Rows past N enter the sums as +0, which changes none.
+// batch of 1000 took 290 us forward and 250 us backward, now 29 and 27.  Rows past N enter the sums as +0, which
+// changes none.
+// COLS is 64 (a 256-byte line per row)
+// where that gives every CU a workgroup, else 16.
 constexpr int kTile = 4096, kTileRegs = kTile / kThreads;
 constexpr int kWideCols = 64, kNarrowCols = 16;
 
@@ -185,6 +218,38 @@ __global__ __launch_bounds__(kThreads) void bn_pa_backward_kernel(const float *_
                                           (int)(n * row), 0);
 }
 
+// One lane per column, as in forward; it walks the column twice.  From six workgroups per CU on the lanes hide the
+// loads' latency, and the tiles' detour over LDS and its barriers cost more than they give.  This against tiles, us:
+// 130 rows of 262144 columns 171 / 144, of 393216 182 / 212, of 524288 237 / 289; 300 rows 383 / 321, 466 / 474 and
+// 562 / 682.
+template <bool RELU>
+__global__ __launch_bounds__(kThreads) void bn_pa_backward_stream_kernel(const float *__restrict__ x,
+                                                                        const float *__restrict__ dy,
+                                                                        float *__restrict__ dx,
+                                                                        const float *__restrict__ save_mean,
+                                                                        const float *__restrict__ save_istd,
+                                                                        int N, int64_t L) {
+  const int64_t l = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (l >= L) return;
+  const float mean = save_mean[l], istd = save_istd[l];
+  float s1 = 0.f, s2 = 0.f;
+  for (int n = 0; n < N; ++n) {
+    const float xh = (x[(int64_t)n * L + l] - mean) * istd;
+    float g = dy[(int64_t)n * L + l];
+    if (RELU) g = xh > 0.f ? g : 0.f;
+    s1 += g;
+    s2 += g * xh;
+  }
+  const float m = (float)N;
+  const float scale = istd / m;
+  for (int n = 0; n < N; ++n) {
+    const float xh = (x[(int64_t)n * L + l] - mean) * istd;
+    float g = dy[(int64_t)n * L + l];
+    if (RELU) g = xh > 0.f ? g : 0.f;
+    dx[(int64_t)n * L + l] = scale * (m * g - s1 - xh * s2);
+  }
+}
+
 struct GradPair {
   float g, xh;
 };
@@ -228,6 +293,9 @@ __global__ __launch_bounds__(kThreads) void bn_pa_backward_tiles_kernel(const fl
     dx[(int64_t)n * L + l] = scale * (m * p.g - s1 - p.xh * s2);
   }
 }
+
+// Whether one lane per column gives every CU six workgroups.
+bool many_columns(int64_t L) { return L >= (int64_t)num_cus() * kThreads * 6; }
 
 // Whether COLS = kWideCols gives every CU a workgroup.
 bool wide_column_blocks(int64_t L) { return L >= (int64_t)num_cus() * kWideCols; }
@@ -545,6 +613,8 @@ static int bn_forward_impl(const DLArrayHandle input, DLArrayHandle output, int 
         pa_forward<64, RELU>(grid, block, s, x, y, mean, istd, d->N, l32);
       else if (d->N <= 128 && pa_rows_addressable(128, L))
         pa_forward<128, RELU>(grid, block, s, x, y, mean, istd, d->N, l32);
+      else if (d->N < kFewRows)
+        hipLaunchKernelGGL(bn_pa_forward_stream_kernel<RELU>, grid, block, 0, s, x, y, mean, istd, d->N, L);
       else
         bn_pa_forward_tiles<RELU>(s, x, y, mean, istd, d->N, L);
     };
@@ -635,6 +705,8 @@ static int bn_backward_impl(const DLArrayHandle input, const DLArrayHandle doutp
           hipLaunchKernelGGL((bn_pa_backward_kernel<64, RELU>), grid, block, 0, s, x, dy, dx, mean, istd, d->N, l32);
         else if (d->N <= 128 && pa_rows_addressable(128, L))
           hipLaunchKernelGGL((bn_pa_backward_kernel<128, RELU>), grid, block, 0, s, x, dy, dx, mean, istd, d->N, l32);
+        else if (many_columns(L))
+          hipLaunchKernelGGL(bn_pa_backward_stream_kernel<RELU>, grid, block, 0, s, x, dy, dx, mean, istd, d->N, L);
         else
           bn_pa_backward_tiles<RELU>(s, x, dy, dx, mean, istd, d->N, L);
       };
