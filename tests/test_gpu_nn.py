@@ -258,9 +258,9 @@ def test_batch_norm(rt, shape, mode):
 
 
 # more rows than the register kernels hold: fewest rows, one and two narrow column blocks, one to four tiles of
-# 256 rows, whole and ragged; the wide column blocks (16 384 columns and more on 256 units), whole and ragged
+# 256 rows, whole and ragged; the wide column blocks (32 768 columns and more on 256 units), whole and ragged
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape", [(129, 1, 1), (1000, 1, 10), (256, 1, 16), (257, 1, 17), (129, 1, 16384), (130, 4, 64, 65)], ids=str)
+@pytest.mark.parametrize("shape", [(129, 1, 1), (1000, 1, 10), (256, 1, 16), (257, 1, 17), (129, 1, 16384), (130, 4, 64, 65), (129, 1, 32768), (130, 8, 64, 65)], ids=str)
 def test_batch_norm_with_rows_walked_in_tiles(rt, shape):
     test_batch_norm(rt, shape, "pre_activation")
     if len(shape) == 4:

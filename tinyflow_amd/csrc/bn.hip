@@ -116,8 +116,9 @@ __global__ __launch_bounds__(kThreads) void bn_pa_forward_stream_kernel(const fl
 // that chain's; taken straight from memory, each link waited for a load: the ten logits of a
 // batch of 1000 took 290 us forward and 250 us backward, now 29 and 27.  Rows past N enter the sums as +0, which
 // changes none.
-// COLS is 64 (a 256-byte line per row)
-// where that gives every CU a workgroup, else 16.
+// COLS is 64 (a 256-byte line per row) where that gives every CU two workgroups, else 16.  16 against 64 columns, us,
+// forward and backward: 130 rows of 4096 columns 8 / 13 and 7 / 11, of 16384 9.9 / 13.7 and 12.5 / 11.2, of 33000
+// 27 / 23 and 35 / 25; 1000 rows of 16384 77 / 115 and 92 / 107, of 33000 182 / 156 and 236 / 223.
 constexpr int kTile = 4096, kTileRegs = kTile / kThreads;
 constexpr int kWideCols = 64, kNarrowCols = 16;
 
@@ -297,8 +298,8 @@ __global__ __launch_bounds__(kThreads) void bn_pa_backward_tiles_kernel(const fl
 // Whether one lane per column gives every CU six workgroups.
 bool many_columns(int64_t L) { return L >= (int64_t)num_cus() * kThreads * 6; }
 
-// Whether COLS = kWideCols gives every CU a workgroup.
-bool wide_column_blocks(int64_t L) { return L >= (int64_t)num_cus() * kWideCols; }
+// Whether COLS = kWideCols gives every CU two workgroups.
+bool wide_column_blocks(int64_t L) { return L >= (int64_t)num_cus() * kWideCols * 2; }
 
 template <bool RELU>
 void bn_pa_forward_tiles(hipStream_t s, const float *x, float *y, float *mean, float *istd, int N, int64_t L) {
