@@ -298,6 +298,38 @@ def test_batch_norm_of_very_many_columns(rt, rows, columns):
         test_fused_batch_norm_relu_equals_the_two_ops(rt, shape)
 
 
+# spatial mode with the chunks folded by a kernel of its own: one and several chunks of a channel per lane, channels that
+# do not fill a workgroup, 16-byte and single accesses; and maps of one pixel whose chunks the apply pass folds
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1024, 3, 10, 10), (300, 1, 7, 9), (1100, 37, 1, 1), (4000, 333, 1, 1), (150, 50, 2, 2),
+                                   (600, 70, 1, 1)], ids=str)
+def test_spatial_batch_norm_of_many_chunks(rt, shape):
+    test_batch_norm(rt, shape, "spatial")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,mode", [
+    ((8, 12, 6, 6), "spatial"), ((8, 12, 5, 7), "spatial"), ((1024, 3, 10, 10), "spatial"), ((1100, 37, 1, 1), "spatial"),
+    ((20, 12, 6, 6), "pre_activation"), ((300, 12, 6, 6), "pre_activation"), ((130, 33000, 1, 1), "pre_activation"),
+], ids=str)
+def test_batch_norm_in_place(rt, shape, mode):
+    """An output that is the input's own array (forward), or the upstream gradient's (backward): the bits of the call
+    with arrays of their own."""
+    from tinyflow_amd import gpu_op, ndarray
+    rng = np.random.RandomState(41)
+    x = rng.normal(0.5, 2, shape).astype(np.float32)
+    dy = rng.normal(0, 1, shape).astype(np.float32)
+    results = []
+    for in_place in (False, True):
+        mean_p, var_p, lst = gpu_op.bn_get_cudnnlist(shape, "NCHW", mode)
+        gx, gdy, again = _gpu(x, rt), _gpu(dy, rt), _gpu(x, rt)
+        gy, gdx = (gx, gdy) if in_place else (ndarray.empty(shape, rt.ctx), ndarray.empty(shape, rt.ctx))
+        assert gpu_op.bn_forward(gx, gy, mode, 0, mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+        assert gpu_op.bn_backward(again, gdy, gdx, mode, mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+        results.append((gy.asnumpy().tobytes(), gdx.asnumpy().tobytes()))
+    assert results[0] == results[1]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["pre_activation", "spatial"])
 def test_batch_norm_with_mean_far_from_zero(rt, mode):

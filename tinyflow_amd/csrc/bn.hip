@@ -10,10 +10,11 @@
 //   single pass: forward reads x and writes y (8 B/element), backward reads x, dy
 //   and writes dx (12 B/element).  Lanes of a wave read 64 consecutive columns,
 //   so every access is a full 256-byte line.
-// spatial mode: one statistic per channel over (N,H,W).  Two kernels: per-(channel,
-//   image-chunk) partial sums (fp32 per lane, fp64 across lanes and chunks), and a
-//   streaming normalise pass over the flat tensor whose workgroups first fold the chunks
-//   of the channels they meet, in a fixed order (12 B/element forward, 20 backward).
+// spatial mode: one statistic per channel over (N,H,W).  Per-(channel, image-chunk)
+//   partial sums (fp32 per lane, fp64 across lanes and chunks), and a streaming
+//   normalise pass over the flat tensor (12 B/element forward, 20 backward).  The chunks
+//   of a channel are folded in a fixed order, by the workgroups of the second pass
+//   themselves or, where that costs more than a launch, by a small kernel in between.
 //
 // Saved statistics protocol (as the reference): forward allocates mean and
 // inverse-std buffers and publishes them through *mean_p / *Variance_p; backward
@@ -425,73 +426,125 @@ __global__ __launch_bounds__(kThreads) void bn_sp_partial_kernel(const float *__
   }
 }
 
+// What the apply pass needs of a channel, from the sums of its chunk partials: forward (mean,
+// 1/sqrt(var + eps)), which are also the saved statistics; backward (sum dy, sum dy*xhat).
+template <bool BWD>
+__device__ inline void channel_floats(double s, double q, double m, float pivot, float &f0, float &f1) {
+  f0 = (float)s;
+  f1 = (float)q;
+  if (BWD) return;
+  const double shifted_mean = s / m;  // mean of x - pivot; the variance does not depend on the pivot
+  double var = q / m - shifted_mean * shifted_mean;
+  if (var < 0.0) var = 0.0;
+  f0 = (float)((double)pivot + shifted_mean);
+  f1 = (float)(1.0 / sqrt(var + (double)kEps));
+}
+
+// Folds the chunk partials of every channel, in chunk order.  A workgroup takes CH channels; all lanes fetch, 256 / CH
+// chunks of a channel at a time, so that the chain of additions runs out of LDS:
+// 1024 chunks of one channel took 77 us with a lane per channel that reads them from memory, and take 4 so.
+template <bool BWD>
+__global__ __launch_bounds__(kThreads) void bn_sp_finish_kernel(const double *__restrict__ partial,
+                                                               const float *__restrict__ pivots,
+                                                               float *__restrict__ out0, float *__restrict__ out1,
+                                                               int C, int chunks, double m, int log_ch) {
+  __shared__ double part[2][kThreads];
+  const int tid = threadIdx.x, ch = 1 << log_ch, depth = kThreads >> log_ch;
+  const int local = tid & (ch - 1), c = blockIdx.x * ch + local;
+  const int sums_of = tid >> log_ch;  // 0: first sum of the pair, 1: second, beyond: fetches only
+  double sum = 0.0;
+  for (int k0 = 0; k0 < chunks; k0 += depth) {
+    const int n = min(depth, chunks - k0);
+    if ((tid >> log_ch) < n && c < C) {
+      const double *p = partial + ((int64_t)(k0 + (tid >> log_ch)) * C + c) * 2;
+      part[0][tid] = p[0];
+      part[1][tid] = p[1];
+    }
+    __syncthreads();
+    if (sums_of < 2 && c < C) {
+#pragma unroll 8
+      for (int k = 0; k < n; ++k) sum += part[sums_of][(k << log_ch) + local];
+    }
+    __syncthreads();
+  }
+  if (sums_of < 2) part[sums_of][local] = sum;
+  __syncthreads();
+  if (sums_of == 0 && c < C) channel_floats<BWD>(part[0][local], part[1][local], m, BWD ? 0.f : pivots[c], out0[c], out1[c]);
+}
+
+// Channels per workgroup of the kernel above, as a power of two: as many as leave lanes for all chunks of each.
+int finish_log_channels(int chunks) {
+  int log_ch = 6;  // at least four lanes per channel
+  while (log_ch > 0 && (kThreads >> log_ch) < chunks) --log_ch;
+  return log_ch;
+}
+
 // Apply pass over the flat tensor, one contiguous run of 1024 units (16 KiB when
 // VEC) per workgroup as in the elementwise engine; a unit (float4 or float) lies
 // inside one (image, channel) row, whose channel is (unit / units per row) % C.
-// Each workgroup first folds, in chunk order, the chunk partials of the channels of its
-// rows: a few KB from the L2 while its elements are on their way.  The fold as a
-// kernel of its own is a launch that does next to nothing: of the 43 + 10 layers of ResNet-50 at batch 8,
-// 160 pixels it cost 3.3 us each forward and 2.5 us backward.
-// FWD: y = (x - mean) * istd, and the saved statistics, by the workgroup that holds the
+// FOLD: each workgroup first folds, in chunk order, the chunk partials of the channels of its
+// rows: a few KB from the L2 while its elements are on their way (fold_in_apply says when).
+// Else p0, p1 hold what bn_sp_finish_kernel made of them.
+// FWD: y = (x - mean) * istd; with FOLD also the saved statistics, by the workgroup that holds the
 // first unit of the channel's row in image 0.  BWD: dx = istd/m * (m*dy - s1 - xhat*s2).
-template <bool BWD, bool VEC>
+template <bool BWD, bool VEC, bool FOLD>
 __global__ __launch_bounds__(kThreads) void bn_sp_apply_kernel(const float *__restrict__ x,
                                                               const float *__restrict__ dy,
                                                               float *__restrict__ out,
                                                               const double *__restrict__ partial,
                                                               const float *__restrict__ pivot, int chunks, double m,
+                                                              const float *__restrict__ p0,
+                                                              const float *__restrict__ p1,
                                                               float *__restrict__ save_mean,
                                                               float *__restrict__ save_istd, FastDiv div_row,
                                                               FastDiv div_c, uint32_t units) {
   constexpr int W = Unit<VEC>::W;
   constexpr int kUnroll = 4;
-  __shared__ float fold[2][kThreads * kUnroll];  // per row: FWD mean, istd; BWD sum dy, sum dy*xhat
+  __shared__ float fold[2][FOLD ? kThreads * kUnroll : 1];  // per row: FWD mean, istd; BWD sum dy, sum dy*xhat
   const uint32_t first = blockIdx.x * (kThreads * kUnroll), base = first + threadIdx.x;
-  float xv[kUnroll][W], gv[kUnroll][W] = {};
+  float xv[kUnroll][W], gv[kUnroll][W];
+  uint32_t row_of[kUnroll], ch[kUnroll];
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
-    const uint32_t unit = base + u * kThreads;
-    if (unit >= units) continue;
+    const uint32_t unit = min(base + u * kThreads, units - 1u);  // no branch between the loads
+    uint32_t img;
+    row_of[u] = div_row.div(unit);
+    div_c.divmod(row_of[u], img, ch[u]);
     Unit<VEC>::load(x + (int64_t)unit * W, xv[u]);
     if (BWD) Unit<VEC>::load(dy + (int64_t)unit * W, gv[u]);
   }
   const uint32_t first_row = div_row.div(first);
-  const uint32_t last_row = div_row.div(min(first + kThreads * kUnroll, units) - 1u);
-  for (uint32_t row = first_row + threadIdx.x; row <= last_row; row += kThreads) {
-    uint32_t img, c;
-    div_c.divmod(row, img, c);
-    double s = 0.0, q = 0.0;
+  if (FOLD) {
+    const uint32_t last_row = div_row.div(min(first + kThreads * kUnroll, units) - 1u);
+    for (uint32_t row = first_row + threadIdx.x; row <= last_row; row += kThreads) {
+      uint32_t img, c;
+      div_c.divmod(row, img, c);
+      double s = 0.0, q = 0.0;
 #pragma unroll 4
-    for (int k = 0; k < chunks; ++k) {
-      s += partial[((int64_t)k * div_c.d + c) * 2 + 0];
-      q += partial[((int64_t)k * div_c.d + c) * 2 + 1];
-    }
-    float f0 = (float)s, f1 = (float)q;
-    if (!BWD) {
-      const double shifted_mean = s / m;  // mean of x - pivot; the variance does not depend on the pivot
-      double var = q / m - shifted_mean * shifted_mean;
-      if (var < 0.0) var = 0.0;
-      f0 = (float)((double)pivot[c] + shifted_mean);
-      f1 = (float)(1.0 / sqrt(var + (double)kEps));
-      if (img == 0 && row * div_row.d >= first) {
+      for (int k = 0; k < chunks; ++k) {
+        s += partial[((int64_t)k * div_c.d + c) * 2 + 0];
+        q += partial[((int64_t)k * div_c.d + c) * 2 + 1];
+      }
+      float f0, f1;
+      channel_floats<BWD>(s, q, m, BWD ? 0.f : pivot[c], f0, f1);
+      if (!BWD && img == 0 && row * div_row.d >= first) {
         save_mean[c] = f0;
         save_istd[c] = f1;
       }
+      fold[0][row - first_row] = f0;
+      fold[1][row - first_row] = f1;
     }
-    fold[0][row - first_row] = f0;
-    fold[1][row - first_row] = f1;
+    __syncthreads();
   }
-  __syncthreads();
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
     const uint32_t unit = base + u * kThreads;
     if (unit >= units) continue;
-    const uint32_t row = div_row.div(unit);
-    const float f0 = fold[0][row - first_row], f1 = fold[1][row - first_row];
+    const uint32_t c = ch[u];
+    const float f0 = FOLD ? fold[0][row_of[u] - first_row] : p0[c];
+    const float f1 = FOLD ? fold[1][row_of[u] - first_row] : p1[c];
     float r[W];
     if (BWD) {
-      uint32_t img, c;
-      div_c.divmod(row, img, c);
       const float mean = save_mean[c], istd = save_istd[c];
       const float scale = istd / (float)m;
 #pragma unroll
@@ -524,6 +577,18 @@ int sp_chunks(int N, int C) {
   int chunks = cdiv((int64_t)num_cus() * 4, C);
   if (chunks > N) chunks = N;
   return chunks < 1 ? 1 : chunks;
+}
+
+// Whether the apply pass folds the chunks itself.  That saves a launch of about 3 us, but every workgroup pays the
+// lanes' chain of additions straight from the L2 and, forward, a square root in fp64 that costs as much as eight of
+// them: with few rounds of workgroups and short chains.  Folding in the apply pass / before it, us forward: 32 images
+// of 256 channels of 14 x 14 8.3 / 11.9, 8 of 64 of 56 x 56 8.8 / 9.4, 512 of 32 of 14 x 14 12.6 / 12.7, 300 of 16 of
+// 112 x 112 141 / 119, 1000 of 1 of 224 x 224 449 / 113, 100000 of 64 of one pixel 88 / 48, 65536 of 1 of one pixel
+// 138 / 22.
+bool fold_in_apply(int chunks, int units_per_row, uint32_t units) {
+  const int lane_rows = cdiv(cdiv(kThreads * 4 - 1, units_per_row) + 1, kThreads);  // rows that a lane folds
+  const int64_t per_cu = units / (kThreads * 4) / num_cus();
+  return lane_rows * (chunks + 8) * (4 + per_cu) <= 384;
 }
 
 int check_bn_arrays(const BNDesc *d, const DLArray *a, const DLArray *b) {
@@ -643,9 +708,19 @@ static int bn_forward_impl(const DLArrayHandle input, DLArrayHandle output, int 
       constexpr bool VEC = decltype(vec_c)::value;
       hipLaunchKernelGGL((bn_sp_partial_kernel<false, VEC>), pgrid, dim3(kThreads), 0, s, x, (const float *)nullptr,
                          (const float *)nullptr, (const float *)nullptr, partial, pivots, d->N, d->C, d->HW, ipc, div_row);
-      hipLaunchKernelGGL((bn_sp_apply_kernel<false, VEC>), agrid, dim3(kThreads), 0, s, x, (const float *)nullptr, y,
-                         (const double *)partial, (const float *)pivots, real_chunks, (double)d->N * (double)d->HW,
-                         mean, istd, div_row, div_c, units);
+      const double m = (double)d->N * (double)d->HW;
+      if (fold_in_apply(real_chunks, div_row.d, units)) {
+        hipLaunchKernelGGL((bn_sp_apply_kernel<false, VEC, true>), agrid, dim3(kThreads), 0, s, x,
+                           (const float *)nullptr, y, (const double *)partial, (const float *)pivots, real_chunks, m,
+                           (const float *)nullptr, (const float *)nullptr, mean, istd, div_row, div_c, units);
+      } else {
+        const int log_ch = finish_log_channels(real_chunks);
+        hipLaunchKernelGGL(bn_sp_finish_kernel<false>, dim3(cdiv(d->C, 1 << log_ch)), dim3(kThreads), 0, s,
+                           (const double *)partial, (const float *)pivots, mean, istd, d->C, real_chunks, m, log_ch);
+        hipLaunchKernelGGL((bn_sp_apply_kernel<false, VEC, false>), agrid, dim3(kThreads), 0, s, x,
+                           (const float *)nullptr, y, (const double *)nullptr, (const float *)nullptr, 0, m,
+                           (const float *)mean, (const float *)istd, mean, istd, div_row, div_c, units);
+      }
     };
     if (vec) run(std::true_type{}); else run(std::false_type{});
     device_free(partial);
@@ -716,12 +791,14 @@ static int bn_backward_impl(const DLArrayHandle input, const DLArrayHandle doutp
       const int chunks = sp_chunks(d->N, d->C);
       const int ipc = cdiv(d->N, chunks);
       const int real_chunks = cdiv(d->N, ipc);
-      const size_t pbytes = (size_t)real_chunks * d->C * 2 * sizeof(double);
+      // chunk partials of every channel and, behind them, the channels' two sums
+      const size_t pbytes = (size_t)d->C * (real_chunks * 2 * sizeof(double) + 2 * sizeof(float));
       double *partial = (double *)device_alloc(pbytes);
       if (!partial) {
         if (memorytoSaving) *memorytoSaving = shortfall(pbytes);
         return 0;  // statistics stay published so the call can be repeated
       }
+      float *sums = reinterpret_cast<float *>(partial + (size_t)real_chunks * d->C * 2);
       const bool vec = d->HW % 4 == 0 &&
                        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) |
                          reinterpret_cast<uintptr_t>(dx)) & 15u) == 0;
@@ -733,9 +810,21 @@ static int bn_backward_impl(const DLArrayHandle input, const DLArrayHandle doutp
         constexpr bool VEC = decltype(vec_c)::value;
         hipLaunchKernelGGL((bn_sp_partial_kernel<true, VEC>), pgrid, dim3(kThreads), 0, s, x, dy, mean, istd, partial,
                            (float *)nullptr, d->N, d->C, d->HW, ipc, div_row);
-        hipLaunchKernelGGL((bn_sp_apply_kernel<true, VEC>), agrid, dim3(kThreads), 0, s, x, dy, dx,
-                           (const double *)partial, (const float *)nullptr, real_chunks, (double)d->N * (double)d->HW,
-                           const_cast<float *>(mean), const_cast<float *>(istd), div_row, div_c, units);
+        const double m = (double)d->N * (double)d->HW;
+        float *stat0 = const_cast<float *>(mean), *stat1 = const_cast<float *>(istd);
+        if (fold_in_apply(real_chunks, div_row.d, units)) {
+          hipLaunchKernelGGL((bn_sp_apply_kernel<true, VEC, true>), agrid, dim3(kThreads), 0, s, x, dy, dx,
+                             (const double *)partial, (const float *)nullptr, real_chunks, m, (const float *)nullptr,
+                             (const float *)nullptr, stat0, stat1, div_row, div_c, units);
+        } else {
+          const int log_ch = finish_log_channels(real_chunks);
+          hipLaunchKernelGGL(bn_sp_finish_kernel<true>, dim3(cdiv(d->C, 1 << log_ch)), dim3(kThreads), 0, s,
+                             (const double *)partial, (const float *)nullptr, sums, sums + d->C, d->C, real_chunks, m,
+                             log_ch);
+          hipLaunchKernelGGL((bn_sp_apply_kernel<true, VEC, false>), agrid, dim3(kThreads), 0, s, x, dy, dx,
+                             (const double *)nullptr, (const float *)nullptr, 0, m, (const float *)sums,
+                             (const float *)(sums + d->C), stat0, stat1, div_row, div_c, units);
+        }
       };
       if (vec) run(std::true_type{}); else run(std::false_type{});
       device_free(partial);
