@@ -83,7 +83,8 @@ def test_pooling(rt, case, ties):
 
 
 # planes at the edges of the workgroup sizes of the plane kernels (64, 256 and 1024 lanes, sixteen elements and four
-# windows each): full, one row more, no multiple of four elements, few lanes' worth
+# windows each): full, one row more, no multiple of four elements, few lanes' worth; few planes and as many as turn
+# the forward (4097, 1025 on 256 units) and the backward pass (2049, 513) to the smaller workgroups
 @pytest.mark.parametrize("case", [
     ((5, 3, 32, 32), "max", 0, 0, 2, 2, 2, 2),
     ((5, 3, 34, 32), "max", 0, 0, 2, 2, 2, 2),
@@ -93,6 +94,13 @@ def test_pooling(rt, case, ties):
     ((2, 3, 63, 65), "max", 1, 1, 2, 2, 3, 3),
     ((1000, 16, 10, 10), "max", 0, 0, 2, 2, 2, 2),
     ((3, 5, 3, 3), "max", 1, 1, 2, 2, 3, 3),
+    ((3, 5, 16, 16), "max", 1, 1, 2, 2, 3, 3),
+    ((4097, 1, 32, 32), "max", 0, 0, 2, 2, 2, 2),
+    ((241, 17, 31, 31), "max", 1, 1, 2, 2, 3, 3),
+    ((1025, 1, 64, 64), "max", 0, 0, 2, 2, 2, 2),
+    ((205, 5, 61, 63), "max", 1, 1, 2, 2, 3, 3),
+    ((2049, 1, 32, 32), "max", 0, 0, 2, 2, 2, 2),
+    ((27, 19, 34, 32), "max", 0, 0, 2, 2, 2, 2),
 ], ids=str)
 def test_pooling_at_the_edges_of_the_workgroup_sizes(rt, case):
     for ties in (False, True):

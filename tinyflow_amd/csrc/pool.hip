@@ -343,8 +343,7 @@ __global__ __launch_bounds__(kThreads) void pool_max_backward_tile_kernel(const 
 // are summed in round order rather than in (p, q) order, so the last bit of such a sum
 // can differ from the other forms; run to run it is the same.
 // VEC: H*W a multiple of 4 and 16-byte aligned planes.
-// LANES: the smallest workgroup whose lanes cover the plane with four vectors and four windows each
-// (with_plane_lanes).  A workgroup of 1024 lanes on a 28 x 28 plane leaves four of five idle and two of
+// LANES: see with_plane_lanes.  A workgroup of 1024 lanes on a 28 x 28 plane leaves four of five idle and two of
 // them fill a CU: the two pools of LeNet-5 at batch 1000 took 58 us forward and 84 us backward.
 constexpr int kPlaneMaxFloats = 16384, kPlaneThreads = 1024, kPlaneWindowsPerLane = 4;
 
@@ -536,11 +535,21 @@ bool shape_is(const DLArray *a, int d0, int d1, int d2, int d3) {
   return a->ndim == 4 && a->shape[0] == d0 && a->shape[1] == d1 && a->shape[2] == d2 && a->shape[3] == d3;
 }
 
+// Lanes per workgroup of the plane kernels: the fewest that take one vector and one window each, more of them gain
+// nothing; or the fewest that take four each where there are planes for `enough` lanes per CU, below which the depth of
+// a lane's work is what takes the time: backward, 3 x 3 windows, 512 planes of 32 x 32 4.7 us with 256 lanes, 6.1 with
+// 64, and of 64 x 64 6.6 with 1024, 7.5 with 256; but 1024 of 34 x 34 8.0 with 1024, 5.9 with 256, and 4096 of
+// 24 x 24 9.1 with 256, 7.8 with 64.  A forward pass has less to hide and turns later: 768 of 60 x 60 5.7 with 1024,
+// 6.3 with 256; 2500 of 28 x 28 5.1 with 256, 6.4 with 64.
 template <class F>
-void with_plane_lanes(int floats, int windows, F &&f) {
-  const auto covers = [&](int lanes) { return floats <= 16 * lanes && windows <= kPlaneWindowsPerLane * lanes; };
-  if (covers(64)) f(std::integral_constant<int, 64>{});
-  else if (covers(256)) f(std::integral_constant<int, 256>{});
+void with_plane_lanes(int floats, int windows, int64_t planes, int enough, F &&f) {
+  const auto fits = [&](int lanes) {
+    const bool covers = floats <= 16 * lanes && windows <= kPlaneWindowsPerLane * lanes;
+    const bool one_each = floats <= 4 * lanes && windows <= lanes;
+    return one_each || (covers && planes * lanes > (int64_t)num_cus() * enough);
+  };
+  if (fits(64)) f(std::integral_constant<int, 64>{});
+  else if (fits(256)) f(std::integral_constant<int, 256>{});
   else f(std::integral_constant<int, kPlaneThreads>{});
 }
 
@@ -635,7 +644,7 @@ extern "C" int DLGpuPooling2DForward(const DLArrayHandle input, DLArrayHandle ou
     auto run = [&](auto f_c, auto vec_c) {
       constexpr int F = decltype(f_c)::value;
       constexpr bool VEC = decltype(vec_c)::value;
-      with_plane_lanes(HW, bp.P * bp.Q, [&](auto lanes_c) {
+      with_plane_lanes(HW, bp.P * bp.Q, planes, 1024, [&](auto lanes_c) {
         constexpr int LANES = decltype(lanes_c)::value;
         hipLaunchKernelGGL((pool_max_forward_plane_kernel<F, F, VEC, LANES>), dim3(planes), dim3(LANES), lds, s, xp, yp, bp);
       });
@@ -698,7 +707,7 @@ extern "C" int DLGpuPooling2DBackward(const DLArrayHandle input, const DLArrayHa
       auto run = [&](auto f_c, auto vec_c) {
         constexpr int F = decltype(f_c)::value;
         constexpr bool VEC = decltype(vec_c)::value;
-        with_plane_lanes(HW, bp.P * bp.Q, [&](auto lanes_c) {
+        with_plane_lanes(HW, bp.P * bp.Q, planes, 512, [&](auto lanes_c) {
           constexpr int LANES = decltype(lanes_c)::value;
           hipLaunchKernelGGL((pool_max_backward_plane_kernel<F, F, VEC, LANES>), dim3(planes), dim3(LANES), lds, s, xp, gp,
                              dp, bp);
