@@ -86,30 +86,43 @@ def test_conv_forward_and_gradients(rt, case):
     _check_conv_case(rt, case)
 
 
-# grad-data of strided filters by phases: u*v = 2, 3 and 4, a phase without taps (filter smaller than the stride
-# one way), a phase without pixels (one input row), rows and columns that no tap reaches (rows past the last window),
-# padding larger than a phase's offset, both filter loaders (channels a multiple of 4 or not), every tile shape
-PHASE_CASES = [
-    (2, 5, 9, 11, 7, 3, 3, "SAME", 2, 1),
-    (2, 8, 9, 11, 7, 2, 5, "VALID", 1, 2),
-    (3, 6, 10, 8, 9, 3, 4, "VALID", 1, 3),
-    (2, 4, 13, 9, 3, 3, 1, "VALID", 4, 1),
-    (2, 12, 8, 8, 6, 2, 1, "VALID", 2, 2),
-    (2, 12, 8, 7, 6, 1, 3, "VALID", 2, 2),
-    (5, 3, 1, 9, 4, 1, 3, "VALID", 2, 2),
-    (2, 8, 12, 14, 10, 5, 5, "SAME", 2, 2),
-    (1, 70, 31, 29, 20, 7, 7, "SAME", 2, 2),
-    (4, 130, 56, 56, 33, 3, 3, "SAME", 2, 2),
-    (16, 128, 57, 55, 64, 3, 3, "VALID", 2, 2),
+# grad-data of strided filters: u*v = 2, 3 and 4, a phase without taps (filter smaller than the stride one way), a phase
+# without pixels (one input row), rows and columns that no tap reaches (rows past the last window), padding larger than
+# a phase's offset.  By phases, each tile shape with both filter loaders (channels a multiple of 4 or not); and too
+# little work for the phases, which walks every tap
+STRIDED_CASES = [
+    ((2, 5, 9, 11, 48, 3, 3, "SAME", 2, 1), "dgrad_phases 64x64", "PlainAlong"),
+    ((2, 8, 9, 11, 32, 2, 5, "VALID", 1, 2), "dgrad_phases 64x64", "Along4"),
+    ((3, 6, 10, 8, 17, 3, 4, "VALID", 1, 3), "dgrad_phases 64x64", "PlainAlong"),
+    ((2, 4, 13, 9, 50, 3, 1, "VALID", 4, 1), "dgrad_phases 64x64", "Along4"),
+    ((2, 12, 8, 8, 97, 2, 1, "VALID", 2, 2), "dgrad_phases 64x64", "Along4"),
+    ((2, 12, 8, 7, 97, 1, 3, "VALID", 2, 2), "dgrad_phases 64x64", "Along4"),
+    ((5, 3, 1, 9, 98, 1, 3, "VALID", 2, 2), "dgrad_phases 64x64", "PlainAlong"),
+    ((2, 8, 12, 14, 10, 5, 5, "SAME", 2, 2), "dgrad_phases 64x64", "Along4"),
+    ((1, 70, 31, 29, 20, 7, 7, "SAME", 2, 2), "dgrad_phases 64x64", "PlainAlong"),
+    ((4, 130, 56, 56, 33, 3, 3, "SAME", 2, 2), "dgrad_phases 64x64", "PlainAlong"),
+    ((16, 128, 57, 55, 64, 3, 3, "VALID", 2, 2), "dgrad_phases 64x128", "Along4"),
+    ((16, 66, 57, 55, 20, 3, 3, "SAME", 2, 2), "dgrad_phases 64x128", "PlainAlong"),
+    ((32, 128, 57, 55, 20, 3, 3, "SAME", 2, 2), "dgrad_phases 128x128", "Along4"),
+    ((32, 126, 57, 55, 20, 3, 3, "SAME", 2, 2), "dgrad_phases 128x128", "PlainAlong"),
+    ((2, 5, 9, 11, 7, 3, 3, "SAME", 2, 1), "dgrad_strided 64x64", "PlainAlong"),
+    ((2, 8, 9, 11, 7, 2, 5, "VALID", 1, 2), "dgrad_strided 64x64", "PlainAlong"),
+    ((3, 6, 10, 8, 9, 3, 4, "VALID", 1, 3), "dgrad_strided 64x64", "PlainAlong"),
+    ((2, 4, 13, 9, 3, 3, 1, "VALID", 4, 1), "dgrad_strided 64x64", "PlainAlong"),
+    ((2, 12, 8, 8, 6, 2, 1, "VALID", 2, 2), "dgrad_strided 64x64", "PlainAlong"),
+    ((2, 12, 8, 7, 6, 1, 3, "VALID", 2, 2), "dgrad_strided 64x64", "PlainAlong"),
+    ((5, 3, 1, 9, 4, 1, 3, "VALID", 2, 2), "dgrad_strided 64x64", "PlainAlong"),
 ]
 
 
-@pytest.mark.parametrize("case", PHASE_CASES, ids=lambda c: "x".join(str(v) for v in c))
-def test_strided_grad_data_by_phases(rt, case):
+@pytest.mark.parametrize("case,kernel,filter_loader", STRIDED_CASES,
+                         ids=lambda v: v if isinstance(v, str) else "x".join(str(e) for e in v))
+def test_strided_grad_data(rt, case, kernel, filter_loader):
     from tinyflow_amd import gpu_op
     N, C, H, W, K, R, S, padding, u, v = case
     _, lst = gpu_op.convolution_2d_forward_get_out_shape((N, C, H, W), (K, C, R, S), "NCHW", padding, u, v)
-    assert "dgrad_phases" in _describe(lst, 1)
+    described = _describe(lst, 1)
+    assert described.startswith(kernel + " ") and filter_loader + "<" in described
     _check_conv_case(rt, case)
 
 

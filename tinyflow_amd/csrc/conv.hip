@@ -42,8 +42,8 @@ typedef unsigned i32x4v __attribute__((__vector_size__(4 * sizeof(unsigned)))); 
 // MODE 0: taps are always inside the image (no padding)      -> no range test
 // MODE 1: range test (zero padding)
 // MODE 2: additionally the tapped coordinate must be divisible by the conv
-//         stride and is divided by it (grad-data of a filter larger than 1x1 whose
-//         strides multiply to more than kMaxPhases, see below)
+//         stride and is divided by it (grad-data of a strided filter larger than 1x1
+//         that does not run by phases, see dgrad_by_phases)
 template <int D, int BK, int MODE>
 struct GatherAlong {
   using Map = AlongMap<D, BK>;
@@ -1296,11 +1296,7 @@ ConvPlan plan_forward(const ConvDesc *d) {
   return p;
 }
 
-bool dgrad_by_phases(const ConvDesc *d) {
-  return d->R * d->S > 1 && d->u * d->v > 1 && d->u * d->v <= kMaxPhases;
-}
-
-// Geometry of the phases; in the order a*v + b the first has the most taps and pixels.
+// Geometry of the phases; in the order a*v + b the first has the most taps.
 Phases dgrad_phases(const ConvDesc *d) {
   Phases all;
   int row = 0;
@@ -1328,6 +1324,26 @@ Phases dgrad_phases(const ConvDesc *d) {
     p.div_row = FastDiv((uint32_t)cols);
   }
   return all;
+}
+
+// Whether the phases are worth it: they cost 4.5 us over the walk.  What they give is the stages of the reduction that a
+// workgroup of the walk fetches and a workgroup of the average phase does not (`saved`), each time the chip is filled
+// (`rounds`; a chip that is never full pays for the whole of one workgroup); for v > 1 half of that, since their
+// stores are every v-th word; and for v = 1 the cheaper gather by itself from eight rounds on.  Walk / phases, us:
+//   8 x 28 x 28 of 3 channels from 2, 2x2 stride 2: no stage, 8.5 / 13.1, and alike for all small layers
+//   64 x 7 x 7 of 256 from 32, 2x2 stride 2: 3 stages, 14.1 / 15.1;  64 x 7 x 7 of 16 from 16, 3x3: 3.8, 15.1 / 13.5
+//   64 x 28 x 28 of 256 from 8, 2x2 stride 2: no stage, 30 / 42;  3x3 strides (1, 2): 1.5 x 12 rounds, 57 / 36
+//   64 x 28 x 28 of 1024 from 1, 3x3 strides (2, 1): no stage, 49 rounds, 93 / 58
+//   16 x 57 x 57 of 1024 from 64, 5x5 stride 2: 37 x 51, 2474 / 445
+bool dgrad_by_phases(const ConvDesc *d) {
+  const int RS = d->R * d->S, uv = d->u * d->v;
+  if (RS == 1 || uv == 1 || uv > kMaxPhases) return false;
+  constexpr int kStage = 32;
+  const Phases phases = dgrad_phases(d);
+  double saved = cdiv((int64_t)d->K * RS, kStage);
+  for (int q = 0; q < uv; ++q) saved -= (double)cdiv(phases.p[q].k_extent, kStage) / uv;
+  const double rounds = (double)cdiv(d->C, 64) * cdiv((int64_t)d->N * d->H * d->W, 64) / num_cus();
+  return saved >= 3.5 || saved * rounds >= (d->v == 1 ? 2.0 : 4.0) || (d->v == 1 && rounds >= 8.0);
 }
 
 ConvPlan plan_dgrad(const ConvDesc *d) {
@@ -1886,7 +1902,7 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
     device_free(wt);
     return finish(s, "DLGpuConvolutionBackwardData");
   }
-  // a strided filter larger than 1x1 in more than kMaxPhases phases always runs on the small tile, unsplit
+  // a strided filter larger than 1x1 that does not run by phases always runs on the small tile, unsplit
   const bool strided_taps = RS > 1 && !(d->u == 1 && d->v == 1);
   const int g_bm = strided_taps ? 64 : plan.bm, g_bn = strided_taps ? 64 : plan.bn;
   Geometry g = make_geometry(M, plan.N, K, g_bm, g_bn, strided_taps ? 1 : plan.splits, stage_depth(g_bm, g_bn));
