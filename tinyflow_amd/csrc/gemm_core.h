@@ -3,8 +3,8 @@
 //
 //   D[m, n] = sum_k A(m, k) * B(k, n)
 //
-// One 256-lane workgroup (four wave64 waves in a 2 x 2 arrangement) owns a
-// BM x BN tile of D and walks the reduction in steps of BK (16 or 32, a template
+// One 256-lane workgroup (four wave64 waves, 2 x 2 over the tile or, on a tile of 32
+// rows, side by side) owns a BM x BN tile of D and walks the reduction in steps of BK (16 or 32, a template
 // parameter chosen with the tile shape).  Operand tiles
 // are fetched with bounds-checked buffer loads (an out-of-range or padded
 // element is given an offset beyond the buffer and reads as zero, so tails and

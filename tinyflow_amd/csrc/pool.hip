@@ -344,7 +344,7 @@ __global__ __launch_bounds__(kThreads) void pool_max_backward_tile_kernel(const 
 // can differ from the other forms; run to run it is the same.
 // VEC: H*W a multiple of 4 and 16-byte aligned planes.
 // LANES: see with_plane_lanes.  A workgroup of 1024 lanes on a 28 x 28 plane leaves four of five idle and two of
-// them fill a CU: the two pools of LeNet-5 at batch 1000 took 58 us forward and 84 us backward.
+// them fill a CU: the two pools of LeNet-5 at batch 1000 took 58 us forward and 84 us backward, with 64 lanes 15 and 19.
 constexpr int kPlaneMaxFloats = 16384, kPlaneThreads = 1024, kPlaneWindowsPerLane = 4;
 
 template <int FH, int FW, bool VEC, int LANES>
