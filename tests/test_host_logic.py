@@ -689,3 +689,22 @@ def test_recompute_schedule_invariants():
         # released once after the forward pass and once for good
         rel = sorted(t2 for t2, ns in release.items() if n in ns)
         assert len(rel) == 2 and rel[0] < first_backward <= rel[1] and rel[0] < t <= rel[1]
+
+
+@pytest.mark.parametrize("case,split", [
+    (((64, 256, 14, 14), (1024, 256, 1, 1), "VALID", 1), (True, True, True)),
+    (((20, 50, 61, 59), (70, 50, 5, 5), "VALID", 2), (True, True, True)),
+    (((64, 47, 14, 14), (1024, 47, 1, 1), "VALID", 1), (False, False, False)),    # fewer than 48 channels on a side
+    (((64, 1024, 14, 14), (47, 1024, 1, 1), "VALID", 1), (False, False, False)),
+    (((64, 256, 14, 14), (256, 256, 3, 3), "SAME", 1), (False, False, False)),    # 3x3 / stride 1
+    (((64, 1024, 14, 14), (2048, 1024, 1, 1), "VALID", 2), (True, True, False)),  # 49 outputs, x gathered by elements
+    (((64, 64, 56, 56), (256, 64, 1, 1), "VALID", 1), (True, False, True)),       # grad-data of 64 rows
+], ids=str)
+def test_planner_picks_the_engine_by_shape(monkeypatch, case, split):
+    monkeypatch.delenv("TINYFLOW_SPLIT", raising=False)
+    x_shape, w_shape, padding, stride = case
+    _, lst = gpu_op.convolution_2d_forward_get_out_shape(x_shape, w_shape, "NCHW", padding, stride, stride)
+    name = ctypes.create_string_buffer(256)
+    for which in range(3):
+        assert _LIB.DLGpuConvolutionDescribeKernel(lst, which, name, 256, None) == 0
+        assert (b"Split" in name.value) == split[which], name.value

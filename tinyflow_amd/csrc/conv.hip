@@ -20,6 +20,7 @@
 // layout change of the activations.
 #include "gemm_core.h"
 #include "gemm_launch.h"
+#include "gemm_split.h"
 #include "internal.h"
 
 #include <algorithm>
@@ -31,7 +32,7 @@ using namespace tf;
 using namespace tf::gemm;
 
 namespace {
-typedef float f32x2v __attribute__((ext_vector_type(2)));
+using split::f32x2v;
 typedef unsigned i32x2v __attribute__((__vector_size__(2 * sizeof(unsigned))));   // operand types of the 8- and 16-byte
 typedef unsigned i32x4v __attribute__((__vector_size__(4 * sizeof(unsigned))));   // buffer builtins
 
@@ -44,9 +45,9 @@ typedef unsigned i32x4v __attribute__((__vector_size__(4 * sizeof(unsigned)))); 
 // MODE 2: additionally the tapped coordinate must be divisible by the conv
 //         stride and is divided by it (grad-data of a strided filter larger than 1x1
 //         that does not run by phases, see dgrad_by_phases)
-template <int D, int BK, int MODE>
-struct GatherAlong {
-  using Map = AlongMap<D, BK>;
+template <int MODE, class LaneMap>
+struct GatherAlongLanes {
+  using Map = LaneMap;
   static constexpr int EPT = Map::EPT;
   const float *base;
   uint32_t bytes;
@@ -140,6 +141,18 @@ struct GatherAlong {
 #pragma unroll
     for (int e = 0; e < EPT; ++e) tile[st.map.k_of(e)][st.map.d_local] = reg[e];
   }
+  __device__ inline void put(const State &st, char *planes, const float (&reg)[EPT]) const { st.map.put(planes, reg); }
+  template <class F>
+  __device__ inline void each(const State &st, const float (&reg)[EPT], F &&f) const {
+    st.map.each(reg, f);
+  }
+};
+template <int D, int BK, int MODE>
+struct GatherAlong : GatherAlongLanes<MODE, AlongMap<D, BK>> {};
+template <int D, int BK, int MODE>
+struct SplitGatherAlong : GatherAlongLanes<MODE, split::AlongRuns<D, BK>> {
+  using Layout = typename split::AlongRuns<D, BK>::Layout;
+  static constexpr bool kSplit = true;
 };
 
 // ---- gathered operand, lanes along the reduction (grad-filter's x) --------------
@@ -239,6 +252,155 @@ struct DyAcross {
   __device__ inline void store(const State &st, float (*tile)[LD], const float (&reg)[EPT]) const {
 #pragma unroll
     for (int e = 0; e < EPT; ++e) tile[st.map.k_local][st.map.d_of(e)] = reg[e];
+  }
+};
+
+// ---- the same two for the split engine: four consecutive k a lane --------------
+// col -> (c, r, s) fixed per lane for the whole kernel,
+// k -> (img, p, q): the first of a lane's four consecutive ones is taken apart per stage, the
+// others are counted on from it; reads x[img][c][p*u+r-pad_h][q*v+s-pad_w].
+// MODE 0 and 1: one element per load, without and with padding.  MODE 2 (v = 1) and 3 (v = 2): no padding and rows of
+// a multiple of four outputs, whose four inputs are inside four or eight consecutive elements (the last of
+// those may lie past the row; nothing is taken from there).
+template <int D, int BK, int MODE>
+struct SplitGatherAcross {
+  using Map = split::AcrossRuns<D, BK>;
+  using Layout = typename Map::Layout;
+  static constexpr bool kSplit = true;
+  static constexpr int EPT = Map::EPT;
+  const float *base;
+  uint32_t bytes;
+  int k_extent, n_extent;    // N*P*Q, C*R*S
+  FastDiv div_pq, div_q, div_rs, div_s;
+  int img_stride, chan_stride;  // C*H*W, H*W
+  int H, W, P, u, v, pad_h, pad_w;
+  uint32_t pix_valid;        // pixels per image where div_pq counts more of them (ragged segments), else no limit
+
+  struct State {
+    Map map;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t col_off[Map::VPT];  // byte offset of (channel, tap) from the window's first element, or OOB
+    int taps[Map::VPT];          // packed (r, s)
+  };
+  __device__ inline void init(State &st, int origin, int tid) const {
+    st.map.init(tid);
+    st.rsrc = make_rsrc(base, bytes);
+#pragma unroll
+    for (int e = 0; e < Map::VPT; ++e) {
+      const int col = origin + st.map.d_of(e);
+      const bool ok = col < n_extent;
+      uint32_t c, rs, r, s;
+      div_rs.divmod((uint32_t)(ok ? col : 0), c, rs);
+      div_s.divmod(rs, r, s);
+      st.col_off[e] = ok ? (uint32_t)((int)c * chan_stride + (int)r * W + (int)s) * 4u : OOB;
+      st.taps[e] = (int)((r << 16) | s);
+    }
+  }
+  __device__ inline void load(const State &st, int k0, int k_limit, float (&reg)[EPT]) const {
+    const int kidx = k0 + st.map.k_local;
+    uint32_t img, rem, p, q;
+    div_pq.divmod((uint32_t)min(kidx, k_limit - 1), img, rem);
+    div_q.divmod(rem, p, q);
+    int y0 = (int)p * u - pad_h, x0 = (int)q * v - pad_w, img_off = (int)img * img_stride;
+    if constexpr (MODE >= 2) {  // the four are in one row: one or two vectors hold them
+      const uint32_t at = (uint32_t)(img_off + y0 * W + x0) * 4u;
+      const uint32_t k_bad = kidx < k_limit ? 0u : OOB;
+#pragma unroll
+      for (int e = 0; e < Map::VPT; ++e) {
+        const uint32_t off = (at + (st.col_off[e] & ~OOB)) | (k_bad | (st.col_off[e] & OOB));
+        const f32x4v lo = buf_load4(st.rsrc, off);
+        if constexpr (MODE == 2) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) reg[4 * e + i] = lo[i];
+        } else {
+          const f32x4v hi = buf_load4(st.rsrc, off + 16u);
+          reg[4 * e] = lo[0];
+          reg[4 * e + 1] = lo[2];
+          reg[4 * e + 2] = hi[0];
+          reg[4 * e + 3] = hi[2];
+        }
+      }
+      return;
+    }
+    const int x_end = (int)div_q.d * v - pad_w, y_end = P * u - pad_h;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t at = (uint32_t)(img_off + y0 * W + x0) * 4u;
+      const uint32_t k_bad = kidx + i < k_limit && rem + i < pix_valid ? 0u : OOB;
+#pragma unroll
+      for (int e = 0; e < Map::VPT; ++e) {
+        uint32_t bad = k_bad | (st.col_off[e] & OOB);
+        if (MODE == 1) {
+          const int yy = y0 + (st.taps[e] >> 16), xx = x0 + (st.taps[e] & 0xffff);
+          if ((uint32_t)yy >= (uint32_t)H || (uint32_t)xx >= (uint32_t)W) bad = OOB;
+        }
+        reg[4 * e + i] = buf_load(st.rsrc, (at + (st.col_off[e] & ~OOB)) | bad);
+      }
+      x0 += v;
+      if (x0 == x_end) {
+        x0 = -pad_w;
+        y0 += u;
+        if (y0 == y_end) {
+          y0 = -pad_h;
+          img_off += img_stride;
+        }
+      }
+    }
+  }
+  __device__ inline void put(const State &st, char *planes, const float (&reg)[EPT]) const { st.map.put(planes, reg); }
+  template <class F>
+  __device__ inline void each(const State &st, const float (&reg)[EPT], F &&f) const {
+    st.map.each(reg, f);
+  }
+};
+
+template <int D, int BK>
+struct SplitDyAcross {
+  using Map = split::AcrossRuns<D, BK>;
+  using Layout = typename Map::Layout;
+  static constexpr bool kSplit = true;
+  static constexpr int EPT = Map::EPT;
+  const float *base;
+  uint32_t bytes;
+  int k_extent, m_extent;  // N*P*Q, K
+  FastDiv div_pq;
+  int img_stride, PQ;      // K*P*Q
+
+  struct State {
+    Map map;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t row_off[Map::VPT];
+  };
+  __device__ inline void init(State &st, int origin, int tid) const {
+    st.map.init(tid);
+    st.rsrc = make_rsrc(base, bytes);
+#pragma unroll
+    for (int e = 0; e < Map::VPT; ++e) {
+      const int m = origin + st.map.d_of(e);
+      st.row_off[e] = m < m_extent ? (uint32_t)m * (uint32_t)PQ * 4u : OOB;
+    }
+  }
+  __device__ inline void load(const State &st, int k0, int k_limit, float (&reg)[EPT]) const {
+    const int kidx = k0 + st.map.k_local;
+    uint32_t img, pq;
+    div_pq.divmod((uint32_t)min(kidx, k_limit - 1), img, pq);
+    int img_off = (int)img * img_stride;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t k_off = kidx + i < k_limit ? (uint32_t)(img_off + (int)pq) * 4u : OOB;
+#pragma unroll
+      for (int e = 0; e < Map::VPT; ++e)
+        reg[4 * e + i] = buf_load(st.rsrc, (st.row_off[e] + k_off) | ((st.row_off[e] | k_off) & OOB));
+      if (++pq == (uint32_t)PQ) {
+        pq = 0;
+        img_off += img_stride;
+      }
+    }
+  }
+  __device__ inline void put(const State &st, char *planes, const float (&reg)[EPT]) const { st.map.put(planes, reg); }
+  template <class F>
+  __device__ inline void each(const State &st, const float (&reg)[EPT], F &&f) const {
+    st.map.each(reg, f);
   }
 };
 
@@ -366,8 +528,20 @@ struct Phases {
   }
 };
 
-template <class L>  // Along4 or PlainAlong over the whole re-laid filter
+// Loaders of the split engine say so; their planes' layout, if they are.
+template <class L, class = void>
+struct is_split : std::false_type {
+  using Layout = void;
+};
+template <class L>
+struct is_split<L, std::enable_if_t<L::kSplit>> : std::true_type {
+  using Layout = typename L::Layout;
+};
+
+template <class L>  // Along4, PlainAlong or SplitAlong4 over the whole re-laid filter
 struct PhasedFilter {
+  using Layout = typename is_split<L>::Layout;
+  static constexpr bool kSplit = is_split<L>::value;
   static constexpr int EPT = L::EPT;
   L whole;
   Phases phases;
@@ -390,11 +564,17 @@ struct PhasedFilter {
   __device__ inline void store(const State &s, float (*tile)[LD], const float (&reg)[EPT]) const {
     s.one.template store<LD>(s.st, tile, reg);
   }
+  __device__ inline void put(const State &s, char *planes, const float (&reg)[EPT]) const { s.one.put(s.st, planes, reg); }
+  template <class F>
+  __device__ inline void each(const State &s, const float (&reg)[EPT], F &&f) const {
+    s.one.each(s.st, reg, f);
+  }
 };
 
-template <int D, int BK>
-struct PhasedGather {
-  using L = GatherAlong<D, BK, 1>;
+template <class L>  // GatherAlong or SplitGatherAlong
+struct PhasedGatherOf {
+  using Layout = typename is_split<L>::Layout;
+  static constexpr bool kSplit = is_split<L>::value;
   static constexpr int EPT = L::EPT;
   L whole;  // the members that a phase does not replace
   Phases phases;
@@ -425,7 +605,17 @@ struct PhasedGather {
   __device__ inline void store(const State &s, float (*tile)[LD], const float (&reg)[EPT]) const {
     s.one.template store<LD>(s.st, tile, reg);
   }
+  __device__ inline void put(const State &s, char *planes, const float (&reg)[EPT]) const { s.one.put(s.st, planes, reg); }
+  template <class F>
+  __device__ inline void each(const State &s, const float (&reg)[EPT], F &&f) const {
+    s.one.each(s.st, reg, f);
+  }
 };
+
+template <int D, int BK>
+struct PhasedGather : PhasedGatherOf<GatherAlong<D, BK, 1>> {};
+template <int D, int BK>
+struct SplitPhasedGather : PhasedGatherOf<SplitGatherAlong<D, BK, 1>> {};
 
 // D[m = c][n = (img, i, j)] -> dx[img][c][y0 + u*i][x0 + v*j]
 struct StorePhase {
@@ -953,7 +1143,7 @@ using IC = std::integral_constant<int, V>;
 // Tile shapes and the stage depth that goes with each (measured): 16-deep stages
 // for the wide tiles, 32-deep for the 64 x 64 tile, whose per-stage overhead is
 // otherwise as large as its eight MFMAs per wave.
-inline int stage_depth(int bm, int bn) { return (bm == 64 && bn == 64) ? 32 : 16; }
+constexpr int stage_depth(int bm, int bn) { return (bm == 64 && bn == 64) ? 32 : 16; }
 
 // Forward, the 1x1 grad-data and the Winograd products run the 64 x 64 tile with 16-deep
 // stages when the reduction (per k-split) is short (at most 512): half the LDS per workgroup lets eight instead of four share a CU,
@@ -983,9 +1173,14 @@ thread_local hipEvent_t next_kernel_start = nullptr, next_kernel_stop = nullptr;
 
 template <int BM, int BN, int BK, class AL, class BL, class EP>
 void launch(const AL &al, const BL &bl, const EP &ep, int K, const Geometry &g, hipStream_t s, int batch = 1) {
+  if constexpr (is_split<AL>::value && BK != stage_depth(BM, BN)) return;  // only the fp32 engine has those (run_depth)
   if (next_kernel_start) (void)hipEventRecord(next_kernel_start, s);
-  hipLaunchKernelGGL((gemm_kernel<BM, BN, BK, AL, BL, EP>), dim3(g.blocks(), batch), dim3(THREADS), 0, s, al, bl, ep,
-                     K, g.k_per_split, g.tiles_m, g.tiles_n, g.fold());
+  if constexpr (is_split<AL>::value)
+    hipLaunchKernelGGL((split::gemm_kernel<BM, BN, BK, AL, BL, EP>), dim3(g.blocks(), batch), dim3(THREADS), 0, s, al, bl,
+                       ep, K, g.k_per_split, g.tiles_m, g.tiles_n, g.fold());
+  else
+    hipLaunchKernelGGL((gemm::gemm_kernel<BM, BN, BK, AL, BL, EP>), dim3(g.blocks(), batch), dim3(THREADS), 0, s, al, bl, ep,
+                       K, g.k_per_split, g.tiles_m, g.tiles_n, g.fold());
   if (next_kernel_stop) (void)hipEventRecord(next_kernel_stop, s);
   next_kernel_start = next_kernel_stop = nullptr;
 }
@@ -1010,6 +1205,7 @@ struct ConvPlan {
                           // to a multiple of 4 (ragged segments); 0 when they are not used
   bool winograd = false;  // 3x3 / stride-1 layers: transformed-domain products (bm x bn is their tile)
   int wino_tile = 2;      // F(2x2, 3x3) or F(4x4, 3x3)
+  bool split = false;     // on the split engine (gemm_split.h)
 };
 
 // Pixels per image as the 16-byte loaders index a [image][channel][pixel] block: the
@@ -1060,8 +1256,9 @@ double predict_us(int M, int N, int K, int bm, int bn, int splits, bool wgrad, b
 // Fills p.bm / p.bn / p.splits with the cheapest candidate.  `may_split` is false
 // where the epilogue cannot write partial sums (scatter); grad-filter only has
 // the square tiles.
+// `traffic` given: for the split engine.
 double choose_tile_and_splits(ConvPlan &p, bool wgrad, bool padded, bool scatter, bool may_split,
-                              double out_bytes) {
+                              double out_bytes, const SplitTraffic *traffic = nullptr) {
   static const int tiles[3][2] = {{128, 128}, {64, 128}, {64, 64}};
   const size_t max_scratch = (size_t)512 << 20;
   double best = 1e30;
@@ -1079,6 +1276,9 @@ double choose_tile_and_splits(ConvPlan &p, bool wgrad, bool padded, bool scatter
         // aim at 1, 1.5, 2, 3, 4 and 6 workgroups per CU
         static const int per_cu_x2[] = {2, 3, 4, 6, 8, 12};
         for (int x : per_cu_x2) cand[n_cand++] = std::max(1, (num_cus() * x / 2 + n_tiles / 2) / n_tiles);
+        // so few tiles and so short a reduction that none of these is allowed below: as many splits as are
+        // (15 x 27 x 27, 49 -> 144 channels, 1x1 stride 2: 87 us unsplit)
+        if (traffic && p.K / 64 < cand[1]) cand[n_cand++] = std::max(1, p.K / 64);
       } else {
         static const int few[] = {2, 3, 4, 5, 6, 8, 10, 12};
         for (int x : few) cand[n_cand++] = x;
@@ -1087,7 +1287,8 @@ double choose_tile_and_splits(ConvPlan &p, bool wgrad, bool padded, bool scatter
     for (int i = 0; i < n_cand; ++i) {
       const int splits = cand[i];
       if (splits > 1 && (p.K / splits < 64 || (double)splits * out_bytes > (double)max_scratch)) continue;
-      const double us = predict_us(p.M, p.N, p.K, bm, bn, splits, wgrad, padded, scatter, out_bytes);
+      const double us = traffic ? predict_split_us(p.M, p.N, p.K, bm, bn, splits, stage_depth(bm, bn), *traffic)
+                                : predict_us(p.M, p.N, p.K, bm, bn, splits, wgrad, padded, scatter, out_bytes);
       if (us < best) {
         best = us;
         p.bm = bm;
@@ -1097,6 +1298,62 @@ double choose_tile_and_splits(ConvPlan &p, bool wgrad, bool padded, bool scatter
     }
   }
   return best;
+}
+
+// Whether a layer's direct forms may run on the split engine (gemm_split.h).  TINYFLOW_SPLIT in the environment forces
+// the choice (tests and measurements): 0 the fp32 engine, 1 the split engine wherever it has the loaders.
+//   * Fewer than 48 channels on either side leave most of a tile's rows or of its reduction empty, and the time is
+//     the gather's: 5x5, 6 -> 16 channels, 1 000 images 28 us on either.
+//   * 3x3 / stride-1 layers keep the fp32 engine whichever form the planner picks.  Their transformed-domain products
+//     are the form that counts, and networks of such layers under a batch-norm head (VGG-16 with dropout, Adam)
+//     turn any change of rounding into steps of Adam the other way: a different summation order of the fp32 engine
+//     alone moves their gradients by more than half their size.
+int forced_engine() {
+  const char *e = getenv("TINYFLOW_SPLIT");
+  return e && *e ? atoi(e) : -1;
+}
+bool may_use_split(const ConvDesc *d) {
+  const int forced = forced_engine();
+  if (forced >= 0) return forced != 0;
+  return !(d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1) && d->C >= 48 && d->K >= 48;
+}
+
+// Grad-filter's gathered x by vectors (SplitGatherAcross MODE 2 and 3): four outputs of one row at a time.
+bool vector_gather(const ConvDesc *d) { return d->pad_h == 0 && d->pad_w == 0 && d->Q % 4 == 0 && d->v <= 2; }
+
+// What the split engine's cost model wants to know of forward / grad-data / grad-filter (which = 0 / 1 / 2) with the
+// pixel operand fetched by vectors or gathered.
+SplitTraffic split_traffic(const ConvDesc *d, int which, bool vec) {
+  const int RS = d->R * d->S;
+  const double x = 4.0 * d->N * d->C * (RS == 1 ? (double)d->P * d->Q : (double)d->H * d->W);
+  const double y = 4.0 * d->N * d->K * (double)d->P * d->Q;
+  SplitTraffic t;
+  t.which = which;
+  t.in_bytes = which == 0 ? x : which == 1 ? y : x + y;
+  t.out_bytes = which == 0 ? y : which == 1 ? 4.0 * d->N * d->C * (double)d->H * d->W : 4.0 * d->K * d->C * RS;
+  t.gather = which != 2 ? (vec ? 1.0 : 1.4) : vec ? 1.04 : vector_gather(d) ? 1.2 : 1.82;
+  t.scatter = which == 1 && RS == 1 && (d->u > 1 || d->v > 1);
+  return t;
+}
+
+// The direct form on the engine, with the tile and splits, that the models give the least time.  `on_split`: the plan so
+// far for the split engine.  The fp32 model leaves out what every launch costs (4 us here) and underestimates large
+// ones by a seventh: with both corrected, over 300 layers of ResNet-50 at five sizes and random ones (48 - 512 channels,
+// 1x1 to 7x7), 0.86 of the fp32 engine's time in all, the choice within 3 % of the better one except where it keeps fp32.
+double choose_direct(ConvPlan &p, ConvPlan on_split, const ConvDesc *d, const SplitTraffic &traffic, bool wgrad, bool padded,
+                     bool scatter, bool may_split, double out_bytes) {
+  double us = choose_tile_and_splits(p, wgrad, padded, scatter, may_split, out_bytes);
+  // Not faster there (us, fp32 / split): grad-data of at most 64 rows 64 <- 256 channels 56 x 56, batch 64, 69 / 74; strided
+  // grad-filter whose x comes one element at a time 512 -> 1024 channels 28 x 28 stride 2, 130 / 142.
+  const bool slow = wgrad ? on_split.b_vec == false && d->v > 1 && !vector_gather(d) : traffic.which == 1 && p.M <= 64;
+  if (!may_use_split(d) || (slow && forced_engine() != 1)) return us;
+  on_split.split = true;
+  const double split_us = choose_tile_and_splits(on_split, wgrad, padded, scatter, may_split, out_bytes, &traffic);
+  if (split_us < 1.15 * us + 4.0 || forced_engine() == 1) {
+    p = on_split;
+    us = split_us;
+  }
+  return us;
 }
 
 // Geometry of the Winograd form of a 3x3 / stride-1 convolution (forward) or of its
@@ -1286,7 +1543,8 @@ ConvPlan plan_forward(const ConvDesc *d) {
             (int64_t)d->N * p.seg < (1ll << 31);
   if (p.b_vec) p.N = d->N * p.seg;  // columns in the loaders' (possibly padded) index space
   else p.seg = 0;
-  const double direct_us = choose_tile_and_splits(p, false, padded, false, true, 4.0 * p.M * d->N * d->P * d->Q);
+  const double direct_us = choose_direct(
+      p, p, d, split_traffic(d, 0, p.b_vec), false, padded, false, true, 4.0 * p.M * d->N * d->P * d->Q);
   p.variant = padded ? "fwd_pad" : "fwd_nopad";
   p.epilogue = "StoreNCHW";
   p.a_loader = p.a_vec ? "Across4" : "PlainAcross";
@@ -1366,13 +1624,13 @@ ConvPlan plan_dgrad(const ConvDesc *d) {
     p.a_vec = p.b_vec;
     if (p.b_vec) p.N = d->N * p.seg;
     else p.seg = 0;
-    choose_tile_and_splits(p, false, false, !dense, dense, 4.0 * p.M * d->N * d->H * d->W);
+    choose_direct(p, p, d, split_traffic(d, 1, p.b_vec), false, false, !dense, dense, 4.0 * p.M * d->N * d->H * d->W);
     p.variant = dense ? "dgrad_1x1" : "dgrad_1x1_scatter";
     if (!dense) p.epilogue = "StoreScatter";
   } else {
     p.N = d->N * d->H * d->W;
     if (d->u == 1 && d->v == 1) {
-      direct_us = choose_tile_and_splits(p, false, true, false, true, 4.0 * p.M * p.N);
+      direct_us = choose_direct(p, p, d, split_traffic(d, 1, false), false, true, false, true, 4.0 * p.M * p.N);
       p.variant = "dgrad_pad";
       p.b_mode = 1;
     } else if (dgrad_by_phases(d)) {
@@ -1397,6 +1655,7 @@ ConvPlan plan_dgrad(const ConvDesc *d) {
           p.bn = t[1];
         }
       }
+      p.split = may_use_split(d);
       p.variant = "dgrad_phases";
       p.epilogue = "StorePhase";
       p.b_mode = 1;
@@ -1430,12 +1689,18 @@ ConvPlan plan_wgrad(const ConvDesc *d) {
   p.a_vec = p.b_vec || PQ % 4 == 0;
   if (!p.b_vec) p.seg = p.a_vec ? PQ : 0;
   p.K = d->N * (p.seg ? p.seg : PQ);
-  const double direct_us = choose_tile_and_splits(p, true, padded, false, true, 4.0 * p.M * p.N);
+  ConvPlan other = p;  // on the split engine: whatever x is, dy's segments may be ragged
+  if (!p.b_vec) {
+    other.seg = vector_segment(PQ);
+    other.a_vec = other.seg != 0;
+    other.K = d->N * (other.seg ? other.seg : PQ);
+  }
+  const double direct_us = choose_direct(p, other, d, split_traffic(d, 2, p.b_vec), true, padded, false, true, 4.0 * p.M * p.N);
   p.variant = padded ? "wgrad_pad" : "wgrad_nopad";
   p.epilogue = "StoreRowMajor";
   p.a_loader = p.a_vec ? "Across4" : "DyAcross";
   p.b_loader = p.b_vec ? "Across4" : "GatherAcross";
-  p.b_mode = p.b_vec ? -1 : padded ? 1 : 0;
+  p.b_mode = p.b_vec ? -1 : padded ? 1 : p.split && vector_gather(d) ? 1 + d->v : 0;
   consider_winograd_wgrad(p, d, direct_us);
   return p;
 }
@@ -1664,7 +1929,7 @@ extern "C" int DLGpuConvolutionDescribeKernel(void ***list, int which, char *nam
   TF_REQUIRE(which >= 0 && which <= 2 && name && name_len > 0, "bad arguments");
   const ConvPlan p = which == 0 ? plan_forward(d) : which == 1 ? plan_dgrad(d) : plan_wgrad(d);
   // forward and the 1x1 grad-data run short reductions with 16-deep stages (run_depth)
-  const bool short_stages = !p.winograd && (which == 0 || (which == 1 && d->R * d->S == 1));
+  const bool short_stages = !p.winograd && !p.split && (which == 0 || (which == 1 && d->R * d->S == 1));
   const int bk = short_stages ? run_depth(p.bm, p.bn, p.K) : stage_depth(p.bm, p.bn);
   if (p.winograd) {
     // the batched product is the contraction kernel; its flop count is what it
@@ -1681,6 +1946,25 @@ extern "C" int DLGpuConvolutionDescribeKernel(void ***list, int which, char *nam
       wino_shape(d, which == 1, w, which == 2, p.wino_tile);
       *flops = 2.0 * w.positions * d->K * (double)d->C * w.T;
     }
+    return 0;
+  }
+  if (p.split) {
+    char a[48], b[48];
+    const bool phases = which == 1 && dgrad_by_phases(d);
+    const bool ragged = which == 2 ? p.seg != 0 && p.seg != d->P * d->Q : which == 0 && p.K % 4 != 0;
+    if (which == 1)
+      snprintf(a, sizeof a, phases ? "PhasedFilter<SplitAlong4<%d, %d>>" : "SplitAlong4<%d, %d>", p.bm, bk);
+    else if (which == 2 && !p.a_vec)
+      snprintf(a, sizeof a, "SplitDyAcross<%d, %d>", p.bm, bk);
+    else
+      snprintf(a, sizeof a, "SplitAcross4<%d, %d, %s, %s>", p.bm, bk, ragged ? "true" : "false", which == 2 ? "true" : "false");
+    if (phases) snprintf(b, sizeof b, "SplitPhasedGather<%d, %d>", p.bn, bk);
+    else if (p.b_vec && which == 2) snprintf(b, sizeof b, "SplitAcross4<%d, %d, %s, true>", p.bn, bk, ragged ? "true" : "false");
+    else if (p.b_vec) snprintf(b, sizeof b, "SplitAlong4<%d, %d>", p.bn, bk);
+    else snprintf(b, sizeof b, "%s<%d, %d, %d>", which == 2 ? "SplitGatherAcross" : "SplitGatherAlong", p.bn, bk, p.b_mode);
+    snprintf(name, (size_t)name_len, "%s %dx%d s%d | gemm_kernel<%d, %d, %d, %s, %s, %s>", p.variant, p.bm, p.bn, p.splits,
+             p.bm, p.bn, bk, a, b, p.epilogue);
+    if (flops) *flops = 2.0 * d->N * d->K * d->C * d->R * d->S * (double)d->P * d->Q;
     return 0;
   }
   if (which == 1 && dgrad_by_phases(d)) {
@@ -1800,7 +2084,7 @@ extern "C" int DLGpuConvolution2DForward(const DLArrayHandle input, const DLArra
   const int PQ = d->P * d->Q;
   // (a plan with ragged segments counts its columns in the padded index space, so it
   // keeps the 16-byte loaders whatever the alignment: they only need 4 bytes)
-  const bool aligned = (vec4_ok(filter->data, 0) && vec4_ok(input->data, 0)) || (plan.seg != 0 && plan.seg != PQ);
+  const bool aligned = plan.split || (vec4_ok(filter->data, 0) && vec4_ok(input->data, 0)) || (plan.seg != 0 && plan.seg != PQ);
   const bool a_vec = plan.a_vec && aligned, b_vec = plan.b_vec && aligned;
   const uint32_t w_bytes = (uint32_t)(numel(filter) * 4), x_bytes = (uint32_t)(numel(input) * 4);
   with_tile(bm, bn, [&](auto bm_c, auto bn_c, auto bk_c) {
@@ -1808,6 +2092,27 @@ extern "C" int DLGpuConvolution2DForward(const DLArrayHandle input, const DLArra
     // with the 16-byte loader the columns are (image, pixel) in its segment index space
     const int seg = b_vec ? plan.seg : PQ;
     StoreNCHW ep{partial ? partial : (float *)output->data, M, N, FastDiv((uint32_t)seg), PQ, numel(output)};
+    if (plan.split) {
+      auto with_a = [&](const auto &al) {
+        if (b_vec) {
+          launch<BM, BN, BK>(al, split::SplitAlong4<BN, BK>{(const float *)input->data, x_bytes, PQ, N, K,
+                                                            FastDiv((uint32_t)seg), d->C * PQ}, ep, K, g, s);
+          return;
+        }
+        auto run = [&](auto mode_c) {
+          SplitGatherAlong<BN, BK, decltype(mode_c)::value> bl{
+              (const float *)input->data, x_bytes, K, N, FastDiv((uint32_t)(d->R * d->S)), FastDiv((uint32_t)d->S),
+              d->H * d->W, FastDiv((uint32_t)PQ), FastDiv((uint32_t)d->Q), d->C * d->H * d->W, d->H, d->W, d->u, d->v,
+              -d->pad_h, -d->pad_w, 1, d->R, d->S, FastDiv(1), FastDiv(1)};
+          launch<BM, BN, BK>(al, bl, ep, K, g, s);
+        };
+        if (padded) run(IC<1>{}); else run(IC<0>{});
+      };
+      const float *w = (const float *)filter->data;
+      if (K % 4 == 0) with_a(split::SplitAcross4<BM, BK>{w, w_bytes, K, M, K, FastDiv(ONE_SEGMENT), 0});
+      else with_a(split::SplitAcross4<BM, BK, true>{w, w_bytes, K, M, K, FastDiv(ONE_SEGMENT), 0, K});
+      return;
+    }
     auto with_b = [&](const auto &al, auto a_is_vec) {
       if constexpr (decltype(a_is_vec)::value) {  // a vectorised input only comes with a vectorised filter
         if (b_vec) {
@@ -1832,7 +2137,7 @@ extern "C" int DLGpuConvolution2DForward(const DLArrayHandle input, const DLArra
              std::true_type{});
     else
       with_b(PlainAcross<BM, BK>{(const float *)filter->data, w_bytes, K, M, K}, std::false_type{});
-  }, run_depth(bm, bn, K));
+  }, plan.split ? stage_depth(bm, bn) : run_depth(bm, bn, K));
   if (partial) {
     launch_split_sum(partial, (float *)output->data, numel(output), g.splits, s);
     device_free(partial);
@@ -1857,6 +2162,15 @@ static void run_dgrad_phases(const ConvDesc *d, const ConvPlan &plan, const floa
                                          d->K * PQ, d->P, d->Q, 1, 1, 0, 0, -1, 0, 0, FastDiv(1), FastDiv(1)},
                                   phases};
     const StorePhase ep{dx, dx_bytes, plan.M, d->H, d->W, d->u, d->v, phases};
+    if (plan.split) {
+      using SplitGather = SplitGatherAlong<BN, BK, 1>;
+      const SplitPhasedGather<BN, BK> sbl{{SplitGather{dy, dy_bytes, 0, 0, FastDiv(1), FastDiv(1), PQ, FastDiv(1), FastDiv(1),
+                                                       d->K * PQ, d->P, d->Q, 1, 1, 0, 0, -1, 0, 0, FastDiv(1), FastDiv(1)},
+                                           phases}};
+      const PhasedFilter<split::SplitAlong4<BM, BK>> al{{wt, w_bytes, d->C, plan.M, plan.K, FastDiv(ONE_SEGMENT), 0}, phases};
+      launch<BM, BN, BK>(al, sbl, ep, plan.K, g, s, d->u * d->v);
+      return;
+    }
     auto go = [&](const auto &filter) { launch<BM, BN, BK>(filter, bl, ep, plan.K, g, s, d->u * d->v); };
     if (plan.a_vec)
       go(PhasedFilter<Along4<BM, BK>>{{wt, w_bytes, d->C, plan.M, plan.K, FastDiv(ONE_SEGMENT), 0}, phases});
@@ -1949,7 +2263,7 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
   const int64_t dx_count = numel(dinput);
 
   // (a plan with ragged segments keeps the 16-byte loaders whatever the alignment)
-  const bool aligned = (vec4_ok(wt, 0) && vec4_ok(doutput->data, 0)) || (plan.seg != 0 && plan.seg != PQ);
+  const bool aligned = plan.split || (vec4_ok(wt, 0) && vec4_ok(doutput->data, 0)) || (plan.seg != 0 && plan.seg != PQ);
   const bool a_vec = plan.a_vec && aligned, b_vec = plan.b_vec && aligned;
   const FastDiv whole(ONE_SEGMENT);
   if (RS == 1) {
@@ -1972,7 +2286,16 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
           launch<BM, BN, BK>(al, bl, ep, K, g, s);
         }
       };
-      if (a_vec && b_vec) {
+      if (plan.split) {
+        const split::SplitAlong4<BM, BK> al{wt, w_bytes, d->C, M, K, whole, 0};
+        if (b_vec)
+          with_epilogue(al, split::SplitAlong4<BN, BK>{(const float *)doutput->data, dy_bytes, PQ, N, K,
+                                                       FastDiv((uint32_t)seg), d->K * PQ});
+        else
+          with_epilogue(al, SplitGatherAlong<BN, BK, 0>{
+              (const float *)doutput->data, dy_bytes, K, N, FastDiv(1), FastDiv(1), PQ, FastDiv((uint32_t)PQ),
+              FastDiv((uint32_t)d->Q), d->K * PQ, d->P, d->Q, 1, 1, 0, 0, -1, 1, 1, FastDiv(1), FastDiv(1)});
+      } else if (a_vec && b_vec) {
         with_epilogue(Along4<BM, BK>{wt, w_bytes, d->C, M, K, whole, 0},
                       Along4<BN, BK>{(const float *)doutput->data, dy_bytes, PQ, N, K, FastDiv((uint32_t)seg),
                                      d->K * PQ});
@@ -1982,7 +2305,7 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
                                              PQ, FastDiv((uint32_t)PQ), FastDiv((uint32_t)d->Q), d->K * PQ, d->P,
                                              d->Q, 1, 1, 0, 0, -1, 1, 1, FastDiv(1), FastDiv(1)});
       }
-    }, run_depth(bm, bn, K));
+    }, plan.split ? stage_depth(bm, bn) : run_depth(bm, bn, K));
   } else {
     const int N = plan.N;
     const int HW = d->H * d->W;
@@ -1995,7 +2318,13 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
                               FastDiv((uint32_t)d->S), PQ,
                               FastDiv((uint32_t)HW), FastDiv((uint32_t)d->W), d->K * PQ, d->P, d->Q,
                               1, 1, d->pad_h, d->pad_w, -1, d->R, d->S, FastDiv(1), FastDiv(1)};
-        if (a_vec) launch<BM, BN, BK>(Along4<BM, BK>{wt, w_bytes, d->C, M, K, whole, 0}, bl, ep, K, g, s);
+        if (plan.split) {
+          SplitGatherAlong<BN, BK, 1> sbl{(const float *)doutput->data, dy_bytes, K, N, FastDiv((uint32_t)RS),
+                                          FastDiv((uint32_t)d->S), PQ, FastDiv((uint32_t)HW), FastDiv((uint32_t)d->W),
+                                          d->K * PQ, d->P, d->Q, 1, 1, d->pad_h, d->pad_w, -1, d->R, d->S, FastDiv(1),
+                                          FastDiv(1)};
+          launch<BM, BN, BK>(split::SplitAlong4<BM, BK>{wt, w_bytes, d->C, M, K, whole, 0}, sbl, ep, K, g, s);
+        } else if (a_vec) launch<BM, BN, BK>(Along4<BM, BK>{wt, w_bytes, d->C, M, K, whole, 0}, bl, ep, K, g, s);
         else launch<BM, BN, BK>(PlainAlong<BM, BK>{wt, w_bytes, d->C, M, K}, bl, ep, K, g, s);
       });
     } else {
@@ -2062,13 +2391,52 @@ extern "C" int DLGpuConvolutionBackwardFilter(const DLArrayHandle input, const D
   }
   const bool padded = d->pad_h != 0 || d->pad_w != 0;
   const bool ragged = plan.seg != 0 && plan.seg != PQ;  // both operands in the padded reduction index
-  const bool aligned = (vec4_ok(doutput->data, 0) && vec4_ok(input->data, 0)) || ragged;
+  const bool aligned = plan.split || (vec4_ok(doutput->data, 0) && vec4_ok(input->data, 0)) || ragged;
   const bool a_vec = plan.a_vec && aligned, b_vec = plan.b_vec && aligned;
   const uint32_t dy_bytes = (uint32_t)(numel(doutput) * 4), x_bytes = (uint32_t)(numel(input) * 4);
   with_tile(bm, bn, [&](auto bm_c, auto bn_c, auto bk_c) {
     constexpr int BM = decltype(bm_c)::value, BN = decltype(bn_c)::value, BK = decltype(bk_c)::value;
     if constexpr (BM == BN) {  // only the square tiles are used for grad-filter
       StoreRowMajor ep{dst, N, M, N, (int64_t)M * N};
+      if (plan.split) {
+        const float *x = (const float *)input->data, *dy = (const float *)doutput->data;
+        const FastDiv div_seg((uint32_t)(plan.seg ? plan.seg : PQ));
+        if (ragged && b_vec) {
+          split::SplitAcross4<BM, BK, true, true> al{dy, dy_bytes, PQ, M, K, div_seg, d->K * PQ, PQ};
+          split::SplitAcross4<BN, BK, true, true> bl{x, x_bytes, PQ, N, K, div_seg, d->C * PQ, PQ};
+          launch<BM, BN, BK>(al, bl, ep, K, g, s);
+          return;
+        }
+        const split::SplitAcross4<BM, BK, false, true> al{dy, dy_bytes, PQ, M, K, div_seg, d->K * PQ};
+        if (b_vec) {
+          launch<BM, BN, BK>(al, split::SplitAcross4<BN, BK, false, true>{x, x_bytes, PQ, N, K, div_seg, d->C * PQ}, ep, K, g, s);
+          return;
+        }
+        auto run = [&](auto mode_c) {
+          SplitGatherAcross<BN, BK, decltype(mode_c)::value> bl{
+              x, x_bytes, K, N, div_seg, FastDiv((uint32_t)d->Q), FastDiv((uint32_t)RS), FastDiv((uint32_t)d->S),
+              d->C * d->H * d->W, d->H * d->W, d->H, d->W, d->P, d->u, d->v, d->pad_h, d->pad_w,
+              plan.seg && plan.seg != PQ ? (uint32_t)PQ : ~0u};
+          if constexpr (decltype(mode_c)::value < 2) {  // rows of a multiple of four are whole vectors of dy, too
+            if (ragged) {
+              launch<BM, BN, BK>(split::SplitAcross4<BM, BK, true, true>{dy, dy_bytes, PQ, M, K, div_seg, d->K * PQ, PQ}, bl,
+                                 ep, K, g, s);
+              return;
+            }
+            if (!a_vec) {
+              launch<BM, BN, BK>(SplitDyAcross<BM, BK>{dy, dy_bytes, K, M, FastDiv((uint32_t)PQ), d->K * PQ, PQ}, bl, ep, K, g, s);
+              return;
+            }
+          }
+          launch<BM, BN, BK>(al, bl, ep, K, g, s);
+        };
+        const int mode = plan.b_mode;
+        if (mode == 1) run(IC<1>{});
+        else if (mode == 2) run(IC<2>{});
+        else if (mode == 3) run(IC<3>{});
+        else run(IC<0>{});
+        return;
+      }
       if (ragged) {  // 1x1, stride 1, pixels per image not a multiple of 4: masked 16-byte loads on both sides
         const FastDiv div_seg((uint32_t)plan.seg);
         Across4<BM, BK, true> al{(const float *)doutput->data, dy_bytes, PQ, M, K, div_seg, d->K * PQ, PQ};

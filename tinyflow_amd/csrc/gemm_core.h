@@ -368,6 +368,138 @@ struct ProblemExtent<L, std::void_t<decltype(&L::problem_k_extent)>> {
   static __device__ inline int of(const L &loader, int) { return loader.problem_k_extent(); }
 };
 
+// Which tile a workgroup owns and which part of the reduction (all of this is scalar arithmetic).
+struct TileWork {
+  bool folded;
+  int tile, split, k_begin, k_end, fold_tile, piece;
+};
+template <class BLoader>
+__device__ inline TileWork tile_work(const BLoader &bl, int k_extent, int k_per_split, int tiles, const Fold &fold) {
+  TileWork w;
+  const bool folding = fold.pieces > 1;
+  w.folded = folding && (int)blockIdx.x >= fold.plain_blocks;
+  w.fold_tile = w.piece = 0;
+  if (!w.folded) {
+    const int plain_tiles = folding ? fold.first_tile : tiles;
+    const int logical = xcd_contiguous((int)blockIdx.x, folding ? fold.plain_blocks : (int)gridDim.x);
+    w.tile = logical % plain_tiles;
+    w.split = logical / plain_tiles;
+    w.k_begin = w.split * k_per_split;
+    w.k_end = w.k_begin + k_per_split;
+  } else {
+    const int fold_tiles = tiles - fold.first_tile;
+    const int logical = xcd_contiguous((int)blockIdx.x - fold.plain_blocks, (int)gridDim.x - fold.plain_blocks);
+    w.fold_tile = logical % fold_tiles;
+    w.piece = logical / fold_tiles;
+    w.tile = fold.first_tile + w.fold_tile;
+    w.split = 0;
+    w.k_begin = w.piece * fold.k_per_piece;
+    w.k_end = w.k_begin + fold.k_per_piece;
+  }
+  const int own_extent = ProblemExtent<BLoader>::of(bl, k_extent);
+  if (w.k_end > own_extent) w.k_end = own_extent;
+  return w;
+}
+
+// Writes a finished tile, or adds it to the other pieces of its tile (see Fold).  (m_wave, n_wave): first row and
+// column of this wave's accumulators; `is_last`: a word of LDS that nobody reads any more.
+// PAIRS: the pieces are added two by two, with both in flight.
+template <int BM, int BN, bool PAIRS, int TM, int TN, class Epilogue>
+__device__ inline void write_tile(const f32x16 (&acc)[TM][TN], const Epilogue &ep, const TileWork &w, int tiles,
+                                  const Fold &fold, int m_wave, int n_wave, int tid, unsigned &is_last) {
+  const int lane = tid & 63, lrow = lane >> 5, lcol = lane & 31;
+  if (w.folded) {  // uniform over the workgroup
+    // The pieces travel through scratch with device-scope ("sc1") stores and loads:
+    // such an access is coherent across the XCDs' L2s by itself, so no cache-wide
+    // write-back or invalidate is needed (a __threadfence() here costs exactly that
+    // and slows every workgroup of the XCD down).  Ordering: all stores of the piece
+    // have been acknowledged (s_waitcnt 0) before the barrier that precedes the ticket.
+    constexpr int SC1 = 16;  // device scope in the cache-policy operand of the buffer instructions
+    const int fold_tiles = tiles - fold.first_tile;
+    const size_t slot = (size_t)blockIdx.y * fold_tiles + w.fold_tile;
+    constexpr uint32_t kPieceBytes = (uint32_t)(BM * BN) * 4u;
+    const __amdgpu_buffer_rsrc_t pieces_of_tile =
+        make_rsrc(fold.scratch + slot * fold.pieces * (size_t)(BM * BN), (uint32_t)fold.pieces * kPieceBytes);
+    const uint32_t lane_off = (uint32_t)tid * 16u;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4v v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+          __builtin_amdgcn_raw_buffer_store_b128(
+              __builtin_bit_cast(__attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned, v), pieces_of_tile,
+              (int)((uint32_t)w.piece * kPieceBytes + (uint32_t)((i * TN + j) * 4 + q) * (THREADS * 16u) + lane_off), 0,
+              SC1);
+        }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (tid == 0) is_last = atomicAdd(fold.tickets + slot, 1u) == (unsigned)(fold.pieces - 1);
+    __syncthreads();
+    if (!is_last) return;
+    // Last piece of the tile: add the pieces in piece order, four accumulator
+    // registers at a time (the sums go straight to the epilogue, so the fold needs
+    // no registers beyond the loads in flight), and clear the ticket.
+    typename Epilogue::State sf;
+    ep.template init<TN>(sf, n_wave, lane, 0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        f32x4v sum[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sum[q] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        auto fetch = [&](int p, f32x4v (&part)[4]) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            part[q] = __builtin_bit_cast(
+                f32x4v, __builtin_amdgcn_raw_buffer_load_b128(
+                            pieces_of_tile,
+                            (int)((uint32_t)p * kPieceBytes + (uint32_t)((i * TN + j) * 4 + q) * (THREADS * 16u) + lane_off),
+                            0, SC1));
+        };
+        int p = 0;
+        if constexpr (PAIRS) {
+          for (; p + 1 < fold.pieces; p += 2) {
+            f32x4v one[4], two[4];
+            fetch(p, one);
+            fetch(p + 1, two);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sum[q] += one[q] + two[q];
+          }
+        }
+        for (; p < fold.pieces; ++p) {
+          f32x4v part[4];
+          fetch(p, part);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sum[q] += part[q];
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int m = m_wave + 32 * i + 8 * (v >> 2) + 4 * lrow + (v & 3);
+          const int n = n_wave + 32 * j + lcol;
+          ep.store(sf, m, n, j, sum[v >> 2][v & 3]);
+        }
+      }
+    if (tid == 0) fold.tickets[slot] = 0u;  // ready for the next launch on this stream
+    return;
+  }
+
+  typename Epilogue::State se;
+  ep.template init<TN>(se, n_wave, lane, w.split);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = m_wave + 32 * i + 8 * (v >> 2) + 4 * lrow + (v & 3);
+        const int n = n_wave + 32 * j + lcol;
+        ep.store(se, m, n, j, acc[i][j][v]);
+      }
+}
+
 // ---- the kernel ----------------------------------------------------------------------
 // Work decomposition: gridDim.x = tiles_m * tiles_n * splits (plus, with a fold, the
 // pieces of the folded tiles behind the plain workgroups).  Hardware hands
@@ -406,32 +538,10 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(const ALoader al, const B
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WAVES_M, wn = wave / WAVES_M;
 
-  // which tile, and which part of the reduction (all of this is scalar arithmetic)
   const int tiles = tiles_m * tiles_n;
-  const bool folding = fold.pieces > 1;
-  const bool folded = folding && (int)blockIdx.x >= fold.plain_blocks;
-  int tile, split, k_begin, k_end, fold_tile = 0, piece = 0;
-  if (!folded) {
-    const int plain_tiles = folding ? fold.first_tile : tiles;
-    const int logical = xcd_contiguous((int)blockIdx.x, folding ? fold.plain_blocks : (int)gridDim.x);
-    tile = logical % plain_tiles;
-    split = logical / plain_tiles;
-    k_begin = split * k_per_split;
-    k_end = k_begin + k_per_split;
-  } else {
-    const int fold_tiles = tiles - fold.first_tile;
-    const int logical = xcd_contiguous((int)blockIdx.x - fold.plain_blocks, (int)gridDim.x - fold.plain_blocks);
-    fold_tile = logical % fold_tiles;
-    piece = logical / fold_tiles;
-    tile = fold.first_tile + fold_tile;
-    split = 0;
-    k_begin = piece * fold.k_per_piece;
-    k_end = k_begin + fold.k_per_piece;
-  }
-  const int own_extent = ProblemExtent<BLoader>::of(bl, k_extent);
-  if (k_end > own_extent) k_end = own_extent;
-  const int tm = tile % tiles_m, tn = tile / tiles_m;
-  const int m0 = tm * BM, n0 = tn * BN;
+  const TileWork work = tile_work(bl, k_extent, k_per_split, tiles, fold);
+  const int k_begin = work.k_begin, k_end = work.k_end;
+  const int m0 = work.tile % tiles_m * BM, n0 = work.tile / tiles_m * BN;
 
   typename ALoader::State sa;
   typename BLoader::State sb;
@@ -547,88 +657,12 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(const ALoader al, const B
     buf ^= 1;
   }
 
-  if (folded) {  // uniform over the workgroup
-    // The pieces travel through scratch with device-scope ("sc1") stores and loads:
-    // such an access is coherent across the XCDs' L2s by itself, so no cache-wide
-    // write-back or invalidate is needed (a __threadfence() here costs exactly that
-    // and slows every workgroup of the XCD down).  Ordering: all stores of the piece
-    // have been acknowledged (s_waitcnt 0) before the barrier that precedes the ticket.
-    constexpr int SC1 = 16;  // device scope in the cache-policy operand of the buffer instructions
-    // the flag lives in the first word of the A planes, which nobody reads any more (every
-    // wave has passed the barrier that ended the reduction loop): the two 128 x 128 planes
-    // of [m][k] operands fill a quarter of a CU's LDS to the byte, and four workgroups
-    // per CU are what the kernel is tuned for
-    unsigned &is_last = *reinterpret_cast<unsigned *>(&As[0][0][0]);
-    const int fold_tiles = tiles - fold.first_tile;
-    const size_t slot = (size_t)blockIdx.y * fold_tiles + fold_tile;
-    constexpr uint32_t kPieceBytes = (uint32_t)(BM * BN) * 4u;
-    const __amdgpu_buffer_rsrc_t pieces_of_tile =
-        make_rsrc(fold.scratch + slot * fold.pieces * (size_t)(BM * BN), (uint32_t)fold.pieces * kPieceBytes);
-    const uint32_t lane_off = (uint32_t)tid * 16u;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4v v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-          __builtin_amdgcn_raw_buffer_store_b128(
-              __builtin_bit_cast(__attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned, v), pieces_of_tile,
-              (int)((uint32_t)piece * kPieceBytes + (uint32_t)((i * TN + j) * 4 + q) * (THREADS * 16u) + lane_off), 0,
-              SC1);
-        }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (tid == 0) is_last = atomicAdd(fold.tickets + slot, 1u) == (unsigned)(fold.pieces - 1);
-    __syncthreads();
-    if (!is_last) return;
-    // Last piece of the tile: add the pieces in piece order, four accumulator
-    // registers at a time (the sums go straight to the epilogue, so the fold needs
-    // no registers beyond the loads in flight), and clear the ticket.
-    typename Epilogue::State sf;
-    ep.template init<TN>(sf, n0 + wn * WN, lane, 0);
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        f32x4v sum[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sum[q] = f32x4v{0.f, 0.f, 0.f, 0.f};
-        for (int p = 0; p < fold.pieces; ++p) {
-          f32x4v part[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            part[q] = __builtin_bit_cast(
-                f32x4v, __builtin_amdgcn_raw_buffer_load_b128(
-                            pieces_of_tile,
-                            (int)((uint32_t)p * kPieceBytes + (uint32_t)((i * TN + j) * 4 + q) * (THREADS * 16u) + lane_off),
-                            0, SC1));
-#pragma unroll
-          for (int q = 0; q < 4; ++q) sum[q] += part[q];
-        }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = m0 + wm * WM + 32 * i + 8 * (v >> 2) + 4 * lrow + (v & 3);
-          const int n = n0 + wn * WN + 32 * j + lcol;
-          ep.store(sf, m, n, j, sum[v >> 2][v & 3]);
-        }
-      }
-    if (tid == 0) fold.tickets[slot] = 0u;  // ready for the next launch on this stream
-    return;
-  }
-
-  typename Epilogue::State se;
-  ep.template init<TN>(se, n0 + wn * WN, lane, split);
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = m0 + wm * WM + 32 * i + 8 * (v >> 2) + 4 * lrow + (v & 3);
-        const int n = n0 + wn * WN + 32 * j + lcol;
-        ep.store(se, m, n, j, acc[i][j][v]);
-      }
+  // the fold's flag lives in the first word of the A planes, which nobody reads any more (every
+  // wave has passed the barrier that ended the reduction loop): the two 128 x 128 planes
+  // of [m][k] operands fill a quarter of a CU's LDS to the byte, and four workgroups
+  // per CU are what the kernel is tuned for
+  write_tile<BM, BN, false>(acc, ep, work, tiles, fold, m0 + wm * WM, n0 + wn * WN, tid,
+                     *reinterpret_cast<unsigned *>(&As[0][0][0]));
 }
 
 // Host-side launch geometry shared by the users.

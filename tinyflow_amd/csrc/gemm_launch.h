@@ -35,8 +35,8 @@ constexpr int kMaxTailPieces = 8;      // 4, 8 and 16 measured the same
 //     floor(CUs / R) pieces along the reduction, about one short piece per CU,
 //     instead of R whole tiles that keep R CUs busy while the rest idle.
 // Depends on the shape and the CU count only, so a layer always gets the same
-// summation order.  `tail_ok` = false keeps the remainder round as it is.
-inline void plan_fold(Geometry &g, int K, int BK, int batch, bool tail_ok = true) {
+// summation order.
+inline void plan_fold(Geometry &g, int K, int BK, int batch) {
   const int mode = fold_switch();
   const int tiles = g.tiles();
   const int k_steps = (K + BK - 1) / BK;
@@ -48,7 +48,7 @@ inline void plan_fold(Geometry &g, int K, int BK, int batch, bool tail_ok = true
     g.splits = 1;
     return;
   }
-  if (!(mode & 2) || !tail_ok || batch != 1) return;
+  if (!(mode & 2) || batch != 1) return;
   const int cus = num_cus();
   if (tiles <= cus) return;
   const int rest = tiles % cus;
@@ -88,6 +88,39 @@ inline int acquire_fold(Geometry &g, int bm, int bn, int batch, hipStream_t s, F
 inline void release_fold(FoldBuffers &fb) {
   if (fb.scratch) device_free(fb.scratch);  // stream-ordered reuse: later users are enqueued behind the kernel
   fb.scratch = nullptr;
+}
+
+// ---- cost model of the split engine (gemm_split.h) ------------------------------------------
+struct SplitTraffic {
+  int which = 0;                         // 0 forward or a plain product, 1 grad-data, 2 grad-filter
+  double in_bytes = 0, out_bytes = 0;    // the operand that is not a filter, and the result
+  double gather = 1.0;                   // time of a reduction step next to that of one fetched by vectors
+  bool scatter = false;                  // the result goes to every u-th row and v-th column, zeros between
+};
+
+// Microseconds, fitted to sweeps of every tile and split over 300 layers (ResNet-50 at batch 8 to 128 and 64 to 224
+// pixels, random ones of 48 - 512 channels and 1x1 to 7x7 filters): rms error 11 %, its picks within 1.1 % of the
+// sweeps' best on average.
+//   workgroup time   = a(tile) * gather * (k per split + o(tile)); a tile's start and end cost as much as 70 - 80 steps
+//   rounds           = workgroups / CUs, rounded up three quarters of the way
+//   latency hiding   = a CU that only ever holds 1 / 2 workgroups runs them at 0.73 / 0.92 of the rate
+//   bytes            = nothing runs faster than 5.6 TB/s over operand and result, and 5.8 us a launch
+//   split-sum pass   = 7.75 TB/s over the partial results, folds in the kernel 3.8 TB/s
+inline double predict_split_us(int M, int N, int K, int bm, int bn, int splits, int stage, const SplitTraffic &t) {
+  const Geometry g = make_geometry(M, N, K, bm, bn, splits, stage);
+  const double a = bm == 128 ? 0.0316 : bn == 128 ? 0.0223 : 0.0126;
+  const double o = bm == 128 ? 69.0 : bn == 128 ? 70.0 : 81.0;
+  const double per_cu = (double)g.blocks() / num_cus();
+  const double whole = std::ceil(per_cu);
+  const double rounds = per_cu <= 1.0 ? 1.0 : std::min(whole, per_cu + 0.75);
+  const double hiding = whole <= 1 ? 0.725 : whole <= 2 ? 0.918 : 1.0;
+  const bool second_pass = g.splits > kMaxFoldedSplits;
+  double us = rounds * a * t.gather * (g.k_per_split + o) / hiding;
+  us = std::max(us, (t.out_bytes * (second_pass ? g.splits : 1) + t.in_bytes) / 5.6e6) + 5.8;
+  if (second_pass) us += (2.0 * g.splits + 1.0) * t.out_bytes / 7.75e6 + 0.8;
+  else if (g.splits > 1) us += (g.splits + 1.0) * t.out_bytes / 3.8e6;
+  if (t.scatter) us += t.out_bytes / 14.9e6;
+  return us;
 }
 
 }  // namespace gemm

@@ -11,6 +11,7 @@
 // fixed-order pass adds up, so results do not depend on scheduling.
 #include "gemm_core.h"
 #include "gemm_launch.h"
+#include "gemm_split.h"
 #include "internal.h"
 
 using namespace tf;
@@ -18,6 +19,8 @@ using namespace tf::gemm;
 
 namespace {
 
+template <int V>
+using IC = std::integral_constant<int, V>;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // out[i] = sum_s partial[s * count + i] for 16-byte aligned data with count % 4 == 0, with the
@@ -139,6 +142,26 @@ void dispatch(const float *A, bool tA, int lda, uint32_t a_bytes, const float *B
   }
 }
 
+template <int BM, int BN, int BK, bool RAGGED>
+void dispatch_split(const float *A, bool tA, int lda, uint32_t a_bytes, const float *B, bool tB, int ldb,
+                    uint32_t b_bytes, const StoreRowMajor &ep, int M, int N, int K, const Geometry &g, hipStream_t s) {
+  const FastDiv whole(ONE_SEGMENT);
+  auto go = [&](const auto &al, const auto &bl) {
+    using AL = std::decay_t<decltype(al)>;
+    using BL = std::decay_t<decltype(bl)>;
+    hipLaunchKernelGGL((split::gemm_kernel<BM, BN, BK, AL, BL, StoreRowMajor>), dim3(g.blocks()), dim3(THREADS), 0, s, al,
+                       bl, ep, K, g.k_per_split, g.tiles_m, g.tiles_n, g.fold());
+  };
+  const split::SplitAcross4<BM, BK, RAGGED> a_across{A, a_bytes, lda, M, K, whole, 0, K};
+  const split::SplitAcross4<BN, BK, RAGGED> b_across{B, b_bytes, ldb, N, K, whole, 0, K};
+  const split::SplitAlong4<BM, BK> a_along{A, a_bytes, lda, M, K, whole, 0};
+  const split::SplitAlong4<BN, BK> b_along{B, b_bytes, ldb, N, K, whole, 0};
+  if (!tA && !tB) go(a_across, b_along);
+  else if (tA && !tB) go(a_along, b_along);
+  else if (!tA && tB) go(a_across, b_across);
+  else go(a_along, b_across);
+}
+
 }  // namespace
 
 namespace tf {
@@ -183,7 +206,20 @@ struct Plan {
   int tile, splits;  // square tile that the reduction is planned for, k-splits asked for
   Geometry g;        // of that tile
   bool flat;         // launched on 32 x 128 tiles
+  bool split;        // on the split engine (gemm_split.h)
 };
+
+// Products of more than 256 rows, columns and reduction steps run on the split engine (1000 x 1537 x 777 and both its
+// gradients 117 us on the fp32 engine, 4096^3 1000 against 670).  With fewer of one the time is mostly that of
+// streaming the largest operand or of the launch (256 x 256 x 12544: 22 against 21 us, 128 x 784 x 256 11.5 against 10),
+// and products with one extent the batch are the classifiers under a batch-norm head whose steps take no other rounding
+// (see may_use_split in conv.hip).  TINYFLOW_SPLIT=0 / 1 forces the fp32 / the split engine.
+bool product_on_split(int M, int N, int K) {
+  const char *e = getenv("TINYFLOW_SPLIT");
+  if (e && *e) return atoi(e) != 0;
+  return M > 256 && N > 256 && K > 256;
+}
+constexpr int split_stage(int tile) { return tile == 128 ? 16 : 32; }
 
 // Two 64 x 64 tiles of at most 32 rows side by side are one 32 x 128 tile, with as many floats to fold.  Every
 // output element keeps the pieces of the reduction that it has on the 64 x 64 tiles and the order in which they
@@ -195,6 +231,29 @@ void to_flat_tiles(Geometry &g, int N) {
 
 Plan plan_product(int M, int N, int K, bool vec) {
   Plan p;
+  p.split = product_on_split(M, N, K);
+  if (p.split) {
+    SplitTraffic t;
+    t.in_bytes = 4.0 * ((double)M * K + (double)K * N);
+    t.out_bytes = 4.0 * (double)M * N;
+    double best = 1e30;
+    for (int tile : {128, 64}) {
+      if (tile == 128 && (M <= 64 || N <= 64)) continue;
+      for (int splits : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        if (splits > 1 && K / splits < 64) break;
+        const double us = predict_split_us(M, N, K, tile, tile, splits, split_stage(tile), t);
+        if (us < best) {
+          best = us;
+          p.tile = tile;
+          p.splits = splits;
+        }
+      }
+    }
+    p.g = make_geometry(M, N, K, p.tile, p.tile, p.splits, split_stage(p.tile));
+    plan_fold(p.g, K, split_stage(p.tile), 1);
+    p.flat = false;
+    return p;
+  }
   p.tile = M > 64 && N > 64 && cdiv(M, 128) * cdiv(N, 128) >= num_cus() ? 128 : 64;
   p.splits = choose_splits(cdiv(M, p.tile) * cdiv(N, p.tile), K, 256);
   p.g = make_geometry(M, N, K, p.tile, p.tile, p.splits);
@@ -252,7 +311,7 @@ extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, co
   FoldBuffers fb;
   if (acquire_fold(g, plan.tile, plan.tile, 1, s, fb) != 0) {  // no scratch (this entry point cannot report it): no fold
     release_fold(fb);
-    g = make_geometry((int)M, (int)N, (int)K, plan.tile, plan.tile, plan.splits);
+    g = make_geometry((int)M, (int)N, (int)K, plan.tile, plan.tile, plan.splits, plan.split ? split_stage(plan.tile) : 32);
   }
 
   float *dst = (float *)matC->data;
@@ -267,7 +326,19 @@ extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, co
   }
   if (plan.flat) to_flat_tiles(g, (int)N);
   StoreRowMajor ep{dst, (int)N, (int)M, (int)N, M * N};
-  if (plan.tile == 128)
+  if (plan.split) {
+    auto run = [&](auto tile, auto ragged) {
+      constexpr int T = decltype(tile)::value;
+      dispatch_split<T, T, split_stage(T), decltype(ragged)::value>(
+          (const float *)matA->data, transposeA, lda, (uint32_t)a_bytes, (const float *)matB->data, transposeB, ldb,
+          (uint32_t)b_bytes, ep, (int)M, (int)N, (int)K, g, s);
+    };
+    const bool ragged = K % 4 != 0;  // the last vector along the reduction holds other elements behind it
+    if (plan.tile == 128 && ragged) run(IC<128>{}, std::true_type{});
+    else if (plan.tile == 128) run(IC<128>{}, std::false_type{});
+    else if (ragged) run(IC<64>{}, std::true_type{});
+    else run(IC<64>{}, std::false_type{});
+  } else if (plan.tile == 128)
     dispatch<128, 128, 16>((const float *)matA->data, transposeA, lda, (uint32_t)a_bytes, (const float *)matB->data,
                        transposeB, ldb, (uint32_t)b_bytes, ep, (int)M, (int)N, (int)K, g, s);
   else if (plan.flat)
