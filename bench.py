@@ -222,7 +222,6 @@ class HbmTimer(object):
         self.hip, self.pool = hip, pool
         self.enabled = False
         self.pairs = []
-        self.streamless = None   # stream the library uses for entry points without a stream argument
         self.mask_counts = gpu_op.relu_mask_counts
         n = lambda a: int(np.prod(a.shape))
         bn_b = (8, 12) if bn_mode == "pre_activation" else (12, 20)
@@ -237,8 +236,8 @@ class HbmTimer(object):
             "matrix_elementwise_add": lambda a: 12 * n(a[2]),
             "pooling_2d_backward": lambda a: 4 * (n(a[0]) + n(a[1]) + n(a[2]) + n(a[3])),
             "sgd_update": lambda a: 12 * n(a[0]),
-            # all updates of the step in one launch on the default stream: (tables, tables, count, lr)
-            "sgd_compute_o": lambda a: 12 * int(a[2]),
+            # all updates of the step in one launch: (tables, tables, count, lr, written arrays, stream)
+            "sgd_compute_o_on_stream": lambda a: 12 * int(a[2]),
         }
         for name, nbytes in table.items():
             setattr(gpu_op, name, self._wrap(name, getattr(gpu_op, name), nbytes))
@@ -247,7 +246,7 @@ class HbmTimer(object):
         def timed(*args):
             if not self.enabled:
                 return fn(*args)
-            s = self.streamless if name == "sgd_compute_o" else stream_handle(args[-1])
+            s = stream_handle(args[-1])
             e0 = self.pool.pop() if self.pool else self.hip.event()
             e1 = self.pool.pop() if self.pool else self.hip.event()
             counts = self.mask_counts() if name.startswith("activation_") else None
@@ -448,7 +447,6 @@ def main():
     # pairs would weigh on `value`) with an event pair around each such call.
     hbm_kernels = None
     if not args.no_kernel_events:
-        hbm_timer.streamless = s   # the executor's stream is the only one that runs kernels
         hbm_timer.enabled = True
         for _ in range(2):
             ex.run(resident)

@@ -84,6 +84,16 @@ int DLArrayCopyWaitsForCompletion(int kind, int stream_runs_kernels, int sync_ev
  * stream cell as for DLArrayCopyFromTo (not NULL); returns after the copy. */
 int DLArrayCopyIntoFresh(DLArrayHandle from, DLArrayHandle to, DLStreamHandle stream);
 
+/* No counterpart in the reference.  Copies n host arrays into device arrays in front of what is
+ * enqueued next on `stream` (a stream cell), without waiting for what is enqueued already: the host
+ * arrays may be reused on return, the device arrays change behind the stream's earlier work.  Where that
+ * cannot be had (no stream cell, a device-memory budget, TINYFLOW_SYNC_EVERY_OP, more than 1 GiB, no
+ * pinned or device memory for it) the arrays are copied by DLArrayCopyFromTo. */
+int DLArrayFeed(DLArrayHandle *from, DLArrayHandle *to, int n, DLStreamHandle stream);
+
+/* Makes the room that feeds of these device arrays need ahead of the first one; it goes with the stream. */
+int DLArrayFeedReserve(DLArrayHandle *to, int n, DLStreamHandle stream);
+
 /* No counterpart in the reference.  Call right after DLArrayAlloc on an array that
  * DLArrayCopyIntoFresh will fill later: records, now, the fence that covers the
  * last release of the array's storage, so that the copy waits for nothing enqueued
@@ -416,6 +426,14 @@ int DLGpuGetN4CudaPointer(void **output, void **m, void **v, void **g, int numbe
 int DLGpuAdam_o(void ****n4list, const void ***indexlist, const int count,
                 const float b1, const float b2, const float b1t, const float b2t,
                 const float e, const float learning_rate);
+
+/* No counterpart in the reference, where these run on the default stream: the same on `stream`.  With several
+ * streams that run kernels the default stream makes the host wait for all of them. */
+int DLGpuRelu_onStream(const DLArrayHandle in, DLArrayHandle out, void **stream);
+int DLGpuReluGradient_onStream(const DLArrayHandle in, const DLArrayHandle grad, DLArrayHandle out, void **stream);
+/* `written` are the parameters. */
+int DLGpuSgd_o_onStream(void ****n2list, const void ***indexlist, int count, float learning_rate,
+                        const DLArrayHandle *written, int n_written, void **stream);
 
 /* No counterpart in the reference, whose fused update runs on the default stream: DLGpuAdam_o on `stream`.
  * `written` are the arrays behind the first three pointer tables (parameters and moments), so that what

@@ -1,0 +1,84 @@
+"""Feeding a step from host memory (csrc/feed.hip): every step sees the batch it was given, whatever the caller does with
+the host arrays afterwards and however far the host is ahead of the GPU."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# one element, no multiple of four, the largest feed that a kernel reads from pinned memory (1 MiB) and the next one, more
+# than one chunk of the copy stream (4 MiB), several arrays, more than eight of them
+@pytest.mark.parametrize("sizes", [[1], [5, 3], [262144], [262145], [2500003], [1 << 21, 7, 4097], [3] * 19], ids=str)
+def test_arrays_arrive_in_order(rt, sizes):
+    from tinyflow_amd import gpu_op, ndarray
+    rng = np.random.RandomState(len(sizes))
+    targets = [ndarray.empty((n,), rt.ctx) for n in sizes]
+    seen, sent = [], []
+    hosts = [np.empty(n, np.float32) for n in sizes]
+    for step in range(7):
+        for h in hosts:   # the same host arrays, overwritten right after the call before
+            h[:] = rng.uniform(-1, 1, h.shape)
+        sent.append([h.copy() for h in hosts])
+        ndarray.feed(list(zip(targets, hosts)), rt.stream)
+        kept = [ndarray.empty((n,), rt.ctx) for n in sizes]
+        for t, k in zip(targets, kept):
+            gpu_op.matrix_elementwise_multiply_by_const(t, 1.0, k, rt.stream)
+        seen.append(kept)
+    for s, k in zip(sent, seen):
+        for a, b in zip(s, k):
+            np.testing.assert_array_equal(a, b.asnumpy())
+
+
+def test_what_is_refused(rt):
+    from tinyflow_amd import ndarray
+    target = ndarray.empty((4, 5), rt.ctx)
+    with pytest.raises(ValueError):
+        ndarray.feed([(target, np.zeros((5, 4), np.float32))], rt.stream)
+    with pytest.raises(TypeError):
+        ndarray.feed([(target, "not an array")], rt.stream)
+    ndarray.feed([(target, np.arange(20).reshape(4, 5).tolist())], rt.stream)   # converted, as a synchronous copy would
+    np.testing.assert_array_equal(target.asnumpy(), np.arange(20, dtype=np.float32).reshape(4, 5))
+    ndarray.feed([], rt.stream)
+    ndarray.feed([(target, np.ones((4, 5), np.float64).T.copy().T)], rt.stream)   # another type and order
+    np.testing.assert_array_equal(target.asnumpy(), np.ones((4, 5), np.float32))
+
+
+@pytest.mark.parametrize("batch", [64, 600], ids=str)   # a feed of 0.2 MB and one of 1.9 MB
+def test_steps_equal_those_of_synchronous_feeds(batch):
+    """Several executors in turn, batches that change every step; with a device-memory budget the feeds are synchronous."""
+    from tinyflow_amd import gpu_op, models
+    from tinyflow_amd.TrainExecute import TrainExecutor
+
+    def train(synchronous):
+        if synchronous:
+            gpu_op.set_device_memory_limit(8 << 30)
+        try:
+            executors = []
+            for seed in (1, 2):
+                model = models.lenet5(np.random.RandomState(seed), batch=batch)
+                ex = TrainExecutor(model.loss, 1e-4)
+                ex.init_Variable(dict(model.variables))
+                executors.append((model, ex))
+            losses = []
+            rng = np.random.RandomState(9)
+            X = np.empty(executors[0][0].input_shape, np.float32)
+            y = np.zeros((batch, 10), np.float32)
+            for step in range(6):
+                X[:] = rng.uniform(0, 1, X.shape)
+                y[:] = 0
+                y[np.arange(batch), rng.randint(0, 10, batch)] = 1
+                for model, ex in executors:
+                    out = ex.run({model.X: X, model.y_: y})
+                    if step in (0, 3, 5):
+                        losses.append(out[0].asnumpy())
+            weights = [a.asnumpy() for _, ex in executors for a in ex.run({executors[0][0].X: X, executors[0][0].y_: y}
+                       if ex is executors[0][1] else {executors[1][0].X: X, executors[1][0].y_: y})[1:]]
+            for _, ex in executors:
+                ex.close()
+            return losses + weights
+        finally:
+            if synchronous:
+                gpu_op.set_device_memory_limit(0)
+
+    for a, b in zip(train(False), train(True)):
+        assert a.tobytes() == b.tobytes()

@@ -8,13 +8,15 @@ last reader of its parameter (``swapsgd``).  The first ``run`` infers shapes
 later runs copy the feeds in and recompute every node in place.
 
 A step only enqueues work: nothing waits for the GPU except the read-back of a
-(1,)-shaped operand inside Add/Mul (the upstream-gradient scalar) and whatever
+(1,)-shaped operand inside Add/Mul (the upstream-gradient scalar), a feed for the last but
+one before it, and whatever
 the caller reads afterwards with ``asnumpy``.
 """
 import numpy as np
 
 from . import autodiff as ad
 from . import gpu_op, ndarray
+from ._base import c_array
 
 
 class TrainExecutor(object):
@@ -144,17 +146,26 @@ class TrainExecutor(object):
                 self._fused_sgd = None
             if self._fused_sgd is None:
                 plan += [(node.op.compute, node, input_vals, None) for node, input_vals in fused_updates]
+        if ndarray.is_gpu_ctx(self.ctx):   # the second step's feed finds its room made
+            ndarray.reserve_feed([self.node_to_arr_map[node] for node in feed_dict
+                                  if node.isw != 1 and node in self.node_to_arr_map], self.cudaStream)
         self.isfirstrun = 1
+
+    def _feed(self, pairs):
+        """The batch of a step, in front of it on the executor's stream; the step before may still run."""
+        if ndarray.is_gpu_ctx(self.ctx):
+            ndarray.feed(pairs, self.cudaStream)
+            return
+        for array, value in pairs:
+            array._sync_copyfrom(value)
 
     def run(self, feed_dict, Accuracy_node=None, convert_to_numpy_ret_vals=False):
         """One step.  Returns [loss, variables in network order (, accuracy node)]."""
         if self.isfirstrun == 0:
             self._first_run(feed_dict)
         else:
-            for node, value in feed_dict.items():
-                if node.isw == 1:
-                    continue  # variables live on the device; only data is re-fed
-                self.node_to_arr_map[node]._sync_copyfrom(value)
+            # variables live on the device; only data is re-fed
+            self._feed([(self.node_to_arr_map[node], value) for node, value in feed_dict.items() if node.isw != 1])
         handles = (self.cudnnHandle, self.cublasHandle, self.cudaStream)
         for compute, node, input_vals, node_val in self._plan:
             wanted = compute(node, input_vals, node_val, *handles)
@@ -239,21 +250,20 @@ class FusedUpdate(object):
 
 
 class _FusedSgd(FusedUpdate):
-    """The call has no stream argument: it runs on the default stream, which is ordered behind
-    the executor's stream and in front of its next launch."""
-
     def __init__(self, updates):
         rates = set(node.learning_rate for node, _ in updates)
         assert len(rates) == 1, "one learning rate per step"
         self.learning_rate = rates.pop()
         FusedUpdate.__init__(self, updates)
+        self.written = c_array(ndarray.DLArrayHandle, [arrays[0].handle for arrays in self.arrays])
 
     @staticmethod
     def _pointer_tables(columns, n):
         return gpu_op.get_n2_cuda_pointer(*columns, n)
 
     def apply(self, cudnnHandle, cublasHandle, cudaStream):
-        gpu_op.sgd_compute_o(self.pointers, self.tables, self.count, self.learning_rate)
+        gpu_op.sgd_compute_o_on_stream(self.pointers, self.tables, self.count, self.learning_rate, self.written,
+                                       cudaStream)
 
 
 def find_bn_relu_pairs(topo_order, outputs):

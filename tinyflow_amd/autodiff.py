@@ -412,7 +412,7 @@ class ReluOp(Op):
 
     def compute(self, node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream, use_numpy=False):
         _no_numpy(use_numpy)
-        gpu_op.relu(input_vals[0], output_val)
+        gpu_op.relu_on_stream(input_vals[0], output_val, cudaStream)
         return 0
 
     def gradient(self, node, output_grad):
@@ -431,7 +431,7 @@ class ReluGradientOp(Op):
 
     def compute(self, node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream, use_numpy=False):
         _no_numpy(use_numpy)
-        gpu_op.relu_gradient(input_vals[0], input_vals[1], output_val)
+        gpu_op.relu_gradient_on_stream(input_vals[0], input_vals[1], output_val, cudaStream)
         return 0
 
     def infer_shape(self, node, input_shapes, cudnnHandle):

@@ -274,24 +274,40 @@ extern "C" int DLGpuMatrixMultiplyByConst(const DLArrayHandle in, float val, DLA
                                         numel(out), stream_of(stream), "DLGpuMatrixMultiplyByConst");
 }
 
-// The two stream-less entry points run on the legacy default stream, which is
-// ordered after all work already enqueued on the blocking streams created by
-// DLGpuCreatecudaStream and before any work enqueued on them later.
-extern "C" int DLGpuRelu(const DLArrayHandle in, DLArrayHandle out) {
+static int launch_relu(const DLArrayHandle in, DLArrayHandle out, hipStream_t s, const char *what) {
   announce_write(out);
   TF_REQUIRE(on_gpu(in) && on_gpu(out), "arrays must live on the GPU");
   TF_REQUIRE(same_shape(in, out), "shape mismatch");
-  return launch_ew<OpRelu, true, false>(OpRelu{}, (float *)out->data, (const float *)in->data, nullptr,
-                                        numel(out), streamless_launch_stream(), "DLGpuRelu");
+  return launch_ew<OpRelu, true, false>(OpRelu{}, (float *)out->data, (const float *)in->data, nullptr, numel(out), s, what);
 }
 
-extern "C" int DLGpuReluGradient(const DLArrayHandle in, const DLArrayHandle grad, DLArrayHandle out) {
+static int launch_relu_gradient(const DLArrayHandle in, const DLArrayHandle grad, DLArrayHandle out, hipStream_t s,
+                                const char *what) {
   announce_write(out);
   TF_REQUIRE(on_gpu(in) && on_gpu(grad) && on_gpu(out), "arrays must live on the GPU");
   TF_REQUIRE(same_shape(in, out) && same_shape(grad, out), "shape mismatch");
   return launch_ew<OpReluGrad, true, true>(OpReluGrad{}, (float *)out->data, (const float *)in->data,
-                                           (const float *)grad->data, numel(out), streamless_launch_stream(),
-                                           "DLGpuReluGradient");
+                                           (const float *)grad->data, numel(out), s, what);
+}
+
+// The two stream-less entry points run on the legacy default stream, which is
+// ordered after all work already enqueued on the blocking streams created by
+// DLGpuCreatecudaStream and before any work enqueued on them later.
+extern "C" int DLGpuRelu(const DLArrayHandle in, DLArrayHandle out) {
+  return launch_relu(in, out, streamless_launch_stream(), "DLGpuRelu");
+}
+
+extern "C" int DLGpuReluGradient(const DLArrayHandle in, const DLArrayHandle grad, DLArrayHandle out) {
+  return launch_relu_gradient(in, grad, out, streamless_launch_stream(), "DLGpuReluGradient");
+}
+
+extern "C" int DLGpuRelu_onStream(const DLArrayHandle in, DLArrayHandle out, void **stream) {
+  return launch_relu(in, out, stream_of(stream), "DLGpuRelu_onStream");
+}
+
+extern "C" int DLGpuReluGradient_onStream(const DLArrayHandle in, const DLArrayHandle grad, DLArrayHandle out,
+                                          void **stream) {
+  return launch_relu_gradient(in, grad, out, stream_of(stream), "DLGpuReluGradient_onStream");
 }
 
 extern "C" int DLGpuSgdUpdate(DLArrayHandle w, const DLArrayHandle g, float lr, void **stream) {
@@ -618,13 +634,10 @@ extern "C" int DLGpuAdam_o_onStream(void ****n4list, const void ***indexlist, in
                            "DLGpuAdam_o_onStream");
 }
 
-extern "C" int DLGpuSgd_o(void ****n2list, const void ***indexlist, const int count,
-                          const float learning_rate) {
-  note_write_everything();  // the pointer tables name the written tensors, not their sizes
+static int launch_multi_sgd(void ****n2list, const void ***indexlist, int count, float learning_rate, hipStream_t s,
+                            const char *what) {
   TF_REQUIRE(n2list && *n2list && indexlist && *indexlist && count >= 0, "bad arguments");
   if (count == 0) return 0;
-  // no stream argument: ordered against all streams that run kernels
-  hipStream_t s = streamless_launch_stream();
   RunTable runs;
   const int found = find_run_table((*indexlist)[0], count, runs);
   TF_REQUIRE(found >= 0, "count %d is not the count the index tables were built for", count);
@@ -632,10 +645,24 @@ extern "C" int DLGpuSgd_o(void ****n2list, const void ***indexlist, const int co
     hipLaunchKernelGGL((multi_tensor_kernel<2, MultiSgd>), dim3(runs.n_pieces), dim3(kThreads), 0, s,
                        MultiSgd{learning_rate}, (float *const *)((*n2list)[0]), (float *const *)((*n2list)[1]),
                        (float *const *)nullptr, (float *const *)nullptr, (const RunPiece *)runs.pieces);
-    return finish(s, "DLGpuSgd_o");
+    return finish(s, what);
   }
   hipLaunchKernelGGL(sgd_multi_kernel, dim3(grid_for(count)), dim3(kThreads), 0, s,
                      (float **)((*n2list)[0]), (float **)((*n2list)[1]), (const int *)((*indexlist)[0]),
                      (const int *)((*indexlist)[1]), learning_rate, count);
-  return finish(s, "DLGpuSgd_o");
+  return finish(s, what);
+}
+
+extern "C" int DLGpuSgd_o(void ****n2list, const void ***indexlist, const int count,
+                          const float learning_rate) {
+  note_write_everything();  // the pointer tables name the written tensors, not their sizes
+  // no stream argument: ordered against all streams that run kernels
+  return launch_multi_sgd(n2list, indexlist, count, learning_rate, streamless_launch_stream(), "DLGpuSgd_o");
+}
+
+extern "C" int DLGpuSgd_o_onStream(void ****n2list, const void ***indexlist, int count, float learning_rate,
+                                   const DLArrayHandle *written, int n_written, void **stream) {
+  TF_REQUIRE(n_written >= 0 && (written || n_written == 0), "bad arguments");
+  for (int i = 0; i < n_written; ++i) announce_write(written[i]);
+  return launch_multi_sgd(n2list, indexlist, count, learning_rate, stream_of(stream), "DLGpuSgd_o_onStream");
 }

@@ -24,6 +24,12 @@ void pinned_free(void *p);
 // ---- streams ----------------------------------------------------------------
 hipStream_t stream_of(void **cell);      // cell written by DLGpuCreatecudaStream; NULL -> default stream
 hipStream_t streamless_launch_stream();  // for entry points without a stream argument
+void *pinned_alloc(size_t bytes);
+void pinned_free(void *p);
+int wait_for_other_streams(hipStream_t s);  // `s` behind everything enqueued on the other kernel-running streams
+bool other_streams_busy(hipStream_t s);     // whether there is any such thing
+bool idle(hipStream_t s);                   // nothing of what was enqueued on it is left to run
+void feed_forget_stream(hipStream_t s);     // feed.hip: gives back what feeds on the stream keep (waits for it)
 bool sync_every_op();                    // TINYFLOW_SYNC_EVERY_OP=1
 int finish(hipStream_t s, const char *what);  // launch-error check (+ optional sync)
 

@@ -680,14 +680,12 @@ extern "C" int DLArrayFree(DLArrayHandle handle) {
   return 0;
 }
 
-namespace {
+namespace tf {
 
-hipMemcpyKind copy_kind(const DLArray *from, const DLArray *to) {
-  const bool fg = from->ctx.device_type == kGPU, tg = to->ctx.device_type == kGPU;
-  if (fg && tg) return hipMemcpyDeviceToDevice;
-  if (fg) return hipMemcpyDeviceToHost;
-  if (tg) return hipMemcpyHostToDevice;
-  return hipMemcpyHostToHost;
+bool idle(hipStream_t s) {
+  const bool nothing_pending = hipStreamQuery(s) == hipSuccess;
+  if (!nothing_pending) (void)hipGetLastError();
+  return nothing_pending;
 }
 
 // Make `s` wait for everything already enqueued on the other kernel-running
@@ -699,11 +697,31 @@ int wait_for_other_streams(hipStream_t s) {
   Runtime &r = rt();
   std::lock_guard<std::mutex> g(r.mu);
   for (auto &rec : r.streams) {
-    if (rec.stream == s || !rec.runs_kernels) continue;
+    if (rec.stream == s || !rec.runs_kernels || idle(rec.stream)) continue;
     TF_HIP(hipEventRecord(rec.event, rec.stream));
     TF_HIP(hipStreamWaitEvent(s, rec.event, 0));
   }
   return 0;
+}
+
+bool other_streams_busy(hipStream_t s) {
+  Runtime &r = rt();
+  std::lock_guard<std::mutex> g(r.mu);
+  for (auto &rec : r.streams)
+    if (rec.stream != s && rec.runs_kernels && !idle(rec.stream)) return true;
+  return false;
+}
+
+}  // namespace tf
+
+namespace {
+
+hipMemcpyKind copy_kind(const DLArray *from, const DLArray *to) {
+  const bool fg = from->ctx.device_type == kGPU, tg = to->ctx.device_type == kGPU;
+  if (fg && tg) return hipMemcpyDeviceToDevice;
+  if (fg) return hipMemcpyDeviceToHost;
+  if (tg) return hipMemcpyHostToDevice;
+  return hipMemcpyHostToHost;
 }
 
 // True when an op entry point has launched on `s`: later kernels of the step are
@@ -861,6 +879,7 @@ extern "C" int DLGpuDestroycudaStream(void **cell) {
   TF_REQUIRE(cell, "null cell");
   note_write_everything();  // kept blocks are ordered by the stream that made them
   hipStream_t s = reinterpret_cast<hipStream_t>(*cell);
+  feed_forget_stream(s);
   hipEvent_t ev = nullptr;
   bool found = false;
   {

@@ -154,6 +154,18 @@ def relu_gradient(in_arr, in_grad_arr, out_arr):
     check_call(_LIB.DLGpuReluGradient(in_arr.handle, in_grad_arr.handle, out_arr.handle))
 
 
+def relu_on_stream(in_arr, out_arr, cudaStream):
+    """``relu`` on ``cudaStream`` instead of the default stream (no counterpart in the reference)."""
+    _nd_args(in_arr, out_arr)
+    check_call(_LIB.DLGpuRelu_onStream(in_arr.handle, out_arr.handle, cudaStream))
+
+
+def relu_gradient_on_stream(in_arr, in_grad_arr, out_arr, cudaStream):
+    """``relu_gradient`` on ``cudaStream`` instead of the default stream (no counterpart in the reference)."""
+    _nd_args(in_arr, in_grad_arr, out_arr)
+    check_call(_LIB.DLGpuReluGradient_onStream(in_arr.handle, in_grad_arr.handle, out_arr.handle, cudaStream))
+
+
 def softmax(in_arr, out_arr, cudaStream):
     _nd_args(in_arr, out_arr)
     check_call(_LIB.DLGpuSoftmax(in_arr.handle, out_arr.handle, cudaStream))
@@ -455,6 +467,13 @@ def adam_compute_o(n4list, indexinfolist, count, b1, b2, b1t, b2t, e, learning_r
     check_call(_LIB.DLGpuAdam_o(n4list, indexinfolist, ctypes.c_int(count), ctypes.c_float(b1),
                                 ctypes.c_float(b2), ctypes.c_float(b1t), ctypes.c_float(b2t),
                                 ctypes.c_float(e), ctypes.c_float(learning_rate)))
+
+
+def sgd_compute_o_on_stream(n2list, indexinfolist, count, learning_rate, written, cudaStream):
+    """``sgd_compute_o`` on ``cudaStream`` instead of the default stream (no counterpart in the
+    reference); ``written``: a ``c_array`` of the handles of the parameters."""
+    check_call(_LIB.DLGpuSgd_o_onStream(n2list, indexinfolist, ctypes.c_int(count), ctypes.c_float(learning_rate),
+                                        written, ctypes.c_int(len(written)), cudaStream))
 
 
 def adam_compute_o_on_stream(n4list, indexinfolist, count, b1, b2, b1t, b2t, e, learning_rate, written, cudaStream):

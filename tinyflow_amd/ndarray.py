@@ -104,6 +104,12 @@ class NDArray(object):
 
     def _sync_copyfrom(self, source_array):
         """Synchronous host -> this array copy of an fp32-convertible array."""
+        borrowed, keep = NDArray._numpyasarray(self._as_source(source_array))
+        check_call(_LIB.DLArrayCopyFromTo(ctypes.byref(borrowed), self.handle, None))
+        del keep
+
+    def _as_source(self, source_array):
+        """``source_array`` as the contiguous fp32 numpy array that can be copied into this one."""
         if not isinstance(source_array, np.ndarray):
             try:
                 source_array = np.array(source_array, dtype=np.float32)
@@ -113,9 +119,7 @@ class NDArray(object):
         source_array = np.ascontiguousarray(source_array, dtype=np.float32)
         if source_array.shape != self.shape:
             raise ValueError("array shape do not match the shape of NDArray")
-        borrowed, keep = NDArray._numpyasarray(source_array)
-        check_call(_LIB.DLArrayCopyFromTo(ctypes.byref(borrowed), self.handle, None))
-        del keep
+        return source_array
 
     @staticmethod
     def _numpyasarray(np_data):
@@ -159,6 +163,23 @@ class NDArray(object):
         for everything enqueued (the prefetch of the swap path)."""
         check_call(_LIB.DLArrayCopyIntoFresh(self.handle, target.handle, cudaStream))
         return target
+
+
+def feed(pairs, cudaStream):
+    """Copies host arrays into device arrays, given as (device array, array_like) pairs, in front of what is enqueued
+    next on ``cudaStream`` and without waiting for what is enqueued already.  The host arrays may be changed on return."""
+    sources = [target._as_source(value) for target, value in pairs]
+    borrowed = [NDArray._numpyasarray(source) for source in sources]
+    n = len(pairs)
+    from_handles = (DLArrayHandle * n)(*[ctypes.pointer(arr) for arr, _ in borrowed])
+    to_handles = (DLArrayHandle * n)(*[target.handle for target, _ in pairs])
+    check_call(_LIB.DLArrayFeed(from_handles, to_handles, n, cudaStream))
+
+
+def reserve_feed(arrays, cudaStream):
+    """Makes the room that ``feed`` of these device arrays on this stream needs."""
+    handles = (DLArrayHandle * len(arrays))(*[a.handle for a in arrays])
+    check_call(_LIB.DLArrayFeedReserve(handles, len(arrays), cudaStream))
 
 
 def empty(shape, ctx=cpu(0)):
