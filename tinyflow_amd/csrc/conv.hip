@@ -18,6 +18,7 @@
 // All four lane-parallel directions ((n,p,q), (n,h,w), (c,r,s)) are contiguous
 // in memory for NCHW/KCRS, so global loads and stores coalesce without any
 // layout change of the activations.
+#include "conv_few.h"
 #include "gemm_core.h"
 #include "gemm_launch.h"
 #include "gemm_split.h"
@@ -1529,6 +1530,84 @@ void consider_winograd_wgrad(ConvPlan &p, const ConvDesc *d, double direct_us) {
   p.K = best_tp;
 }
 
+// ---- few output channels on the vector units (conv_few.h) ---------------------------------
+// Taken by forward and stride-1 grad-data of at most eight output channels where every CU gets a workgroup (us, engine /
+// here: 6 <- 16 channels, 5x5, 14 x 14, 64 images 25 / 28, 300 images 50 / 34, 1 000 121 / 51; 1 -> 6 channels, 28 x 28, 64
+// images forward 9.4 / 9.1, grad-data 25 / 11, 4 096 216 / 61 and 705 / 169).  With sixteen channels the filter values of a tap
+// row no longer fit the scalar registers: 6 -> 16 channels, 1 000 images 31 / 39.  Not for
+//   * reductions of more than 512 steps, a lane's chain: the engine cuts them up for the whole chip;
+//   * a forward reduction of a multiple of four, which the engine walks in another order, and 1x1 filters (no gather);
+//   * plans whose pieces a second pass sums, which takes them in an order of its own.
+constexpr int kFewChannels = 8, kFewSteps = 512, kFewLds = 32 << 10;
+struct FewLaunch {
+  few::Conv c;
+  unsigned blocks = 0, lds = 0;
+};
+bool few_channels(const ConvDesc *d, const ConvPlan &p, bool dgrad, const Geometry &g, FewLaunch &l) {
+  if (p.winograd || p.split || p.M > kFewChannels || p.K > kFewSteps || p.b_vec || g.splits > 1) return false;
+  if (d->S != 3 && d->S != 5 && d->S != 7) return false;
+  if (dgrad ? d->u != 1 || d->v != 1 : p.a_vec) return false;
+  few::Conv &c = l.c;
+  c.N = d->N;
+  c.M = p.M;
+  c.C = dgrad ? d->K : d->C;
+  c.Hs = dgrad ? d->P : d->H;
+  c.Ws = dgrad ? d->Q : d->W;
+  const int OH = dgrad ? d->H : d->P;
+  c.OW = dgrad ? d->W : d->Q;
+  c.OHW = OH * c.OW;
+  c.R = d->R;
+  c.u = d->u;
+  c.v = d->v;
+  c.row0 = dgrad ? d->pad_h - (d->R - 1) : -d->pad_h;
+  c.col0 = dgrad ? d->pad_w - (d->S - 1) : -d->pad_w;
+  c.images = std::max(1, few::kThreads / c.OHW);
+  c.ranges = cdiv(c.OHW, few::kThreads);
+  c.span = cdiv(c.OHW, c.ranges);
+  const int out_rows = c.ranges == 1 ? OH : std::min(OH, (c.span + c.OW - 2) / c.OW + 1);
+  c.rows = (out_rows - 1) * c.u + c.R;
+  c.width = (c.OW - 1) * c.v + d->S;
+  const int64_t plane = (int64_t)c.images * c.rows * c.width * 4;
+  if (plane > kFewLds) return false;
+  c.chunk = (int)std::min<int64_t>(c.C, kFewLds / plane);
+  c.piece = g.fold_pieces > 1 ? g.fold_k_per_piece : 0;
+  c.tile = p.bn;
+  c.first_tile = g.fold_first_tile;
+  c.div_ow = FastDiv((uint32_t)c.OW);
+  c.div_ohw = FastDiv((uint32_t)c.OHW);
+  c.div_width = FastDiv((uint32_t)c.width);
+  c.div_rows = FastDiv((uint32_t)c.rows);
+  c.div_chunk = FastDiv((uint32_t)c.chunk);
+  c.div_ranges = FastDiv((uint32_t)c.ranges);
+  c.div_tile = FastDiv((uint32_t)c.tile);
+  l.blocks = (unsigned)(cdiv(c.N, c.images) * c.ranges);
+  l.lds = (unsigned)(plane * c.chunk);
+  return l.blocks >= (unsigned)num_cus();
+}
+// The kernel's channels: the smallest of its sizes that holds M.
+int few_size(int M) { return M <= 4 ? 4 : M <= 6 ? 6 : 8; }
+
+template <bool DGRAD>
+void launch_few(const FewLaunch &l, int S, const float *src, const float *w, float *out, hipStream_t s) {
+  if (next_kernel_start) (void)hipEventRecord(next_kernel_start, s);
+  auto go = [&](auto m, auto taps) {
+    hipLaunchKernelGGL((few::gemm_kernel<decltype(m)::value, decltype(taps)::value, DGRAD>),
+                       dim3(l.blocks), dim3(few::kThreads), l.lds, s, src, w, out, l.c);
+  };
+  auto with_taps = [&](auto m) {
+    if (S == 3) go(m, IC<3>{});
+    else if (S == 5) go(m, IC<5>{});
+    else go(m, IC<7>{});
+  };
+  switch (few_size(l.c.M)) {
+    case 4: with_taps(IC<4>{}); break;
+    case 6: with_taps(IC<6>{}); break;
+    default: with_taps(IC<8>{});
+  }
+  if (next_kernel_stop) (void)hipEventRecord(next_kernel_stop, s);
+  next_kernel_start = next_kernel_stop = nullptr;
+}
+
 ConvPlan plan_forward(const ConvDesc *d) {
   ConvPlan p;
   p.M = d->K;
@@ -1973,6 +2052,17 @@ extern "C" int DLGpuConvolutionDescribeKernel(void ***list, int which, char *nam
     if (flops) *flops = 2.0 * d->N * d->K * d->C * d->R * d->S * (double)d->P * d->Q;
     return 0;
   }
+  if (which != 2) {
+    Geometry g = make_geometry(p.M, p.N, p.K, p.bm, p.bn, p.splits, stage_depth(p.bm, p.bn));
+    plan_fold(g, p.K, stage_depth(p.bm, p.bn), 1);
+    FewLaunch few;
+    if (few_channels(d, p, which == 1, g, few)) {
+      snprintf(name, (size_t)name_len, "%s %dx%d s%d | gemm_kernel<%d, %d, %s>", p.variant, p.bm, p.bn, p.splits,
+               few_size(p.M), d->S, which == 1 ? "true" : "false");
+      if (flops) *flops = 2.0 * d->N * d->K * d->C * d->R * d->S * (double)d->P * d->Q;
+      return 0;
+    }
+  }
   // Across4 carries its RAGGED flag in the symbol (a profiler prints defaulted arguments too)
   char b_args[32];
   const bool ragged_wgrad = which == 2 && p.b_vec && p.seg != d->P * d->Q;
@@ -2066,6 +2156,11 @@ extern "C" int DLGpuConvolution2DForward(const DLArrayHandle input, const DLArra
   const int bm = plan.bm, bn = plan.bn;
   Geometry g = make_geometry(M, N, K, bm, bn, plan.splits, stage_depth(bm, bn));
   if (fold_tickets(s)) plan_fold(g, K, stage_depth(bm, bn), 1);  // no ticket words: the unfolded plan
+  FewLaunch few;
+  if (few_channels(d, plan, false, g, few)) {
+    launch_few<false>(few, d->S, (const float *)input->data, (const float *)filter->data, (float *)output->data, s);
+    return finish(s, "DLGpuConvolution2DForward");
+  }
   FoldBuffers fb;
   if (const int rc = acquire_fold(g, bm, bn, 1, s, fb)) {
     if (rc == 1 && memorytoSaving) *memorytoSaving = shortfall(fb.bytes);
@@ -2221,6 +2316,11 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
   const int g_bm = strided_taps ? 64 : plan.bm, g_bn = strided_taps ? 64 : plan.bn;
   Geometry g = make_geometry(M, plan.N, K, g_bm, g_bn, strided_taps ? 1 : plan.splits, stage_depth(g_bm, g_bn));
   if (fold_tickets(s)) plan_fold(g, K, stage_depth(g_bm, g_bn), 1);  // no ticket words: the unfolded plan
+  FewLaunch few;
+  if (few_channels(d, plan, true, g, few)) {
+    launch_few<true>(few, d->S, (const float *)doutput->data, (const float *)filter->data, (float *)dinput->data, s);
+    return finish(s, "DLGpuConvolutionBackwardData");
+  }
   // Scratch: the re-laid filter, the fold pieces or the k-split partials.  Whichever of them
   // cannot be had, the call reports all of them, so that a caller who makes that much room
   // can repeat it.
