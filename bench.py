@@ -233,6 +233,10 @@ class HbmTimer(object):
             # backward call that uses them reads dy and the bits instead of dy and x
             "activation_forward": lambda a, bits=False: (8.125 if bits else 8) * n(a[0]),
             "activation_backward": lambda a, bits=False: (8.125 if bits else 12) * n(a[0]),
+            # a sum with the ReLU behind it, and two adjoints' sum with the ReLU's gradient: with the bits two
+            # arrays are read and two written, without them one array more is read
+            "add_activation_forward": lambda a, bits=False: (16.125 if bits else 20) * n(a[2]),
+            "add_activation_backward": lambda a, bits=False: (16.125 if bits else 20) * n(a[2]),
             "matrix_elementwise_add": lambda a: 12 * n(a[2]),
             "pooling_2d_backward": lambda a: 4 * (n(a[0]) + n(a[1]) + n(a[2]) + n(a[3])),
             "sgd_update": lambda a: 12 * n(a[0]),
@@ -249,7 +253,7 @@ class HbmTimer(object):
             s = stream_handle(args[-1])
             e0 = self.pool.pop() if self.pool else self.hip.event()
             e1 = self.pool.pop() if self.pool else self.hip.event()
-            counts = self.mask_counts() if name.startswith("activation_") else None
+            counts = self.mask_counts() if "activation_" in name else None
             self.hip.record(e0, s)
             ret = fn(*args)
             self.hip.record(e1, s)

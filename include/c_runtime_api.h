@@ -325,6 +325,15 @@ int DLGpuActivationBackward(const DLArrayHandle input, DLArrayHandle dinput,
                             const DLArrayHandle output, const DLArrayHandle doutput,
                             int activationMode, void ***list, void **handle, void **stream);
 
+/* No counterpart in the reference: sum = matA + matB and output = max(sum, 0), a residual join and its
+ * ReLU; and sum = matA + matB and dinput = input > 0 ? sum : 0, the adjoints that meet there and the
+ * ReLU's gradient.  Both results are written, the bytes are those of the two calls each stands for. */
+int DLGpuMatrixElementwiseAddReluForward(const DLArrayHandle matA, const DLArrayHandle matB, DLArrayHandle sum,
+                                         DLArrayHandle output, void ***list, void **handle, void **stream);
+int DLGpuMatrixElementwiseAddReluBackward(const DLArrayHandle matA, const DLArrayHandle matB, DLArrayHandle sum,
+                                          const DLArrayHandle input, DLArrayHandle dinput,
+                                          const DLArrayHandle output, void ***list, void **handle, void **stream);
+
 /* No counterpart in the reference: introspection for tests and for the benchmark's
  * byte accounting.  Once a ReLU descriptor has seen a backward call, its forward calls
  * also write one bit per element (x > 0) into a block of the library's own, and the

@@ -102,7 +102,19 @@ class TrainExecutor(object):
         for role in fused.values():   # a fused call reads its sources as arrays
             if len(role) == 3:
                 unread_zeros -= set(role[2])
+        joined = find_joins(self.topo_order, self.node_to_shape_map, set(feed_dict) | unread_zeros, fused)
+        by_join = set(joined.values())
         for node in self.topo_order:
+            if node in by_join:
+                continue   # computed with its first operand
+            if node in joined:
+                relu = joined[node]
+                outputs = [self._alloc(self.node_to_shape_map[n]) for n in (node, relu)]
+                self.node_to_arr_map[node], self.node_to_arr_map[relu] = outputs
+                sources = fused[relu][2] if relu in fused else relu.inputs
+                plan.append((_join_compute, relu, [self.node_to_arr_map[i] for i in list(node.inputs) + list(sources)],
+                             outputs))
+                continue
             if node in unread_zeros:
                 continue   # every reader adds it as the constant 0.0: never materialised
             role = fused.get(node)
@@ -333,6 +345,49 @@ def find_add_relu_pairs(topo_order, outputs, shapes):
         roles[r] = ("add_relu", s, list(s.inputs))
         roles[a] = ("mask_from_output", s, [r, a.inputs[1], r])
     return roles
+
+
+def find_joins(topo_order, shapes, unavailable, roles):
+    """Elementwise sums S that are computed together with the ReLU R that reads them, or with the ReLU backward A whose
+    upstream gradient they are: one pass that writes both, where the second of two passes would read S again (64 images
+    of 256 channels of 56 x 56: 20 bytes per element become 16).  Returns S -> R or A.
+
+    Both run at S's place: R reads nothing else, and A's other operands have to precede S.  Other readers of either do
+    not matter, both arrays hold what they would.  ``unavailable`` nodes are fed or never materialised; ``roles`` are
+    the fused roles, of which only a backward that takes its mask from the ReLU's output can join."""
+    at = {n: i for i, n in enumerate(topo_order)}
+    joins, taken = {}, unavailable | {n for n, role in roles.items() if role[0] != "mask_from_output"}
+    for r in topo_order:
+        if r in taken:
+            continue
+        if isinstance(r.op, ad.ActivationForwardOp):
+            s, before = r.inputs[0], []
+        elif isinstance(r.op, ad.ActivationBackwardOp):
+            s, before = r.inputs[1], roles[r][2] if r in roles else r.inputs
+            before = [n for n in before if n is not s]
+        else:
+            continue
+        if r.activationMode != "relu" or s in taken or s in joins or not isinstance(s.op, ad.AddOp):
+            continue
+        if not (len(s.inputs) == 2 and shapes[s.inputs[0]] == shapes[s.inputs[1]] == shapes[s]):
+            continue   # a (1,)-shaped operand is applied as a constant
+        if unavailable & set(s.inputs) or any(at[n] > at[s] for n in before):
+            continue
+        joins[s] = r
+    return joins
+
+
+def _join_compute(node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream):
+    """Plan entry of a join: ``node`` is the ReLU or its backward, ``input_vals`` the two operands of the sum and then
+    what ``node`` reads, ``output_val`` the arrays of the sum and of ``node``."""
+    a, b = input_vals[:2]
+    total, out = output_val
+    if isinstance(node.op, ad.ActivationForwardOp):
+        gpu_op.add_activation_forward(a, b, total, out, node.cudnnlist[0], cudnnHandle, cudaStream)
+    else:
+        x, y = input_vals[2], input_vals[4]
+        gpu_op.add_activation_backward(a, b, total, x, out, y, node.cudnnlist[0], cudnnHandle, cudaStream)
+    return 0
 
 
 def _known_scalar_compute(node, shapes):

@@ -323,6 +323,21 @@ def activation_backward(input, dinput, output, doutput, activationMode, cudnnlis
                                             doutput.handle, mode, cudnnlist, cudnnHandle, cudaStream))
 
 
+def add_activation_forward(matA, matB, total, output, cudnnlist, cudnnHandle, cudaStream):
+    """total = matA + matB and output = max(total, 0) in one pass (extension)"""
+    _nd_args(matA, matB, total, output)
+    check_call(_LIB.DLGpuMatrixElementwiseAddReluForward(matA.handle, matB.handle, total.handle, output.handle,
+                                                         cudnnlist, cudnnHandle, cudaStream))
+
+
+def add_activation_backward(matA, matB, total, input, dinput, output, cudnnlist, cudnnHandle, cudaStream):
+    """total = matA + matB and dinput = total where input > 0, else 0, in one pass (extension)"""
+    _nd_args(matA, matB, total, input, dinput, output)
+    check_call(_LIB.DLGpuMatrixElementwiseAddReluBackward(matA.handle, matB.handle, total.handle, input.handle,
+                                                          dinput.handle, output.handle, cudnnlist, cudnnHandle,
+                                                          cudaStream))
+
+
 # ---------------------------------------------------------- batch normalisation
 
 def bn_get_cudnnlist(input_shapes, dataformat, batchNormMode):
