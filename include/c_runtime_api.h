@@ -378,6 +378,19 @@ int DLGpuBatchNormalizationReluBackward(const DLArrayHandle input, const DLArray
                                         void **Variance_p, void ***list, void **handle,
                                         int *memorytoSaving, void **stream);
 
+/* No counterpart in the reference: a batch norm and the ReLU that reads it, and their gradients, with both
+ * results written; the bytes are those of the two calls each stands for. */
+int DLGpuBatchNormalizationAndReluForward(const DLArrayHandle input, DLArrayHandle bn_output,
+                                          DLArrayHandle relu_output, int batchNormMode, int n, void **mean_p,
+                                          void **Variance_p, void ***list, void ***activation_list,
+                                          void **handle, int *memorytoSaving, void **stream);
+int DLGpuBatchNormalizationAndReluBackward(const DLArrayHandle input, const DLArrayHandle bn_output,
+                                           const DLArrayHandle relu_output, const DLArrayHandle doutput,
+                                           DLArrayHandle drelu, DLArrayHandle dinput, int batchNormMode,
+                                           void **mean_p, void **Variance_p, void ***list,
+                                           void ***activation_list, void **handle, int *memorytoSaving,
+                                           void **stream);
+
 /* ----------------------------------------------------- dropout, concatenation */
 
 /* Element-count descriptor that dropout takes in place of the reference's cuDNN

@@ -69,6 +69,43 @@ def test_join_in_place_and_with_foreign_bits(rt):
         assert out.asnumpy().tobytes() == O.relu(c + d).tobytes()
 
 
+# the register kernels of 32, 64 and 128 rows, full and not; rows past the last of them and the spatial mode take the two
+# calls; columns that do not fill a workgroup
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["pre_activation", "spatial"])
+@pytest.mark.parametrize("shape", [(1, 3, 5, 7), (31, 4, 9, 9), (32, 16, 16, 16), (33, 5, 11, 3), (64, 3, 17, 5),
+                                   (65, 2, 8, 8), (128, 3, 6, 7), (129, 3, 6, 7)], ids=str)
+def test_batch_norm_with_relu_writes_the_bytes_of_the_separate_calls(rt, shape, mode):
+    from tinyflow_amd import gpu_op, ndarray
+    ctx, cudnn, stream = rt.ctx, rt.cudnn, rt.stream
+    gen = np.random.default_rng(5)
+    x, dy = (gen.standard_normal(shape, dtype=np.float32) for _ in range(2))
+    x[0, 0] = 2.5
+    x[:, 1, 0, 0] = 0.75   # a column of equal values: bn(x) is zero
+    dy[0, 0, 0, :2] = [np.nan, -0.0]
+    gx, gdy = ndarray.array(x, ctx), ndarray.array(dy, ctx)
+    results = []
+    for joined in (False, True):
+        act = gpu_op.activation_get_cudnnlist(shape, "NCHW", "relu")
+        mean_p, var_p, lst = gpu_op.bn_get_cudnnlist(shape, "NCHW", mode)
+        out = [ndarray.empty(shape, ctx) for _ in range(4)]
+        for step in range(2):
+            for arr in out:
+                gpu_op.array_set(arr, 7.0, stream)
+            bn, relu, drelu, dx = out
+            if joined:
+                assert gpu_op.bn_and_relu_forward(gx, bn, relu, mode, step, mean_p, var_p, lst, act, cudnn, stream) == 0
+                assert gpu_op.bn_and_relu_backward(gx, bn, relu, gdy, drelu, dx, mode, mean_p, var_p, lst, act, cudnn,
+                                                   stream) == 0
+            else:
+                assert gpu_op.bn_forward(gx, bn, mode, step, mean_p, var_p, lst, cudnn, stream) == 0
+                gpu_op.activation_forward(bn, relu, "relu", act, cudnn, stream)
+                gpu_op.activation_backward(bn, drelu, relu, gdy, "relu", act, cudnn, stream)
+                assert gpu_op.bn_backward(gx, drelu, dx, mode, mean_p, var_p, lst, cudnn, stream) == 0
+            results.append([arr.asnumpy().tobytes() for arr in out])
+    assert results[0] == results[1] == results[2] == results[3]
+
+
 def test_which_sums_join():
     """A sum joins one ReLU; not where it is fed or applied as a constant, where the ReLU's gradient needs a later
     operand, or where a fused role has it."""
@@ -92,3 +129,24 @@ def test_which_sums_join():
     shapes.update({late: (2, 3), back2: (2, 3)})
     order = [x, y, s, r, g, tanh.inputs[0], tanh, late, back2]
     assert find_joins(order, shapes, set(), {}) == {s: r}
+
+
+def test_which_batch_norms_join():
+    """A per-activation batch norm joins its ReLU, the ReLU's gradient that batch norm's gradient; spatial ones do not, nor
+    a gradient of another batch norm."""
+    from tinyflow_amd import autodiff as ad
+    from tinyflow_amd.TrainExecute import find_joins
+    x, y, dr = ad.Placeholder("x"), ad.Placeholder("y"), ad.Placeholder("dr")
+    for mode in ("pre_activation", "spatial"):
+        b = ad.bn_forward_op(x, "NCHW", mode)
+        r = ad.activation_forward_op(b, "NCHW", "relu")
+        a = ad.activation_backward_op(b, dr, r, "relu", r.cudnnlist)
+        d = ad.bn_backward_op(x, a, mode, b.Save_p, b.cudnnlist)
+        b2 = ad.bn_forward_op(y, "NCHW", mode)
+        d2 = ad.bn_backward_op(y, a, mode, b2.Save_p, b2.cudnnlist)
+        joins = {b: r, a: d} if mode == "pre_activation" else {}
+        order = [x, y, dr, b, b2, r, a, d, d2]
+        shapes = {n: (2, 3, 4, 4) for n in order}
+        assert find_joins(order, shapes, set(), {}) == joins
+        assert find_joins([x, y, dr, b, b2, r, a, d2], shapes, set(), {}) == {s: t for s, t in joins.items() if s is b}
+        assert find_joins(order, shapes, {b}, {}) == {}   # fed: nothing to compute

@@ -108,12 +108,12 @@ class TrainExecutor(object):
             if node in by_join:
                 continue   # computed with its first operand
             if node in joined:
-                relu = joined[node]
-                outputs = [self._alloc(self.node_to_shape_map[n]) for n in (node, relu)]
-                self.node_to_arr_map[node], self.node_to_arr_map[relu] = outputs
-                sources = fused[relu][2] if relu in fused else relu.inputs
-                plan.append((_join_compute, relu, [self.node_to_arr_map[i] for i in list(node.inputs) + list(sources)],
-                             outputs))
+                reader = joined[node]
+                outputs = [self._alloc(self.node_to_shape_map[n]) for n in (node, reader)]
+                self.node_to_arr_map[node], self.node_to_arr_map[reader] = outputs
+                sources = fused[reader][2] if reader in fused else reader.inputs
+                plan.append((_join_compute(node, reader), reader,
+                             [self.node_to_arr_map[i] for i in list(node.inputs) + list(sources)], outputs))
                 continue
             if node in unread_zeros:
                 continue   # every reader adds it as the constant 0.0: never materialised
@@ -348,46 +348,78 @@ def find_add_relu_pairs(topo_order, outputs, shapes):
 
 
 def find_joins(topo_order, shapes, unavailable, roles):
-    """Elementwise sums S that are computed together with the ReLU R that reads them, or with the ReLU backward A whose
-    upstream gradient they are: one pass that writes both, where the second of two passes would read S again (64 images
-    of 256 channels of 56 x 56: 20 bytes per element become 16).  Returns S -> R or A.
+    """Nodes S that are computed together with a reader: one pass that writes both, where the second of two passes would
+    read S again (64 images of 256 channels of 56 x 56, sum and ReLU: 20 bytes per element become 16).  S is
 
-    Both run at S's place: R reads nothing else, and A's other operands have to precede S.  Other readers of either do
-    not matter, both arrays hold what they would.  ``unavailable`` nodes are fed or never materialised; ``roles`` are
+    - an elementwise sum or a per-activation batch norm, its reader a ReLU;
+    - an elementwise sum, its reader a ReLU backward whose upstream gradient it is;
+    - the ReLU backward behind such a batch norm, its reader that batch norm's backward.
+
+    Returns S -> reader.  Both run at S's place: the reader's other operands have to precede S.  Other readers of either
+    do not matter, both arrays hold what they would.  ``unavailable`` nodes are fed or never materialised; ``roles`` are
     the fused roles, of which only a backward that takes its mask from the ReLU's output can join."""
     at = {n: i for i, n in enumerate(topo_order)}
     joins, taken = {}, unavailable | {n for n, role in roles.items() if role[0] != "mask_from_output"}
+
+    def is_sum(s):
+        return (isinstance(s.op, ad.AddOp) and len(s.inputs) == 2   # a (1,)-shaped operand is applied as a constant
+                and shapes[s.inputs[0]] == shapes[s.inputs[1]] == shapes[s])
+
+    def is_norm(s):
+        return isinstance(s.op, ad.BNForwardOp) and s.batchNormMode == "pre_activation"
+
     for r in topo_order:
         if r in taken:
             continue
-        if isinstance(r.op, ad.ActivationForwardOp):
-            s, before = r.inputs[0], []
-        elif isinstance(r.op, ad.ActivationBackwardOp):
-            s, before = r.inputs[1], roles[r][2] if r in roles else r.inputs
-            before = [n for n in before if n is not s]
+        if isinstance(r.op, ad.ActivationForwardOp) and r.activationMode == "relu":
+            s, others = r.inputs[0], []
+            fits = is_sum(s) or is_norm(s)
+        elif isinstance(r.op, ad.ActivationBackwardOp) and r.activationMode == "relu":
+            s, others = r.inputs[1], roles[r][2] if r in roles else r.inputs
+            others = [n for n in others if n is not s]
+            fits = is_sum(s)
+        elif isinstance(r.op, ad.BNBackwardOp) and r.batchNormMode == "pre_activation":
+            s, others = r.inputs[1], r.inputs[:1]
+            fits = (isinstance(s.op, ad.ActivationBackwardOp) and s.activationMode == "relu" and s not in roles
+                    and is_norm(s.inputs[0]) and s.inputs[0].Save_p is r.Save_p and s.inputs[0].inputs[0] is r.inputs[0])
         else:
             continue
-        if r.activationMode != "relu" or s in taken or s in joins or not isinstance(s.op, ad.AddOp):
-            continue
-        if not (len(s.inputs) == 2 and shapes[s.inputs[0]] == shapes[s.inputs[1]] == shapes[s]):
-            continue   # a (1,)-shaped operand is applied as a constant
-        if unavailable & set(s.inputs) or any(at[n] > at[s] for n in before):
+        if not fits or s in taken or unavailable & set(s.inputs) or any(at[n] >= at[s] for n in others):
             continue
         joins[s] = r
+        taken |= {r, s}
     return joins
 
 
-def _join_compute(node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream):
-    """Plan entry of a join: ``node`` is the ReLU or its backward, ``input_vals`` the two operands of the sum and then
-    what ``node`` reads, ``output_val`` the arrays of the sum and of ``node``."""
-    a, b = input_vals[:2]
-    total, out = output_val
-    if isinstance(node.op, ad.ActivationForwardOp):
-        gpu_op.add_activation_forward(a, b, total, out, node.cudnnlist[0], cudnnHandle, cudaStream)
+def _join_compute(first, reader):
+    """Plan entry (same signature as ``Op.compute``) of a join: ``input_vals`` are what ``first`` reads and then what
+    ``reader`` reads, ``output_val`` the arrays of both."""
+    if isinstance(first.op, ad.BNForwardOp):
+        def compute(node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream):
+            wanted = gpu_op.bn_and_relu_forward(input_vals[0], output_val[0], output_val[1], first.batchNormMode, first.n,
+                                                first.Save_p[0], first.Save_p[1], first.cudnnlist[0],
+                                                reader.cudnnlist[0], cudnnHandle, cudaStream)
+            first.n += 1
+            return wanted
+    elif isinstance(first.op, ad.ActivationBackwardOp):
+        def compute(node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream):
+            bn_out, dy, relu_out, x = input_vals[:4]
+            return gpu_op.bn_and_relu_backward(x, bn_out, relu_out, dy, output_val[0], output_val[1],
+                                               reader.batchNormMode, reader.Save_p[0], reader.Save_p[1],
+                                               reader.cudnnlist[0], first.cudnnlist[0], cudnnHandle, cudaStream)
+    elif isinstance(reader.op, ad.ActivationForwardOp):
+        def compute(node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream):
+            a, b = input_vals[:2]
+            gpu_op.add_activation_forward(a, b, output_val[0], output_val[1], reader.cudnnlist[0], cudnnHandle,
+                                          cudaStream)
+            return 0
     else:
-        x, y = input_vals[2], input_vals[4]
-        gpu_op.add_activation_backward(a, b, total, x, out, y, node.cudnnlist[0], cudnnHandle, cudaStream)
-    return 0
+        def compute(node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream):
+            a, b, x, _, y = input_vals
+            gpu_op.add_activation_backward(a, b, output_val[0], x, output_val[1], y, reader.cudnnlist[0], cudnnHandle,
+                                           cudaStream)
+            return 0
+    return compute
 
 
 def _known_scalar_compute(node, shapes):

@@ -44,16 +44,18 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // rows, so rows N..NREG-1 read as zero and their stores are dropped by the bounds
 // check: no per-row branch.  Needs NREG * L * 4 < 2^32 (the row offsets are 32-bit).
 // RELU: y = max(bn(x), 0) in the same pass (the fused entry points below).
+// BOTH: also bn(x) itself, to `plain`: 12 bytes per element where batch norm and ReLU apart move 16.
 // FULL: N == NREG, no row needs masking in the variance.
-template <int NREG, bool RELU, bool FULL>
+template <int NREG, bool RELU, bool BOTH, bool FULL>
 __global__ __launch_bounds__(kThreads) void bn_pa_forward_kernel(const float *__restrict__ x,
-                                                                float *__restrict__ y,
+                                                                float *__restrict__ y, float *__restrict__ plain,
                                                                 float *__restrict__ save_mean,
                                                                 float *__restrict__ save_istd, int N, uint32_t L) {
   const uint32_t l = blockIdx.x * kThreads + threadIdx.x;
   if (l >= L) return;
   const uint32_t col = l * 4u, row = L * 4u;
   const __amdgpu_buffer_rsrc_t rx = gemm::make_rsrc(x, (uint32_t)N * row), ry = gemm::make_rsrc(y, (uint32_t)N * row);
+  const __amdgpu_buffer_rsrc_t rp = BOTH ? gemm::make_rsrc(plain, (uint32_t)N * row) : ry;
   float v[NREG];
 #pragma unroll
   for (int n = 0; n < NREG; ++n)
@@ -74,6 +76,7 @@ __global__ __launch_bounds__(kThreads) void bn_pa_forward_kernel(const float *__
 #pragma unroll
   for (int n = 0; n < NREG; ++n) {
     const float out = (v[n] - mean) * istd;
+    if (BOTH) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, out), rp, (int)col, (int)(n * row), 0);
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, (RELU && out < 0.f) ? 0.f : out), ry, (int)col,
                                           (int)(n * row), 0);
   }
@@ -184,11 +187,12 @@ __global__ __launch_bounds__(kThreads) void bn_pa_forward_tiles_kernel(const flo
 
 // dx = istd/N * (N*dy - sum(dy) - xhat * sum(dy*xhat))
 // RELU: dy is first masked with bn(x) > 0, i.e. the gradient of max(bn(x), 0).
+// BOTH: the masked dy goes to `masked` as well: 16 bytes per element where the two gradients apart move 20.
 // Addressing as in the forward kernel; a row beyond N reads dy = 0 and adds nothing.
-template <int NREG, bool RELU>
+template <int NREG, bool RELU, bool BOTH>
 __global__ __launch_bounds__(kThreads) void bn_pa_backward_kernel(const float *__restrict__ x,
                                                                  const float *__restrict__ dy,
-                                                                 float *__restrict__ dx,
+                                                                 float *__restrict__ dx, float *__restrict__ masked,
                                                                  const float *__restrict__ save_mean,
                                                                  const float *__restrict__ save_istd, int N,
                                                                  uint32_t L) {
@@ -196,7 +200,7 @@ __global__ __launch_bounds__(kThreads) void bn_pa_backward_kernel(const float *_
   if (l >= L) return;
   const uint32_t col = l * 4u, row = L * 4u, all = (uint32_t)N * row;
   const __amdgpu_buffer_rsrc_t rx = gemm::make_rsrc(x, all), rg = gemm::make_rsrc(dy, all),
-                               ro = gemm::make_rsrc(dx, all);
+                               ro = gemm::make_rsrc(dx, all), rm = BOTH ? gemm::make_rsrc(masked, all) : ro;
   const float mean = save_mean[l], istd = save_istd[l];
   float xh[NREG], g[NREG];
 #pragma unroll
@@ -209,6 +213,7 @@ __global__ __launch_bounds__(kThreads) void bn_pa_backward_kernel(const float *_
   for (int n = 0; n < NREG; ++n) {
     xh[n] = (xh[n] - mean) * istd;
     if (RELU) g[n] = xh[n] > 0.f ? g[n] : 0.f;
+    if (BOTH) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, g[n]), rm, (int)col, (int)(n * row), 0);
     s1 += g[n];
     s2 += g[n] * xh[n];
   }
@@ -560,17 +565,23 @@ __global__ __launch_bounds__(kThreads) void bn_sp_apply_kernel(const float *__re
   }
 }
 
-template <int NREG, bool RELU>
-void pa_forward(dim3 grid, dim3 block, hipStream_t s, const float *x, float *y, float *mean, float *istd, int N,
-                uint32_t L) {
+template <int NREG, bool RELU, bool BOTH>
+void pa_forward(dim3 grid, dim3 block, hipStream_t s, const float *x, float *y, float *plain, float *mean, float *istd,
+                int N, uint32_t L) {
   if (N == NREG)
-    hipLaunchKernelGGL((bn_pa_forward_kernel<NREG, RELU, true>), grid, block, 0, s, x, y, mean, istd, N, L);
+    hipLaunchKernelGGL((bn_pa_forward_kernel<NREG, RELU, BOTH, true>), grid, block, 0, s, x, y, plain, mean, istd, N, L);
   else
-    hipLaunchKernelGGL((bn_pa_forward_kernel<NREG, RELU, false>), grid, block, 0, s, x, y, mean, istd, N, L);
+    hipLaunchKernelGGL((bn_pa_forward_kernel<NREG, RELU, BOTH, false>), grid, block, 0, s, x, y, plain, mean, istd, N, L);
 }
 
 // The register kernels address row n at the 32-bit byte offset n * L * 4.
 bool pa_rows_addressable(int nreg, int64_t L) { return (int64_t)nreg * L * 4 < ((int64_t)1 << 32); }
+
+// Rows of the register kernel that takes N rows of L columns, 0 where none does.
+int pa_registers(int N, int64_t L) {
+  const int nreg = N <= 32 ? 32 : N <= 64 ? 64 : 128;
+  return N <= 128 && pa_rows_addressable(nreg, L) ? nreg : 0;
+}
 
 int sp_chunks(int N, int C) {
   // about four workgroups per CU in the partial pass
@@ -633,7 +644,7 @@ extern "C" int DLGpuBatchNormalizationGetCudnnlist(const int *input_shapes, int 
 
 static int bn_forward_impl(const DLArrayHandle input, DLArrayHandle output, int batchNormMode, int n,
                            void **mean_p, void **Variance_p, void ***list, void **handle, int *memorytoSaving,
-                           void **stream, bool relu, const char *what) {
+                           void **stream, bool relu, float *plain, const char *what) {
   (void)handle;
   (void)n;  // would weight running statistics, which the reference never keeps
   BNDesc *d = desc_from_list<BNDesc>(list, kMagicBN);
@@ -670,21 +681,24 @@ static int bn_forward_impl(const DLArrayHandle input, DLArrayHandle output, int 
   if (d->mode == 0) {
     const int64_t L = d->stat_count;
     const dim3 grid(cdiv(L, kThreads)), block(kThreads);  // one lane per column
-    auto run = [&](auto relu_c) {
-      constexpr bool RELU = decltype(relu_c)::value;
+    auto run = [&](auto relu_c, auto both_c) {
+      constexpr bool RELU = decltype(relu_c)::value, BOTH = decltype(both_c)::value;
       const uint32_t l32 = (uint32_t)L;
-      if (d->N <= 32 && pa_rows_addressable(32, L))
-        pa_forward<32, RELU>(grid, block, s, x, y, mean, istd, d->N, l32);
-      else if (d->N <= 64 && pa_rows_addressable(64, L))
-        pa_forward<64, RELU>(grid, block, s, x, y, mean, istd, d->N, l32);
-      else if (d->N <= 128 && pa_rows_addressable(128, L))
-        pa_forward<128, RELU>(grid, block, s, x, y, mean, istd, d->N, l32);
+      const int nreg = pa_registers(d->N, L);
+      if (nreg == 32)
+        pa_forward<32, RELU, BOTH>(grid, block, s, x, y, plain, mean, istd, d->N, l32);
+      else if (nreg == 64)
+        pa_forward<64, RELU, BOTH>(grid, block, s, x, y, plain, mean, istd, d->N, l32);
+      else if (nreg == 128)
+        pa_forward<128, RELU, BOTH>(grid, block, s, x, y, plain, mean, istd, d->N, l32);
       else if (d->N < kFewRows)
         hipLaunchKernelGGL(bn_pa_forward_stream_kernel<RELU>, grid, block, 0, s, x, y, mean, istd, d->N, L);
       else
         bn_pa_forward_tiles<RELU>(s, x, y, mean, istd, d->N, L);
     };
-    if (relu) run(std::true_type{}); else run(std::false_type{});
+    if (plain) run(std::true_type{}, std::true_type{});  // the caller has checked that a register kernel takes it
+    else if (relu) run(std::true_type{}, std::false_type{});
+    else run(std::false_type{}, std::false_type{});
   } else {
     const int chunks = sp_chunks(d->N, d->C);
     const int ipc = cdiv(d->N, chunks);
@@ -734,7 +748,7 @@ extern "C" int DLGpuBatchNormalizationForward(const DLArrayHandle input, DLArray
                                               void **stream) {
   announce_write(output);
   return bn_forward_impl(input, output, batchNormMode, n, mean_p, Variance_p, list, handle, memorytoSaving, stream,
-                         false, "DLGpuBatchNormalizationForward");
+                         false, nullptr, "DLGpuBatchNormalizationForward");
 }
 
 // No counterpart in the reference: y = max(bn(x), 0) in one pass over x (8 bytes per
@@ -746,12 +760,12 @@ extern "C" int DLGpuBatchNormalizationReluForward(const DLArrayHandle input, DLA
                                                   void **stream) {
   announce_write(output);
   return bn_forward_impl(input, output, batchNormMode, n, mean_p, Variance_p, list, handle, memorytoSaving, stream,
-                         true, "DLGpuBatchNormalizationReluForward");
+                         true, nullptr, "DLGpuBatchNormalizationReluForward");
 }
 
 static int bn_backward_impl(const DLArrayHandle input, const DLArrayHandle doutput, DLArrayHandle dinput,
                             int batchNormMode, void **mean_p, void **Variance_p, void ***list, void **handle,
-                            int *memorytoSaving, void **stream, bool relu, const char *what) {
+                            int *memorytoSaving, void **stream, bool relu, float *masked, const char *what) {
   (void)handle;
   BNDesc *d = desc_from_list<BNDesc>(list, kMagicBN);
   TF_REQUIRE(d, "descriptor list was not created by DLGpuBatchNormalizationGetCudnnlist");
@@ -772,21 +786,27 @@ static int bn_backward_impl(const DLArrayHandle input, const DLArrayHandle doutp
     if (d->mode == 0) {
       const int64_t L = d->stat_count;
       const dim3 grid(cdiv(L, kThreads)), block(kThreads);  // one lane per column
-      auto run = [&](auto relu_c) {
-        constexpr bool RELU = decltype(relu_c)::value;
+      auto run = [&](auto relu_c, auto both_c) {
+        constexpr bool RELU = decltype(relu_c)::value, BOTH = decltype(both_c)::value;
         const uint32_t l32 = (uint32_t)L;
-        if (d->N <= 32 && pa_rows_addressable(32, L))
-          hipLaunchKernelGGL((bn_pa_backward_kernel<32, RELU>), grid, block, 0, s, x, dy, dx, mean, istd, d->N, l32);
-        else if (d->N <= 64 && pa_rows_addressable(64, L))
-          hipLaunchKernelGGL((bn_pa_backward_kernel<64, RELU>), grid, block, 0, s, x, dy, dx, mean, istd, d->N, l32);
-        else if (d->N <= 128 && pa_rows_addressable(128, L))
-          hipLaunchKernelGGL((bn_pa_backward_kernel<128, RELU>), grid, block, 0, s, x, dy, dx, mean, istd, d->N, l32);
+        const int nreg = pa_registers(d->N, L);
+        if (nreg == 32)
+          hipLaunchKernelGGL((bn_pa_backward_kernel<32, RELU, BOTH>), grid, block, 0, s, x, dy, dx, masked, mean, istd,
+                             d->N, l32);
+        else if (nreg == 64)
+          hipLaunchKernelGGL((bn_pa_backward_kernel<64, RELU, BOTH>), grid, block, 0, s, x, dy, dx, masked, mean, istd,
+                             d->N, l32);
+        else if (nreg == 128)
+          hipLaunchKernelGGL((bn_pa_backward_kernel<128, RELU, BOTH>), grid, block, 0, s, x, dy, dx, masked, mean, istd,
+                             d->N, l32);
         else if (many_columns(L))
           hipLaunchKernelGGL(bn_pa_backward_stream_kernel<RELU>, grid, block, 0, s, x, dy, dx, mean, istd, d->N, L);
         else
           bn_pa_backward_tiles<RELU>(s, x, dy, dx, mean, istd, d->N, L);
       };
-      if (relu) run(std::true_type{}); else run(std::false_type{});
+      if (masked) run(std::true_type{}, std::true_type{});  // as in the forward pass
+      else if (relu) run(std::true_type{}, std::false_type{});
+      else run(std::false_type{}, std::false_type{});
     } else {
       const int chunks = sp_chunks(d->N, d->C);
       const int ipc = cdiv(d->N, chunks);
@@ -844,7 +864,7 @@ extern "C" int DLGpuBatchNormalizationBackward(const DLArrayHandle input, const 
                                                int *memorytoSaving, void **stream) {
   announce_write(dinput);
   return bn_backward_impl(input, doutput, dinput, batchNormMode, mean_p, Variance_p, list, handle, memorytoSaving,
-                          stream, false, "DLGpuBatchNormalizationBackward");
+                          stream, false, nullptr, "DLGpuBatchNormalizationBackward");
 }
 
 // No counterpart in the reference: gradient of max(bn(x), 0) with respect to x.
@@ -857,5 +877,52 @@ extern "C" int DLGpuBatchNormalizationReluBackward(const DLArrayHandle input, co
                                                    int *memorytoSaving, void **stream) {
   announce_write(dinput);
   return bn_backward_impl(input, doutput, dinput, batchNormMode, mean_p, Variance_p, list, handle, memorytoSaving,
-                          stream, true, "DLGpuBatchNormalizationReluBackward");
+                          stream, true, nullptr, "DLGpuBatchNormalizationReluBackward");
+}
+
+// bn_output = bn(x) and relu_output = max(bn(x), 0): one pass where a register kernel takes the tensor (up to 128 images,
+// per-activation mode), else the two calls that this stands for, with the same bytes.
+extern "C" int DLGpuBatchNormalizationAndReluForward(const DLArrayHandle input, DLArrayHandle bn_output,
+                                                     DLArrayHandle relu_output, int batchNormMode, int n, void **mean_p,
+                                                     void **Variance_p, void ***list, void ***activation_list,
+                                                     void **handle, int *memorytoSaving, void **stream) {
+  const BNDesc *d = desc_from_list<BNDesc>(list, kMagicBN);
+  TF_REQUIRE(d, "descriptor list was not created by DLGpuBatchNormalizationGetCudnnlist");
+  if (check_bn_arrays(d, input, bn_output) != 0 || check_bn_arrays(d, input, relu_output) != 0) return -1;
+  if (d->mode == 0 && batchNormMode == 0 && pa_registers(d->N, d->stat_count) && bn_output->data != relu_output->data) {
+    announce_write(bn_output);
+    announce_write(relu_output);
+    return bn_forward_impl(input, relu_output, batchNormMode, n, mean_p, Variance_p, list, handle, memorytoSaving, stream,
+                           true, (float *)bn_output->data, "DLGpuBatchNormalizationAndReluForward");
+  }
+  int wanted = 0;
+  const int rc = DLGpuBatchNormalizationForward(input, bn_output, batchNormMode, n, mean_p, Variance_p, list, handle,
+                                                &wanted, stream);
+  if (memorytoSaving && wanted) *memorytoSaving = wanted;
+  return rc || wanted ? rc : DLGpuActivationForward(bn_output, relu_output, 1, activation_list, handle, stream);
+}
+
+// drelu = doutput where bn(x) > 0, else 0, and dinput = the batch norm's gradient of it: one pass under the same rule
+// (the mask rebuilt from x and the saved statistics, which has bn_output's bits), else the two calls.
+extern "C" int DLGpuBatchNormalizationAndReluBackward(const DLArrayHandle input, const DLArrayHandle bn_output,
+                                                      const DLArrayHandle relu_output, const DLArrayHandle doutput,
+                                                      DLArrayHandle drelu, DLArrayHandle dinput, int batchNormMode,
+                                                      void **mean_p, void **Variance_p, void ***list,
+                                                      void ***activation_list, void **handle, int *memorytoSaving,
+                                                      void **stream) {
+  const BNDesc *d = desc_from_list<BNDesc>(list, kMagicBN);
+  TF_REQUIRE(d, "descriptor list was not created by DLGpuBatchNormalizationGetCudnnlist");
+  if (check_bn_arrays(d, input, doutput) != 0 || check_bn_arrays(d, drelu, dinput) != 0) return -1;
+  // in place the two calls read what they have written
+  const void *const read[] = {input->data, doutput->data};
+  const bool apart = drelu->data != dinput->data && drelu->data != read[0] && dinput->data != read[1];
+  if (d->mode == 0 && batchNormMode == 0 && pa_registers(d->N, d->stat_count) && apart) {
+    announce_write(drelu);
+    announce_write(dinput);
+    return bn_backward_impl(input, doutput, dinput, batchNormMode, mean_p, Variance_p, list, handle, memorytoSaving,
+                            stream, true, (float *)drelu->data, "DLGpuBatchNormalizationAndReluBackward");
+  }
+  const int rc = DLGpuActivationBackward(bn_output, drelu, relu_output, doutput, 1, activation_list, handle, stream);
+  return rc ? rc : DLGpuBatchNormalizationBackward(input, drelu, dinput, batchNormMode, mean_p, Variance_p, list, handle,
+                                                   memorytoSaving, stream);
 }

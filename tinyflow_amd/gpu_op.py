@@ -396,6 +396,31 @@ def bn_relu_backward(input, doutput, dinput, batchNormMode, mean_p, var_p, cudnn
     return wanted.value
 
 
+def bn_and_relu_forward(input, bn_output, relu_output, batchNormMode, n, mean_p, var_p, cudnnlist, activation_list,
+                        cudnnHandle, cudaStream):
+    """bn_output = bn(input) and relu_output = max(bn_output, 0), in one pass where the batch fits registers (extension)"""
+    _nd_args(input, bn_output, relu_output)
+    mode = _enum(_BATCHNORM, batchNormMode)
+    wanted = ctypes.c_int(0)
+    check_call(_LIB.DLGpuBatchNormalizationAndReluForward(input.handle, bn_output.handle, relu_output.handle, mode, n,
+                                                          mean_p, var_p, cudnnlist, activation_list, cudnnHandle,
+                                                          ctypes.byref(wanted), cudaStream))
+    return wanted.value
+
+
+def bn_and_relu_backward(input, bn_output, relu_output, doutput, drelu, dinput, batchNormMode, mean_p, var_p, cudnnlist,
+                         activation_list, cudnnHandle, cudaStream):
+    """drelu = doutput where bn_output > 0, else 0, and dinput = the batch norm's gradient of it (extension)"""
+    _nd_args(input, bn_output, relu_output, doutput, drelu, dinput)
+    mode = _enum(_BATCHNORM, batchNormMode)
+    wanted = ctypes.c_int(0)
+    check_call(_LIB.DLGpuBatchNormalizationAndReluBackward(input.handle, bn_output.handle, relu_output.handle,
+                                                           doutput.handle, drelu.handle, dinput.handle, mode, mean_p,
+                                                           var_p, cudnnlist, activation_list, cudnnHandle,
+                                                           ctypes.byref(wanted), cudaStream))
+    return wanted.value
+
+
 # ------------------------------------------------------------------- optimizers
 
 def sgd_update(output, g, learning_rate, cudaStream):
