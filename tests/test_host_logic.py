@@ -694,8 +694,9 @@ def test_recompute_schedule_invariants():
 @pytest.mark.parametrize("case,split", [
     (((64, 256, 14, 14), (1024, 256, 1, 1), "VALID", 1), (True, True, True)),
     (((20, 50, 61, 59), (70, 50, 5, 5), "VALID", 2), (True, True, True)),
-    (((64, 47, 14, 14), (1024, 47, 1, 1), "VALID", 1), (False, False, False)),    # fewer than 48 channels on a side
-    (((64, 1024, 14, 14), (47, 1024, 1, 1), "VALID", 1), (False, False, False)),
+    (((64, 23, 14, 14), (1024, 23, 1, 1), "VALID", 1), (False, False, False)),    # fewer than 24 channels on a side
+    (((64, 1024, 14, 14), (23, 1024, 1, 1), "VALID", 1), (False, False, False)),
+    (((32, 24, 56, 56), (96, 24, 5, 5), "SAME", 2), (True, False, False)),        # grad-data by phases: 48 channels
     (((64, 256, 14, 14), (256, 256, 3, 3), "SAME", 1), (False, False, False)),    # 3x3 / stride 1
     (((64, 1024, 14, 14), (2048, 1024, 1, 1), "VALID", 2), (True, True, False)),  # 49 outputs, x gathered by elements
     (((64, 64, 56, 56), (256, 64, 1, 1), "VALID", 1), (True, False, True)),       # grad-data of 64 rows

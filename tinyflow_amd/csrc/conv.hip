@@ -1303,8 +1303,11 @@ double choose_tile_and_splits(ConvPlan &p, bool wgrad, bool padded, bool scatter
 
 // Whether a layer's direct forms may run on the split engine (gemm_split.h).  TINYFLOW_SPLIT in the environment forces
 // the choice (tests and measurements): 0 the fp32 engine, 1 the split engine wherever it has the loaders.
-//   * Fewer than 48 channels on either side leave most of a tile's rows or of its reduction empty, and the time is
-//     the gather's: 5x5, 6 -> 16 channels, 1 000 images 28 us on either.
+//   * Fewer than 24 channels on either side leave most of a tile's rows or of its reduction empty, and the time is
+//     the gather's: 5x5, 6 -> 16 channels, 1 000 images forward 30.7 us on fp32, 27.7 on split, and the networks of
+//     such layers are those of the next point.  Over 17 layers of 24 - 47 channels the choice takes 0.92 of the time of fp32
+//     alone: 7x7, 27 -> 45, 33 x 31, batch 20, 56.6 -> 46.6; 1x1 grad-filter, 40 -> 96, 56 x 56, batch 32, 29.9 -> 22.7;
+//     none is slower, strided grad-data by phases aside (48 channels there, see plan_dgrad).
 //   * 3x3 / stride-1 layers keep the fp32 engine whichever form the planner picks.  Their transformed-domain products
 //     are the form that counts, and networks of such layers under a batch-norm head (VGG-16 with dropout, Adam)
 //     turn any change of rounding into steps of Adam the other way: a different summation order of the fp32 engine
@@ -1316,7 +1319,7 @@ int forced_engine() {
 bool may_use_split(const ConvDesc *d) {
   const int forced = forced_engine();
   if (forced >= 0) return forced != 0;
-  return !(d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1) && d->C >= 48 && d->K >= 48;
+  return !(d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1) && d->C >= 24 && d->K >= 24;
 }
 
 // Grad-filter's gathered x by vectors (SplitGatherAcross MODE 2 and 3): four outputs of one row at a time.
@@ -1339,8 +1342,8 @@ SplitTraffic split_traffic(const ConvDesc *d, int which, bool vec) {
 
 // The direct form on the engine, with the tile and splits, that the models give the least time.  `on_split`: the plan so
 // far for the split engine.  The fp32 model leaves out what every launch costs (4 us here) and underestimates large
-// ones by a seventh: with both corrected, over 300 layers of ResNet-50 at five sizes and random ones (48 - 512 channels,
-// 1x1 to 7x7), 0.86 of the fp32 engine's time in all, the choice within 3 % of the better one except where it keeps fp32.
+// ones by a seventh; the line corrects both.  Over 300 layers of ResNet-50 at five sizes and random ones (48 - 512
+// channels, 1x1 to 7x7) the choice takes 0.86 of the fp32 engine's time in all.
 double choose_direct(ConvPlan &p, ConvPlan on_split, const ConvDesc *d, const SplitTraffic &traffic, bool wgrad, bool padded,
                      bool scatter, bool may_split, double out_bytes) {
   double us = choose_tile_and_splits(p, wgrad, padded, scatter, may_split, out_bytes);
@@ -1734,7 +1737,9 @@ ConvPlan plan_dgrad(const ConvDesc *d) {
           p.bn = t[1];
         }
       }
-      p.split = may_use_split(d);
+      // A phase has a quarter of the taps: below 48 channels fp32 and split take turns, us: 24 -> 24 channels 3x3 stride 2,
+      // 224 x 224, 21.6 and 26.1; 32 -> 64 5x5, 61 x 59, batch 16, 53.8 and 55.5; 30 -> 30, 20 x 20, batch 128, 25.4 and 22.9.
+      p.split = may_use_split(d) && (forced_engine() == 1 || (d->C >= 48 && d->K >= 48));
       p.variant = "dgrad_phases";
       p.epilogue = "StorePhase";
       p.b_mode = 1;
