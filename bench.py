@@ -34,6 +34,8 @@ if ROOT not in sys.path:
 
 PASS_NAMES = {0: "forward", 1: "grad-data", 2: "grad-filter"}
 MFMA_FP32_PEAK_TFLOPS = 157.3
+# dense bf16 over the six products of the three slices that stand for one fp32 product
+MFMA_SPLIT_PEAK_TFLOPS = 2500.0 / 6
 HBM_PEAK_GBPS = 8000.0
 HBM_PEAK_GBS = 8000.0
 
@@ -235,6 +237,9 @@ class HbmTimer(object):
             "activation_backward": lambda a, bits=False: (8.125 if bits else 12) * n(a[0]),
             # a sum with the ReLU behind it, and two adjoints' sum with the ReLU's gradient: with the bits two
             # arrays are read and two written, without them one array more is read
+            # per-activation batch norm with the ReLU behind it, and both gradients, each result written
+            "bn_and_relu_forward": lambda a: 12 * n(a[0]),
+            "bn_and_relu_backward": lambda a: 16 * n(a[0]),
             "add_activation_forward": lambda a, bits=False: (16.125 if bits else 20) * n(a[2]),
             "add_activation_backward": lambda a, bits=False: (16.125 if bits else 20) * n(a[2]),
             "matrix_elementwise_add": lambda a: 12 * n(a[2]),
@@ -502,24 +507,29 @@ def main():
     stats = timer.collect(pair_overhead)
     gpu_step_ms = gpu_ms / args.steps
     traffic = measured_traffic_bytes(args.config, args.batch) if args.bn_mode == "pre_activation" else {}
-    RIDGE = MFMA_FP32_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBPS * 1e9)   # flop per HBM byte where the two roofs meet
+
+    def peak_of(name):
+        """Matrix peak, in fp32 flops, of the engine that a contraction symbol runs on."""
+        return MFMA_SPLIT_PEAK_TFLOPS if "Split" in name else MFMA_FP32_PEAK_TFLOPS
 
     def bound_of(name, launches, total_ms, total_flops):
         """Which roof bounds a contraction symbol: with its counter traffic known, a launch that executes fewer
-        flops per HBM byte than the ridge (19.7) is priced against HBM, not against the matrix pipes."""
+        flops per HBM byte than where the two roofs meet (19.7; 52 on bf16 slices) is priced against HBM, not against the matrix pipes."""
         nbytes = traffic.get(_normalise_symbol(name))
         if not nbytes:
             return {"bound": "mfma", "traffic": None}
         intensity = total_flops / launches / nbytes
         gbps = nbytes * launches / (total_ms * 1e-3) / 1e9
-        return {"bound": "hbm" if intensity < RIDGE else "mfma", "traffic": nbytes, "flop_per_hbm_byte": intensity,
+        ridge = peak_of(name) * 1e12 / (HBM_PEAK_GBPS * 1e9)
+        return {"bound": "hbm" if intensity < ridge else "mfma", "traffic": nbytes, "flop_per_hbm_byte": intensity,
                 "hbm_GBps": gbps, "frac_of_hbm_peak": gbps / HBM_PEAK_GBPS}
 
     def symbol_roofline(which, name, launches, total_ms, total_flops):
         achieved = total_flops / (total_ms * 1e-3) / 1e12
         return {
             "bound": "mfma", "pass": PASS_NAMES[which], "kernel": name, "achieved": achieved,
-            "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / MFMA_FP32_PEAK_TFLOPS,
+            "peak": peak_of(name), "unit": "TFLOP/s", "frac": achieved / peak_of(name),
+            "frac_of_fp32_mfma_peak": achieved / MFMA_FP32_PEAK_TFLOPS,
             "traffic": traffic.get(_normalise_symbol(name)),
             "against_hbm": bound_of(name, launches, total_ms, total_flops),
             "flops_per_launch": total_flops / launches,
@@ -543,13 +553,14 @@ def main():
             return None
         ms = sum(v[1] for _, v in rows)
         flops = sum(v[2] for _, v in rows)
+        at_peak = sum(v[2] / (peak_of(name) * 1e12) for name, v in rows) * 1e3   # ms, each symbol at its engine's peak
         slow_name, slow = min(rows, key=lambda kv: kv[1][2] / kv[1][1])
         return {
-            "executed_tflops": flops / (ms * 1e-3) / 1e12, "frac": flops / (ms * 1e-3) / 1e12 / MFMA_FP32_PEAK_TFLOPS,
-            "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "ms_per_step": ms / event_steps,
+            "executed_tflops": flops / (ms * 1e-3) / 1e12, "frac": at_peak / ms,
+            "peak": flops / (at_peak * 1e-3) / 1e12, "unit": "TFLOP/s", "ms_per_step": ms / event_steps,
             "launches_per_step": sum(v[0] for _, v in rows) / event_steps, "symbols": len(rows),
             "slowest_symbol": dict({"kernel": slow_name, "tflops": slow[2] / (slow[1] * 1e-3) / 1e12,
-                                    "frac": slow[2] / (slow[1] * 1e-3) / 1e12 / MFMA_FP32_PEAK_TFLOPS,
+                                    "frac": slow[2] / (slow[1] * 1e-3) / 1e12 / peak_of(slow_name),
                                     "ms_per_step": slow[1] / event_steps, "launches_per_step": slow[0] / event_steps},
                                    **bound_of(slow_name, slow[0], slow[1], slow[2])),
         }
@@ -567,7 +578,7 @@ def main():
                                 "contraction kernels alone, without transform and split-sum passes"}
         # the single op with the most time in the step, whatever bounds it
         conv_rows = [("%s %s" % (PASS_NAMES[k[0]], k[1]), v[1] / event_steps, "mfma",
-                      v[2] / (v[1] * 1e-3) / 1e12 / MFMA_FP32_PEAK_TFLOPS) for k, v in stats.items()]
+                      v[2] / (v[1] * 1e-3) / 1e12 / peak_of(k[1])) for k, v in stats.items()]
         hbm_rows = [(h["op"], h["avg_launch_us"] * h["launches"] / 2 * 1e-3, "hbm", h["frac_of_hbm_peak"])
                     for h in (hbm_kernels or [])]   # the bandwidth-bound ops were timed over two steps
         if conv_rows or hbm_rows:
