@@ -98,24 +98,61 @@ __global__ __launch_bounds__(kThreads) void midsum_kernel(const float *__restric
 }
 
 // out[j] = sum_chunk partial[chunk*B + j], chunks added in index order.  Bound by the loads' latency (a few
-// KB from the L2): sixteen of them are in flight before the first addition.  One at a time, the 84 to 250
-// chunks of a narrow bias gradient at batch 1000 took 27 us on average.
+// KB from the L2), so all of a round's loads are in flight before its first addition: up to kFinalDepth chunks by
+// the lane that adds them, more by the whole workgroup, which takes 2^log_cols columns and hands the
+// chunks over in LDS, 1024 values a round.  The six sums of a LeNet-5 step at batch 1000, 84
+// chunks and more, us on average: one load at a time 27, kFinalDepth of them 7.0, this way 5.9.
+constexpr int kFinalDepth = 16, kFinalRounds = 4;
+
 __global__ __launch_bounds__(kThreads) void finalsum_kernel(const float *__restrict__ partial,
                                                            float *__restrict__ out, int B, int chunks) {
-  constexpr int DEPTH = 16;
   const int j = blockIdx.x * kThreads + threadIdx.x;
   if (j >= B) return;
-  float s = 0.f;
-  int c = 0;
-  for (; c + DEPTH <= chunks; c += DEPTH) {
-    float v[DEPTH];
+  float v[kFinalDepth], s = 0.f;
 #pragma unroll
-    for (int e = 0; e < DEPTH; ++e) v[e] = partial[(int64_t)(c + e) * B + j];
+  for (int e = 0; e < kFinalDepth; ++e) v[e] = partial[(int64_t)min(e, chunks - 1) * B + j];
 #pragma unroll
-    for (int e = 0; e < DEPTH; ++e) s += v[e];
+  for (int e = 0; e < kFinalDepth; ++e) {
+    if (e < chunks) s += v[e];
   }
-  for (; c < chunks; ++c) s += partial[(int64_t)c * B + j];
   out[j] = s;
+}
+
+__global__ __launch_bounds__(kThreads) void finalsum_tiles_kernel(const float *__restrict__ partial,
+                                                                 float *__restrict__ out, int B, int chunks,
+                                                                 int log_cols) {
+  __shared__ float tile[kFinalRounds * kThreads];
+  const int tid = threadIdx.x, cols = 1 << log_cols, depth = kThreads >> log_cols;
+  const int col = tid & (cols - 1), j = blockIdx.x * cols + col;
+  const float *p = partial + min(j, B - 1);
+  float s = 0.f;
+  for (int c0 = 0; c0 < chunks; c0 += kFinalRounds * depth) {
+    float v[kFinalRounds];
+#pragma unroll
+    for (int e = 0; e < kFinalRounds; ++e) v[e] = p[(int64_t)min(c0 + e * depth + (tid >> log_cols), chunks - 1) * B];
+#pragma unroll
+    for (int e = 0; e < kFinalRounds; ++e) tile[e * kThreads + tid] = v[e];
+    __syncthreads();
+    if (tid < cols) {
+      const int n = min(kFinalRounds * depth, chunks - c0);
+#pragma unroll 16
+      for (int k = 0; k < n; ++k) s += tile[(k << log_cols) + col];
+    }
+    __syncthreads();
+  }
+  if (tid < cols && j < B) out[j] = s;
+}
+
+// 64 columns a workgroup, fewer where that takes the chunks in one round; four at least, a 16-byte piece of a line.
+void launch_finalsum(const float *partial, float *out, int B, int chunks, hipStream_t s) {
+  if (chunks <= kFinalDepth) {
+    hipLaunchKernelGGL(finalsum_kernel, dim3(cdiv(B, kThreads)), dim3(kThreads), 0, s, partial, out, B, chunks);
+    return;
+  }
+  int log_cols = 6;
+  while (log_cols > 2 && (kThreads >> log_cols) * kFinalRounds < chunks) --log_cols;
+  hipLaunchKernelGGL(finalsum_tiles_kernel, dim3(cdiv(B, 1 << log_cols)), dim3(kThreads), 0, s, partial, out, B, chunks,
+                     log_cols);
 }
 
 // Row softmax: one wave per row, max-subtracted.
@@ -310,8 +347,7 @@ int reduce_abc(const float *in, float *out, int64_t A, int64_t B, int64_t C, hip
                        (int)A, (int)B, (int)C, rows_per_chunk);
   }
   if (chunks > 1) {
-    hipLaunchKernelGGL(finalsum_kernel, dim3(cdiv(B, kThreads)), dim3(kThreads), 0, s, partial, out, (int)B,
-                       chunks);
+    launch_finalsum(partial, out, (int)B, chunks, s);
     if (!fixed) device_free(partial);  // stream-ordered reuse: later users are enqueued behind finalsum
   }
   return finish(s, what);
