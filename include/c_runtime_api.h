@@ -449,8 +449,9 @@ int DLGpuAdam_o(void ****n4list, const void ***indexlist, const int count,
                 const float b1, const float b2, const float b1t, const float b2t,
                 const float e, const float learning_rate);
 
-/* No counterpart in the reference, where these run on the default stream: the same on `stream`.  With several
- * streams that run kernels the default stream makes the host wait for all of them. */
+/* No counterpart in the reference, where these run on the default stream: the same on `stream`, with the default
+ * stream's order: behind what other streams that run kernels hold, and in front of what is launched on them later.
+ * (The default stream itself makes the host wait where there are several.) */
 int DLGpuRelu_onStream(const DLArrayHandle in, DLArrayHandle out, void **stream);
 int DLGpuReluGradient_onStream(const DLArrayHandle in, const DLArrayHandle grad, DLArrayHandle out, void **stream);
 /* `written` are the parameters. */
@@ -459,7 +460,8 @@ int DLGpuSgd_o_onStream(void ****n2list, const void ***indexlist, int count, flo
 
 /* No counterpart in the reference, whose fused update runs on the default stream: DLGpuAdam_o on `stream`.
  * `written` are the arrays behind the first three pointer tables (parameters and moments), so that what
- * the library derived from other arrays stays valid. */
+ * the library derived from other arrays stays valid.  Comes in front of what is launched on other streams later, but
+ * does not wait for what they hold. */
 int DLGpuAdam_o_onStream(void ****n4list, const void ***indexlist, int count, float b1, float b2, float b1t,
                          float b2t, float e, float learning_rate, const DLArrayHandle *written,
                          int n_written, void **stream);

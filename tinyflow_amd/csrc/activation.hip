@@ -193,7 +193,7 @@ extern "C" int DLGpuActivationForward(const DLArrayHandle input, DLArrayHandle o
     case 1: {
       const size_t bytes = mask_bytes(n / 4);
       if (d->backward_seen && x != y && mask_shape_ok(n, x, y) && keeping_relu_mask() && keep_has_room(bytes)) {
-        if (mask_t *mask = (mask_t *)device_alloc(bytes)) {
+        if (mask_t *mask = (mask_t *)device_alloc(bytes, s)) {
           hipLaunchKernelGGL(relu_forward_mask_kernel<false>, dim3((unsigned)mask_blocks(n / 4)), dim3(kThreads), 0, s, x,
                              (const float *)nullptr, (float *)nullptr, y, mask, n / 4);
           keep_set(&d->kept_mask, mask, bytes, x, (size_t)n * sizeof(float), s, kMaskTag);
@@ -241,7 +241,7 @@ extern "C" int DLGpuActivationBackward(const DLArrayHandle input, DLArrayHandle 
                              mask, (const float *)nullptr, dy, (const float *)nullptr, (float *)nullptr, dx, n / 4);
           g_masks_used.fetch_add(1);
         }
-        device_free(mask);
+        device_free(mask, s);
         if (usable) return finish(s, "DLGpuActivationBackward");
       }
       return launch_ew<BwdRelu, true, true>(BwdRelu{}, dx, x, dy, n, s, "DLGpuActivationBackward");
@@ -270,10 +270,10 @@ extern "C" int DLGpuMatrixElementwiseAddReluForward(const DLArrayHandle a, const
   if (d->backward_seen && y != ps && mask_shape_ok(n, pa, pb) && mask_shape_ok(n, ps, y) && keeping_relu_mask()) {
     announce_write(sum);
     announce_write(output);
+    hipStream_t s = stream_of(stream);
     const size_t bytes = mask_bytes(n / 4);
-    mask_t *mask = keep_has_room(bytes) ? (mask_t *)device_alloc(bytes) : nullptr;
+    mask_t *mask = keep_has_room(bytes) ? (mask_t *)device_alloc(bytes, s) : nullptr;
     if (mask) {
-      hipStream_t s = stream_of(stream);
       hipLaunchKernelGGL(relu_forward_mask_kernel<true>, dim3((unsigned)mask_blocks(n / 4)), dim3(kThreads), 0, s, pa, pb,
                          ps, y, mask, n / 4);
       keep_set(&d->kept_mask, mask, bytes, ps, (size_t)n * sizeof(float), s, kMaskTag);
@@ -314,7 +314,7 @@ extern "C" int DLGpuMatrixElementwiseAddReluBackward(const DLArrayHandle a, cons
   if (mask_t *mask = (mask_t *)keep_take(&d->kept_mask, x, s, kMaskTag)) {
     hipLaunchKernelGGL((relu_backward_kernel<true, true>), grid, dim3(kThreads), 0, s, mask, x, pa, pb, ps, dx, n / 4);
     g_masks_used.fetch_add(1);
-    device_free(mask);
+    device_free(mask, s);
   } else {
     hipLaunchKernelGGL((relu_backward_kernel<true, false>), grid, dim3(kThreads), 0, s, (const mask_t *)nullptr, x, pa,
                        pb, ps, dx, n / 4);

@@ -656,8 +656,8 @@ static int bn_forward_impl(const DLArrayHandle input, DLArrayHandle output, int 
   hipStream_t s = stream_of(stream);
   const size_t stat_bytes = (size_t)d->stat_count * sizeof(float);
   if (d->saved_mean) {  // a forward whose backward never ran: recycle its statistics
-    device_free(d->saved_mean);
-    device_free(d->saved_istd);
+    device_free(d->saved_mean, d->saved_on);
+    device_free(d->saved_istd, d->saved_on);
     d->saved_mean = d->saved_istd = nullptr;
   }
   // Everything this call allocates, which is what it reports when any of it cannot be had:
@@ -666,15 +666,16 @@ static int bn_forward_impl(const DLArrayHandle input, DLArrayHandle output, int 
   // chunk partials of every channel and, behind them, the channels' pivots
   const size_t sp_partial_bytes = sp_real_chunks ? (size_t)d->C * (sp_real_chunks * 2 * sizeof(double) + sizeof(float)) : 0;
   const size_t all_bytes = 2 * block_bytes(stat_bytes) + (sp_partial_bytes ? block_bytes(sp_partial_bytes) : 0);
-  float *mean = (float *)device_alloc(stat_bytes);
-  float *istd = mean ? (float *)device_alloc(stat_bytes) : nullptr;
+  float *mean = (float *)device_alloc(stat_bytes, s);
+  float *istd = mean ? (float *)device_alloc(stat_bytes, s) : nullptr;
   if (!mean || !istd) {
-    if (mean) device_free(mean);
+    if (mean) device_free(mean, s);
     if (memorytoSaving) *memorytoSaving = shortfall(all_bytes);
     return 0;
   }
   *mean_p = d->saved_mean = mean;
   *Variance_p = d->saved_istd = istd;
+  d->saved_on = s;
   const float *x = (const float *)input->data;
   float *y = (float *)output->data;
   if (numel(input) == 0) return 0;
@@ -703,10 +704,10 @@ static int bn_forward_impl(const DLArrayHandle input, DLArrayHandle output, int 
     const int chunks = sp_chunks(d->N, d->C);
     const int ipc = cdiv(d->N, chunks);
     const int real_chunks = sp_real_chunks;
-    double *partial = (double *)device_alloc(sp_partial_bytes);
+    double *partial = (double *)device_alloc(sp_partial_bytes, s);
     if (!partial) {
-      device_free(mean);
-      device_free(istd);
+      device_free(mean, s);
+      device_free(istd, s);
       *mean_p = d->saved_mean = nullptr;
       *Variance_p = d->saved_istd = nullptr;
       if (memorytoSaving) *memorytoSaving = shortfall(all_bytes);
@@ -737,7 +738,7 @@ static int bn_forward_impl(const DLArrayHandle input, DLArrayHandle output, int 
       }
     };
     if (vec) run(std::true_type{}); else run(std::false_type{});
-    device_free(partial);
+    device_free(partial, s);
   }
   return finish(s, what);
 }
@@ -813,7 +814,7 @@ static int bn_backward_impl(const DLArrayHandle input, const DLArrayHandle doutp
       const int real_chunks = cdiv(d->N, ipc);
       // chunk partials of every channel and, behind them, the channels' two sums
       const size_t pbytes = (size_t)d->C * (real_chunks * 2 * sizeof(double) + 2 * sizeof(float));
-      double *partial = (double *)device_alloc(pbytes);
+      double *partial = (double *)device_alloc(pbytes, s);
       if (!partial) {
         if (memorytoSaving) *memorytoSaving = shortfall(pbytes);
         return 0;  // statistics stay published so the call can be repeated
@@ -847,12 +848,12 @@ static int bn_backward_impl(const DLArrayHandle input, const DLArrayHandle doutp
         }
       };
       if (vec) run(std::true_type{}); else run(std::false_type{});
-      device_free(partial);
+      device_free(partial, s);
     }
   }
   // the saved statistics are consumed (stream-ordered release)
-  device_free(d->saved_mean);
-  device_free(d->saved_istd);
+  device_free(d->saved_mean, s);
+  device_free(d->saved_istd, s);
   *mean_p = d->saved_mean = nullptr;
   *Variance_p = d->saved_istd = nullptr;
   return finish(s, what);

@@ -1846,29 +1846,29 @@ int run_winograd(ConvDesc *d, bool dgrad, const ConvPlan &plan, const float *in,
   const size_t bytes = (w.u_elems + w.v_elems + w.m_elems) * sizeof(float);
   float *kept_V = nullptr;
   if (!dgrad && d->grad_filter_tile == w.tile && keeping_transformed_input() && keep_has_room(w.v_elems * sizeof(float)))
-    kept_V = (float *)device_alloc(w.v_elems * sizeof(float));  // no room: this call keeps nothing
+    kept_V = (float *)device_alloc(w.v_elems * sizeof(float), s);  // no room: this call keeps nothing
   // The transformed filter: a forward call also writes the one grad-data will want (a block
   // of its own, valid until anything writes to the filter); grad-data takes that over.
   float *U_for_dgrad = nullptr, *U_kept = nullptr;
   if (dgrad) d->grad_data_tile = w.tile;
   if (dgrad && keeping_transformed_input()) U_kept = (float *)keep_take(&d->kept_u, filter, s, w.tile);
   if (!dgrad && d->grad_data_tile == w.tile && keeping_transformed_input() && keep_has_room(w.u_elems * sizeof(float)))
-    U_for_dgrad = (float *)device_alloc(w.u_elems * sizeof(float));
+    U_for_dgrad = (float *)device_alloc(w.u_elems * sizeof(float), s);
   // dy: grad-filter may have left grad-data's transform of it, or will want its own
   float *V_kept = nullptr, *dM_for_wgrad = nullptr;
   if (dgrad && w.tile == 4 && dy_transforms_shareable(d) && keeping_transformed_input()) {
     V_kept = (float *)keep_take(&d->kept_dy, in, s, kKeptDyForDgrad | 4);
     if (!V_kept && d->grad_filter_tile == 4 && keep_has_room(w.v_elems * sizeof(float)))
-      dM_for_wgrad = (float *)device_alloc(w.v_elems * sizeof(float));
+      dM_for_wgrad = (float *)device_alloc(w.v_elems * sizeof(float), s);
   }
   const size_t own = bytes - ((kept_V || V_kept) ? w.v_elems * sizeof(float) : 0) - (U_kept ? w.u_elems * sizeof(float) : 0);
-  float *scratch = (float *)device_alloc(own);
+  float *scratch = (float *)device_alloc(own, s);
   if (!scratch) {
-    if (kept_V) device_free(kept_V);
-    if (U_for_dgrad) device_free(U_for_dgrad);
-    if (U_kept) device_free(U_kept);
-    if (V_kept) device_free(V_kept);
-    if (dM_for_wgrad) device_free(dM_for_wgrad);
+    if (kept_V) device_free(kept_V, s);
+    if (U_for_dgrad) device_free(U_for_dgrad, s);
+    if (U_kept) device_free(U_kept, s);
+    if (V_kept) device_free(V_kept, s);
+    if (dM_for_wgrad) device_free(dM_for_wgrad, s);
     if (memorytoSaving) *memorytoSaving = shortfall(bytes);
     return 0;
   }
@@ -1912,9 +1912,9 @@ int run_winograd(ConvDesc *d, bool dgrad, const ConvPlan &plan, const float *in,
   else
     hipLaunchKernelGGL(wino_output_kernel<4>, ogrid, block, 0, s, (const float *)Mt, out, w.Mo, w.out_h, w.out_w,
                        div_tiles, div_tw, w.T, w.Tp, rows_vec, out_bytes);
-  device_free(scratch);
-  if (U_kept) device_free(U_kept);
-  if (V_kept) device_free(V_kept);
+  device_free(scratch, s);
+  if (U_kept) device_free(U_kept, s);
+  if (V_kept) device_free(V_kept, s);
   if (dM_for_wgrad)
     keep_set(&d->kept_dy, dM_for_wgrad, w.v_elems * sizeof(float), in, (size_t)d->N * d->K * d->P * d->Q * sizeof(float),
              s, kKeptDyForWgrad | 4);
@@ -1940,18 +1940,18 @@ int run_winograd_wgrad(ConvDesc *d, const ConvPlan &plan, const float *x, const 
   if (w.tile == 4 && dy_transforms_shareable(d) && keeping_transformed_input()) {
     dM_kept = (float *)keep_take(&d->kept_dy, dy, s, kKeptDyForWgrad | 4);
     if (!dM_kept && d->grad_data_tile == 4 && keep_has_room(w.m_elems * sizeof(float)))
-      V_for_dgrad = (float *)device_alloc(w.m_elems * sizeof(float));
+      V_for_dgrad = (float *)device_alloc(w.m_elems * sizeof(float), s);
   }
   const int KC = d->K * d->C;
   const int bk = stage_depth(plan.bm, plan.bn);
   const Geometry g = make_geometry(d->K, d->C, w.Tp, plan.bm, plan.bn, plan.splits, bk);
   const size_t du_elems = (size_t)g.splits * w.positions * KC;
   const size_t bytes = ((kept_V ? 0 : w.v_elems) + (dM_kept ? 0 : w.m_elems) + du_elems) * sizeof(float);
-  float *scratch = (float *)device_alloc(bytes);
+  float *scratch = (float *)device_alloc(bytes, s);
   if (!scratch) {
-    if (kept_V) device_free(kept_V);
-    if (dM_kept) device_free(dM_kept);
-    if (V_for_dgrad) device_free(V_for_dgrad);
+    if (kept_V) device_free(kept_V, s);
+    if (dM_kept) device_free(dM_kept, s);
+    if (V_for_dgrad) device_free(V_for_dgrad, s);
     if (memorytoSaving) *memorytoSaving = shortfall(bytes);
     return 0;
   }
@@ -1990,9 +1990,9 @@ int run_winograd_wgrad(ConvDesc *d, const ConvPlan &plan, const float *x, const 
     hipLaunchKernelGGL(wino_dfilter_kernel<2>, dim3(cdiv(KC, 64)), block, 0, s, (const float *)dU, dw, KC, g.splits);
   else
     hipLaunchKernelGGL(wino_dfilter_kernel<4>, dim3(cdiv(KC, 64)), block, 0, s, (const float *)dU, dw, KC, g.splits);
-  device_free(scratch);
-  if (kept_V) device_free(kept_V);
-  if (dM_kept) device_free(dM_kept);
+  device_free(scratch, s);
+  if (kept_V) device_free(kept_V, s);
+  if (dM_kept) device_free(dM_kept, s);
   if (V_for_dgrad)
     keep_set(&d->kept_dy, V_for_dgrad, w.m_elems * sizeof(float), dy, (size_t)d->N * d->K * d->P * d->Q * sizeof(float), s,
              kKeptDyForDgrad | 4);
@@ -2174,7 +2174,7 @@ extern "C" int DLGpuConvolution2DForward(const DLArrayHandle input, const DLArra
   float *partial = nullptr;
   if (g.splits > 1) {
     const size_t bytes = (size_t)g.splits * numel(output) * sizeof(float);
-    partial = (float *)device_alloc(bytes);
+    partial = (float *)device_alloc(bytes, s);
     if (!partial) {
       if (memorytoSaving) *memorytoSaving = shortfall(bytes);
       return 0;
@@ -2240,7 +2240,7 @@ extern "C" int DLGpuConvolution2DForward(const DLArrayHandle input, const DLArra
   }, plan.split ? stage_depth(bm, bn) : run_depth(bm, bn, K));
   if (partial) {
     launch_split_sum(partial, (float *)output->data, numel(output), g.splits, s);
-    device_free(partial);
+    device_free(partial, s);
   }
   release_fold(fb);
   return finish(s, "DLGpuConvolution2DForward");
@@ -2304,7 +2304,7 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
   const uint32_t w_bytes = (uint32_t)(numel(filter) * 4), dy_bytes = (uint32_t)(numel(doutput) * 4);
   const int PQ = d->P * d->Q;
   if (dgrad_by_phases(d)) {
-    float *wt = (float *)device_alloc((size_t)numel(filter) * sizeof(float));
+    float *wt = (float *)device_alloc((size_t)numel(filter) * sizeof(float), s);
     if (!wt) {
       if (memorytoSaving) *memorytoSaving = shortfall(block_bytes((size_t)numel(filter) * sizeof(float)));
       return 0;
@@ -2313,7 +2313,7 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
     hipLaunchKernelGGL(filter_to_phases_kernel, dim3(min(cdiv(total, 256), num_cus() * 8)), dim3(256), 0, s,
                        (const float *)filter->data, wt, d->K, d->C, d->R, d->S, d->u, d->v);
     run_dgrad_phases(d, plan, (const float *)doutput->data, wt, (float *)dinput->data, s);
-    device_free(wt);
+    device_free(wt, s);
     return finish(s, "DLGpuConvolutionBackwardData");
   }
   // a strided filter larger than 1x1 that does not run by phases always runs on the small tile, unsplit
@@ -2338,7 +2338,7 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
   const float *wt = (const float *)filter->data;
   float *wt_scratch = nullptr;
   if (wt_bytes) {
-    wt_scratch = (float *)device_alloc(wt_bytes);
+    wt_scratch = (float *)device_alloc(wt_bytes, s);
     if (!wt_scratch) {
       if (memorytoSaving) *memorytoSaving = shortfall(all_bytes);
       return 0;
@@ -2350,15 +2350,15 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
   }
   FoldBuffers fb;
   if (const int rc = acquire_fold(g, g_bm, g_bn, 1, s, fb)) {
-    if (wt_scratch) device_free(wt_scratch);
+    if (wt_scratch) device_free(wt_scratch, s);
     if (rc == 1 && memorytoSaving) *memorytoSaving = shortfall(all_bytes);
     return rc == 1 ? 0 : -1;
   }
   float *partial = nullptr;
   if (partial_bytes) {
-    partial = (float *)device_alloc(partial_bytes);
+    partial = (float *)device_alloc(partial_bytes, s);
     if (!partial) {
-      if (wt_scratch) device_free(wt_scratch);
+      if (wt_scratch) device_free(wt_scratch, s);
       release_fold(fb);
       if (memorytoSaving) *memorytoSaving = shortfall(all_bytes);
       return 0;
@@ -2445,10 +2445,10 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
   }
   if (partial) {
     launch_split_sum(partial, (float *)dinput->data, dx_count, g.splits, s);
-    device_free(partial);
+    device_free(partial, s);
   }
   release_fold(fb);
-  if (wt_scratch) device_free(wt_scratch);
+  if (wt_scratch) device_free(wt_scratch, s);
   return finish(s, "DLGpuConvolutionBackwardData");
 }
 
@@ -2486,7 +2486,7 @@ extern "C" int DLGpuConvolutionBackwardFilter(const DLArrayHandle input, const D
   float *partial = nullptr;
   if (g.splits > 1) {
     const size_t bytes = (size_t)g.splits * M * N * sizeof(float);
-    partial = (float *)device_alloc(bytes);
+    partial = (float *)device_alloc(bytes, s);
     if (!partial) {
       release_fold(fb);
       if (memorytoSaving) *memorytoSaving = shortfall(bytes);
@@ -2577,7 +2577,7 @@ extern "C" int DLGpuConvolutionBackwardFilter(const DLArrayHandle input, const D
   });
   if (partial) {
     launch_split_sum(partial, (float *)dfilter->data, (int64_t)M * N, g.splits, s);
-    device_free(partial);
+    device_free(partial, s);
   }
   release_fold(fb);
   return finish(s, "DLGpuConvolutionBackwardFilter");

@@ -182,14 +182,14 @@ extern "C" int DLGpuDropoutForward(const DLArrayHandle input, DLArrayHandle outp
   // The mask goes back to the pool; the two small host records are only invalidated,
   // not freed, because the caller's old cells still point at them.
   if (in->pending) {
-    device_free(in->pending->reserve);
+    device_free(in->pending->reserve);  // the forward's stream is not kept
     in->pending->reserve = nullptr;
     in->pending->magic = 0;
     in->pending = nullptr;
     in->pending_slots = nullptr;
   }
   const int64_t groups = (in->count + 7) / 8;
-  unsigned char *mask = (unsigned char *)device_alloc((size_t)(groups > 0 ? groups : 1));
+  unsigned char *mask = (unsigned char *)device_alloc((size_t)(groups > 0 ? groups : 1), s);
   if (!mask) {
     if (memorytoSaving) *memorytoSaving = shortfall(groups);
     return 0;
@@ -237,7 +237,7 @@ extern "C" int DLGpuDropoutBackward(const DLArrayHandle doutput, DLArrayHandle d
     in->pending = nullptr;
     in->pending_slots = nullptr;
   }
-  device_free(d->reserve);
+  device_free(d->reserve, s);
   *reserveSpace_p = nullptr;
   d->magic = 0;
   delete d;

@@ -301,13 +301,27 @@ extern "C" int DLGpuReluGradient(const DLArrayHandle in, const DLArrayHandle gra
   return launch_relu_gradient(in, grad, out, streamless_launch_stream(), "DLGpuReluGradient");
 }
 
+// What the *_onStream forms stand for was ordered against every stream by the default stream, and programs of several
+// streams rely on it (an update against the readers of the parameters on other streams): `launch` on the stream, behind what
+// the others hold and in front of what they launch later.  With one stream that runs kernels there is nothing to do.
+template <class F>
+static int ordered_like_default_stream(void **stream, F &&launch) {
+  hipStream_t s = stream_of(stream);
+  if (wait_for_other_streams(s) != 0) return -1;
+  const int rc = launch(s);
+  order_others_behind(s);
+  return rc;
+}
+
 extern "C" int DLGpuRelu_onStream(const DLArrayHandle in, DLArrayHandle out, void **stream) {
-  return launch_relu(in, out, stream_of(stream), "DLGpuRelu_onStream");
+  return ordered_like_default_stream(stream, [&](hipStream_t s) { return launch_relu(in, out, s, "DLGpuRelu_onStream"); });
 }
 
 extern "C" int DLGpuReluGradient_onStream(const DLArrayHandle in, const DLArrayHandle grad, DLArrayHandle out,
                                           void **stream) {
-  return launch_relu_gradient(in, grad, out, stream_of(stream), "DLGpuReluGradient_onStream");
+  return ordered_like_default_stream(stream, [&](hipStream_t s) {
+    return launch_relu_gradient(in, grad, out, s, "DLGpuReluGradient_onStream");
+  });
 }
 
 extern "C" int DLGpuSgdUpdate(DLArrayHandle w, const DLArrayHandle g, float lr, void **stream) {
@@ -630,8 +644,12 @@ extern "C" int DLGpuAdam_o_onStream(void ****n4list, const void ***indexlist, in
                                     int n_written, void **stream) {
   TF_REQUIRE(n_written >= 0 && (written || n_written == 0), "bad arguments");
   for (int i = 0; i < n_written; ++i) announce_write(written[i]);
-  return launch_multi_adam(n4list, indexlist, count, MultiAdam{b1, b2, b1t, b2t, e, learning_rate}, stream_of(stream),
-                           "DLGpuAdam_o_onStream");
+  // does not wait for what other streams hold; what they launch later sees the update
+  hipStream_t s = stream_of(stream);
+  const int rc = launch_multi_adam(n4list, indexlist, count, MultiAdam{b1, b2, b1t, b2t, e, learning_rate}, s,
+                                   "DLGpuAdam_o_onStream");
+  order_others_behind(s);
+  return rc;
 }
 
 static int launch_multi_sgd(void ****n2list, const void ***indexlist, int count, float learning_rate, hipStream_t s,
@@ -664,5 +682,7 @@ extern "C" int DLGpuSgd_o_onStream(void ****n2list, const void ***indexlist, int
                                    const DLArrayHandle *written, int n_written, void **stream) {
   TF_REQUIRE(n_written >= 0 && (written || n_written == 0), "bad arguments");
   for (int i = 0; i < n_written; ++i) announce_write(written[i]);
-  return launch_multi_sgd(n2list, indexlist, count, learning_rate, stream_of(stream), "DLGpuSgd_o_onStream");
+  return ordered_like_default_stream(stream, [&](hipStream_t s) {
+    return launch_multi_sgd(n2list, indexlist, count, learning_rate, s, "DLGpuSgd_o_onStream");
+  });
 }

@@ -68,6 +68,7 @@ struct FoldBuffers {
   float *scratch = nullptr;
   unsigned *tickets = nullptr;
   size_t bytes = 0;
+  hipStream_t stream = nullptr;
 };
 
 // Scratch and tickets for the folded tiles of `g`, entered into `g`: 0 ok (also when
@@ -80,13 +81,14 @@ inline int acquire_fold(Geometry &g, int bm, int bn, int batch, hipStream_t s, F
     fprintf(stderr, "[tinyflow_amd] no memory for the fold counters\n");
     return -1;
   }
-  fb.scratch = (float *)device_alloc(fb.bytes);
+  fb.stream = s;
+  fb.scratch = (float *)device_alloc(fb.bytes, s);
   g.fold_scratch = fb.scratch;
   g.fold_ticket_words = fb.tickets;
   return fb.scratch ? 0 : 1;
 }
 inline void release_fold(FoldBuffers &fb) {
-  if (fb.scratch) device_free(fb.scratch);  // stream-ordered reuse: later users are enqueued behind the kernel
+  if (fb.scratch) device_free(fb.scratch, fb.stream);  // stream-ordered reuse
   fb.scratch = nullptr;
 }
 

@@ -12,11 +12,15 @@
 namespace tf {
 
 // ---- device scratch / array storage: caching allocator (runtime.hip) -------
-// Blocks are recycled by size; a freed block may still be read by kernels that
-// are already enqueued, which is safe because every consumer is ordered after
-// them (same stream, or cross-stream wait inserted by DLArrayCopyFromTo).
-void *device_alloc(size_t bytes);  // nullptr when the device (or the cap) is exhausted
-void device_free(void *p);
+// Blocks are recycled by size; a freed block may still be read by kernels that are
+// already enqueued, so its next user has to come behind them.  `s` is the one stream that
+// the block is used on: a block given back on the stream that takes it next needs nothing,
+// for any other stream device_alloc makes that stream wait for the others.  kAnyStream: the users are
+// not known (arrays, tables); everything launched after device_alloc comes behind
+// everything enqueued before it, on every stream.  Copies order themselves (DLArrayCopyFromTo).
+const hipStream_t kAnyStream = reinterpret_cast<hipStream_t>(~(uintptr_t)0);
+void *device_alloc(size_t bytes, hipStream_t s = kAnyStream);  // nullptr when the device (or the cap) is exhausted
+void device_free(void *p, hipStream_t s = kAnyStream);
 size_t block_bytes(size_t bytes);  // what a block of that many bytes occupies (the allocator's rounding)
 void *pinned_alloc(size_t bytes);
 void pinned_free(void *p);
@@ -24,9 +28,8 @@ void pinned_free(void *p);
 // ---- streams ----------------------------------------------------------------
 hipStream_t stream_of(void **cell);      // cell written by DLGpuCreatecudaStream; NULL -> default stream
 hipStream_t streamless_launch_stream();  // for entry points without a stream argument
-void *pinned_alloc(size_t bytes);
-void pinned_free(void *p);
 int wait_for_other_streams(hipStream_t s);  // `s` behind everything enqueued on the other kernel-running streams
+void order_others_behind(hipStream_t s);    // what is launched from now on on another stream: behind what `s` holds now
 bool other_streams_busy(hipStream_t s);     // whether there is any such thing
 bool idle(hipStream_t s);                   // nothing of what was enqueued on it is left to run
 void feed_forget_stream(hipStream_t s);     // feed.hip: gives back what feeds on the stream keep (waits for it)
@@ -171,6 +174,7 @@ struct BNDesc {
   int64_t stat_count;  // C*HW (per-activation) or C (spatial)
   // statistics published by the last forward and not yet consumed by a backward
   float *saved_mean, *saved_istd;
+  hipStream_t saved_on;  // stream of that forward
 };
 
 struct ReduceDesc {

@@ -317,7 +317,7 @@ extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, co
   float *dst = (float *)matC->data;
   float *partial = nullptr;
   if (g.splits > 1) {
-    partial = (float *)device_alloc((size_t)g.splits * M * N * sizeof(float));
+    partial = (float *)device_alloc((size_t)g.splits * M * N * sizeof(float), s);
     if (!partial) {  // no scratch: fall back to one pass over the whole reduction
       g = make_geometry((int)M, (int)N, (int)K, plan.tile, plan.tile, 1);
     } else {
@@ -349,7 +349,7 @@ extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, co
                      transposeB, ldb, (uint32_t)b_bytes, ep, (int)M, (int)N, (int)K, g, s);
   if (partial) {
     launch_split_sum(partial, (float *)matC->data, M * N, g.splits, s);
-    device_free(partial);
+    device_free(partial, s);
   }
   release_fold(fb);
   return finish(s, "DLGpuMatrixMultiply");

@@ -733,7 +733,7 @@ extern "C" int DLGpuPooling2DBackward(const DLArrayHandle input, const DLArrayHa
     const int64_t windows = numel(doutput);
     // this entry point has no way to report a failed allocation to the caller
     // (no memorytoSaving argument), so it must also work without the scratch
-    unsigned char *tap = (unsigned char *)device_alloc((size_t)windows);
+    unsigned char *tap = (unsigned char *)device_alloc((size_t)windows, s);
     if (tap)
       hipLaunchKernelGGL(pool_argmax_kernel, dim3(grid_for(windows)), dim3(kThreads), 0, s,
                          (const float *)input->data, tap, pp, (uint32_t)windows);
@@ -750,7 +750,7 @@ extern "C" int DLGpuPooling2DBackward(const DLArrayHandle input, const DLArrayHa
                          (const float *)input->data, (const float *)doutput->data, (float *)dinput->data, pp,
                          (uint32_t)total);
     }
-    if (tap) device_free(tap);  // stream-ordered reuse
+    if (tap) device_free(tap, s);  // stream-ordered reuse
   } else {
     hipLaunchKernelGGL(pool_backward_kernel<false>, dim3(grid_for(total)), dim3(kThreads), 0, s,
                        (const unsigned char *)nullptr, (const float *)nullptr, (const float *)doutput->data,

@@ -324,7 +324,7 @@ int reduce_abc(const float *in, float *out, int64_t A, int64_t B, int64_t C, hip
       }
       partial = fixed;
     } else {
-      partial = (float *)device_alloc(bytes);
+      partial = (float *)device_alloc(bytes, s);
     }
     if (!partial) {
       if (scratch_bytes) {
@@ -348,7 +348,7 @@ int reduce_abc(const float *in, float *out, int64_t A, int64_t B, int64_t C, hip
   }
   if (chunks > 1) {
     launch_finalsum(partial, out, (int)B, chunks, s);
-    if (!fixed) device_free(partial);  // stream-ordered reuse: later users are enqueued behind finalsum
+    if (!fixed) device_free(partial, s);  // stream-ordered reuse: later users are enqueued behind finalsum
   }
   return finish(s, what);
 }
@@ -550,12 +550,12 @@ extern "C" int DLGpuSoftmaxCrossEntropy(const DLArrayHandle logits, const DLArra
   hipStream_t s = stream_of(stream);
   const int rows = (int)logits->shape[0], cols = (int)logits->shape[1];
   // this entry point cannot report exhausted scratch: without it the one-launch form runs
-  float *row_loss = rows > 16 ? (float *)device_alloc((size_t)rows * sizeof(float)) : nullptr;
+  float *row_loss = rows > 16 ? (float *)device_alloc((size_t)rows * sizeof(float), s) : nullptr;
   if (row_loss) {
     hipLaunchKernelGGL(softmax_xent_rows_kernel, dim3(cdiv(rows, kThreads / 64)), dim3(kThreads), 0, s,
                        (const float *)logits->data, (const float *)labels->data, row_loss, rows, cols);
     hipLaunchKernelGGL(xent_mean_kernel, dim3(1), dim3(1024), 0, s, (const float *)row_loss, (float *)out->data, rows);
-    device_free(row_loss);
+    device_free(row_loss, s);
   } else {
     hipLaunchKernelGGL(softmax_xent_kernel, dim3(1), dim3(1024), 0, s, (const float *)logits->data,
                        (const float *)labels->data, (float *)out->data, rows, cols);

@@ -25,6 +25,11 @@ struct StreamRec {
   hipEvent_t event;   // reusable marker for cross-stream ordering
   bool runs_kernels;  // an op entry point has launched on it (copy-only streams stay false)
   unsigned *fold_tickets = nullptr;  // counters of the contraction kernels' in-kernel fold (see fold_tickets)
+  // Order points (Runtime::order_points): the last one set on this stream with its event (not recorded while this
+  // was the only stream: there was nobody to order), and the last one that this stream's launches are behind of.
+  uint64_t order_point = 0, ordered_to = 0;
+  hipEvent_t point_event = nullptr;
+  bool point_recorded = false;
 };
 
 __global__ void zero_words_kernel(unsigned *p, int n) {
@@ -33,6 +38,7 @@ __global__ void zero_words_kernel(unsigned *p, int n) {
 }
 
 struct Runtime {
+  static constexpr uint64_t kNoFence = 0;  // storage never handed back since it came from HIP
   std::mutex mu;
   // caching allocator state (one per memory kind)
   struct Pool {
@@ -45,6 +51,18 @@ struct Runtime {
   Pool dev, host;
   size_t dev_limit = 0;  // 0 = unlimited; TINYFLOW_GPU_MEM_LIMIT_MB
 
+  // How a block's storage was last given back: the fence (below) that covers its last use, and the stream of that use.
+  struct Release {
+    uint64_t fence = kNoFence;
+    hipStream_t stream = kAnyStream;
+    bool operator==(const Release &o) const { return fence == o.fence && stream == o.stream; }
+    // A use on `s` needs no wait: the storage is fresh, was used on the same stream, or one of the two is the legacy
+    // default stream, which the streams created here order themselves against.
+    bool in_order_for(hipStream_t s) const {
+      return fence == kNoFence || stream == nullptr || s == nullptr || (s == stream && s != kAnyStream);
+    }
+  };
+
   // Under a budget, device memory comes from one arena obtained with a single
   // hipMalloc and sub-allocated best-fit with coalescing: a step that runs at the
   // budget then never calls hipMalloc / hipFree (hipFree waits for the whole
@@ -56,11 +74,11 @@ struct Runtime {
     bool retired = false;                        // budget changed: serve no new requests
     std::map<size_t, size_t> free_by_off;        // offset -> length
     std::multimap<size_t, size_t> free_by_len;   // length -> offset
-    // release fences by address: non-overlapping segments covering the arena, each with the
-    // fence of the last release that touched it (free ranges coalesce, their histories must not:
+    // releases by address: non-overlapping segments covering the arena, each with the
+    // last release that touched it (free ranges coalesce, their histories must not:
     // a merged range would inherit its youngest neighbour's fence)
-    struct Seg { size_t len; uint64_t fence; };
-    std::map<size_t, Seg> fence_seg;             // offset -> segment
+    struct Seg { size_t len; Release release; };
+    std::map<size_t, Seg> release_seg;           // offset -> segment
     std::unordered_map<void *, size_t> used;     // pointer -> length
   } arena;
   // Release fences.  Every device block remembers the number of the first fence
@@ -72,13 +90,16 @@ struct Runtime {
   // a ring of events; a slot that has been reused holds a later fence of the same
   // stream, which is just as safe to wait for.
   static constexpr int kFenceRing = 1024;
-  static constexpr uint64_t kNoFence = 0;                  // storage never handed back since it came from HIP
   static constexpr uint64_t kConservative = ~(uint64_t)0;  // no single stream to fence on: wait for all
   hipEvent_t fence_ring[kFenceRing] = {};
   uint64_t fence_count = 0;
-  std::unordered_map<void *, uint64_t> pool_fence;   // cached / handed-out pool block -> fence of its last release
+  std::unordered_map<void *, Release> pool_release;  // cached / handed-out pool block -> its last release
   std::unordered_map<void *, uint64_t> block_fence;  // handed-out device block -> fence to honour before reuse
   std::vector<StreamRec> streams;
+  // Order points, counted: whatever another stream launches after one comes behind all that the point's stream held.
+  // The waits are enqueued with the next launch on each other stream (stream_of); a program of one stream records no
+  // event and waits for none.
+  uint64_t order_points = 0;
   bool sync_ops = false;
   int cus = 0;
   bool inited = false;
@@ -111,7 +132,7 @@ void release_cached(Runtime::Pool &p, bool device, size_t need, size_t limit) {
     auto it = std::prev(p.free_blocks.end());
     if (device) {
       (void)hipFree(it->second);
-      rt().pool_fence.erase(it->second);
+      rt().pool_release.erase(it->second);
     } else {
       (void)hipHostFree(it->second);
     }
@@ -139,53 +160,58 @@ void arena_insert_free(Runtime::Arena &a, size_t off, size_t len) {
 // Fence numbers grow along the one stream they are recorded on, so the later of two is the larger.
 uint64_t later_fence(uint64_t x, uint64_t y) { return x > y ? x : y; }
 
-// Stamps [off, off + len) with `fence`, splitting the segments it overlaps.
-void arena_set_fence(Runtime::Arena &a, size_t off, size_t len, uint64_t fence) {
+// Stamps [off, off + len) with `release`, splitting the segments it overlaps.
+void arena_set_release(Runtime::Arena &a, size_t off, size_t len, const Runtime::Release &release) {
   const size_t end = off + len;
-  auto it = a.fence_seg.upper_bound(off);
-  if (it != a.fence_seg.begin()) --it;
-  while (it != a.fence_seg.end() && it->first < end) {
+  auto it = a.release_seg.upper_bound(off);
+  if (it != a.release_seg.begin()) --it;
+  while (it != a.release_seg.end() && it->first < end) {
     const size_t s_off = it->first, s_end = it->first + it->second.len;
-    const uint64_t s_fence = it->second.fence;
+    const Runtime::Release s_release = it->second.release;
     if (s_end <= off) {
       ++it;
       continue;
     }
-    it = a.fence_seg.erase(it);
-    if (s_off < off) a.fence_seg[s_off] = {off - s_off, s_fence};          // part in front survives
-    if (s_end > end) it = a.fence_seg.emplace(end, Runtime::Arena::Seg{s_end - end, s_fence}).first;  // part behind
+    it = a.release_seg.erase(it);
+    if (s_off < off) a.release_seg[s_off] = {off - s_off, s_release};      // part in front survives
+    if (s_end > end) it = a.release_seg.emplace(end, Runtime::Arena::Seg{s_end - end, s_release}).first;  // part behind
   }
-  auto mine = a.fence_seg.emplace(off, Runtime::Arena::Seg{len, fence}).first;
+  auto mine = a.release_seg.emplace(off, Runtime::Arena::Seg{len, release}).first;
   // fold equal neighbours together so the map stays as small as the arena's block structure
   auto next = std::next(mine);
-  if (next != a.fence_seg.end() && next->second.fence == fence && mine->first + mine->second.len == next->first) {
+  if (next != a.release_seg.end() && next->second.release == release && mine->first + mine->second.len == next->first) {
     mine->second.len += next->second.len;
-    a.fence_seg.erase(next);
+    a.release_seg.erase(next);
   }
-  if (mine != a.fence_seg.begin()) {
+  if (mine != a.release_seg.begin()) {
     auto prev = std::prev(mine);
-    if (prev->second.fence == fence && prev->first + prev->second.len == mine->first) {
+    if (prev->second.release == release && prev->first + prev->second.len == mine->first) {
       prev->second.len += mine->second.len;
-      a.fence_seg.erase(mine);
+      a.release_seg.erase(mine);
     }
   }
 }
 
-// Latest fence among the segments that [off, off + len) overlaps.
-uint64_t arena_fence_of(const Runtime::Arena &a, size_t off, size_t len) {
-  uint64_t fence = Runtime::kNoFence;
-  auto it = a.fence_seg.upper_bound(off);
-  if (it != a.fence_seg.begin()) --it;
-  for (; it != a.fence_seg.end() && it->first < off + len; ++it)
-    if (it->first + it->second.len > off) fence = later_fence(fence, it->second.fence);
-  return fence;
+// The releases of all segments that [off, off + len) overlaps as one: the latest fence, and a stream only
+// where they agree on it.
+Runtime::Release arena_release_of(const Runtime::Arena &a, size_t off, size_t len) {
+  Runtime::Release all;
+  auto it = a.release_seg.upper_bound(off);
+  if (it != a.release_seg.begin()) --it;
+  for (; it != a.release_seg.end() && it->first < off + len; ++it) {
+    const Runtime::Release &one = it->second.release;
+    if (it->first + it->second.len <= off || one.fence == Runtime::kNoFence) continue;
+    all.stream = all.fence == Runtime::kNoFence || all.stream == one.stream ? one.stream : kAnyStream;
+    all.fence = later_fence(all.fence, one.fence);
+  }
+  return all;
 }
 
-void *arena_alloc(Runtime::Arena &a, size_t want, uint64_t *fence) {
+void *arena_alloc(Runtime::Arena &a, size_t want, Runtime::Release *release) {
   auto it = a.free_by_len.lower_bound(want);  // best fit
   if (it == a.free_by_len.end()) return nullptr;
   const size_t len = it->first, off = it->second;
-  *fence = arena_fence_of(a, off, want);
+  *release = arena_release_of(a, off, want);
   arena_erase_free(a, off, len);
   if (len > want) arena_insert_free(a, off + want, len - want);
   void *ptr = a.base + off;
@@ -194,15 +220,14 @@ void *arena_alloc(Runtime::Arena &a, size_t want, uint64_t *fence) {
   return ptr;
 }
 
-// Returns false when `ptr` does not belong to the arena.  `fence` is the release
-// fence of the block.
-bool arena_free(Runtime::Arena &a, void *ptr, uint64_t fence) {
+// Returns false when `ptr` does not belong to the arena.
+bool arena_free(Runtime::Arena &a, void *ptr, const Runtime::Release &release) {
   auto it = a.used.find(ptr);
   if (it == a.used.end()) return false;
   size_t off = (size_t)((char *)ptr - a.base), len = it->second;
   a.used_bytes -= len;
   a.used.erase(it);
-  arena_set_fence(a, off, len, fence);
+  arena_set_release(a, off, len, release);
   auto next = a.free_by_off.lower_bound(off);
   if (next != a.free_by_off.end() && next->first == off + len) {  // merge with the range behind
     const size_t nlen = next->second;
@@ -227,12 +252,27 @@ bool arena_free(Runtime::Arena &a, void *ptr, uint64_t fence) {
   return true;
 }
 
-void *pool_alloc(Runtime::Pool &p, size_t bytes, bool device, size_t limit) {
+bool several_kernel_streams(const Runtime &r) {
+  int n = 0;
+  for (const auto &rec : r.streams) n += rec.runs_kernels ? 1 : 0;
+  return n > 1;
+}
+
+// `s`: of the cached blocks that fit, one that this stream can use without a wait is taken first.
+void *pool_alloc(Runtime::Pool &p, size_t bytes, bool device, size_t limit, hipStream_t s) {
   const size_t want = round_size(bytes);
   void *ptr = nullptr;
   auto it = p.free_blocks.lower_bound(want);
   // accept a cached block when it wastes at most 1/8 of its size
-  if (it != p.free_blocks.end() && it->first - want <= it->first / 8) {
+  auto fits = [&](auto at) { return at != p.free_blocks.end() && at->first - want <= at->first / 8; };
+  if (fits(it)) {
+    if (device && s != kAnyStream && several_kernel_streams(rt())) {
+      for (auto at = it; fits(at); ++at)
+        if (rt().pool_release[at->second].in_order_for(s)) {
+          it = at;
+          break;
+        }
+    }
     ptr = it->second;
     p.free_blocks.erase(it);
   }
@@ -285,7 +325,7 @@ void arena_open(Runtime &r) {
   r.arena.base = (char *)base;
   r.arena.size = size;
   arena_insert_free(r.arena, 0, size);
-  r.arena.fence_seg[0] = {size, Runtime::kNoFence};
+  r.arena.release_seg[0] = {size, Runtime::Release{}};
 }
 
 // Records a release fence on the one stream that runs kernels and returns its
@@ -317,26 +357,96 @@ uint64_t record_release_fence(Runtime &r) {
 
 size_t block_bytes(size_t bytes) { return round_size(bytes); }
 
+// ---- order between streams ----------------------------------------------------------
+bool idle(hipStream_t s) {
+  const bool nothing_pending = hipStreamQuery(s) == hipSuccess;
+  if (!nothing_pending) (void)hipGetLastError();
+  return nothing_pending;
+}
+
+// A stream that is being captured into a graph can neither be asked nor wait for work outside of the graph; when that
+// runs is its owner's affair.
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) (void)hipGetLastError();
+  return status != hipStreamCaptureStatusNone;
+}
+
+// `s` behind all that is enqueued on `other`; false when that cannot be had.  With the lock held.
+static bool wait_for_stream(StreamRec &other, hipStream_t s) {
+  if (other.stream == s || !other.runs_kernels || capturing(s) || capturing(other.stream) || idle(other.stream)) return true;
+  return hipEventRecord(other.event, other.stream) == hipSuccess && hipStreamWaitEvent(s, other.event, 0) == hipSuccess;
+}
+
+static void host_waits_instead() {
+  (void)hipGetLastError();
+  (void)hipDeviceSynchronize();
+}
+
+// With the lock held.
+static void set_order_point(Runtime &r, StreamRec &rec) {
+  if (capturing(rec.stream)) return;
+  if (rec.ordered_to == r.order_points) ++rec.ordered_to;  // a stream's own point asks nothing of it
+  rec.order_point = ++r.order_points;
+  rec.point_recorded = false;
+  if (!several_kernel_streams(r)) return;
+  rec.point_recorded = hipEventRecord(rec.point_event, rec.stream) == hipSuccess;
+  if (!rec.point_recorded) host_waits_instead();
+}
+
+// The launches that follow on `rec` behind the order points that other streams have set.  With the lock held.
+static void come_behind_order_points(Runtime &r, StreamRec &rec) {
+  if (rec.ordered_to == r.order_points || capturing(rec.stream)) return;
+  for (auto &other : r.streams) {
+    if (other.order_point <= rec.ordered_to || &other == &rec) continue;
+    if (!(other.point_recorded ? hipStreamWaitEvent(rec.stream, other.point_event, 0) == hipSuccess
+                               : wait_for_stream(other, rec.stream)))
+      host_waits_instead();
+  }
+  rec.ordered_to = r.order_points;
+}
+
+// The next use of a block with the history `last`, on `s` (kAnyStream: wherever) comes behind it.  With the lock held.
+static void come_behind_release(Runtime &r, const Runtime::Release &last, hipStream_t s) {
+  if (last.in_order_for(s)) return;
+  for (auto &rec : r.streams) {
+    if (!rec.runs_kernels || (last.stream != kAnyStream && last.stream != rec.stream)) continue;
+    if (s != kAnyStream) {
+      if (!wait_for_stream(rec, s)) host_waits_instead();
+    } else if (!several_kernel_streams(r) || capturing(rec.stream) || !idle(rec.stream)) {
+      set_order_point(r, rec);
+    }
+  }
+}
+
+void order_others_behind(hipStream_t s) {
+  Runtime &r = rt();
+  std::lock_guard<std::mutex> g(r.mu);
+  for (auto &rec : r.streams)
+    if (rec.stream == s) set_order_point(r, rec);
+}
+
 int drop_all_kept();  // below, with the registry of kept blocks
-static void *device_alloc_once(size_t bytes);
+static void *device_alloc_once(size_t bytes, hipStream_t s);
 // Blocks kept for a later call (keep_set) are a convenience, never a reason to fail:
 // when the device has no room, they are given back and the request is tried again.
-void *device_alloc(size_t bytes) {
-  void *p = device_alloc_once(bytes);
-  if (!p && drop_all_kept() > 0) p = device_alloc_once(bytes);
+void *device_alloc(size_t bytes, hipStream_t s) {
+  void *p = device_alloc_once(bytes, s);
+  if (!p && drop_all_kept() > 0) p = device_alloc_once(bytes, s);
   return p;
 }
-static void *device_alloc_once(size_t bytes) {
+static void *device_alloc_once(size_t bytes, hipStream_t s) {
   Runtime &r = rt();
   std::lock_guard<std::mutex> g(r.mu);
   r.init();
   if (r.dev_limit != 0) {
     if (!r.arena.base) arena_open(r);
     if (r.arena.base && !r.arena.retired) {
-      uint64_t fence = Runtime::kNoFence;
-      void *ptr = arena_alloc(r.arena, round_size(bytes), &fence);
+      Runtime::Release last;
+      void *ptr = arena_alloc(r.arena, round_size(bytes), &last);
       if (ptr) {
-        r.block_fence[ptr] = fence;
+        r.block_fence[ptr] = last.fence;
+        come_behind_release(r, last, s);
         const size_t total = r.dev.in_use + r.arena.used_bytes;
         if (total > r.dev.peak_in_use) r.dev.peak_in_use = total;
       }
@@ -346,23 +456,25 @@ static void *device_alloc_once(size_t bytes) {
   // blocks still alive in an arena that an earlier budget left behind count against this one
   size_t limit = r.dev_limit;
   if (limit != 0 && r.arena.base) limit = limit > r.arena.used_bytes ? limit - r.arena.used_bytes : 1;
-  void *ptr = pool_alloc(r.dev, bytes, true, limit);
+  void *ptr = pool_alloc(r.dev, bytes, true, limit, s);
   if (ptr) {
-    auto it = r.pool_fence.find(ptr);
-    r.block_fence[ptr] = it == r.pool_fence.end() ? Runtime::kNoFence : it->second;
+    auto it = r.pool_release.find(ptr);
+    const Runtime::Release last = it == r.pool_release.end() ? Runtime::Release{} : it->second;
+    r.block_fence[ptr] = last.fence;
+    come_behind_release(r, last, s);
   }
   return ptr;
 }
-void device_free(void *p) {
+void device_free(void *p, hipStream_t s) {
   if (!p) return;
   Runtime &r = rt();
   std::lock_guard<std::mutex> g(r.mu);
   if (r.block_fence.erase(p) == 0) return;  // not a block handed out by device_alloc
   // the next fence to be recorded covers this release (an event per release would put
   // a marker into the compute stream each time: measured 0.75 ms per ResNet-50 step)
-  const uint64_t fence = r.fence_count + 1;
-  if (r.arena.base && arena_free(r.arena, p, fence)) return;
-  r.pool_fence[p] = fence;
+  const Runtime::Release release{r.fence_count + 1, s};
+  if (r.arena.base && arena_free(r.arena, p, release)) return;
+  r.pool_release[p] = release;
   pool_free(r.dev, p);
   // a pool block returned while a budget is active must not linger in the cache
   if (r.dev_limit != 0 && r.arena.base) release_cached(r.dev, true, 0, 0);
@@ -389,7 +501,7 @@ void *pinned_alloc(size_t bytes) {
   Runtime &r = rt();
   std::lock_guard<std::mutex> g(r.mu);
   r.init();
-  return pool_alloc(r.host, bytes, false, 0);
+  return pool_alloc(r.host, bytes, false, 0, kAnyStream);
 }
 void pinned_free(void *p) {
   Runtime &r = rt();
@@ -398,7 +510,8 @@ void pinned_free(void *p) {
 }
 
 // Stream an op launches on.  Marks the stream as one that runs kernels, so that
-// copies on other streams know to order themselves behind it.
+// copies on other streams know to order themselves behind it, and brings it behind the
+// order points of the others.
 hipStream_t stream_of(void **cell) {
   if (!cell) return nullptr;
   hipStream_t s = reinterpret_cast<hipStream_t>(*cell);
@@ -407,6 +520,7 @@ hipStream_t stream_of(void **cell) {
   for (auto &rec : r.streams)
     if (rec.stream == s) {
       rec.runs_kernels = true;
+      come_behind_order_points(r, rec);
       break;
     }
   return s;
@@ -587,7 +701,7 @@ size_t kept_cap() {
 
 // with kept_mu held
 void drop_at(size_t i) {
-  if (*kept[i].slot) device_free(*kept[i].slot);
+  if (*kept[i].slot) device_free(*kept[i].slot, kept[i].stream);
   *kept[i].slot = nullptr;
   kept_bytes -= kept[i].block_bytes;
   kept[i] = kept.back();
@@ -682,12 +796,6 @@ extern "C" int DLArrayFree(DLArrayHandle handle) {
 
 namespace tf {
 
-bool idle(hipStream_t s) {
-  const bool nothing_pending = hipStreamQuery(s) == hipSuccess;
-  if (!nothing_pending) (void)hipGetLastError();
-  return nothing_pending;
-}
-
 // Make `s` wait for everything already enqueued on the other kernel-running
 // streams created through DLGpuCreatecudaStream: whatever produced the source, or
 // still reads the destination's recycled storage, was launched on one of them.
@@ -696,11 +804,8 @@ bool idle(hipStream_t s) {
 int wait_for_other_streams(hipStream_t s) {
   Runtime &r = rt();
   std::lock_guard<std::mutex> g(r.mu);
-  for (auto &rec : r.streams) {
-    if (rec.stream == s || !rec.runs_kernels || idle(rec.stream)) continue;
-    TF_HIP(hipEventRecord(rec.event, rec.stream));
-    TF_HIP(hipStreamWaitEvent(s, rec.event, 0));
-  }
+  for (auto &rec : r.streams)
+    TF_REQUIRE(wait_for_stream(rec, s), "cannot order a stream behind another: %s", hipGetErrorString(hipGetLastError()));
   return 0;
 }
 
@@ -708,7 +813,7 @@ bool other_streams_busy(hipStream_t s) {
   Runtime &r = rt();
   std::lock_guard<std::mutex> g(r.mu);
   for (auto &rec : r.streams)
-    if (rec.stream != s && rec.runs_kernels && !idle(rec.stream)) return true;
+    if (rec.stream != s && rec.runs_kernels && !capturing(rec.stream) && !idle(rec.stream)) return true;
   return false;
 }
 
@@ -863,13 +968,16 @@ extern "C" int DLGpuCreatecudaStream(void **cell) {
   // stream-less entry points (DLGpuRelu, DLGpuReluGradient) launch on the
   // default stream and are ordered against every stream created here.
   TF_HIP(hipStreamCreateWithFlags(&s, hipStreamDefault));
-  hipEvent_t ev = nullptr;
+  hipEvent_t ev = nullptr, point = nullptr;
   TF_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  TF_HIP(hipEventCreateWithFlags(&point, hipEventDisableTiming));
   {
     Runtime &r = rt();
     std::lock_guard<std::mutex> g(r.mu);
     r.init();
-    r.streams.push_back({s, ev, false, nullptr});
+    StreamRec rec{s, ev, false};
+    rec.point_event = point;
+    r.streams.push_back(rec);
   }
   *cell = s;
   return 0;
@@ -880,14 +988,17 @@ extern "C" int DLGpuDestroycudaStream(void **cell) {
   note_write_everything();  // kept blocks are ordered by the stream that made them
   hipStream_t s = reinterpret_cast<hipStream_t>(*cell);
   feed_forget_stream(s);
-  hipEvent_t ev = nullptr;
+  hipEvent_t ev = nullptr, point = nullptr;
   bool found = false;
   {
     Runtime &r = rt();
     std::lock_guard<std::mutex> g(r.mu);
     for (size_t i = 0; i < r.streams.size(); ++i)
       if (r.streams[i].stream == s) {
+        // blocks that were given back on it go to other streams without a wait from here on
+        TF_HIP(hipStreamSynchronize(s));
         ev = r.streams[i].event;
+        point = r.streams[i].point_event;
         if (r.streams[i].fold_tickets) (void)hipFree(r.streams[i].fold_tickets);  // waits for the device
         r.streams.erase(r.streams.begin() + i);
         found = true;
@@ -895,8 +1006,8 @@ extern "C" int DLGpuDestroycudaStream(void **cell) {
       }
   }
   TF_REQUIRE(found, "not a stream created by DLGpuCreatecudaStream");
-  TF_HIP(hipStreamSynchronize(s));
   TF_HIP(hipEventDestroy(ev));
+  TF_HIP(hipEventDestroy(point));
   TF_HIP(hipStreamDestroy(s));
   *cell = nullptr;
   return 0;
