@@ -278,7 +278,7 @@ int feed(DLArrayHandle *from, DLArrayHandle *to, int n, DLStreamHandle stream) {
   }
   if (total == 0) return 0;
   if (!asynchronous(total, stream)) return copy_synchronously(from, to, n);
-  hipStream_t s = stream_of(reinterpret_cast<void **>(stream));
+  hipStream_t s = reinterpret_cast<hipStream_t>(*reinterpret_cast<void **>(stream));
   Feed *f = feed_of(s);
   std::lock_guard<std::mutex> g(f->mu);
   if (const int rc = make_room(*f, total)) return rc > 0 ? copy_synchronously(from, to, n) : -1;
@@ -305,7 +305,7 @@ int feed(DLArrayHandle *from, DLArrayHandle *to, int n, DLStreamHandle stream) {
   // the next one's: what runs there ends first.  The host waits for it, as a synchronous copy would; a queue that waits
   // for another's event slows that one's launches down (ResNet-50 spatial at batch 8, three executors in turn: 4.55 ms a step
   // so, 3.97 with one executor, 4.25 with synchronous copies).
-  if (other_streams_busy(s)) TF_HIP(hipDeviceSynchronize());
+  if (host_waits_for_other_streams(s) != 0) return -1;
   if (direct) {
     if (launch_feed(to, offset.data(), n, slot.host, s) != 0) return -1;
   } else {

@@ -30,6 +30,7 @@ hipStream_t stream_of(void **cell);      // cell written by DLGpuCreatecudaStrea
 hipStream_t streamless_launch_stream();  // for entry points without a stream argument
 int wait_for_other_streams(hipStream_t s);  // `s` behind everything enqueued on the other kernel-running streams
 void order_others_behind(hipStream_t s);    // what is launched from now on on another stream: behind what `s` holds now
+int host_waits_for_other_streams(hipStream_t s);  // the same before a launch on `s`, by waiting here
 bool other_streams_busy(hipStream_t s);     // whether there is any such thing
 bool idle(hipStream_t s);                   // nothing of what was enqueued on it is left to run
 void feed_forget_stream(hipStream_t s);     // feed.hip: gives back what feeds on the stream keep (waits for it)

@@ -25,11 +25,9 @@ struct StreamRec {
   hipEvent_t event;   // reusable marker for cross-stream ordering
   bool runs_kernels;  // an op entry point has launched on it (copy-only streams stay false)
   unsigned *fold_tickets = nullptr;  // counters of the contraction kernels' in-kernel fold (see fold_tickets)
-  // Order points (Runtime::order_points): the last one set on this stream with its event (not recorded while this
-  // was the only stream: there was nobody to order), and the last one that this stream's launches are behind of.
+  // Order points (Runtime::order_points): the last one set on this stream, and the last one that this stream's
+  // launches are behind of.
   uint64_t order_point = 0, ordered_to = 0;
-  hipEvent_t point_event = nullptr;
-  bool point_recorded = false;
 };
 
 __global__ void zero_words_kernel(unsigned *p, int n) {
@@ -97,8 +95,9 @@ struct Runtime {
   std::unordered_map<void *, uint64_t> block_fence;  // handed-out device block -> fence to honour before reuse
   std::vector<StreamRec> streams;
   // Order points, counted: whatever another stream launches after one comes behind all that the point's stream held.
-  // The waits are enqueued with the next launch on each other stream (stream_of); a program of one stream records no
-  // event and waits for none.
+  // Setting one costs nothing.  The wait is enqueued with the next launch on each other stream (stream_of), for what the
+  // point's stream holds by then: an event at each point would cover less, and cost a step as much as its smallest kernels
+  // (MLP at batch 128 in turn with other executors: 208 us a step so, 300 with one).
   uint64_t order_points = 0;
   bool sync_ops = false;
   int cus = 0;
@@ -388,21 +387,13 @@ static void set_order_point(Runtime &r, StreamRec &rec) {
   if (capturing(rec.stream)) return;
   if (rec.ordered_to == r.order_points) ++rec.ordered_to;  // a stream's own point asks nothing of it
   rec.order_point = ++r.order_points;
-  rec.point_recorded = false;
-  if (!several_kernel_streams(r)) return;
-  rec.point_recorded = hipEventRecord(rec.point_event, rec.stream) == hipSuccess;
-  if (!rec.point_recorded) host_waits_instead();
 }
 
 // The launches that follow on `rec` behind the order points that other streams have set.  With the lock held.
 static void come_behind_order_points(Runtime &r, StreamRec &rec) {
   if (rec.ordered_to == r.order_points || capturing(rec.stream)) return;
-  for (auto &other : r.streams) {
-    if (other.order_point <= rec.ordered_to || &other == &rec) continue;
-    if (!(other.point_recorded ? hipStreamWaitEvent(rec.stream, other.point_event, 0) == hipSuccess
-                               : wait_for_stream(other, rec.stream)))
-      host_waits_instead();
-  }
+  for (auto &other : r.streams)
+    if (other.order_point > rec.ordered_to && !wait_for_stream(other, rec.stream)) host_waits_instead();
   rec.ordered_to = r.order_points;
 }
 
@@ -809,12 +800,35 @@ int wait_for_other_streams(hipStream_t s) {
   return 0;
 }
 
-bool other_streams_busy(hipStream_t s) {
-  Runtime &r = rt();
-  std::lock_guard<std::mutex> g(r.mu);
+static bool others_busy(Runtime &r, hipStream_t s) {
   for (auto &rec : r.streams)
     if (rec.stream != s && rec.runs_kernels && !capturing(rec.stream) && !idle(rec.stream)) return true;
   return false;
+}
+
+bool other_streams_busy(hipStream_t s) {
+  Runtime &r = rt();
+  std::lock_guard<std::mutex> g(r.mu);
+  return others_busy(r, s);
+}
+
+int host_waits_for_other_streams(hipStream_t s) {
+  Runtime &r = rt();
+  bool busy;
+  uint64_t points;  // those set meanwhile are not waited for
+  {
+    std::lock_guard<std::mutex> g(r.mu);
+    points = r.order_points;
+    busy = others_busy(r, s);
+  }
+  if (busy) TF_HIP(hipDeviceSynchronize());
+  std::lock_guard<std::mutex> g(r.mu);
+  for (auto &rec : r.streams)
+    if (rec.stream == s) {
+      rec.runs_kernels = true;
+      if (rec.ordered_to < points) rec.ordered_to = points;
+    }
+  return 0;
 }
 
 }  // namespace tf
@@ -968,16 +982,13 @@ extern "C" int DLGpuCreatecudaStream(void **cell) {
   // stream-less entry points (DLGpuRelu, DLGpuReluGradient) launch on the
   // default stream and are ordered against every stream created here.
   TF_HIP(hipStreamCreateWithFlags(&s, hipStreamDefault));
-  hipEvent_t ev = nullptr, point = nullptr;
+  hipEvent_t ev = nullptr;
   TF_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  TF_HIP(hipEventCreateWithFlags(&point, hipEventDisableTiming));
   {
     Runtime &r = rt();
     std::lock_guard<std::mutex> g(r.mu);
     r.init();
-    StreamRec rec{s, ev, false};
-    rec.point_event = point;
-    r.streams.push_back(rec);
+    r.streams.push_back({s, ev, false, nullptr});
   }
   *cell = s;
   return 0;
@@ -988,7 +999,7 @@ extern "C" int DLGpuDestroycudaStream(void **cell) {
   note_write_everything();  // kept blocks are ordered by the stream that made them
   hipStream_t s = reinterpret_cast<hipStream_t>(*cell);
   feed_forget_stream(s);
-  hipEvent_t ev = nullptr, point = nullptr;
+  hipEvent_t ev = nullptr;
   bool found = false;
   {
     Runtime &r = rt();
@@ -998,7 +1009,6 @@ extern "C" int DLGpuDestroycudaStream(void **cell) {
         // blocks that were given back on it go to other streams without a wait from here on
         TF_HIP(hipStreamSynchronize(s));
         ev = r.streams[i].event;
-        point = r.streams[i].point_event;
         if (r.streams[i].fold_tickets) (void)hipFree(r.streams[i].fold_tickets);  // waits for the device
         r.streams.erase(r.streams.begin() + i);
         found = true;
@@ -1007,7 +1017,6 @@ extern "C" int DLGpuDestroycudaStream(void **cell) {
   }
   TF_REQUIRE(found, "not a stream created by DLGpuCreatecudaStream");
   TF_HIP(hipEventDestroy(ev));
-  TF_HIP(hipEventDestroy(point));
   TF_HIP(hipStreamDestroy(s));
   *cell = nullptr;
   return 0;
