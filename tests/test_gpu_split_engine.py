@@ -96,6 +96,35 @@ def test_products_are_no_further_from_float64_than_the_fp32_engine(rt, monkeypat
             assert err[1] <= err[0], (m, k, n, positive, err)
 
 
+@pytest.mark.parametrize("scale_a,scale_b", [
+    (1e-33, 1.0), (1e-35, 1.0), (1e-37, 1.0), (1e-40, 1.0), (1e-44, 1.0),     # down to one bit of a subnormal number
+    (1e-36, 1e30), (1e-37, 1e37), (1e-40, 1e30), (1e-44, 1e37),               # tiny operands of ordinary results
+    (1e-19, 1e-19), (1e-20, 1e-20), (1e-22, 1e-22),                           # results below the normal numbers
+    (1.0, 1e24), (1e30, 1.0), (1e-38, 3e31), (1e12, 1e12), (1e18, 1e18),      # around the scaled range's upper end and past it
+], ids=str)
+@pytest.mark.parametrize("swapped", [False, True], ids=["a", "b"])
+def test_operands_of_any_size_keep_their_bits(rt, monkeypatch, scale_a, scale_b, swapped):
+    """The error is not above the fp32 engine's whatever the exponents are; tiles of ordinary numbers beside tiny ones, rows
+    of zeros and single tiny elements do not matter."""
+    rng = np.random.RandomState(6)
+    m, k, n = 320, 264, 288
+    a, b = rng.normal(0, 1, (m, k)) * scale_a, rng.normal(0, 1, (k, n)) * scale_b
+    ordinary, tiny = np.arange(0, 128), np.arange(128, m)
+    if scale_a < 1:
+        a[ordinary] *= min(1.0, 1.0 / scale_b) / scale_a
+        a[40, 261] = scale_a
+    a[2::9] = 0.0
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    err = []
+    for engine in ("0", "1"):
+        monkeypatch.setenv("TINYFLOW_SPLIT", engine)
+        got = _product(rt, b.T.copy(), False, a.T.copy(), False).T if swapped else _product(rt, a, False, b, False)
+        np.testing.assert_array_equal(got[2::9], 0.0)
+        err.append([np.linalg.norm((got - ref)[rows]) for rows in (ordinary, tiny)])
+    assert err[1][0] <= err[0][0] and err[1][1] <= err[0][1], err
+
+
 def test_what_bf16_cannot_hold_is_computed_in_fp32(rt, monkeypatch):
     """Infinities, NaN, values above the largest bf16 and sums that overflow part way: tiles that meet one have the
     fp32 engine's results, elements of other tiles are not touched by them."""

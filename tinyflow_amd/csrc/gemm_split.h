@@ -18,13 +18,16 @@
 // show.  (In one accumulator the instruction's own rounding adds up to a bias: error against float64 of
 // 4096^3 from 8.1e-7 of the fp32 instruction to 9.4e-7, with two 3.2e-7; 256 x 64 x 200704: 1.05e-7, 1.08e-7, 4.1e-8.)
 //
-// Where the split does not hold - an infinity (its rest is not a number), a finite
-// value above the largest bf16, a sum that overflows part way - some accumulator ends
-// up infinite or NaN.  A workgroup that finds one computes its tile again with
-// the fp32 instruction, so such problems have the results of a plain fp32 product.  (Slices
-// below 2^-133 are lost, so an element under 2^-109 keeps fewer than 24 bits.)
+// Every element is multiplied by 2^23 before it is split, and the sums by 2^-46 at the end: all slices of every
+// fp32 number, subnormal ones included, are then normal bf16 numbers.  (Unscaled, the slices below 2^-133 are lost: error
+// against float64 of K = 264 with operands of 1e-36 2.7e-5, of 1e-40 0.26; scaled 6.7e-8, fp32 engine 2.9e-7.)
 //
-// Operand tiles are fetched as in gemm_core.h, split in registers (eleven vector
+// Where the split does not hold - an infinity (its rest is not a number), a value or a sum that
+// the scaling takes past the largest number (from 2^104 and 2^82 on) - some accumulator ends
+// up infinite or NaN.  A workgroup that finds one computes its tile again with
+// the fp32 instruction, so such problems have the results of a plain fp32 product.
+//
+// Operand tiles are fetched as in gemm_core.h, split in registers (thirteen vector
 // instructions for two elements) and staged through
 // double-buffered LDS as planes [slice][k / 8][row] of 16-byte units: a unit is the eight
 // reduction elements that one lane feeds to one MFMA.  Per MFMA a lane supplies
@@ -32,7 +35,7 @@
 // D[8*(v/4) + 4*(lane/32) + v%4][lane%32], as with the fp32 instruction, so the epilogues are shared.
 //
 // What bounds it: power.  4096^3 runs at 205 TFLOP/s (fp32 engine: 137) and with zeros for data at 300; the
-// matrix instructions alone, out of LDS, at 324.  So the work beside them counts: the splitting (88 of the 98 vector instructions
+// matrix instructions alone, out of LDS, at 324.  So the work beside them counts: the splitting (104 of the 114 vector instructions
 // of a 128 x 128 stage) sits between the matrix instructions, addresses are a lane's constant plus a scalar, and
 // the LDS layouts have no bank conflicts.
 #pragma once
@@ -55,8 +58,12 @@ __device__ inline uint32_t pack_bf16(float a, float b) {
   const f32x2v v = {a, b};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
-// The three slices of two neighbouring reduction elements: eleven instructions.
+constexpr float kScale = 0x1p23f, kUnscale = 0x1p-46f;  // of an element, of a sum of products
+
+// The three slices of two neighbouring reduction elements: thirteen instructions.
 __device__ inline void split_pair(float a, float b, uint32_t (&slice)[3]) {
+  a *= kScale;
+  b *= kScale;
 #pragma unroll
   for (int s = 0; s < 3; ++s) {
     slice[s] = pack_bf16(a, b);
@@ -412,9 +419,12 @@ __global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : 1) void gemm_ker
     al.put(sa, lds + (cur ^ 1) * STAGE, ra[cur ^ 1]);
     bl.put(sb, lds + (cur ^ 1) * STAGE + PA::BYTES, rb[cur ^ 1]);
     // Interleave: the first matrix instructions need the highest slices only; the splitting of the next stage's
-    // values (some 5.5 vector instructions an element) goes between the others, which leave the issue port free.
-    constexpr int MFMAS = 6 * TM * TN * (BK / 16), SPLIT = 6 * (ALoader::EPT + BLoader::EPT) + 8;
-    constexpr int FIRST = MFMAS / 3, PER = (SPLIT + MFMAS - FIRST - 1) / (MFMAS - FIRST);
+    // values (some 6.5 vector instructions an element) goes between the others, which leave the issue port free.  A sixth
+    // of them first: 5x5 stride 2 layer with both gradients 144 us, with a third 149; groups of 9 an element on the 64 x 64
+    // tile: 1000 x 1537 x 777 with both gradients 86 us, of 7 92, which the other tiles like better.
+    constexpr int MFMAS = 6 * TM * TN * (BK / 16);
+    constexpr int SPLIT = (BM == 64 && BN == 64 ? 9 : 7) * (ALoader::EPT + BLoader::EPT) + 8;
+    constexpr int FIRST = MFMAS / 6, PER = (SPLIT + MFMAS - FIRST - 1) / (MFMAS - FIRST);
     __builtin_amdgcn_sched_group_barrier(0x100, 3 * (TM + TN), 0);
     __builtin_amdgcn_sched_group_barrier(0x008, FIRST, 0);
 #pragma unroll
@@ -432,7 +442,7 @@ __global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : 1) void gemm_ker
     stage(std::integral_constant<int, 1>{}, k0 + BK);
   }
 
-  // The split does not hold for infinities and on the way over the largest fp32: see the head of this file.
+  // The split does not hold for infinities and on the way over the largest number: see the head of this file.
   {
     float largest = 0.f;  // propagates NaN
 #pragma unroll
@@ -464,16 +474,32 @@ __global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : 1) void gemm_ker
         al.each(sa, ra[0], [&](int k, int d, float v) { fa[k * LDA + d] = v; });
         bl.each(sb, rb[0], [&](int k, int d, float v) { fb[k * LDB + d] = v; });
         __syncthreads();
+        // a stage is summed apart: the rounding of one long chain would exceed that of the slices
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) low[i][j][v] = 0.f;
 #pragma unroll 1
         for (int k = lhalf; k < BK; k += 2)
 #pragma unroll
           for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[k * LDA + m_wave + 32 * i + lcol],
-                                                               fb[k * LDB + n_wave + 32 * j + lcol], acc[i][j], 0, 0, 0);
+              low[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[k * LDA + m_wave + 32 * i + lcol],
+                                                               fb[k * LDB + n_wave + 32 * j + lcol], low[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
       }
       __syncthreads();
+    } else {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] *= kUnscale;
     }
   }
 
