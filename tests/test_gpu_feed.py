@@ -1,5 +1,7 @@
 """Feeding a step from host memory (csrc/feed.hip): every step sees the batch it was given, whatever the caller does with
 the host arrays afterwards and however far the host is ahead of the GPU."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -82,3 +84,41 @@ def test_steps_equal_those_of_synchronous_feeds(batch):
 
     for a, b in zip(train(False), train(True)):
         assert a.tobytes() == b.tobytes()
+
+
+def _held(rt):
+    from tinyflow_amd import gpu_op
+    return gpu_op.device_memory_stats()[1]
+
+
+@pytest.mark.parametrize("why", ["no room", "a budget"])
+def test_the_buffers_of_feeds_are_given_back(rt, why):
+    """Device memory that feeds hold between steps is there for whoever finds no room, and for a budget.  An array of
+    4 TiB fits no device, so asking for it is a device without room."""
+    from tinyflow_amd import gpu_op, ndarray
+    stream = gpu_op.create_cudaStream()
+    n = 3000017
+    target, kept = ndarray.empty((n,), rt.ctx), ndarray.empty((n,), rt.ctx)
+    gc.collect()   # arrays of other tests
+    before = _held(rt)
+    ndarray.reserve_feed([target], stream)
+    assert _held(rt) >= before + 2 * 4 * n
+    if why == "no room":
+        assert isinstance(ndarray.empty((1 << 40,), rt.ctx), int)
+    else:
+        gpu_op.set_device_memory_limit(4 << 30)
+        gpu_op.set_device_memory_limit(0)
+    assert _held(rt) == before
+    for step in range(3):   # feeds arrive without it, and take it again only where nobody had to go without
+        values = np.full(n, step + 0.5, np.float32)
+        values[step] = -1
+        ndarray.reserve_feed([target], stream)
+        ndarray.feed([(target, values)], stream)
+        gpu_op.matrix_elementwise_multiply_by_const(target, 1.0, kept, stream)
+        assert kept.asnumpy().tobytes() == values.tobytes()
+    if why == "no room":
+        assert _held(rt) == before
+    else:
+        assert _held(rt) >= before + 2 * 4 * n
+    gpu_op.destroy_cudaStream(stream)
+    assert _held(rt) == before

@@ -11,7 +11,9 @@
 //     the host, overlapping with what the caller's stream still runs, and a kernel behind it distributes the buffer.
 //     More than that with nothing to overlap with, a plain copy.
 // Two slots of pinned memory and buffer per stream: a call waits for the last but one before it, so the host is
-// at most two steps ahead.  They belong to the stream and go with it.
+// at most two steps ahead.  They belong to the stream and go with it, or before: when anything else finds no room on the
+// device, or a budget is set (feed_give_back).  A stream whose room could not be had, or was taken back, copies its
+// large feeds synchronously from then on: asking again at every step would empty the allocator's cache each time.
 #include "internal.h"
 
 #include <atomic>
@@ -144,7 +146,14 @@ struct Feed {
   hipEvent_t landed = nullptr;
   Slot slot[2];
   size_t host_bytes = 0, dev_bytes = 0;  // of a slot; both are halves of one block of the pools
+  size_t refused = ~(size_t)0;           // feeds of this many bytes and more have no room
   int next = 0;
+};
+thread_local Feed *feed_in_hand = nullptr;  // whose mutex this thread holds
+struct HoldFeed {
+  explicit HoldFeed(Feed &f) : lock(f.mu) { feed_in_hand = &f; }
+  ~HoldFeed() { feed_in_hand = nullptr; }
+  std::lock_guard<std::mutex> lock;
 };
 std::mutex feeds_mu;
 std::unordered_map<hipStream_t, std::unique_ptr<Feed>> *feeds = nullptr;  // leaked on purpose
@@ -178,7 +187,9 @@ int wait_for_readers(Feed &f) {
   return 0;
 }
 
+// Behind wait_for_readers.
 void drop_memory(Feed &f) {
+  if (f.dev_bytes) (void)hipStreamSynchronize(copy_stream());  // a feed that failed part way leaves copies behind
   if (f.slot[0].host) pinned_free(f.slot[0].host);
   if (f.slot[0].dev) device_free(f.slot[0].dev);
   for (Slot &slot : f.slot) slot.host = slot.dev = nullptr;
@@ -193,16 +204,22 @@ int make_room(Feed &f, size_t bytes) {
   if (!direct && !f.landed) TF_HIP(hipEventCreateWithFlags(&f.landed, hipEventDisableTiming));
   if (!direct && !copy_stream()) return 1;
   if (f.host_bytes >= bytes && (direct || f.dev_bytes >= bytes)) return 0;
+  if (bytes >= f.refused) return 1;
   if (wait_for_readers(f) != 0) return -1;
   drop_memory(f);
+  f.refused = bytes;  // until there is room
   char *host = (char *)pinned_alloc(2 * bytes);
   if (!host) return 1;
+  char *dev = direct ? nullptr : (char *)device_alloc(2 * bytes);
+  if (!direct && !dev) {
+    pinned_free(host);
+    return 1;
+  }
+  f.refused = ~(size_t)0;
   f.slot[0].host = host;
   f.slot[1].host = host + bytes;
   f.host_bytes = bytes;
   if (direct) return 0;
-  char *dev = (char *)device_alloc(2 * bytes);
-  if (!dev) return 1;
   f.slot[0].dev = dev;
   f.slot[1].dev = dev + bytes;
   f.dev_bytes = bytes;
@@ -249,13 +266,29 @@ void feed_forget_stream(hipStream_t s) {
     f = std::move(it->second);
     feeds->erase(it);
   }
-  if (f->dev_bytes) (void)hipStreamSynchronize(copy_stream());
   (void)hipStreamSynchronize(s);
   drop_memory(*f);
   for (Slot &slot : f->slot) {
     if (slot.read) (void)hipEventDestroy(slot.read);
   }
   if (f->landed) (void)hipEventDestroy(f->landed);
+}
+
+// Returns whether any device memory was given back.  A feed that is under way on another thread keeps its own.
+bool feed_give_back(bool for_good) {
+  bool any = false;
+  std::lock_guard<std::mutex> g(feeds_mu);
+  if (!feeds) return false;
+  for (auto &entry : *feeds) {
+    Feed &f = *entry.second;
+    if (&f == feed_in_hand || !f.mu.try_lock()) continue;
+    std::lock_guard<std::mutex> held(f.mu, std::adopt_lock);
+    if (f.dev_bytes == 0 || wait_for_readers(f) != 0) continue;
+    drop_memory(f);
+    if (for_good) f.refused = std::min(f.refused, kDirectBytes + 1);
+    any = true;
+  }
+  return any;
 }
 
 }  // namespace tf
@@ -280,10 +313,10 @@ int feed(DLArrayHandle *from, DLArrayHandle *to, int n, DLStreamHandle stream) {
   if (!asynchronous(total, stream)) return copy_synchronously(from, to, n);
   hipStream_t s = reinterpret_cast<hipStream_t>(*reinterpret_cast<void **>(stream));
   Feed *f = feed_of(s);
-  std::lock_guard<std::mutex> g(f->mu);
-  if (const int rc = make_room(*f, total)) return rc > 0 ? copy_synchronously(from, to, n) : -1;
+  HoldFeed hold(*f);
   // nothing to overlap with: a plain copy is through sooner
   if (total > kDirectBytes && idle(s) && !other_streams_busy(s)) return copy_synchronously(from, to, n);
+  if (const int rc = make_room(*f, total)) return rc > 0 ? copy_synchronously(from, to, n) : -1;
   Slot &slot = f->slot[f->next];
   f->next ^= 1;
   if (slot.pending) TF_HIP(hipEventSynchronize(slot.read));
@@ -346,7 +379,7 @@ extern "C" int DLArrayFeedReserve(DLArrayHandle *to, int n, DLStreamHandle strea
   if (total == 0 || !asynchronous(total, stream)) return 0;
   try {
     Feed *f = feed_of(stream_of(reinterpret_cast<void **>(stream)));
-    std::lock_guard<std::mutex> g(f->mu);
+    HoldFeed hold(*f);
     return make_room(*f, total) < 0 ? -1 : 0;  // without room the feeds are synchronous
   } catch (const std::exception &e) {
     TF_REQUIRE(false, "%s", e.what());

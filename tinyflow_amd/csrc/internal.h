@@ -34,6 +34,7 @@ int host_waits_for_other_streams(hipStream_t s);  // the same before a launch on
 bool other_streams_busy(hipStream_t s);     // whether there is any such thing
 bool idle(hipStream_t s);                   // nothing of what was enqueued on it is left to run
 void feed_forget_stream(hipStream_t s);     // feed.hip: gives back what feeds on the stream keep (waits for it)
+bool feed_give_back(bool for_good);         // the device memory of all feeds; for good: they do without from then on
 bool sync_every_op();                    // TINYFLOW_SYNC_EVERY_OP=1
 int finish(hipStream_t s, const char *what);  // launch-error check (+ optional sync)
 

@@ -419,11 +419,12 @@ void order_others_behind(hipStream_t s) {
 
 int drop_all_kept();  // below, with the registry of kept blocks
 static void *device_alloc_once(size_t bytes, hipStream_t s);
-// Blocks kept for a later call (keep_set) are a convenience, never a reason to fail:
+// Blocks kept for a later call (keep_set) and the feeds' buffers are a convenience, never a reason to fail:
 // when the device has no room, they are given back and the request is tried again.
 void *device_alloc(size_t bytes, hipStream_t s) {
   void *p = device_alloc_once(bytes, s);
   if (!p && drop_all_kept() > 0) p = device_alloc_once(bytes, s);
+  if (!p && feed_give_back(true)) p = device_alloc_once(bytes, s);
   return p;
 }
 static void *device_alloc_once(size_t bytes, hipStream_t s) {
@@ -488,11 +489,16 @@ int wait_for_previous_life(void *ptr, hipStream_t s) {
   }
   return 0;
 }
-void *pinned_alloc(size_t bytes) {
+static void *pinned_alloc_once(size_t bytes) {
   Runtime &r = rt();
   std::lock_guard<std::mutex> g(r.mu);
   r.init();
   return pool_alloc(r.host, bytes, false, 0, kAnyStream);
+}
+void *pinned_alloc(size_t bytes) {
+  void *p = pinned_alloc_once(bytes);
+  if (!p && feed_give_back(true)) p = pinned_alloc_once(bytes);  // the large feeds' pinned memory goes with their buffers
+  return p;
 }
 void pinned_free(void *p) {
   Runtime &r = rt();
@@ -942,6 +948,7 @@ extern "C" int getInt(int *intp) { return intp ? *intp : 0; }
 // are given back until the budget holds; arrays in use are not touched.
 extern "C" int DLGpuSetDeviceMemoryLimit(int64_t bytes) {
   note_write_everything();  // nothing is kept from call to call under a budget
+  if (bytes > 0) (void)feed_give_back(false);
   Runtime &r = rt();
   std::lock_guard<std::mutex> g(r.mu);
   r.init();
