@@ -1161,11 +1161,16 @@ inline int run_depth(int bm, int bn, int K) {
 }
 
 template <class F>
-void with_tile(int bm, int bn, F &&f, int depth = 0) {
-  if (bm == 128 && bn == 128) f(IC<128>{}, IC<128>{}, IC<16>{});
-  else if (bm == 64 && bn == 128) f(IC<64>{}, IC<128>{}, IC<16>{});
-  else if (depth == 16) f(IC<64>{}, IC<64>{}, IC<16>{});
-  else f(IC<64>{}, IC<64>{}, IC<32>{});
+void with_tile(int bm, int bn, F &&f) {
+  auto go = [&](auto bm_c, auto bn_c) { f(bm_c, bn_c, IC<stage_depth(decltype(bm_c)::value, decltype(bn_c)::value)>{}); };
+  if (bm == 128 && bn == 128) go(IC<128>{}, IC<128>{});
+  else if (bm == 64 && bn == 128) go(IC<64>{}, IC<128>{});
+  else go(IC<64>{}, IC<64>{});
+}
+template <class F>
+void with_tile(int bm, int bn, F &&f, int depth) {
+  if (depth != stage_depth(bm, bn)) f(IC<64>{}, IC<64>{}, IC<16>{});  // run_depth has no other
+  else with_tile(bm, bn, f);
 }
 
 // Events a measuring caller wants recorded around the next contraction kernel only
@@ -1174,7 +1179,7 @@ thread_local hipEvent_t next_kernel_start = nullptr, next_kernel_stop = nullptr;
 
 template <int BM, int BN, int BK, class AL, class BL, class EP>
 void launch(const AL &al, const BL &bl, const EP &ep, int K, const Geometry &g, hipStream_t s, int batch = 1) {
-  if constexpr (is_split<AL>::value && BK != stage_depth(BM, BN)) return;  // only the fp32 engine has those (run_depth)
+  static_assert(!is_split<AL>::value || BK == stage_depth(BM, BN), "only the fp32 engine has other depths (run_depth)");
   if (next_kernel_start) (void)hipEventRecord(next_kernel_start, s);
   if constexpr (is_split<AL>::value)
     hipLaunchKernelGGL((split::gemm_kernel<BM, BN, BK, AL, BL, EP>), dim3(g.blocks(), batch), dim3(THREADS), 0, s, al, bl,
@@ -2193,6 +2198,7 @@ extern "C" int DLGpuConvolution2DForward(const DLArrayHandle input, const DLArra
     const int seg = b_vec ? plan.seg : PQ;
     StoreNCHW ep{partial ? partial : (float *)output->data, M, N, FastDiv((uint32_t)seg), PQ, numel(output)};
     if (plan.split) {
+      constexpr int BK = stage_depth(BM, BN);
       auto with_a = [&](const auto &al) {
         if (b_vec) {
           launch<BM, BN, BK>(al, split::SplitAlong4<BN, BK>{(const float *)input->data, x_bytes, PQ, N, K,
@@ -2237,7 +2243,7 @@ extern "C" int DLGpuConvolution2DForward(const DLArrayHandle input, const DLArra
              std::true_type{});
     else
       with_b(PlainAcross<BM, BK>{(const float *)filter->data, w_bytes, K, M, K}, std::false_type{});
-  }, plan.split ? stage_depth(bm, bn) : run_depth(bm, bn, K));
+  }, run_depth(bm, bn, K));
   if (partial) {
     launch_split_sum(partial, (float *)output->data, numel(output), g.splits, s);
     device_free(partial, s);
@@ -2378,39 +2384,40 @@ extern "C" int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLA
     const int seg = (a_vec && b_vec) ? plan.seg : PQ;  // pixels per image in the column index
     with_tile(bm, bn, [&](auto bm_c, auto bn_c, auto bk_c) {
       constexpr int BM = decltype(bm_c)::value, BN = decltype(bn_c)::value, BK = decltype(bk_c)::value;
-      auto with_epilogue = [&](const auto &al, const auto &bl) {
+      auto with_epilogue = [&](auto depth, const auto &al, const auto &bl) {
         if (d->u == 1 && d->v == 1) {
           StoreNCHW ep{dst, M, N, FastDiv((uint32_t)seg), PQ, dx_count};
-          launch<BM, BN, BK>(al, bl, ep, K, g, s);
+          launch<BM, BN, decltype(depth)::value>(al, bl, ep, K, g, s);
         } else {
           StoreScatter ep{(float *)dinput->data, M, N, FastDiv((uint32_t)seg), FastDiv((uint32_t)d->Q),
                           d->H, d->W, d->u, d->v,
                           d->u == 2 && d->v == 2 && d->H % 2 == 0 && d->W % 2 == 0 &&
                               (reinterpret_cast<uintptr_t>(dinput->data) & 7u) == 0,
                           PQ};
-          launch<BM, BN, BK>(al, bl, ep, K, g, s);
+          launch<BM, BN, decltype(depth)::value>(al, bl, ep, K, g, s);
         }
       };
       if (plan.split) {
+        constexpr int BK = stage_depth(BM, BN);
         const split::SplitAlong4<BM, BK> al{wt, w_bytes, d->C, M, K, whole, 0};
         if (b_vec)
-          with_epilogue(al, split::SplitAlong4<BN, BK>{(const float *)doutput->data, dy_bytes, PQ, N, K,
+          with_epilogue(IC<BK>{}, al, split::SplitAlong4<BN, BK>{(const float *)doutput->data, dy_bytes, PQ, N, K,
                                                        FastDiv((uint32_t)seg), d->K * PQ});
         else
-          with_epilogue(al, SplitGatherAlong<BN, BK, 0>{
+          with_epilogue(IC<BK>{}, al, SplitGatherAlong<BN, BK, 0>{
               (const float *)doutput->data, dy_bytes, K, N, FastDiv(1), FastDiv(1), PQ, FastDiv((uint32_t)PQ),
               FastDiv((uint32_t)d->Q), d->K * PQ, d->P, d->Q, 1, 1, 0, 0, -1, 1, 1, FastDiv(1), FastDiv(1)});
       } else if (a_vec && b_vec) {
-        with_epilogue(Along4<BM, BK>{wt, w_bytes, d->C, M, K, whole, 0},
+        with_epilogue(bk_c, Along4<BM, BK>{wt, w_bytes, d->C, M, K, whole, 0},
                       Along4<BN, BK>{(const float *)doutput->data, dy_bytes, PQ, N, K, FastDiv((uint32_t)seg),
                                      d->K * PQ});
       } else {
-        with_epilogue(PlainAlong<BM, BK>{wt, w_bytes, d->C, M, K},
+        with_epilogue(bk_c, PlainAlong<BM, BK>{wt, w_bytes, d->C, M, K},
                       GatherAlong<BN, BK, 0>{(const float *)doutput->data, dy_bytes, K, N, FastDiv(1), FastDiv(1),
                                              PQ, FastDiv((uint32_t)PQ), FastDiv((uint32_t)d->Q), d->K * PQ, d->P,
                                              d->Q, 1, 1, 0, 0, -1, 1, 1, FastDiv(1), FastDiv(1)});
       }
-    }, plan.split ? stage_depth(bm, bn) : run_depth(bm, bn, K));
+    }, run_depth(bm, bn, K));
   } else {
     const int N = plan.N;
     const int HW = d->H * d->W;

@@ -126,7 +126,7 @@ __device__ inline void put_run(char *planes, int row_off, int k, const float *v)
 //
 // "Along" lanes: the 256 lanes run along the tile's rows, every lane holds a run of
 // consecutive reduction elements of one row, and one load instruction of a wave reads 64
-// consecutive rows for a single, wave-uniform k (two such k on a tile of 32 rows).
+// consecutive rows for a single, wave-uniform k.
 template <int D, int BK>
 struct AlongRuns {
   static_assert(D == 64 || D == 128, "tile extent");
@@ -324,9 +324,8 @@ template <int BM, int BN, int BK, class ALoader, class BLoader, class Epilogue>
 __global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : 1) void gemm_kernel(const ALoader al, const BLoader bl, const Epilogue ep,
                                                       int k_extent, int k_per_split, int tiles_m, int tiles_n,
                                                       const Fold fold) {
-  // four waves, 2 x 2 over the tile, or side by side over a tile that is one MFMA high
-  constexpr int WAVES_M = BM == 32 ? 1 : 2;
-  constexpr int WM = BM / WAVES_M, WN = BN / (4 / WAVES_M);  // wave tile
+  // four waves, 2 x 2 over the tile
+  constexpr int WM = BM / 2, WN = BN / 2;  // wave tile
   constexpr int TM = WM / 32, TN = WN / 32;
   static_assert(TM >= 1 && TN >= 1, "tile too small for the wave grid");
   using PA = typename ALoader::Layout;
@@ -340,7 +339,7 @@ __global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : 1) void gemm_ker
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m_wave = wave % WAVES_M * WM, n_wave = wave / WAVES_M * WN;  // this wave's part of the tile
+  const int m_wave = wave % 2 * WM, n_wave = wave / 2 * WN;  // this wave's part of the tile
 
   const int tiles = tiles_m * tiles_n;
   const TileWork work = tile_work(bl, k_extent, k_per_split, tiles, fold);
