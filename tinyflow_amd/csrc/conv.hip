@@ -1546,12 +1546,15 @@ void consider_winograd_wgrad(ConvPlan &p, const ConvDesc *d, double direct_us) {
 //   * reductions of more than 512 steps, a lane's chain: the engine cuts them up for the whole chip;
 //   * a forward reduction of a multiple of four, which the engine walks in another order, and 1x1 filters (no gather);
 //   * plans whose pieces a second pass sums, which takes them in an order of its own.
+// TINYFLOW_FEW_CHANNELS=0 in the environment leaves them to the engine (tests: both have the same bits).
 constexpr int kFewChannels = 8, kFewSteps = 512, kFewLds = 32 << 10;
 struct FewLaunch {
   few::Conv c;
   unsigned blocks = 0, lds = 0;
 };
 bool few_channels(const ConvDesc *d, const ConvPlan &p, bool dgrad, const Geometry &g, FewLaunch &l) {
+  const char *e = getenv("TINYFLOW_FEW_CHANNELS");
+  if (e && *e && atoi(e) == 0) return false;
   if (p.winograd || p.split || p.M > kFewChannels || p.K > kFewSteps || p.b_vec || g.splits > 1) return false;
   if (d->S != 3 && d->S != 5 && d->S != 7) return false;
   if (dgrad ? d->u != 1 || d->v != 1 : p.a_vec) return false;
