@@ -94,6 +94,9 @@ int DLArrayFeed(DLArrayHandle *from, DLArrayHandle *to, int n, DLStreamHandle st
 /* Makes the room that feeds of these device arrays need ahead of the first one; it goes with the stream. */
 int DLArrayFeedReserve(DLArrayHandle *to, int n, DLStreamHandle stream);
 
+/* Feeds so far that a kernel read from pinned memory, that went over the copy stream, and that were plain copies. */
+int DLArrayFeedCounts(long long *direct, long long *overlapped, long long *synchronous);
+
 /* No counterpart in the reference.  Call right after DLArrayAlloc on an array that
  * DLArrayCopyIntoFresh will fill later: records, now, the fence that covers the
  * last release of the array's storage, so that the copy waits for nothing enqueued

@@ -8,26 +8,56 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(scope="module")
+def ballast(rt):
+    from tinyflow_amd import ndarray
+    return [ndarray.array(np.full((4096, 4096), 1e-3, np.float32), ctx=rt.ctx) for _ in range(2)] + [
+        ndarray.empty((4096, 4096), rt.ctx)]
+
+
+def _busy(rt, ballast, products):
+    """Two thirds of a millisecond each on the stream."""
+    from tinyflow_amd import gpu_op
+    a, b, c = ballast
+    for _ in range(products):
+        gpu_op.matrix_multiply(a, False, b, False, c, rt.cublas, rt.stream)
+
+
 # one element, no multiple of four, the largest feed that a kernel reads from pinned memory (1 MiB) and the next one, more
-# than one chunk of the copy stream (4 MiB), several arrays, more than eight of them
-@pytest.mark.parametrize("sizes", [[1], [5, 3], [262144], [262145], [2500003], [1 << 21, 7, 4097], [3] * 19], ids=str)
-def test_arrays_arrive_in_order(rt, sizes):
+# than one chunk of the copy stream (4 MiB), several arrays, more than eight of them, arrays that straddle chunks
+@pytest.mark.parametrize("busy", [False, True], ids=["idle", "busy"])
+@pytest.mark.parametrize("sizes", [[1], [5, 3], [262144], [262145], [2500003], [1 << 21, 7, 4097], [3] * 19,
+                                   [300000] * 11], ids=lambda s: "x".join(str(n) for n in s[:3]) + "...%d" % len(s))
+def test_arrays_arrive_in_order(rt, ballast, sizes, busy):
+    """Seven feeds in a row.  On a stream that is busy for longer than the host needs for all of them, the large ones go
+    over the copy stream while it still works, two at a time; on an idle one they are plain copies."""
     from tinyflow_amd import gpu_op, ndarray
     rng = np.random.RandomState(len(sizes))
     targets = [ndarray.empty((n,), rt.ctx) for n in sizes]
-    seen, sent = [], []
+    batches = [[rng.uniform(-1, 1, n).astype(np.float32) for n in sizes] for _ in range(7)]
+    copies = [[ndarray.empty((n,), rt.ctx) for n in sizes] for _ in batches]
     hosts = [np.empty(n, np.float32) for n in sizes]
-    for step in range(7):
-        for h in hosts:   # the same host arrays, overwritten right after the call before
-            h[:] = rng.uniform(-1, 1, h.shape)
-        sent.append([h.copy() for h in hosts])
+    ndarray.reserve_feed(targets, rt.stream)
+    before = ndarray.feed_counts()
+    for batch, kept in zip(batches, copies):
+        if busy:
+            _busy(rt, ballast, 15)   # 10 ms; the host is at most two feeds ahead
+        for h, values in zip(hosts, batch):   # the same host arrays, overwritten right after the call before
+            h[:] = values
         ndarray.feed(list(zip(targets, hosts)), rt.stream)
-        kept = [ndarray.empty((n,), rt.ctx) for n in sizes]
+        for h in hosts:
+            h[:] = np.nan
         for t, k in zip(targets, kept):
             gpu_op.matrix_elementwise_multiply_by_const(t, 1.0, k, rt.stream)
-        seen.append(kept)
-    for s, k in zip(sent, seen):
-        for a, b in zip(s, k):
+        if not busy:
+            copies[0][0].asnumpy()
+    direct, overlapped, synchronous = (a - b for a, b in zip(ndarray.feed_counts(), before))
+    if sum(-(-n // 64) * 64 for n in sizes) <= 1 << 18:   # every array starts at a multiple of 256 bytes
+        assert (direct, overlapped, synchronous) == (7, 0, 0)
+    else:
+        assert (direct, overlapped, synchronous) == ((0, 7, 0) if busy else (0, 0, 7))
+    for batch, kept in zip(batches, copies):
+        for a, b in zip(batch, kept):
             np.testing.assert_array_equal(a, b.asnumpy())
 
 
@@ -40,9 +70,26 @@ def test_what_is_refused(rt):
         ndarray.feed([(target, "not an array")], rt.stream)
     ndarray.feed([(target, np.arange(20).reshape(4, 5).tolist())], rt.stream)   # converted, as a synchronous copy would
     np.testing.assert_array_equal(target.asnumpy(), np.arange(20, dtype=np.float32).reshape(4, 5))
-    ndarray.feed([], rt.stream)
+    ndarray.feed([], rt.stream)   # nothing to feed
     ndarray.feed([(target, np.ones((4, 5), np.float64).T.copy().T)], rt.stream)   # another type and order
     np.testing.assert_array_equal(target.asnumpy(), np.ones((4, 5), np.float32))
+
+
+def test_a_feed_waits_for_the_other_streams(rt, ballast):
+    """A late kernel of another stream still reads the array that is fed."""
+    from tinyflow_amd import gpu_op, ndarray
+    stream = gpu_op.create_cudaStream()
+    for n in (1000, 2500003):
+        target, kept, fed = (ndarray.empty((n,), rt.ctx) for _ in range(3))
+        old, new = np.arange(n, dtype=np.float32), -np.arange(n, dtype=np.float32)
+        target._sync_copyfrom(old)
+        _busy(rt, ballast, 15)
+        gpu_op.matrix_elementwise_multiply_by_const(target, 1.0, kept, rt.stream)
+        ndarray.feed([(target, new)], stream)
+        gpu_op.matrix_elementwise_multiply_by_const(target, 1.0, fed, stream)
+        np.testing.assert_array_equal(kept.asnumpy(), old)
+        np.testing.assert_array_equal(fed.asnumpy(), new)
+    gpu_op.destroy_cudaStream(stream)
 
 
 @pytest.mark.parametrize("batch", [64, 600], ids=str)   # a feed of 0.2 MB and one of 1.9 MB

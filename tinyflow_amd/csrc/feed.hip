@@ -246,7 +246,11 @@ int launch_feed(DLArrayHandle *to, const size_t *offset, int n, const char *base
   return 0;
 }
 
+// Feeds that went each way, for tests: kernels reading pinned memory, the copy stream, plain copies.
+std::atomic<long long> feeds_direct{0}, feeds_overlapped{0}, feeds_synchronous{0};
+
 int copy_synchronously(DLArrayHandle *from, DLArrayHandle *to, int n) {
+  feeds_synchronous.fetch_add(1);
   for (int i = 0; i < n; ++i)
     if (DLArrayCopyFromTo(from[i], to[i], nullptr) != 0) return -1;
   return 0;
@@ -348,6 +352,7 @@ int feed(DLArrayHandle *from, DLArrayHandle *to, int n, DLStreamHandle stream) {
   }
   TF_HIP(hipEventRecord(slot.read, s));
   slot.pending = true;
+  (direct ? feeds_direct : feeds_overlapped).fetch_add(1);
   return 0;
 }
 
@@ -384,4 +389,11 @@ extern "C" int DLArrayFeedReserve(DLArrayHandle *to, int n, DLStreamHandle strea
   } catch (const std::exception &e) {
     TF_REQUIRE(false, "%s", e.what());
   }
+}
+
+extern "C" int DLArrayFeedCounts(long long *direct, long long *overlapped, long long *synchronous) {
+  if (direct) *direct = feeds_direct.load();
+  if (overlapped) *overlapped = feeds_overlapped.load();
+  if (synchronous) *synchronous = feeds_synchronous.load();
+  return 0;
 }

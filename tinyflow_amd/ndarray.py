@@ -182,6 +182,13 @@ def reserve_feed(arrays, cudaStream):
     check_call(_LIB.DLArrayFeedReserve(handles, len(arrays), cudaStream))
 
 
+def feed_counts():
+    """Feeds so far: (read from pinned memory by a kernel, over the copy stream, plain copies)."""
+    counts = [ctypes.c_longlong(0) for _ in range(3)]
+    check_call(_LIB.DLArrayFeedCounts(*[ctypes.byref(c) for c in counts]))
+    return tuple(c.value for c in counts)
+
+
 def empty(shape, ctx=cpu(0)):
     """Uninitialised array; returns the wanted byte count (int) when out of memory."""
     shape = tuple(int(s) for s in shape)
