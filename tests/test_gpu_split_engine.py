@@ -2,8 +2,8 @@
 
 TINYFLOW_SPLIT=1 forces the engine wherever it has loaders, so that small cases reach every loader; 0 is the fp32
 engine.  Bounds: an element of a product is off by at most gamma = (K + 8) 2^-24 times the sum of its terms'
-magnitudes (one rounding per reduction step, the omitted slices 2^-26 and the last addition), the classical bound of an
-fp32 sum in any order."""
+magnitudes (one rounding per reduction step, the omitted slices 2^-24 at most and the last addition), the classical bound of
+an fp32 sum in any order."""
 import math
 
 import numpy as np
@@ -94,6 +94,42 @@ def test_products_are_no_further_from_float64_than_the_fp32_engine(rt, monkeypat
                 monkeypatch.setenv("TINYFLOW_SPLIT", engine)
                 err.append(np.linalg.norm(_product(rt, a, False, b, False) - ref))
             assert err[1] <= err[0], (m, k, n, positive, err)
+
+
+# 1 + 2^-8 - 2^-17 - 2^-23: the middle slice all but 2^-8 and the last 2^-17 of it, so the products that are left out, all of
+# one sign, are 0.97 of 2^-24 of the whole
+WORST = 1 + 2.0 ** -8 - 2.0 ** -17 - 2.0 ** -23
+
+
+@pytest.mark.parametrize("k", [1, 16, 24, 100, 264, 4096])
+def test_the_largest_omission_stays_within_roundings(rt, split, monkeypatch, k):
+    """Equal operands: the omissions add up to 2^-24 of the result, beside the final rounding (2^-24) and those of the
+    sums, where the fp32 engine's chain of equal summands adds up to more."""
+    a, b = np.full((70, k), WORST, np.float32), np.full((k, 70), WORST, np.float32)
+    ref = k * float(np.float32(WORST)) ** 2
+    err = []
+    for engine in ("0", "1"):
+        monkeypatch.setenv("TINYFLOW_SPLIT", engine)
+        err.append(np.abs(_product(rt, a, False, b, False) - ref).max() / ref)
+    assert err[1] <= max(err[0], 2.0 ** -23), err
+
+
+@pytest.mark.parametrize("k", [24, 264, 1024])
+@pytest.mark.parametrize("signed", [False, True])
+def test_slices_of_extreme_rests_are_no_further_from_float64(rt, monkeypatch, k, signed):
+    """Every element has the rests of WORST behind eight leading bits of its own."""
+    rng = np.random.RandomState(7)
+    a = rng.randint(128, 256, (320, k)) / 128.0 + (WORST - 1)
+    b = rng.randint(128, 256, (k, 320)) / 128.0 + (WORST - 1)
+    if signed:
+        b *= rng.choice([-1, 1], b.shape)
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    err = []
+    for engine in ("0", "1"):
+        monkeypatch.setenv("TINYFLOW_SPLIT", engine)
+        err.append(np.linalg.norm(_product(rt, a, False, b, False) - ref))
+    assert err[1] <= err[0], err
 
 
 @pytest.mark.parametrize("scale_a,scale_b", [

@@ -9,9 +9,9 @@
 // computes the six largest,
 //   h h'   and   (h m' + m h') + (m m' + h l' + l h'),
 // each exact in the multiplier, accumulated in fp32 by v_mfma_f32_32x32x16_bf16.  What
-// is left out (m l', l m', l l') is at most 2^-26 of the product, a quarter of an fp32
-// rounding.  Six such instructions for 16 reduction steps cost 192 cycles where the eight
-// fp32 ones cost 512.
+// is left out (m l', l m', l l') is at most 2^-24 of the product, an fp32 rounding (|m| up to 2^-8, |l| up to 2^-17 of a value
+// near 1; more than 2^-26 for one pair of random operands in 36).  Six such instructions for 16 reduction steps cost 192
+// cycles where the eight fp32 ones cost 512.
 //
 // The h h' products and the smaller ones have accumulators of their own, added at the end: a sum of h h' is rounded
 // once where the fp32 instruction rounds eight times, and the roundings of the others do not
