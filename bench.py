@@ -235,11 +235,11 @@ class HbmTimer(object):
             # backward call that uses them reads dy and the bits instead of dy and x
             "activation_forward": lambda a, bits=False: (8.125 if bits else 8) * n(a[0]),
             "activation_backward": lambda a, bits=False: (8.125 if bits else 12) * n(a[0]),
-            # a sum with the ReLU behind it, and two adjoints' sum with the ReLU's gradient: with the bits two
-            # arrays are read and two written, without them one array more is read
             # per-activation batch norm with the ReLU behind it, and both gradients, each result written
             "bn_and_relu_forward": lambda a: 12 * n(a[0]),
             "bn_and_relu_backward": lambda a: 16 * n(a[0]),
+            # a sum with the ReLU behind it, and two adjoints' sum with the ReLU's gradient: with the bits two
+            # arrays are read and two written, without them one array more is read
             "add_activation_forward": lambda a, bits=False: (16.125 if bits else 20) * n(a[2]),
             "add_activation_backward": lambda a, bits=False: (16.125 if bits else 20) * n(a[2]),
             "matrix_elementwise_add": lambda a: 12 * n(a[2]),

@@ -1316,7 +1316,8 @@ double choose_tile_and_splits(ConvPlan &p, bool wgrad, bool padded, bool scatter
 //   * 3x3 / stride-1 layers keep the fp32 engine whichever form the planner picks.  Their transformed-domain products
 //     are the form that counts, and networks of such layers under a batch-norm head (VGG-16 with dropout, Adam)
 //     turn any change of rounding into steps of Adam the other way: a different summation order of the fp32 engine
-//     alone moves their gradients by more than half their size.
+//     alone moves their gradients by more than half their size.  A descriptor does not know its optimizer, so SGD and
+//     single calls, which amplify nothing, keep the fp32 engine with them.
 int forced_engine() {
   const char *e = getenv("TINYFLOW_SPLIT");
   return e && *e ? atoi(e) : -1;
@@ -1346,8 +1347,8 @@ SplitTraffic split_traffic(const ConvDesc *d, int which, bool vec) {
 }
 
 // The direct form on the engine, with the tile and splits, that the models give the least time.  `on_split`: the plan so
-// far for the split engine.  The fp32 model leaves out what every launch costs (4 us here) and underestimates large
-// ones by a seventh; the line corrects both.  Over 300 layers of ResNet-50 at five sizes and random ones (48 - 512
+// far for the split engine, taken unless its model says more than 1.15 times the fp32 one's time and 4 us.  The fp32 model
+// leaves out what every launch costs (4 us here) and underestimates large ones by a seventh; the line corrects both.  Over 300 layers of ResNet-50 at five sizes and random ones (48 - 512
 // channels, 1x1 to 7x7) the choice takes 0.86 of the fp32 engine's time in all.
 double choose_direct(ConvPlan &p, ConvPlan on_split, const ConvDesc *d, const SplitTraffic &traffic, bool wgrad, bool padded,
                      bool scatter, bool may_split, double out_bytes) {

@@ -34,8 +34,11 @@
 // A[m = lane%32][k = 8*(lane/32) + 0..7], the same of B, and owns 16 accumulators
 // D[8*(v/4) + 4*(lane/32) + v%4][lane%32], as with the fp32 instruction, so the epilogues are shared.
 //
-// What bounds it: power.  4096^3 runs at 205 TFLOP/s (fp32 engine: 137) and with zeros for data at 300; the
-// matrix instructions alone, out of LDS, at 324.  So the work beside them counts: the splitting (104 of the 114 vector instructions
+// What bounds it, for long reductions: power.  4096^3 runs at 195 to 205 TFLOP/s by card (fp32 engine: 137), with zeros for data
+// at 300; the matrix instructions alone, out of LDS, at 324.  Short reductions (the 1x1 layers of a ResNet: 120 to 150) are
+// bound by a tile's start and end, as long as 70 to 80 reduction steps and not overlapped with another tile's
+// multiplications: the matrix pipes are busy in 0.3 to 0.5 of their cycles.  The work beside the matrix instructions counts:
+// the splitting (104 of the 114 vector instructions
 // of a 128 x 128 stage) sits between the matrix instructions, addresses are a lane's constant plus a scalar, and
 // the LDS layouts have no bank conflicts.
 #pragma once

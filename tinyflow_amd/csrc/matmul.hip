@@ -210,10 +210,10 @@ struct Plan {
 };
 
 // Products of more than 256 rows, columns and reduction steps run on the split engine (1000 x 1537 x 777 and both its
-// gradients 117 us on the fp32 engine, 4096^3 1000 against 670).  With fewer of one the time is mostly that of
-// streaming the largest operand or of the launch (256 x 256 x 12544: 22 against 21 us, 128 x 784 x 256 11.5 against 10),
-// and products with one extent the batch are the classifiers under a batch-norm head whose steps take no other rounding
-// (see may_use_split in conv.hip).  TINYFLOW_SPLIT=0 / 1 forces the fp32 / the split engine.
+// gradients 117 us on the fp32 engine, 86 here; 4096^3 1000 and 690).  With fewer of one the time is mostly that of
+// streaming the largest operand or of the launch (256 x 256 x 12544: 22 against 21 us, 128 x 784 x 256 11.5 against 10).
+// A line on sizes, no more: it keeps the rounding of classifiers under a batch-norm head (see may_use_split in conv.hip) as
+// long as the batch or a layer's width is at most 256.  TINYFLOW_SPLIT=0 / 1 forces the fp32 / the split engine.
 bool product_on_split(int M, int N, int K) {
   const char *e = getenv("TINYFLOW_SPLIT");
   if (e && *e) return atoi(e) != 0;
