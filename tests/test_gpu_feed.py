@@ -40,10 +40,10 @@ def test_arrays_arrive_in_order(rt, ballast, sizes, busy):
     ndarray.reserve_feed(targets, rt.stream)
     before = ndarray.feed_counts()
     for batch, kept in zip(batches, copies):
-        if busy:
-            _busy(rt, ballast, 15)   # 10 ms; the host is at most two feeds ahead
         for h, values in zip(hosts, batch):   # the same host arrays, overwritten right after the call before
             h[:] = values
+        if busy:
+            _busy(rt, ballast, 15)   # 10 ms, right in front of the feed; the host is at most two feeds ahead
         ndarray.feed(list(zip(targets, hosts)), rt.stream)
         for h in hosts:
             h[:] = np.nan

@@ -187,7 +187,7 @@ def test_an_arrays_storage_goes_from_one_stream_to_the_other(rt, streams, ballas
     on the other stream."""
     from tinyflow_amd import gpu_op
     one, two = streams
-    n = 3_000_017
+    n = 7_340_033   # of no other test: the pool prefers the block that fits best, so it is the one just freed
     values = np.random.RandomState(3).normal(0, 1, n).astype(np.float32)
     for _ in range(3):
         source, kept = _array(rt, values), _empty(rt, (n,))
