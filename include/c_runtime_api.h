@@ -276,6 +276,11 @@ int DLGpuConvolutionBackwardData(const DLArrayHandle input, const DLArrayHandle 
 int DLGpuConvolutionDescribeKernel(void ***list, int which, char *name, int name_len,
                                    double *flops);
 
+/* No counterpart in the reference.  Whether the three convolutions of a 3x3 / stride-1 descriptor may run on
+ * bf16 slices (not before this is called): fp32 results as close to the exact ones, in another rounding.  An owner whose program turns a change
+ * of rounding into steps of another sign (Adam on gradients that are nothing but rounding) leaves it. */
+int DLGpuConvolutionAllowSlices(void ***list, int allow);
+
 /* No counterpart in the reference: measurement aid.  The next convolution entry
  * point called on this host thread records the two HIP events (hipEvent_t, either
  * may be NULL) on its stream immediately before and after its contraction kernel,

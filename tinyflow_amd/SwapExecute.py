@@ -524,6 +524,8 @@ class SwapExecutor(object):
         for node in self.topo_order:
             if node not in shapes:
                 shapes[node] = tuple(node.op.infer_shape(node, [shapes[i] for i in node.inputs], self.cudnnHandle))
+                if self.optimizer == "sgd" and isinstance(node.op, ad.Convolution2DForwardOp):
+                    gpu_op.convolution_allow_slices(node.cudnnlist[0])   # the plain executor's kernels, hence its bits
         self.tensors = {node: _Tensor(node, shapes[node]) for node in self.topo_order}
         self.keep = set(n for n in self.topo_order if n.isw in (1, 2)) | {self.targetloss} | self.keep_values
         self._plan()

@@ -75,6 +75,8 @@ class TrainExecutor(object):
             input_shapes = [self.node_to_shape_map[i] for i in node.inputs]
             assert None not in input_shapes
             self.node_to_shape_map[node] = tuple(node.op.infer_shape(node, input_shapes, self.cudnnHandle))
+            if self._update_op is ad.SgdOp and isinstance(node.op, ad.Convolution2DForwardOp):
+                gpu_op.convolution_allow_slices(node.cudnnlist[0])   # an update scales the rounding, Adam's may not
 
     def init_Variable(self, feed_dict):
         """Initial values (numpy) of the trainable variables, used by the first run."""

@@ -1313,11 +1313,10 @@ double choose_tile_and_splits(ConvPlan &p, bool wgrad, bool padded, bool scatter
 //     such layers are those of the next point.  Over 17 layers of 24 - 47 channels the choice takes 0.92 of the time of fp32
 //     alone: 7x7, 27 -> 45, 33 x 31, batch 20, 56.6 -> 46.6; 1x1 grad-filter, 40 -> 96, 56 x 56, batch 32, 29.9 -> 22.7;
 //     none is slower, strided grad-data by phases aside (48 channels there, see plan_dgrad).
-//   * 3x3 / stride-1 layers keep the fp32 engine whichever form the planner picks.  Their transformed-domain products
-//     are the form that counts, and networks of such layers under a batch-norm head (VGG-16 with dropout, Adam)
-//     turn any change of rounding into steps of Adam the other way: a different summation order of the fp32 engine
-//     alone moves their gradients by more than half their size.  A descriptor does not know its optimizer, so SGD and
-//     single calls, which amplify nothing, keep the fp32 engine with them.
+//   * 3x3 / stride-1 layers, their transformed-domain products included, run on slices only where the descriptor's owner has said
+//     so (DLGpuConvolutionAllowSlices; the executors do for SGD).  Networks of such layers under a batch-norm head (VGG-16
+//     with dropout, Adam) turn any change of rounding into steps of Adam the other way: a different summation order of
+//     the fp32 engine alone moves their gradients by more than half their size.
 int forced_engine() {
   const char *e = getenv("TINYFLOW_SPLIT");
   return e && *e ? atoi(e) : -1;
@@ -1325,7 +1324,8 @@ int forced_engine() {
 bool may_use_split(const ConvDesc *d) {
   const int forced = forced_engine();
   if (forced >= 0) return forced != 0;
-  return !(d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1) && d->C >= 24 && d->K >= 24;
+  const bool dense_3x3 = d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1;
+  return (!dense_3x3 || d->slices_3x3) && d->C >= 24 && d->K >= 24;
 }
 
 // Grad-filter's gathered x by vectors (SplitGatherAcross MODE 2 and 3): four outputs of one row at a time.
@@ -1361,7 +1361,9 @@ double choose_direct(ConvPlan &p, ConvPlan on_split, const ConvDesc *d, const Sp
   const double split_us = choose_tile_and_splits(on_split, wgrad, padded, scatter, may_split, out_bytes, &traffic);
   if (split_us < 1.15 * us + 4.0 || forced_engine() == 1) {
     p = on_split;
-    us = split_us;
+    // 3x3 / stride 1: what the transformed domain is compared with stays the fp32 form.  The gather bounds the direct form on slices
+    // (56 x 56, 64 channels, batch 64, three calls 462 us against 335), and a call that leaves the domain takes its transforms from the others.
+    if (!(d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1)) us = split_us;
   }
   return us;
 }
@@ -1411,6 +1413,39 @@ bool wino_shape(const ConvDesc *d, bool dgrad, WinoShape &w, bool wgrad = false,
   return true;
 }
 
+// Whether the products of this tile size may run on slices.  2x2 tiles do only where 4x4 ones are not allowed: on slices
+// the products are the smaller part, the transforms count, and the calls of a layer share theirs if their tiles agree.
+bool slices_for_tile(const ConvDesc *d, int tile, bool four_allowed) {
+  return may_use_split(d) && (tile == 4 || !four_allowed || forced_engine() == 1);
+}
+
+// Takes the cheaper engine for one tile shape and k-split if it beats the best so far (`fold`: the sum over the k-splits, which `fp32`
+// holds).  Neither is faster than the bytes (5 TB/s); what
+// the fp32 model leaves out of a launch is a microsecond more than what the other one leaves out.  Over 348 products of 64 - 512 channels
+// and 32 - 25 088 tiles the picks are within 2.8 % of the sweep's best on average and take 0.85 of the fp32 engine's time.
+template <class F>
+void take_engine(double fp32, double sliced, double stream_us, bool slices, double &best, bool &split, F &&take,
+                 double fold = 0.0) {
+  if (!slices) {  // the comparison that the fp32 tiles were tuned with
+    if (fp32 < best) {
+      best = fp32;
+      take();
+    }
+    return;
+  }
+  fp32 = std::max(fp32 - fold + 1.0, stream_us) + fold;
+  sliced = std::max(sliced, stream_us) + fold;
+  if (forced_engine() != 1 && fp32 < best && fp32 <= sliced) {
+    best = fp32;
+    split = false;
+    take();
+  } else if (sliced < best) {
+    best = sliced;
+    split = true;
+    take();
+  }
+}
+
 // Decides between the direct and the Winograd forms and fills the plan of the latter.
 // Model: the transformed-domain products as one batched launch of the tile engine,
 // plus the transform passes at their measured memory rate.  TINYFLOW_WINOGRAD in the
@@ -1428,6 +1463,7 @@ void consider_winograd(ConvPlan &p, const ConvDesc *d, bool dgrad, double direct
   static const int tiles[3][2] = {{128, 128}, {64, 128}, {64, 64}};
   double best_us = 1e30;
   int best_tile = 0, best_bm = 64, best_bn = 64;
+  bool best_split = false;
   WinoShape best_w;
   const char *cap = getenv("TINYFLOW_WINOGRAD_MAX_TILE");
   const int max_tile = cap && *cap ? atoi(cap) : 4;
@@ -1435,27 +1471,31 @@ void consider_winograd(ConvPlan &p, const ConvDesc *d, bool dgrad, double direct
     if ((forced == 2 || forced == 4) ? tile != forced : tile > max_tile) continue;
     WinoShape w;
     if (!wino_shape(d, dgrad, w, false, tile)) continue;
-    double best = 1e30;
-    int bm = 64, bn = 64;
-    for (auto &t : tiles) {
-      if (t[0] == 128 && w.Mo <= 64) continue;
-      const double us = predict_us(w.Mo, w.Tp, w.Cr, t[0], t[1], 1, false, false, false, 0.0, w.positions);
-      if (us < best) {
-        best = us;
-        bm = t[0];
-        bn = t[1];
-      }
-    }
+    const bool slices = slices_for_tile(d, tile, w.Cr <= kMaxChannelsF4);
     const double in_bytes = 4.0 * d->N * w.Cr * w.in_h * w.in_w, out_bytes = 4.0 * d->N * w.Mo * w.out_h * w.out_w;
     const double moved = in_bytes + out_bytes + 4.0 * (w.v_elems + w.m_elems) + 8.0 * w.u_elems;
     // short reductions: the products themselves stream V and M once more
     const double stream_us = 4.0 * (w.v_elems + w.m_elems) / 5.0e6;
+    double best = 1e30;
+    int bm = 64, bn = 64;
+    bool split = false;
+    for (auto &t : tiles) {
+      if (t[0] == 128 && w.Mo <= 64) continue;
+      const double fp32 = predict_us(w.Mo, w.Tp, w.Cr, t[0], t[1], 1, false, false, false, 0.0, w.positions);
+      const double sliced = slices ? predict_split_batched_us(w.Mo, w.Tp, w.Cr, t[0], t[1], 1, stage_depth(t[0], t[1]), dgrad,
+                                                              w.positions) : 1e30;
+      take_engine(fp32, sliced, stream_us, slices, best, split, [&] {
+        bm = t[0];
+        bn = t[1];
+      });
+    }
     const double wino_us = std::max(best, stream_us) + moved / 4.0e6 + 6.0;
     if (wino_us < best_us) {
       best_us = wino_us;
       best_tile = tile;
       best_bm = bm;
       best_bn = bn;
+      best_split = split;
       best_w = w;
     }
   }
@@ -1463,6 +1503,7 @@ void consider_winograd(ConvPlan &p, const ConvDesc *d, bool dgrad, double direct
   p.winograd = true;
   p.wino_tile = best_tile;
   p.variant = best_tile == 2 ? variant2 : variant4;
+  p.split = best_split;
   p.bm = best_bm;
   p.bn = best_bn;
   p.splits = 1;
@@ -1483,6 +1524,7 @@ void consider_winograd_wgrad(ConvPlan &p, const ConvDesc *d, double direct_us) {
   static const int cand[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   double best_us = 1e30;
   int best_tile = 0, best_bm = 64, best_bn = 64, best_splits = 1, best_tp = 0;
+  bool best_split = false;
   for (int tile : {2, 4}) {
     // a forced 4 falls back to 2 where the shape does not allow it, so that "forced"
     // always means some Winograd form for grad-filter
@@ -1491,31 +1533,35 @@ void consider_winograd_wgrad(ConvPlan &p, const ConvDesc *d, double direct_us) {
     if (forced == 2 && tile != 2) continue;
     if (forced < 0 && tile > max_tile) continue;
     const double out_bytes = 4.0 * w.positions * d->K * d->C;
+    const double stream_us = 4.0 * (w.v_elems + w.m_elems) / 5.0e6;
+    const bool slices = slices_for_tile(d, tile, d->C <= kMaxChannelsF4 && d->K <= kMaxChannelsF4);
     double best = 1e30;
     int bm = 64, bn = 64, splits_of_best = 1;
+    bool split = false;
     for (auto &t : tiles) {
       if (t[0] == 128 && d->K <= 64) continue;
       if (t[1] == 128 && d->C <= 64) continue;
       for (int splits : cand) {
         if (splits > 1 && (w.Tp / splits < 64 || splits * out_bytes > 256e6)) continue;
-        double us = predict_us(d->K, d->C, w.Tp, t[0], t[1], splits, false, false, false, out_bytes, w.positions);
+        double fp32 = predict_us(d->K, d->C, w.Tp, t[0], t[1], splits, false, false, false, out_bytes, w.positions);
+        const double sliced = slices ? predict_split_batched_us(d->K, d->C, w.Tp, t[0], t[1], splits, stage_depth(t[0], t[1]), 2,
+                                                          w.positions) : 1e30;
         // the kernel that folds the splits and applies G^T . G runs one workgroup per 64
         // filters; with few filters (64 x 64: 64 workgroups) it cannot pull the partial
         // sums at the memory rate (about 25 GB/s per workgroup, measured), which is what
         // the split term of predict_us assumes
         const double fold_rate = std::min(6.0e6, std::ceil(d->K * (double)d->C / 64.0) * 25.0e3);  // bytes per us
-        if (splits > 1) us += splits * out_bytes * (1.0 / fold_rate - 1.0 / 6.0e6);
-        if (us < best) {
-          best = us;
+        if (splits > 1) fp32 += splits * out_bytes * (1.0 / fold_rate - 1.0 / 6.0e6);
+        const double fold = splits > 1 ? splits * out_bytes / fold_rate + (splits + 1.0) * out_bytes / 6.0e6 : 0.0;
+        take_engine(fp32, sliced, stream_us, slices, best, split, [&] {
           bm = t[0];
           bn = t[1];
           splits_of_best = make_geometry(d->K, d->C, w.Tp, bm, bn, splits, stage_depth(bm, bn)).splits;
-        }
+        }, fold);
       }
     }
     const double moved = 4.0 * d->N * ((double)d->C * d->H * d->W + (double)d->K * d->P * d->Q) +
                          4.0 * (w.v_elems + w.m_elems);
-    const double stream_us = 4.0 * (w.v_elems + w.m_elems) / 5.0e6;
     double wino_us = std::max(best, stream_us) + moved / 4.0e6 + 6.0;
     if (forced == 4 && tile == 4) wino_us = 0.0;
     if (wino_us < best_us) {
@@ -1524,6 +1570,7 @@ void consider_winograd_wgrad(ConvPlan &p, const ConvDesc *d, double direct_us) {
       best_bm = bm;
       best_bn = bn;
       best_splits = splits_of_best;
+      best_split = split;
       best_tp = w.Tp;
     }
   }
@@ -1531,6 +1578,7 @@ void consider_winograd_wgrad(ConvPlan &p, const ConvDesc *d, double direct_us) {
   p.winograd = true;
   p.wino_tile = best_tile;
   p.variant = best_tile == 2 ? "wgrad_winograd" : "wgrad_winograd4x4";
+  p.split = best_split;
   p.bm = best_bm;
   p.bn = best_bn;
   p.splits = best_splits;
@@ -1905,6 +1953,19 @@ int run_winograd(ConvDesc *d, bool dgrad, const ConvPlan &plan, const float *in,
     const Batched<Along4<BN, BK>> bl{{V, (uint32_t)((size_t)w.Cr * w.Tp * 4), w.Tp, w.Tp, w.Cr, FastDiv(ONE_SEGMENT), 0},
                                      (int64_t)w.Cr * w.Tp};
     const StoreBatched ep{{Mt, w.Tp, w.Mo, w.Tp, 0}, (int64_t)w.Mo * w.Tp};
+    const FastDiv whole(ONE_SEGMENT);
+    const int64_t u_stride = (int64_t)w.Mo * w.Cr;
+    if (plan.split) {
+      constexpr int BK = stage_depth(BM, BN);
+      const Batched<split::SplitAlong4<BN, BK>> sbl{{V, bl.bytes, w.Tp, w.Tp, w.Cr, whole, 0}, bl.batch_stride};
+      if (dgrad)
+        launch<BM, BN, BK>(Batched<split::SplitAlong4<BM, BK>>{{U, u_bytes, w.Mo, w.Mo, w.Cr, whole, 0}, u_stride}, sbl, ep, w.Cr,
+                           g, s, w.positions);
+      else
+        launch<BM, BN, BK>(Batched<split::SplitAcross4<BM, BK>>{{U, u_bytes, w.Cr, w.Mo, w.Cr, whole, 0}, u_stride}, sbl, ep,
+                           w.Cr, g, s, w.positions);
+      return;
+    }
     if (dgrad) {
       const Batched<Along4<BM, BK>> al{{U, u_bytes, w.Mo, w.Mo, w.Cr, FastDiv(ONE_SEGMENT), 0}, (int64_t)w.Mo * w.Cr};
       launch<BM, BN, BK>(al, bl, ep, w.Cr, g, s, w.positions);
@@ -1912,7 +1973,7 @@ int run_winograd(ConvDesc *d, bool dgrad, const ConvPlan &plan, const float *in,
       const Batched<Across4<BM, BK>> al{{U, u_bytes, w.Cr, w.Mo, w.Cr, FastDiv(ONE_SEGMENT), 0}, (int64_t)w.Mo * w.Cr};
       launch<BM, BN, BK>(al, bl, ep, w.Cr, g, s, w.positions);
     }
-  }, run_depth(plan.bm, plan.bn, w.Cr));
+  }, plan.split ? stage_depth(plan.bm, plan.bn) : run_depth(plan.bm, plan.bn, w.Cr));
   const bool rows_vec = w.out_w % w.tile == 0 && (reinterpret_cast<uintptr_t>(out) & (uintptr_t)(4 * w.tile - 1)) == 0;
   const uint32_t out_bytes = (uint32_t)((size_t)d->N * w.Mo * w.out_h * w.out_w * sizeof(float));  // smaller than M
   if (w.tile == 2)
@@ -1993,8 +2054,16 @@ int run_winograd_wgrad(ConvDesc *d, const ConvPlan &plan, const float *x, const 
     const Batched<Across4<BN, BK>> bl{{V, (uint32_t)((size_t)d->C * w.Tp * 4), w.Tp, d->C, w.Tp, FastDiv(ONE_SEGMENT), 0},
                                       (int64_t)d->C * w.Tp};
     const StoreBatched ep{{dU, d->C, d->K, d->C, (int64_t)w.positions * KC}, (int64_t)KC};
+    if (plan.split) {
+      constexpr int BK = stage_depth(BM, BN);
+      const FastDiv whole(ONE_SEGMENT);
+      launch<BM, BN, BK>(Batched<split::SplitAcross4<BM, BK>>{{dM, al.bytes, w.Tp, d->K, w.Tp, whole, 0}, al.batch_stride},
+                         Batched<split::SplitAcross4<BN, BK>>{{V, bl.bytes, w.Tp, d->C, w.Tp, whole, 0}, bl.batch_stride}, ep,
+                         w.Tp, g, s, w.positions);
+      return;
+    }
     launch<BM, BN, BK>(al, bl, ep, w.Tp, g, s, w.positions);
-  }, run_depth(plan.bm, plan.bn, g.k_per_split));
+  }, plan.split ? bk : run_depth(plan.bm, plan.bn, g.k_per_split));
   if (w.tile == 2)
     hipLaunchKernelGGL(wino_dfilter_kernel<2>, dim3(cdiv(KC, 64)), block, 0, s, (const float *)dU, dw, KC, g.splits);
   else
@@ -2029,11 +2098,13 @@ extern "C" int DLGpuConvolutionDescribeKernel(void ***list, int which, char *nam
     // executes (16 or 36 products), 2.25x or 4x below the direct form's
     const int reduction = which == 2 ? make_geometry(p.M, p.N, p.K, p.bm, p.bn, p.splits, stage_depth(p.bm, p.bn)).k_per_split
                                      : p.K;
-    const int bk = run_depth(p.bm, p.bn, reduction);
+    const int bk = p.split ? stage_depth(p.bm, p.bn) : run_depth(p.bm, p.bn, reduction);
+    const char *across = p.split ? "SplitAcross4" : "Across4", *along = p.split ? "SplitAlong4" : "Along4";
+    const char *flags = p.split ? ", false, false" : ", false";  // of an across loader
     snprintf(name, (size_t)name_len,
              "%s %dx%d s%d | gemm_kernel<%d, %d, %d, Batched<%s<%d, %d%s>>, Batched<%s<%d, %d%s>>, StoreBatched>",
-             p.variant, p.bm, p.bn, p.splits, p.bm, p.bn, bk, which == 1 ? "Along4" : "Across4", p.bm, bk,
-             which == 1 ? "" : ", false", which == 2 ? "Across4" : "Along4", p.bn, bk, which == 2 ? ", false" : "");
+             p.variant, p.bm, p.bn, p.splits, p.bm, p.bn, bk, which == 1 ? along : across, p.bm, bk,
+             which == 1 ? "" : flags, which == 2 ? across : along, p.bn, bk, which == 2 ? flags : "");
     if (flops) {
       WinoShape w;
       wino_shape(d, which == 1, w, which == 2, p.wino_tile);
@@ -2088,6 +2159,13 @@ extern "C" int DLGpuConvolutionDescribeKernel(void ***list, int which, char *nam
            p.bm, p.bn, p.splits, p.bm, p.bn, bk, p.a_loader, p.bm, bk, a_flag, p.b_loader, b_args, p.epilogue);
   if (flops)
     *flops = 2.0 * d->N * d->K * d->C * d->R * d->S * (double)d->P * d->Q;
+  return 0;
+}
+
+extern "C" int DLGpuConvolutionAllowSlices(void ***list, int allow) {
+  ConvDesc *d = desc_from_list<ConvDesc>(list, kMagicConv);
+  TF_REQUIRE(d, "descriptor list was not created by DLGpuConvolution2DForwardGetOutShape");
+  d->slices_3x3 = allow != 0;
   return 0;
 }
 

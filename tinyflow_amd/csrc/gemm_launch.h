@@ -125,5 +125,21 @@ inline double predict_split_us(int M, int N, int K, int bm, int bn, int splits, 
   return us;
 }
 
+// Batched products of the transformed domain (`batch` of them; V and M stream by, the time of the transforms and of the sum
+// over k-splits is the caller's): the same form with constants of their own, from sweeps over 29 layers of VGG-16 at batch 32 and
+// ResNet-50 at batch 64 and 8.  us, measured / model: 256 channels, 6 272 tiles, 128 x 128 178 / 176; 512, 512 tiles 68 / 64, 64 x 128
+// 66 / 69; 128, 3 136 tiles 36 / 33; grad-filter 256, 6 272 tiles in 8 pieces 169 / 161; 64 channels 49.5 / 48.  Grad-data's
+// filter comes eight bytes a lane on tiles of 64 rows: 1.2 times the time.
+inline double predict_split_batched_us(int M, int N, int K, int bm, int bn, int splits, int stage, int which, int batch) {
+  const Geometry g = make_geometry(M, N, K, bm, bn, splits, stage);
+  const double a = (bm == 128 ? 0.0345 : bn == 128 ? 0.0232 : 0.0141) * (which == 2 ? 1.04 : which == 1 && bm == 64 ? 1.2 : 1.0);
+  const double o = bm == 128 ? 109.0 : bn == 128 ? 85.0 : 102.0;
+  const double per_cu = (double)g.blocks() * batch / num_cus();
+  const double whole = std::ceil(per_cu);
+  const double rounds = per_cu <= 1.0 ? 1.0 : std::min(whole, per_cu + 0.75);
+  const double hiding = whole <= 1 ? 0.725 : whole <= 2 ? 0.918 : 1.0;
+  return rounds * a * (g.k_per_split + o) / hiding;
+}
+
 }  // namespace gemm
 }  // namespace tf

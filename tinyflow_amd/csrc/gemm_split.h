@@ -323,8 +323,11 @@ struct SplitAcross4 {
 
 // ---- the kernel ----------------------------------------------------------------------
 // Work decomposition, fold and epilogue are those of the fp32 kernel.
+// Workgroups a CU: two of the 128 x 128 tile (its registers and no more).  Three of the 64 x 128 tile, whose LDS has room for
+// them; left to itself the compiler takes six registers too many for the third (1x1, 256 -> 64 channels, 56 x 56, batch 64: 76 -> 66 us,
+// 64 -> 256 104 -> 86, 512 -> 2048 at 7 x 7 54 -> 52).  LDS holds two of the 64 x 64 tile.
 template <int BM, int BN, int BK, class ALoader, class BLoader, class Epilogue>
-__global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : 1) void gemm_kernel(const ALoader al, const BLoader bl, const Epilogue ep,
+__global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : BN == 128 ? 3 : 1) void gemm_kernel(const ALoader al, const BLoader bl, const Epilogue ep,
                                                       int k_extent, int k_per_split, int tiles_m, int tiles_n,
                                                       const Fold fold) {
   // four waves, 2 x 2 over the tile

@@ -135,6 +135,7 @@ struct ConvDesc {
   int K, R, S;         // filter (K output channels, C input channels)
   int P, Q;            // output spatial
   int pad_h, pad_w, u, v;
+  bool slices_3x3 = false;   // 3x3 / stride-1 layers may run on bf16 slices too (DLGpuConvolutionAllowSlices)
   // Winograd forms: the transformed input V of the last forward call, kept for the
   // grad-filter call of the same step, which needs exactly this array (see keep_set).
   // (the three kept_* pointers are registry slots: written and read only through

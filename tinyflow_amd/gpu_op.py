@@ -242,6 +242,11 @@ def convolution_2d_forward_get_out_shape(input_shapes, filter_shapes, dataformat
     return tuple(c_out), cudnnlist
 
 
+def convolution_allow_slices(cudnnlist, allow=True):
+    """Lets a 3x3 / stride-1 descriptor's convolutions run on bf16 slices (no reference counterpart)."""
+    check_call(_LIB.DLGpuConvolutionAllowSlices(cudnnlist, int(allow)))
+
+
 def convolution_2d_forward(in_arr, in_filter, out_arr, cudnnlist, cudnnHandle, cudaStream):
     _nd_args(in_arr, in_filter, out_arr)
     wanted = ctypes.c_int(0)
