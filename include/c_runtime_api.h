@@ -295,6 +295,24 @@ int DLGpuConvolutionTimeNextKernel(void *start_event, void *stop_event);
  * library was loaded, and how many are held right now; any pointer may be NULL. */
 int DLGpuKeptByproductCounts(long long *kept_blocks, long long *taken_blocks, int *held_now);
 
+/* -------------------------------------------------------- groups of elementwise nodes */
+
+/* No counterpart in the reference.  Up to six elementwise calls as one launch: each step writes its output as the
+ * call that it stands for does, and a step may read what an earlier one wrote.  The outputs have one length, or a single
+ * element; nothing that a step reads from outside may be written by the group.
+ *   kGroupSet out = value; kGroupAdd / kGroupMul out = a + b, a * b; kGroupAddConst / kGroupMulConst with value;
+ *   kGroupRelu out = a < 0 ? 0 : a; kGroupReluGradient out = a > 0 ? b : 0;
+ *   kGroupBroadcast out = a along the trailing dims, or with per_channel along dim 1.
+ * ordered: the launch comes behind what other streams hold and in front of what they launch later (what DLGpuRelu_onStream does). */
+enum { kGroupSet = 0, kGroupAdd, kGroupAddConst, kGroupMul, kGroupMulConst, kGroupRelu, kGroupReluGradient, kGroupBroadcast };
+typedef struct {
+  int kind;
+  float value;
+  int per_channel;
+  DLArrayHandle a, b, out;
+} DLGroupStep;
+int DLGpuElementwiseGroup(const DLGroupStep *steps, int n_steps, int ordered, void **stream);
+
 /* ----------------------------------------------------------------- pooling */
 
 /* out = 1 + (in + 2*pad - window) / stride.

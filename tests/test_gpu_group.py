@@ -1,0 +1,140 @@
+"""Groups of elementwise nodes (csrc/group.hip): the bytes of the separate calls, what is refused, and which nodes the executor
+puts into one launch."""
+import numpy as np
+import pytest
+
+
+def _values(shape, seed):
+    gen = np.random.default_rng(seed)
+    a = gen.standard_normal(shape, dtype=np.float32)
+    flat = a.reshape(-1)
+    flat[::7], flat[3::11] = 0.0, -0.0
+    if flat.size > 20:
+        flat[5::13], flat[6::17] = np.nan, -np.inf
+    return a
+
+
+# one element, remainders of a vector and of a workgroup, rows and planes that are and are not multiples of four
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,per_channel", [
+    ((1, 1), False), ((3, 5), False), ((2, 4), False), ((128, 100), False), ((129, 10), False), ((64, 1030), False),
+    ((2, 3, 5, 7), True), ((4, 6, 28, 28), True), ((5, 4, 2, 2), True), ((3, 1, 1, 1), True), ((7, 16, 10, 10), True),
+], ids=str)
+def test_group_writes_the_bytes_of_the_separate_calls(rt, shape, per_channel):
+    from tinyflow_amd import gpu_op as G, ndarray
+    ctx, stream = rt.ctx, rt.stream
+    x, dy, bias = _values(shape, 1), _values(shape, 2), _values((shape[1],), 3)
+    gx, gdy, gb = (ndarray.array(v, ctx) for v in (x, dy, bias))
+
+    def outputs(n):
+        arrays = [ndarray.empty(shape, ctx) for _ in range(n)] + [ndarray.empty((1,), ctx)]
+        for a in arrays:
+            G.array_set(a, 7.0, stream)
+        return arrays
+
+    spread, total, relu, scaled, one = outputs(4)
+    G.broadcast_to(gb, spread, "NCHW" if per_channel else "NHWC", stream)
+    G.matrix_elementwise_add(gx, spread, total, stream)
+    G.relu_on_stream(total, relu, stream)
+    G.matrix_elementwise_multiply_by_const(relu, -1.7, scaled, stream)
+    G.array_set(one, 1.0, stream)
+    grad, shifted, product, both, _ = outputs(4)
+    G.relu_gradient_on_stream(total, gdy, grad, stream)
+    G.matrix_elementwise_add_by_const(grad, 0.0, shifted, stream)
+    G.matrix_elementwise_multiply(shifted, gx, product, stream)
+    G.matrix_elementwise_add(scaled, product, both, stream)
+    want = [a.asnumpy().tobytes() for a in (spread, total, relu, scaled, one, grad, shifted, product, both)]
+
+    for ordered in (0, 1):
+        spread, total, relu, scaled, one = outputs(4)
+        grad, shifted, product, both, _ = outputs(4)
+        for rows in ([(G.GROUP_BROADCAST, 0, gb, None, spread), (G.GROUP_ADD, 0, gx, spread, total),
+                      (G.GROUP_RELU, 0, total, None, relu), (G.GROUP_MUL_CONST, -1.7, relu, None, scaled),
+                      (G.GROUP_SET, 1.0, None, None, one)],
+                     [(G.GROUP_RELU_GRADIENT, 0, total, gdy, grad), (G.GROUP_ADD_CONST, 0.0, grad, None, shifted),
+                      (G.GROUP_MUL, 0, shifted, gx, product), (G.GROUP_ADD, 0, scaled, product, both)]):
+            G.elementwise_group(_steps(G, rows, per_channel), ordered, stream)
+        got = [a.asnumpy().tobytes() for a in (spread, total, relu, scaled, one, grad, shifted, product, both)]
+        assert [g == w for g, w in zip(got, want)] == [True] * len(want)
+
+
+def _steps(G, rows, per_channel=False):
+    steps = (G.GroupStep * len(rows))()
+    for step, (kind, value, a, b, out) in zip(steps, rows):
+        step.kind, step.value, step.per_channel, step.out = kind, value, per_channel, out.handle
+        if a is not None:
+            step.a = a.handle
+        if b is not None:
+            step.b = b.handle
+    return steps
+
+
+@pytest.mark.gpu
+def test_group_refuses_what_it_cannot_order(rt):
+    from tinyflow_amd import gpu_op as G, ndarray
+    a, b, c = (ndarray.array(np.full((4, 8), v, np.float32), rt.ctx) for v in (1, 2, 3))
+    short = ndarray.array(np.ones((4, 4), np.float32), rt.ctx)
+    add = G.GROUP_ADD_CONST
+    for rows in ([(add, 1.0, a, None, b), (add, 1.0, c, None, b)],          # written twice
+                 [(add, 1.0, a, None, b), (add, 1.0, c, None, a)],          # a later step writes what an earlier one read
+                 [(add, 1.0, a, None, a)],                                  # in place
+                 [(add, 1.0, a, None, b), (add, 1.0, short, None, c)],      # lengths
+                 [(99, 1.0, a, None, b)], [(G.GROUP_ADD, 0.0, a, None, b)],
+                 [(add, 1.0, a, None, b)] * 7):
+        with pytest.raises(RuntimeError):
+            G.elementwise_group(_steps(G, rows), 0, rt.stream)
+    assert (a.asnumpy() == 1).all() and (b.asnumpy() == 2).all() and (c.asnumpy() == 3).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("net,head,optimizer", [("mlp", "softmax_xent", "sgd"), ("lenet5", "softmax_xent", "sgd"),
+                                                ("lenet5", "cross", "adam")])
+def test_steps_with_groups_have_the_bytes_of_steps_without(rt, monkeypatch, net, head, optimizer):
+    from tinyflow_amd import TrainExecute, TrainExecuteAdam, models
+    results = []
+    for grouped in (True, False):
+        if not grouped:
+            monkeypatch.setattr(TrainExecute, "find_groups", lambda *a: {})
+        rng = np.random.RandomState(11)
+        model = getattr(models, net)(rng, batch=96, head=head)
+        X, y = models.synthetic_batch(rng, model.input_shape, model.n_class, "uniform")
+        module = TrainExecuteAdam if optimizer == "adam" else TrainExecute
+        executor = module.TrainExecutor(model.loss, 1e-3)
+        executor.init_Variable(dict(model.variables))
+        for _ in range(3):
+            out = executor.run({model.X: X, model.y_: y})
+        results.append([o.asnumpy().tobytes() for o in out]
+                       + [executor.value_of(n).asnumpy().tobytes() for n in executor.topo_order
+                          if n in executor.node_to_arr_map])
+        executor.close()
+    assert results[0] == results[1]
+
+
+def test_which_nodes_form_a_group():
+    from tinyflow_amd import autodiff as ad
+    from tinyflow_amd.TrainExecute import find_groups, find_joins
+    x, b, dy = ad.Placeholder("x"), ad.Variable("b"), ad.Placeholder("dy")
+    spread = ad.broadcastto_op(b, x)
+    s = x + spread
+    r = ad.activation_forward_op(s, "NCHW", "relu")
+    t = ad.activation_forward_op(r, "NCHW", "tanh")       # no step of a group
+    back = ad.activation_backward_op(s, t, r, "relu", r.cudnnlist)
+    ones = ad.oneslike_op(back)
+    order = [x, b, dy, spread, s, r, t, back, ones]
+    shapes = {n: (8, 12) for n in order}
+    shapes[b], shapes[ones] = (12,), (1,)
+    fed = {x, b, dy}
+    joins = find_joins(order, shapes, fed, {})
+    assert find_groups(order, shapes, fed, {}, {}) == {spread: [spread, s, r, ones]}
+    # the sum has a fed operand and joins nothing; where it joined, the group would take both, and leave both without the operand
+    assert find_groups(order, shapes, fed, {}, {s: r}) == {spread: [spread, s, r, ones]}
+    assert find_groups(order, shapes, fed | {spread}, {}, {s: r}) == {} and joins == {}
+    # the gradient waits for its upstream, which comes behind the ReLU
+    back2 = ad.activation_backward_op(s, dy, r, "relu", r.cudnnlist)
+    shifted = back2 + 2.0
+    order = [x, b, dy, spread, s, r, t, back2, shifted]
+    shapes.update({back2: (8, 12), shifted: (8, 12)})
+    assert find_groups(order, shapes, fed, {}, {}) == {spread: [spread, s, r, back2, shifted]}
+    assert find_groups(order, shapes, fed, {s: ("skip",), r: ("add_relu", s, [x, spread])}, {}) == {back2: [back2, shifted]}
+    shapes.update({n: (2 ** 12, 2 ** 12) for n in (spread, s, r, back2, shifted)})
+    assert find_groups(order, shapes, fed, {}, {}) == {}   # too long

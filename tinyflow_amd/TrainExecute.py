@@ -105,10 +105,17 @@ class TrainExecutor(object):
             if len(role) == 3:
                 unread_zeros -= set(role[2])
         joined = find_joins(self.topo_order, self.node_to_shape_map, set(feed_dict) | unread_zeros, fused)
+        groups = find_groups(self.topo_order, self.node_to_shape_map, set(feed_dict) | unread_zeros, fused, joined)
+        in_group = {n for members in groups.values() for n in members}
+        joined = {n: r for n, r in joined.items() if n not in in_group}
         by_join = set(joined.values())
         for node in self.topo_order:
-            if node in by_join:
-                continue   # computed with its first operand
+            if node in groups:
+                for n in groups[node]:
+                    self.node_to_arr_map[n] = self._alloc(self.node_to_shape_map[n])
+                plan.append((_group_compute(groups[node], self.node_to_shape_map, self.node_to_arr_map), node, None, None))
+            if node in by_join or node in in_group:
+                continue   # computed with its first operand, or with the first of its group
             if node in joined:
                 reader = joined[node]
                 outputs = [self._alloc(self.node_to_shape_map[n]) for n in (node, reader)]
@@ -424,6 +431,125 @@ def _join_compute(first, reader):
     return compute
 
 
+# Longer arrays gain nothing from fewer launches: their joins move as many bytes and keep the ReLU's sign bits.
+MAX_GROUP_ELEMENTS = 1 << 23
+
+
+def _group_step(node, shapes):
+    """How one step of ``elementwise_group`` computes ``node``: (kind, constant, operands), or None."""
+    op, inputs = node.op, node.inputs
+    if isinstance(op, (ad.AddOp, ad.MulOp)) and len(inputs) == 2:
+        which = _added_zeros_operand(node, shapes)
+        if which is not None:
+            return gpu_op.GROUP_ADD_CONST, 0.0, [inputs[1 - which]]
+        add = isinstance(op, ad.AddOp)
+        if shapes[inputs[0]] == shapes[inputs[1]]:
+            return gpu_op.GROUP_ADD if add else gpu_op.GROUP_MUL, 0.0, list(inputs)
+        known = _known_scalar_operand(node, shapes)
+        if known is not None:
+            return gpu_op.GROUP_ADD_CONST if add else gpu_op.GROUP_MUL_CONST, known[1], [inputs[1 - known[0]]]
+    elif isinstance(op, (ad.AddByConstOp, ad.MulByConstOp)):
+        kind = gpu_op.GROUP_ADD_CONST if isinstance(op, ad.AddByConstOp) else gpu_op.GROUP_MUL_CONST
+        return kind, node.const_attr, list(inputs)
+    elif isinstance(op, (ad.OnesLikeOp, ad.ZerosLikeOp)):
+        return gpu_op.GROUP_SET, 1.0 if isinstance(op, ad.OnesLikeOp) else 0.0, []
+    elif isinstance(op, ad.BroadcastToOp):
+        # (1,) spreads over anything; else the operand is the channels, or the trailing dims
+        if node.type == "NCHW" or len(shapes[inputs[0]]) == 1 and shapes[node][-1:] == shapes[inputs[0]]:
+            return gpu_op.GROUP_BROADCAST, 0.0, [inputs[0]]
+    elif isinstance(op, ad.ReluOp):
+        return gpu_op.GROUP_RELU, 0.0, list(inputs)
+    elif isinstance(op, ad.ReluGradientOp):
+        return gpu_op.GROUP_RELU_GRADIENT, 0.0, list(inputs)
+    elif isinstance(op, ad.ActivationForwardOp) and node.activationMode == "relu":
+        return gpu_op.GROUP_RELU, 0.0, list(inputs)
+    elif isinstance(op, ad.ActivationBackwardOp) and node.activationMode == "relu":
+        return gpu_op.GROUP_RELU_GRADIENT, 0.0, [inputs[0], inputs[1]]
+    return None
+
+
+def find_groups(topo_order, shapes, unavailable, roles, joins):
+    """Elementwise nodes of one length that are computed by one launch (``gpu_op.elementwise_group``): a fully connected
+    layer's bias broadcast, sum and ReLU, the ReLU's gradient and the sum with zeros behind it.  Returns first node -> the nodes in
+    order.  They run at the first one's place, so what the others read has to precede it or be in the group; every array
+    holds what it would.  A join of a sum and its ReLU comes apart only where the group brings the sum's operand with it."""
+    at = {n: i for i, n in enumerate(topo_order)}
+    by_join = {r: n for n, r in joins.items()}
+    steps, groups, taken = {}, {}, set()
+    for n in topo_order:
+        if n in unavailable or n in roles or n.issgd or n.isw or int(np.prod(shapes[n])) > MAX_GROUP_ELEMENTS:
+            continue
+        if not all(isinstance(s.op, ad.AddOp) and isinstance(r.op, ad.ActivationForwardOp)
+                   for s, r in joins.items() if n in (s, r)):
+            continue   # joins of a batch norm, or of two adjoints
+        step = _group_step(n, shapes)
+        if step is not None:
+            steps[n] = step
+    for first in topo_order:
+        if first not in steps or first in taken or first in joins or first in by_join or shapes[first] == (1,):
+            continue
+        size = int(np.prod(shapes[first]))
+        members = [first]
+        for n in topo_order[at[first] + 1:]:
+            if len(members) == gpu_op.GROUP_MAX_STEPS:
+                break
+            if n not in steps or n in taken or not (shapes[n] == (1,) and steps[n][0] == gpu_op.GROUP_SET
+                                                    or int(np.prod(shapes[n])) == size):
+                continue
+            kind, _, operands = steps[n]
+            spread = kind == gpu_op.GROUP_BROADCAST
+            if not all(at[i] < at[first] or (i in members and not spread) for i in operands):
+                continue
+            if n in joins and not any(i in members for i in operands):
+                continue   # the sum keeps its ReLU
+            if n in by_join and by_join[n] not in members:
+                continue
+            members.append(n)
+        # a sum whose ReLU found no room stays with it, and with it what reads the two
+        while True:
+            kept = [n for n in members if not (n in joins and joins[n] not in members)
+                    and all(at[i] < at[first] or i in members for i in steps[n][2])]
+            if kept == members:
+                break
+            members = kept
+        if sum(shapes[n] != (1,) for n in members) > 1:   # a single element to set is no reason for a group
+            groups[first] = members
+            taken |= set(members)
+    return groups
+
+
+def _group_compute(members, shapes, arrays):
+    """Plan entry (same signature as ``Op.compute``) of a group."""
+    steps = (gpu_op.GroupStep * len(members))()
+    for entry, n in zip(steps, members):
+        entry.kind, entry.value, operands = _group_step(n, shapes)
+        entry.per_channel = isinstance(n.op, ad.BroadcastToOp) and n.type == "NCHW"
+        entry.out = arrays[n].handle
+        for field, operand in zip(("a", "b"), operands):
+            setattr(entry, field, arrays[operand].handle)
+    # the calls without a stream argument in the reference are ordered against every stream
+    ordered = int(any(isinstance(n.op, (ad.ReluOp, ad.ReluGradientOp)) for n in members))
+
+    def compute(node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream):
+        gpu_op.elementwise_group(steps, ordered, cudaStream)
+        return 0
+    return compute
+
+
+def _known_scalar_operand(node, shapes):
+    """(index, value) of the (1,)-shaped operand of an Add / Mul node that is a ``oneslike`` / ``zeroslike``, or None."""
+    a, b = node.inputs
+    which = 1 if shapes[b] == (1,) else 0 if shapes[a] == (1,) else None
+    if which is None or shapes[a] == shapes[b]:
+        return None
+    producer = node.inputs[which]
+    if isinstance(producer.op, ad.OnesLikeOp):
+        return which, 1.0
+    if isinstance(producer.op, ad.ZerosLikeOp):
+        return which, 0.0
+    return None
+
+
 def _known_scalar_compute(node, shapes):
     """Plan entry for an Add / Mul node one of whose operands is a (1,)-shaped
     ``oneslike`` / ``zeroslike`` value, or None.  The op itself reads a (1,) operand
@@ -433,19 +559,10 @@ def _known_scalar_compute(node, shapes):
     0.0 whatever its input holds, so the constant is known without reading it."""
     if not isinstance(node.op, (ad.AddOp, ad.MulOp)) or len(node.inputs) != 2:
         return None
-    a, b = node.inputs
-    if shapes[a] == shapes[b]:
+    known = _known_scalar_operand(node, shapes)
+    if known is None:
         return None
-    which = 1 if shapes[b] == (1,) else 0 if shapes[a] == (1,) else None
-    if which is None:
-        return None
-    producer = node.inputs[which]
-    if isinstance(producer.op, ad.OnesLikeOp):
-        constant = 1.0
-    elif isinstance(producer.op, ad.ZerosLikeOp):
-        constant = 0.0
-    else:
-        return None
+    which, constant = known
     by_const = (gpu_op.matrix_elementwise_add_by_const if isinstance(node.op, ad.AddOp)
                 else gpu_op.matrix_elementwise_multiply_by_const)
 

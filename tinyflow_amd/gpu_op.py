@@ -228,6 +228,24 @@ def reduce_sum_new(in_arr, out_arr, cudnnlist, cudnnHandle, cudaStream):
     return wanted.value
 
 
+# -------------------------------------------------------- groups of elementwise nodes
+
+GROUP_SET, GROUP_ADD, GROUP_ADD_CONST, GROUP_MUL, GROUP_MUL_CONST, GROUP_RELU, GROUP_RELU_GRADIENT, GROUP_BROADCAST = range(8)
+GROUP_MAX_STEPS = 6
+
+
+class GroupStep(ctypes.Structure):
+    """DLGroupStep of c_runtime_api.h"""
+    _fields_ = [("kind", ctypes.c_int), ("value", ctypes.c_float), ("per_channel", ctypes.c_int),
+                ("a", _nd.DLArrayHandle), ("b", _nd.DLArrayHandle), ("out", _nd.DLArrayHandle)]
+
+
+def elementwise_group(steps, ordered, cudaStream):
+    """One launch for the elementwise calls of ``steps``, a ctypes array of GroupStep (extension: no counterpart in the
+    reference)."""
+    check_call(_LIB.DLGpuElementwiseGroup(steps, len(steps), ordered, cudaStream))
+
+
 # ------------------------------------------------------------------ convolution
 
 def convolution_2d_forward_get_out_shape(input_shapes, filter_shapes, dataformat, padding, u, v):
