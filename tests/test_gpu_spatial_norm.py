@@ -1,0 +1,63 @@
+"""Spatial batch norm of a channel that fits one workgroup: both passes in one launch, alone and with the ReLU."""
+import numpy as np
+import pytest
+
+
+# one to four register slots a lane; one to sixteen chunks; images left over in the last chunk; one lane and one full slot;
+# 16-byte and single accesses; and the first sizes past the limit, which two passes take
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 3, 1, 1), (1, 2, 32, 32), (3, 1100, 5, 5), (5, 300, 9, 9), (8, 256, 10, 10),
+                                   (4, 256, 56, 56), (8, 128, 20, 20), (2, 90, 31, 33), (7, 600, 16, 16), (16, 16, 8, 8),
+                                   (17, 64, 6, 6), (16, 64, 32, 32), (16, 64, 32, 36), (4, 300, 15, 17), (4, 300, 16, 17)],
+                         ids=str)
+def test_against_float64_and_its_joint_form(rt, shape):
+    """A lane adds at most 16 values (64 past the limit) in float32 before float64 takes over, which bounds each sum by that
+    many rounding steps of the sum of magnitudes; the steps behind add one each."""
+    from tinyflow_amd import gpu_op, ndarray
+    rng = np.random.default_rng(3)
+    x = (rng.standard_normal(shape) * 2 + 0.5).astype(np.float32)
+    dy = rng.standard_normal(shape, dtype=np.float32)
+    x[:, -1] = 1.25   # no variance: bn(x) is zero, and not above it
+    mean_p, var_p, lst = gpu_op.bn_get_cudnnlist(shape, "NCHW", "spatial")
+    act = gpu_op.activation_get_cudnnlist(shape, "NCHW", "relu")
+    gx, gdy = ndarray.array(x, rt.ctx), ndarray.array(dy, rt.ctx)
+    y, dx, y2, relu, drelu, dx2, dx3 = (ndarray.empty(shape, rt.ctx) for _ in range(7))
+    for out in (y, dx, y2, relu, drelu, dx2, dx3):
+        gpu_op.array_set(out, 7.0, rt.stream)
+
+    def forward():
+        assert gpu_op.bn_forward(gx, y, "spatial", 0, mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+    forward()
+    assert gpu_op.bn_backward(gx, gdy, dx, "spatial", mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+    assert gpu_op.bn_and_relu_forward(gx, y2, relu, "spatial", 0, mean_p, var_p, lst, act, rt.cudnn, rt.stream) == 0
+    assert gpu_op.bn_and_relu_backward(gx, y2, relu, gdy, drelu, dx2, "spatial", mean_p, var_p, lst, act, rt.cudnn,
+                                       rt.stream) == 0
+    # the joint form has the bytes of the calls that it stands for
+    got = y.asnumpy()
+    assert y2.asnumpy().tobytes() == got.tobytes() and relu.asnumpy().tobytes() == np.where(got < 0, 0, got).tobytes()
+    want_drelu = np.where(got > 0, dy, np.float32(0))
+    assert drelu.asnumpy().tobytes() == want_drelu.tobytes()
+    forward()
+    assert gpu_op.bn_backward(gx, drelu, dx3, "spatial", mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+    assert dx2.asnumpy().tobytes() == dx3.asnumpy().tobytes()
+
+    axes, m, u = (0, 2, 3), x[:, 0].size, 2.0 ** -24
+
+    def over(a):
+        return a.sum(axis=axes, keepdims=True)
+    x64, g = x.astype(np.float64), dy.astype(np.float64)
+    mean, var = x64.mean(axis=axes, keepdims=True), x64.var(axis=axes, keepdims=True) + float(np.float32(1e-5))
+    istd, t = 1 / np.sqrt(var), np.abs(x64 - x64[:1, :, :1, :1])
+    xhat = (x64 - mean) * istd
+    steps = (64 + 3) * u
+    rel_istd = steps * (over(t * t) / m + 2 * (over(t) / m) ** 2) / var / 2 + 2 * u
+    e_xhat = istd * (steps * over(t) / m + 2 * u * np.abs(mean) + u * np.abs(x64 - mean)) + np.abs(xhat) * (rel_istd + 2 * u)
+    assert np.all(np.abs(got - xhat) <= e_xhat)
+    for masked, result in ((g, dx), (want_drelu.astype(np.float64), dx2)):
+        s1, s2 = over(masked), over(masked * xhat)
+        e1 = steps * over(np.abs(masked))
+        e2 = steps * over(np.abs(masked * xhat)) + over(np.abs(masked) * e_xhat)
+        ref = istd * (masked - s1 / m - xhat * s2 / m)
+        bound = istd * (8 * u * (np.abs(masked) + np.abs(s1) / m + np.abs(xhat * s2) / m) +
+                        (e1 + np.abs(xhat) * e2 + e_xhat * np.abs(s2)) / m) + rel_istd * np.abs(ref)
+        assert np.all(np.abs(result.asnumpy() - ref) <= bound)

@@ -421,7 +421,7 @@ def bn_relu_backward(input, doutput, dinput, batchNormMode, mean_p, var_p, cudnn
 
 def bn_and_relu_forward(input, bn_output, relu_output, batchNormMode, n, mean_p, var_p, cudnnlist, activation_list,
                         cudnnHandle, cudaStream):
-    """bn_output = bn(input) and relu_output = max(bn_output, 0), in one pass where the batch fits registers (extension)"""
+    """bn_output = bn(input) and relu_output = max(bn_output, 0), in one pass where a statistic's values fit registers (extension)"""
     _nd_args(input, bn_output, relu_output)
     mode = _enum(_BATCHNORM, batchNormMode)
     wanted = ctypes.c_int(0)
