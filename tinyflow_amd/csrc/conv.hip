@@ -853,18 +853,20 @@ __global__ __launch_bounds__(256) void wino_filter_kernel(const float *__restric
 // output tile of the same index): the input is a dy, and the launch also writes what
 // grad-filter wants of it, dM[pos][cr][t] = (A y A^T)[pos] with y that inner block --
 // grad-data and grad-filter of one layer then read dy once between them.
+// STREAM: the stores are non-temporal (see kStreamTransforms).
 //
 // Addressing: `in`, V and dM are read and written through buffer descriptors, a 32-bit
 // per-lane byte offset plus, for the position planes of V and dM, a uniform plane offset
 // -- one store instruction per value instead of a 64-bit vector address computed for
 // each (every array of a Winograd launch is under 4 GiB: wino_shape bounds the scratch).
-template <int TILE, bool ROW16 = false, bool HALVES = false, bool WITH_DM = false>
+template <int TILE, bool ROW16 = false, bool HALVES = false, bool WITH_DM = false, bool STREAM = false>
 __global__ __launch_bounds__(256) void wino_input_kernel(const float *__restrict__ in, float *__restrict__ V, int Cr,
                                                         int H, int W, FastDiv div_tiles, FastDiv div_tw, int pad_h,
                                                         int pad_w, int T, int Tp, uint32_t in_bytes,
                                                         float *__restrict__ dM = nullptr) {
   static_assert(!ROW16 || TILE == 4, "ROW16 is the 6-wide patch whose columns 1..4 start at a multiple of 4");
   constexpr int A = Wino<TILE>::A;
+  constexpr int kPolicy = STREAM ? 2 : 0;  // of the stores: non-temporal
   const uint32_t t = blockIdx.x * 256 + threadIdx.x;
   const int cr = blockIdx.y;
   if (t >= (uint32_t)Tp) return;
@@ -936,7 +938,7 @@ __global__ __launch_bounds__(256) void wino_input_kernel(const float *__restrict
 #pragma unroll
     for (int j = 0; j < A; ++j)
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, o[j]), rv, (int)lane_off,
-                                            (int)((uint32_t)(i * A + j) * plane_bytes), 0);
+                                            (int)((uint32_t)(i * A + j) * plane_bytes), kPolicy);
   }
   if constexpr (WITH_DM) {
     float q[A][TILE];  // A y, column by column
@@ -957,7 +959,7 @@ __global__ __launch_bounds__(256) void wino_input_kernel(const float *__restrict
 #pragma unroll
       for (int j = 0; j < A; ++j)
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, o[j]), rm, (int)lane_off,
-                                              (int)((uint32_t)(i * A + j) * plane_bytes), 0);
+                                              (int)((uint32_t)(i * A + j) * plane_bytes), kPolicy);
     }
   }
 }
@@ -1857,6 +1859,16 @@ ConvPlan plan_wgrad(const ConvDesc *d) {
 // Nothing is kept under a device-memory budget or with TINYFLOW_KEEP_TRANSFORMED_INPUT=0.
 // Launches the input transform x -> V (and, with dM, the grad-filter form of the same
 // array, see WITH_DM) in the variant the row length and alignment allow.
+//
+// What is written goes past the caches where it is more than the products could find there again (the last-level cache holds 256 MB):
+// a wave writes 256 bytes to each of 36 or 72 planes, and lines that are not to stay make room for each other sooner.
+// One line, dy's pass of 72 planes, us before / after: 512 channels 28 x 28, 32 images, 231 MB 70 / 50 (4.0 -> 5.7 TB/s); 256
+// of 56 x 56, 463 MB 139 / 124; 64 of 224 x 224, 1.85 GB 510 / 491; V alone, 64 of 56 x 56, 64 images, 115 MB 35 / 28.  Of 58 MB
+// it is 16.0 / 14.9 and 24.4 / 25.8 for twice that with dM, and the products read them back slower.  VGG-16, batch 32, a step with lines
+// at none / 300 / 200 / 100 / 50 / 0 MB: 12.63, 12.28, 12.18, 12.16, 12.16, 12.17 ms; ResNet-50, batch 64: 15.91, 15.94, 15.88,
+// 15.84, 15.86, 15.88.
+constexpr double kStreamTransforms = 100e6;
+
 void launch_wino_input(int tile, const float *in, float *V, float *dM, int images, int Cr, int H, int W, int pad_h,
                        int pad_w, const FastDiv &div_tiles, const FastDiv &div_tw, int T, int Tp, hipStream_t s) {
   const dim3 grid(cdiv(Tp, 256), Cr), block(256);
@@ -1868,18 +1880,20 @@ void launch_wino_input(int tile, const float *in, float *V, float *dM, int image
   }
   const bool row16 = pad_w == 1 && W % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
   const bool halves = !row16 && pad_w == 1 && W % 2 == 0 && (reinterpret_cast<uintptr_t>(in) & 7u) == 0;
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, in, V, Cr, H, W, div_tiles, div_tw, pad_h, pad_w, T, Tp, in_bytes, dM);
+  const bool stream = (dM ? 2.0 : 1.0) * 36 * Cr * Tp * sizeof(float) > kStreamTransforms;
+  auto by_form = [&](auto with_dm, auto stream_c) {
+    constexpr bool DM = decltype(with_dm)::value, STREAM = decltype(stream_c)::value;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, 0, s, in, V, Cr, H, W, div_tiles, div_tw, pad_h, pad_w, T, Tp, in_bytes, dM);
+    };
+    if (row16) go(wino_input_kernel<4, true, false, DM, STREAM>);
+    else if (halves) go(wino_input_kernel<4, true, true, DM, STREAM>);
+    else go(wino_input_kernel<4, false, false, DM, STREAM>);
   };
-  if (dM) {
-    if (row16) go(wino_input_kernel<4, true, false, true>);
-    else if (halves) go(wino_input_kernel<4, true, true, true>);
-    else go(wino_input_kernel<4, false, false, true>);
-  } else {
-    if (row16) go(wino_input_kernel<4, true, false, false>);
-    else if (halves) go(wino_input_kernel<4, true, true, false>);
-    else go(wino_input_kernel<4, false, false, false>);
-  }
+  auto by_dm = [&](auto stream_c) {
+    if (dM) by_form(std::true_type{}, stream_c); else by_form(std::false_type{}, stream_c);
+  };
+  if (stream) by_dm(std::true_type{}); else by_dm(std::false_type{});
 }
 
 // dy of a 3x3 / stride-1 layer padded by 1: grad-data's patches and grad-filter's tiles
