@@ -2,7 +2,7 @@
 //
 // Every reduction is a fixed-order, two-stage tree (per-lane serial sums, wave
 // shuffles, then a second pass over per-chunk partials): no atomics, so results
-// are run-to-run deterministic.  The input is read exactly once, which makes the
+// are run-to-run deterministic.  Short sums run both stages in one launch.  The input is read exactly once, which makes the
 // bias gradient HBM-bound at 4*(|dy| + C) bytes.
 //
 // Reference code replaced: src/gpu_op.cu:179-189, 950-963 (axis-0 sum),
@@ -10,6 +10,7 @@
 // :237-302, 1235-1287 (softmax, softmax cross entropy).
 #include "internal.h"
 
+#include <algorithm>
 #include <mutex>
 
 using namespace tf;
@@ -41,14 +42,8 @@ __device__ inline float block_sum(float v, float *smem /*[4]*/) {
   return r;
 }
 
-// in viewed as [A, B] (C == 1): partial[chunk*B + j] = sum over rows of the chunk
-__global__ __launch_bounds__(kThreads) void colsum_kernel(const float *__restrict__ in, float *__restrict__ out,
-                                                         int A, int B, int rows_per_chunk) {
-  const int j = blockIdx.x * kThreads + threadIdx.x;
-  if (j >= B) return;
-  const int a0 = blockIdx.y * rows_per_chunk;
-  int a1 = a0 + rows_per_chunk;
-  if (a1 > A) a1 = A;
+// Sum of rows a0 .. a1-1 of column j of in[A, B].
+__device__ inline float chunk_of_column(const float *__restrict__ in, int a0, int a1, int B, int j) {
   const float *p = in + (int64_t)a0 * B + j;
   float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
   int a = a0;
@@ -63,7 +58,35 @@ __global__ __launch_bounds__(kThreads) void colsum_kernel(const float *__restric
     s0 += p[0];
     p += B;
   }
-  out[(int64_t)blockIdx.y * B + j] = (s0 + s1) + (s2 + s3);
+  return (s0 + s1) + (s2 + s3);
+}
+
+// in viewed as [A, B] (C == 1): partial[chunk*B + j] = sum over rows of the chunk
+__global__ __launch_bounds__(kThreads) void colsum_kernel(const float *__restrict__ in, float *__restrict__ out,
+                                                         int A, int B, int rows_per_chunk) {
+  const int j = blockIdx.x * kThreads + threadIdx.x;
+  if (j >= B) return;
+  const int a0 = blockIdx.y * rows_per_chunk;
+  out[(int64_t)blockIdx.y * B + j] = chunk_of_column(in, a0, min(a0 + rows_per_chunk, A), B, j);
+}
+
+// The same with the chunks folded by the workgroup that has summed them: one launch, the same bits.  A workgroup owns 16
+// columns (64 bytes of a row) and takes up to 64 chunks at a time, a lane each.  Taken where a lane sums few rows: what is left then is the latency
+// of a launch and of its loads, which the pair pays twice (one_launch says where).
+constexpr int kOneCols = 16, kOneSlots = 64, kOneChunks = 256;
+
+__global__ __launch_bounds__(kOneCols * kOneSlots) void colsum_one_kernel(const float *__restrict__ in, float *__restrict__ out, int A, int B,
+                                                         int rows_per_chunk, int chunks) {
+  __shared__ float part[kOneChunks][kOneCols];
+  const int col = threadIdx.x % kOneCols, j = blockIdx.x * kOneCols + col;
+  for (int k = threadIdx.x / kOneCols; k < chunks; k += blockDim.x / kOneCols)
+    part[k][col] = j < B ? chunk_of_column(in, k * rows_per_chunk, min((k + 1) * rows_per_chunk, A), B, j) : 0.f;
+  __syncthreads();
+  if (threadIdx.x >= kOneCols || j >= B) return;
+  float s = 0.f;
+#pragma unroll 16
+  for (int k = 0; k < chunks; ++k) s += part[k][col];
+  out[j] = s;
 }
 
 // in viewed as [A, B, C]: partial[chunk*B + b] = sum_{a in chunk, c} in[a, b, c]
@@ -264,6 +287,43 @@ __global__ __launch_bounds__(1024) void xent_mean_kernel(const float *__restrict
   }
 }
 
+// The same bits in one launch where four rows fit a wave (cols <= 16): a group of 16 lanes takes a row, the lanes past its columns add
+// the zeros that the lanes of a whole wave would.  Four rounds of rows at most; two launches / one, us: 64 x 10 4.6 / 2.6,
+// 128 x 10 5.3 / 3.4, 256 x 16 6.1 / 5.2.
+constexpr int kOneRows = 256;
+__global__ __launch_bounds__(1024) void softmax_xent_one_kernel(const float *__restrict__ logits,
+                                                               const float *__restrict__ labels,
+                                                               float *__restrict__ out, int rows, int cols) {
+  __shared__ float row_loss[kOneRows];
+  const int c = threadIdx.x & 15;
+  for (int r = threadIdx.x >> 4; r < rows; r += 64) {
+    const bool live = c < cols;
+    const float x = live ? logits[(int64_t)r * cols + c] : -INFINITY, t = live ? labels[(int64_t)r * cols + c] : 0.f;
+    float m = fmaxf(-INFINITY, x);
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) m = fmaxf(m, __shfl_down(m, off, 16));
+    m = __shfl(m, 0, 16);
+    float s = live ? expf(x - m) : 0.f;
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) s += __shfl_down(s, off, 16);
+    const float log_s = logf(__shfl(s, 0, 16));
+    float l = 0.f;
+    if (live) l -= t * ((x - m) - log_s);
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) l += __shfl_down(l, off, 16);
+    if (c == 0) row_loss[r] = l;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  float total = 0.f;
+  if (threadIdx.x < 16)
+    for (int r = threadIdx.x; r < rows; r += 16) total += row_loss[r];
+  float s = 0.f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) s += __shfl(total, w, 64);
+  if (threadIdx.x == 0) out[0] = s / (float)rows;
+}
+
 __global__ __launch_bounds__(kThreads) void zero_kernel(float *out, int n) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
   if (i < n) out[i] = 0.f;
@@ -288,6 +348,15 @@ void chunk_rule(int64_t A, int64_t B, int64_t C, int cus, int &chunks, int &rows
   }
   rows_per_chunk = (int)((A + chunks - 1) / chunks);
   chunks = (int)((A + rows_per_chunk - 1) / rows_per_chunk);
+}
+
+// Whether one launch sums the chunks and folds them (us, two launches / one: 64 x 84 3.7 / 2.3, 128 x 256 3.9 / 2.2, 1000 x 120
+// 6.0 / 3.9, 1024 x 1024 6.2 / 3.7, 300 x 4096 5.2 / 2.9, 2048 x 256 7.7 / 5.6).  A lane of long chunks leaves the chip to few waves:
+// 1000 x 4096 7.6 / 7.6, 2000 x 10000 (77 rows) 17.9 / 28.9.
+constexpr int kOneRowsOfLane = 32;
+constexpr int64_t kOneElements = 2 << 20;
+bool one_launch(int64_t A, int64_t B, int64_t C, int chunks, int rows_per_chunk) {
+  return C == 1 && chunks > 1 && chunks <= kOneChunks && cdiv(chunks, kOneSlots) * rows_per_chunk <= kOneRowsOfLane && A * B <= kOneElements;
 }
 
 // out[b] = sum_{a, c} in[a, b, c]; 0 on success, 1 when scratch is exhausted
@@ -315,7 +384,8 @@ int reduce_abc(const float *in, float *out, int64_t A, int64_t B, int64_t C, hip
   int chunks, rows_per_chunk;
   chunk_rule(A, B, C, num_cus(), chunks, rows_per_chunk);
   float *partial = out;
-  if (chunks > 1) {
+  const bool one = one_launch(A, B, C, chunks, rows_per_chunk);
+  if (chunks > 1 && !(one && !fixed)) {
     const size_t bytes = (size_t)chunks * (size_t)B * sizeof(float);
     if (fixed) {
       if (bytes > fixed_bytes) {
@@ -335,6 +405,11 @@ int reduce_abc(const float *in, float *out, int64_t A, int64_t B, int64_t C, hip
       chunks = 1;
       rows_per_chunk = (int)A;
     }
+  }
+  if (one && chunks > 1) {
+    hipLaunchKernelGGL(colsum_one_kernel, dim3(cdiv(B, kOneCols)), dim3(kOneCols * cdiv(std::min(chunks, kOneSlots), 4) * 4), 0, s,
+                       in, out, (int)A, (int)B, rows_per_chunk, chunks);
+    return finish(s, what);
   }
   if (C == 1) {
     hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)blocks_per_chunk, chunks), dim3(kThreads), 0, s, in,
@@ -550,8 +625,12 @@ extern "C" int DLGpuSoftmaxCrossEntropy(const DLArrayHandle logits, const DLArra
   hipStream_t s = stream_of(stream);
   const int rows = (int)logits->shape[0], cols = (int)logits->shape[1];
   // this entry point cannot report exhausted scratch: without it the one-launch form runs
-  float *row_loss = rows > 16 ? (float *)device_alloc((size_t)rows * sizeof(float), s) : nullptr;
-  if (row_loss) {
+  const bool one = rows > 16 && rows <= kOneRows && cols <= 16;
+  float *row_loss = rows > 16 && !one ? (float *)device_alloc((size_t)rows * sizeof(float), s) : nullptr;
+  if (one) {
+    hipLaunchKernelGGL(softmax_xent_one_kernel, dim3(1), dim3(1024), 0, s, (const float *)logits->data,
+                       (const float *)labels->data, (float *)out->data, rows, cols);
+  } else if (row_loss) {
     hipLaunchKernelGGL(softmax_xent_rows_kernel, dim3(cdiv(rows, kThreads / 64)), dim3(kThreads), 0, s,
                        (const float *)logits->data, (const float *)labels->data, row_loss, rows, cols);
     hipLaunchKernelGGL(xent_mean_kernel, dim3(1), dim3(1024), 0, s, (const float *)row_loss, (float *)out->data, rows);
