@@ -277,8 +277,8 @@ int DLGpuConvolutionDescribeKernel(void ***list, int which, char *name, int name
                                    double *flops);
 
 /* No counterpart in the reference.  Whether the three convolutions of a 3x3 / stride-1 descriptor may run on
- * bf16 slices (not before this is called): fp32 results as close to the exact ones, in another rounding.  An owner whose program turns a change
- * of rounding into steps of another sign (Adam on gradients that are nothing but rounding) leaves it. */
+ * bf16 slices (not before this is called): fp32 results as close to the exact ones, in another rounding.  An owner whose program
+ * makes much of a change of rounding (Adam on gradients that are nothing but rounding, batch norms of a spread that is) leaves it. */
 int DLGpuConvolutionAllowSlices(void ***list, int allow);
 
 /* No counterpart in the reference: measurement aid.  The next convolution entry

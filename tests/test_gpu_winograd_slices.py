@@ -57,16 +57,19 @@ def test_error_is_not_above_the_fp32_engines(rt, monkeypatch, case):
     assert all(s <= 1.01 * f for f, s in zip(*errors)), errors
 
 
-def test_executors_give_permission_for_sgd_alone(rt):
+def test_executors_give_permission_for_sgd_without_batch_norm_alone(rt):
     from tinyflow_amd import autodiff as ad, models, TrainExecute, TrainExecuteAdam
-    for module, allowed in ((TrainExecute, True), (TrainExecuteAdam, False)):
+    for module, norms, allowed in ((TrainExecute, False, True), (TrainExecuteAdam, False, False), (TrainExecute, True, False)):
         rng = np.random.RandomState(3)
         X, y = models.synthetic_batch(rng, (4, 3, 64, 64), 10, "normal")
-        model = models.vgg16(rng, batch=4, image=64, n_class=10, fc_width=32)
+        if norms:
+            model = models.resnet(rng, (1, 1, 1, 1), batch=4, image=64, n_class=10, bn_mode="spatial")
+        else:
+            model = models.vgg16(rng, batch=4, image=64, n_class=10, fc_width=32)
         executor = module.TrainExecutor(model.loss, 1e-4)
         executor.init_Variable(dict(model.variables))
         executor.run({model.X: X, model.y_: y})
         plans = [_describe(n.cudnnlist[0], w) for n in executor.topo_order if isinstance(n.op, ad.Convolution2DForwardOp)
-                 for w in range(3)]
+                 and executor.node_to_shape_map[n.inputs[1]][2] == 3 for w in range(3)]
         assert any("Split" in p for p in plans) == allowed, plans
         executor.close()

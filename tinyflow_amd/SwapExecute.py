@@ -28,7 +28,7 @@ import numpy as np
 
 from . import autodiff as ad
 from . import gpu_op, ndarray
-from .TrainExecute import getcomputelist, swapsgd
+from .TrainExecute import getcomputelist, keeps_rounding_small, swapsgd
 
 GPU, HOST, MOVING_OUT, MOVING_IN, FREED = "gpu", "host", "out", "in", "freed"
 
@@ -521,10 +521,11 @@ class SwapExecutor(object):
 
     def _prepare(self, feed_dict):
         shapes = {node: tuple(np.shape(v)) for node, v in feed_dict.items()}
+        slices = keeps_rounding_small(self.topo_order, self.optimizer == "sgd")
         for node in self.topo_order:
             if node not in shapes:
                 shapes[node] = tuple(node.op.infer_shape(node, [shapes[i] for i in node.inputs], self.cudnnHandle))
-                if self.optimizer == "sgd" and isinstance(node.op, ad.Convolution2DForwardOp):
+                if slices and isinstance(node.op, ad.Convolution2DForwardOp):
                     gpu_op.convolution_allow_slices(node.cudnnlist[0])   # the plain executor's kernels, hence its bits
         self.tensors = {node: _Tensor(node, shapes[node]) for node in self.topo_order}
         self.keep = set(n for n in self.topo_order if n.isw in (1, 2)) | {self.targetloss} | self.keep_values

@@ -1316,7 +1316,7 @@ double choose_tile_and_splits(ConvPlan &p, bool wgrad, bool padded, bool scatter
 //     alone: 7x7, 27 -> 45, 33 x 31, batch 20, 56.6 -> 46.6; 1x1 grad-filter, 40 -> 96, 56 x 56, batch 32, 29.9 -> 22.7;
 //     none is slower, strided grad-data by phases aside (48 channels there, see plan_dgrad).
 //   * 3x3 / stride-1 layers, their transformed-domain products included, run on slices only where the descriptor's owner has said
-//     so (DLGpuConvolutionAllowSlices; the executors do for SGD).  Networks of such layers under a batch-norm head (VGG-16
+//     so (DLGpuConvolutionAllowSlices; the executors do for SGD on networks without batch norm).  Networks of such layers under a batch-norm head (VGG-16
 //     with dropout, Adam) turn any change of rounding into steps of Adam the other way: a different summation order of
 //     the fp32 engine alone moves their gradients by more than half their size.
 int forced_engine() {
