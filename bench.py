@@ -399,16 +399,19 @@ def main():
     if args.config.startswith("resnet"):
         kw["bn_mode"] = args.bn_mode
     model, X, y = models.build(args.config, **kw)
+    # VGG-16 has no batch norm: one step of 0.01 from He-normal weights leaves the finite numbers, and steps of NaN
+    # are not what anybody trains (contractions on bf16 slices compute their tiles a second time then)
+    lr = 1e-7 if args.config == "vgg16" else 0.01
     if args.mem_limit_gb > 0:
         from tinyflow_amd.SwapExecute import SwapExecutor
         limit = int(args.mem_limit_gb * (1 << 30))
         gpu_op.set_device_memory_limit(limit)
         # planned for the whole budget; a step that has to evict on demand makes the
         # executor plan for 3 % less (which the warm-up steps absorb)
-        ex = SwapExecutor(model.loss, 0.01, swap=True, memory_budget=limit, prefetch_distance=12,
+        ex = SwapExecutor(model.loss, lr, swap=True, memory_budget=limit, prefetch_distance=12,
                           recompute=not args.no_recompute)
     else:
-        ex = TrainExecutor(model.loss, 0.01, fuse_bn_relu=args.fuse_bn_relu)
+        ex = TrainExecutor(model.loss, lr, fuse_bn_relu=args.fuse_bn_relu)
     ex.init_Variable(dict(model.variables))
     feed = {model.X: X, model.y_: y}
 
@@ -482,7 +485,7 @@ def main():
     if (not args.fuse_bn_relu and not args.no_fused_leg and not args.mem_limit_gb
             and args.config.startswith("resnet") and args.bn_mode == "pre_activation"):
         model2, X2, y2 = models.build(args.config, **kw)
-        ex2 = TrainExecutor(model2.loss, 0.01, fuse_bn_relu=True)
+        ex2 = TrainExecutor(model2.loss, lr, fuse_bn_relu=True)
         ex2.init_Variable(dict(model2.variables))
         ex2.run({model2.X: X2, model2.y_: y2})
         for _ in range(2):
@@ -599,9 +602,9 @@ def main():
         "value": imgs_per_sec, "unit": "imgs/sec", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": ms_per_step, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f32", "data": "synthetic",
-        "config": {"workload": "%s batch %d fp32 3x224x224, fwd+bwd+SGD(lr 0.01), BN mode %s, "
+        "config": {"workload": "%s batch %d fp32 3x224x224, fwd+bwd+SGD(lr %g), BN mode %s, "
                                "softmax-xent over %d random one-hot classes, He-normal weights"
-                               % (args.config, args.batch, args.bn_mode, model.n_class)},
+                               % (args.config, args.batch, lr, args.bn_mode, model.n_class)},
         "gpu_ms_per_step": gpu_ms / args.steps, "loss": loss_val,
         "host_fed": {"ms_per_step": host_fed_ms, "imgs_per_sec": args.batch * 1e3 / host_fed_ms, "steps": host_steps,
                      "note": "batch re-uploaded from pageable host memory every step (PCIe-inclusive)"},
