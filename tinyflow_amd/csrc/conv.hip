@@ -1323,11 +1323,11 @@ int forced_engine() {
   const char *e = getenv("TINYFLOW_SPLIT");
   return e && *e ? atoi(e) : -1;
 }
+bool dense_3x3(const ConvDesc *d) { return d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1; }
 bool may_use_split(const ConvDesc *d) {
   const int forced = forced_engine();
   if (forced >= 0) return forced != 0;
-  const bool dense_3x3 = d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1;
-  return (!dense_3x3 || d->slices_3x3) && d->C >= 24 && d->K >= 24;
+  return (!dense_3x3(d) || d->slices_3x3) && d->C >= 24 && d->K >= 24;
 }
 
 // Grad-filter's gathered x by vectors (SplitGatherAcross MODE 2 and 3): four outputs of one row at a time.
@@ -1356,16 +1356,20 @@ double choose_direct(ConvPlan &p, ConvPlan on_split, const ConvDesc *d, const Sp
                      bool scatter, bool may_split, double out_bytes) {
   double us = choose_tile_and_splits(p, wgrad, padded, scatter, may_split, out_bytes);
   // Not faster there (us, fp32 / split): grad-data of at most 64 rows 64 <- 256 channels 56 x 56, batch 64, 69 / 74; strided
-  // grad-filter whose x comes one element at a time 512 -> 1024 channels 28 x 28 stride 2, 130 / 142.
-  const bool slow = wgrad ? on_split.b_vec == false && d->v > 1 && !vector_gather(d) : traffic.which == 1 && p.M <= 64;
+  // grad-filter whose x comes one element at a time 512 -> 1024 channels 28 x 28 stride 2, 130 / 142; grad-filter of 3x3 / stride 1
+  // out of its transformed domain, short reductions above all, 64 channels 6 x 6, batch 4, 8.8 / 9.7, 64 -> 128, 28 x 28, batch 6,
+  // 20.4 / 22.5, 27 such layers in all 465 / 463.
+  const bool slow = wgrad ? dense_3x3(d) || (!on_split.b_vec && d->v > 1 && !vector_gather(d)) : traffic.which == 1 && p.M <= 64;
   if (!may_use_split(d) || (slow && forced_engine() != 1)) return us;
   on_split.split = true;
   const double split_us = choose_tile_and_splits(on_split, wgrad, padded, scatter, may_split, out_bytes, &traffic);
   if (split_us < 1.15 * us + 4.0 || forced_engine() == 1) {
     p = on_split;
-    // 3x3 / stride 1: what the transformed domain is compared with stays the fp32 form.  The gather bounds the direct form on slices
-    // (56 x 56, 64 channels, batch 64, three calls 462 us against 335), and a call that leaves the domain takes its transforms from the others.
-    if (!(d->R == 3 && d->S == 3 && d->u == 1 && d->v == 1)) us = split_us;
+    // 3x3 / stride 1: what the transformed domain is compared with stays the fp32 form.  Where both fit, the domain is the better one
+    // (56 x 56, 64 channels, batch 64, three calls direct on slices 462 us, there 335), and a call that leaves it takes its transforms
+    // from the others.  Where the direct form stays, on small maps and few channels, slices are faster: 167 layers of 24 - 512 channels,
+    // 2 x 2 to 56 x 56, batch 1 to 64, forward 2091 / 1786 us in all, grad-data 2886 / 2563, none slower.
+    if (!dense_3x3(d)) us = split_us;
   }
   return us;
 }
