@@ -28,3 +28,11 @@ def _plans(n, c, h, w, k, padding="SAME"):
 def test_direct_grad_filter_keeps_its_engine(layer):
     without, with_permission = _plans(*layer)
     assert "winograd" not in without[2] and with_permission[2] == without[2]
+
+
+# ragged channels, many images of small maps, one image of large ones
+@pytest.mark.parametrize("layer", [(5, 96, 40, 40, 72), (32, 96, 14, 14, 72), (60, 240, 7, 7, 92), (1, 64, 102, 102, 96), (5, 320, 22, 22, 96)],
+                         ids=str)
+def test_permission_takes_no_grad_data_out_of_the_transformed_domain(layer):
+    without, with_permission = _plans(*layer)
+    assert "winograd" in without[1] and "winograd" in with_permission[1], with_permission

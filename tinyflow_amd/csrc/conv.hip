@@ -1467,7 +1467,11 @@ void consider_winograd(ConvPlan &p, const ConvDesc *d, bool dgrad, double direct
   const int forced = force && *force ? atoi(force) : -1;
   if (forced == 0) return;
   static const int tiles[3][2] = {{128, 128}, {64, 128}, {64, 64}};
-  double best_us = 1e30;
+  // Grad-data stays in the domain if its fp32 products would run there: grad-filter's transform of dy comes from the same pass.  us of three
+  // calls on slices, grad-data direct / here: 96 -> 72 channels 40 x 40, batch 5, 69 / 60; 320 -> 96, 22 x 22, batch 5, 72 / 60; 240 -> 92,
+  // 7 x 7, batch 60, 77 / 67; of 34 such layers 24 are faster and 5 slower, 0.95 in all (416 -> 32, 27 x 27, batch 21, 120 / 137 is the worst).  Forward
+  // is as often slower (32 -> 96, 105 x 105, 63 / 72; 64 -> 64, 60 x 60, batch 9, 100 / 76) and goes by the model of what it runs on.
+  double best_us = 1e30, fp32_us = 1e30;
   int best_tile = 0, best_bm = 64, best_bn = 64;
   bool best_split = false;
   WinoShape best_w;
@@ -1482,7 +1486,7 @@ void consider_winograd(ConvPlan &p, const ConvDesc *d, bool dgrad, double direct
     const double moved = in_bytes + out_bytes + 4.0 * (w.v_elems + w.m_elems) + 8.0 * w.u_elems;
     // short reductions: the products themselves stream V and M once more
     const double stream_us = 4.0 * (w.v_elems + w.m_elems) / 5.0e6;
-    double best = 1e30;
+    double best = 1e30, best_fp32 = 1e30;
     int bm = 64, bn = 64;
     bool split = false;
     for (auto &t : tiles) {
@@ -1490,12 +1494,14 @@ void consider_winograd(ConvPlan &p, const ConvDesc *d, bool dgrad, double direct
       const double fp32 = predict_us(w.Mo, w.Tp, w.Cr, t[0], t[1], 1, false, false, false, 0.0, w.positions);
       const double sliced = slices ? predict_split_batched_us(w.Mo, w.Tp, w.Cr, t[0], t[1], 1, stage_depth(t[0], t[1]), dgrad,
                                                               w.positions) : 1e30;
+      best_fp32 = std::min(best_fp32, fp32);
       take_engine(fp32, sliced, stream_us, slices, best, split, [&] {
         bm = t[0];
         bn = t[1];
       });
     }
     const double wino_us = std::max(best, stream_us) + moved / 4.0e6 + 6.0;
+    fp32_us = std::min(fp32_us, std::max(best_fp32, stream_us) + moved / 4.0e6 + 6.0);
     if (wino_us < best_us) {
       best_us = wino_us;
       best_tile = tile;
@@ -1505,7 +1511,7 @@ void consider_winograd(ConvPlan &p, const ConvDesc *d, bool dgrad, double direct
       best_w = w;
     }
   }
-  if (best_tile == 0 || (forced < 0 && best_us >= direct_us)) return;
+  if (best_tile == 0 || (forced < 0 && (dgrad ? std::min(best_us, fp32_us) : best_us) >= direct_us)) return;
   p.winograd = true;
   p.wino_tile = best_tile;
   p.variant = best_tile == 2 ? variant2 : variant4;
