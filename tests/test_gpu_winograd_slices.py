@@ -73,3 +73,74 @@ def test_executors_give_permission_for_sgd_without_batch_norm_alone(rt):
                  and executor.node_to_shape_map[n.inputs[1]][2] == 3 for w in range(3)]
         assert any("Split" in p for p in plans) == allowed, plans
         executor.close()
+
+
+def _calls(rt, case, spoil):
+    """Outputs of the three calls of a layer in the transformed domain, and the time of its product-heavy calls, with `spoil` applied to x, w
+    and dy before."""
+    import time
+    from tinyflow_amd import gpu_op, ndarray
+    N, C, H, W, K = case
+    rng = np.random.RandomState(parity.stable_seed(case))
+    x = np.maximum(rng.normal(0, 1, (N, C, H, W)), 0).astype(np.float32)
+    w = rng.normal(0, np.sqrt(2.0 / (C * 9)), (K, C, 3, 3)).astype(np.float32)
+    dy = rng.normal(0, 1, (N, K, H, W)).astype(np.float32)
+    spoil(x, w, dy)
+    gx, gw, gdy = _gpu(x, rt), _gpu(w, rt), _gpu(dy, rt)
+    outs = [ndarray.empty(a.shape, rt.ctx) for a in (dy, x, w)]
+    _, lst = gpu_op.convolution_2d_forward_get_out_shape(x.shape, w.shape, "NCHW", "SAME", 1, 1)
+
+    def step():
+        assert gpu_op.convolution_2d_forward(gx, gw, outs[0], lst, rt.cudnn, rt.stream) == 0
+        assert gpu_op.convolution_backward_data(gx, gdy, gw, outs[1], lst, rt.cudnn, rt.stream) == 0
+        assert gpu_op.convolution_backward_filter(gx, gdy, gw, outs[2], lst, rt.cudnn, rt.stream) == 0
+    step()
+    values = [o.asnumpy() for o in outs]
+    best = 1e9
+    for _ in range(5):
+        start = time.perf_counter()
+        for _ in range(20):
+            step()
+        outs[2].asnumpy()
+        best = min(best, time.perf_counter() - start)
+    return values, best
+
+
+# the first and the last stage of a reduction, one value and all of them, of every operand
+@pytest.mark.parametrize("what", ["x first inf", "x last nan", "w first nan", "w last -inf", "dy first inf", "dy last nan", "all nan"])
+def test_values_that_are_not_finite(rt, monkeypatch, what):
+    """What is finite on the fp32 engine is finite on slices, and within the rounding of two fp32 sums of it."""
+    def spoil(x, w, dy):
+        if what == "all nan":
+            for a in (x, w, dy):
+                a[...] = np.nan
+            return
+        name, place, value = what.split(" ")
+        {"x": x, "w": w, "dy": dy}[name][0, 0 if place == "first" else -1, 1, 1] = float(value)
+    monkeypatch.setenv("TINYFLOW_WINOGRAD", "4")
+    results = []
+    for engine in ("0", "1"):
+        monkeypatch.setenv("TINYFLOW_SPLIT", engine)
+        results.append(_calls(rt, (2, 136, 20, 20, 72), spoil)[0])
+    for fp32, slices, terms in zip(*results, (136 * 9, 72 * 9, 800)):
+        finite = np.isfinite(fp32)
+        assert (np.isfinite(slices) == finite).all()
+        if finite.any():
+            # sums of random signs: 2^-24 sqrt(terms) of their size apart, 2.7 times that in this domain, and the transforms' rounding
+            assert (np.abs(fp32 - slices)[finite] <= 6 * (2.7 * 2.0 ** -24 * np.sqrt(terms) + 4e-6) * np.abs(fp32[finite]).std()).all()
+
+
+def test_steps_on_nan_take_about_the_fp32_engines_time(rt, monkeypatch):
+    """Nothing of the slices' work is done for a tile whose first operands show that the fp32 pass will compute it: with it the three
+    calls took twice the fp32 engine's time, without it they take 1.2 times."""
+    monkeypatch.setenv("TINYFLOW_WINOGRAD", "4")
+
+    def spoil(x, w, dy):
+        for a in (x, w, dy):
+            a[...] = np.nan
+    times = []
+    for engine in ("0", "1"):
+        monkeypatch.setenv("TINYFLOW_SPLIT", engine)
+        times.append(_calls(rt, (32, 512, 28, 28, 512), spoil)[1])
+    print(times)
+    assert times[1] <= 1.6 * times[0], times

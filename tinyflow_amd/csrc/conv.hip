@@ -679,6 +679,7 @@ __global__ __launch_bounds__(256) void filter_to_phases_kernel(const float *__re
 // rotated by 180 degrees.  U, V and M live in scratch memory.
 template <class L>
 struct Batched : L {
+  static constexpr bool kBatched = true;
   int64_t batch_stride;  // elements between the operands of consecutive problems
   __device__ inline void init(typename L::State &st, int origin, int tid) const {
     L one = *this;
@@ -1469,7 +1470,7 @@ void consider_winograd(ConvPlan &p, const ConvDesc *d, bool dgrad, double direct
   static const int tiles[3][2] = {{128, 128}, {64, 128}, {64, 64}};
   // Grad-data stays in the domain if its fp32 products would run there: grad-filter's transform of dy comes from the same pass.  us of three
   // calls on slices, grad-data direct / here: 96 -> 72 channels 40 x 40, batch 5, 69 / 60; 320 -> 96, 22 x 22, batch 5, 72 / 60; 240 -> 92,
-  // 7 x 7, batch 60, 77 / 67; of 34 such layers 24 are faster and 5 slower, 0.95 in all (416 -> 32, 27 x 27, batch 21, 120 / 137 is the worst).  Forward
+  // 7 x 7, batch 60, 77 / 67; of 34 such layers 24 are faster and 6 slower, 0.95 in all (416 -> 32, 27 x 27, batch 21, 120 / 137 is the worst).  Forward
   // is as often slower (32 -> 96, 105 x 105, 63 / 72; 64 -> 64, 60 x 60, batch 9, 100 / 76) and goes by the model of what it runs on.
   double best_us = 1e30, fp32_us = 1e30;
   int best_tile = 0, best_bm = 64, best_bn = 64;
