@@ -1876,9 +1876,10 @@ ConvPlan plan_wgrad(const ConvDesc *d) {
 // One line, dy's pass of 72 planes, us before / after: 512 channels 28 x 28, 32 images, 231 MB 70 / 50 (4.0 -> 5.7 TB/s); 256
 // of 56 x 56, 463 MB 139 / 124; 64 of 224 x 224, 1.85 GB 510 / 491; V alone, 64 of 56 x 56, 64 images, 115 MB 35 / 28.  Of 58 MB
 // it is 16.0 / 14.9 and 24.4 / 25.8 for twice that with dM, and the products read them back slower.  VGG-16, batch 32, a step with lines
-// at none / 300 / 200 / 100 / 50 / 0 MB: 12.63, 12.28, 12.18, 12.16, 12.16, 12.17 ms; fused ResNet-50, batch 32, whose largest are
-// 116 MB, 8.987 / 8.989 / 9.006 at none / 200 / 100.
-constexpr double kStreamTransforms = 200e6;
+// at none / 300 / 200 / 100 / 50 / 0 MB: 12.63, 12.28, 12.18, 12.16, 12.16, 12.17 ms; ResNet-50, batch 64: 15.91, 15.94, 15.88,
+// 15.84, 15.86, 15.88.  Between 100 and 200 MB: 64 channels of 55 x 55, 32 images, 116 MB with dM, three calls 206.0 us at 100 and 208.3 at
+// 200 (runs differ by 0.3 %); fused ResNet-50, batch 32, whose largest are 116 MB, 8.94 and 8.91 ms (0.7 %).
+constexpr double kStreamTransforms = 100e6;
 
 void launch_wino_input(int tile, const float *in, float *V, float *dM, int images, int Cr, int H, int W, int pad_h,
                        int pad_w, const FastDiv &div_tiles, const FastDiv &div_tw, int T, int Tp, hipStream_t s) {
