@@ -380,7 +380,7 @@ __global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : BN == 128 ? 3 : 
   if (tid == 0) flag = 0u;
   // Transformed-domain products: a workgroup that fetches anything infinite or NaN for its first stage leaves its tile to the fp32 pass at
   // once, which for them keeps two stages in LDS and one chain of sums, as the fp32 kernel does.  VGG-16, batch 32, steps on nothing but
-  // NaN: 18.2 ms with all of the slices' work before that pass and one stage in it, now 14.7, with the fp32 kernel 13.7; finite steps are
+  // NaN: 18.2 ms with all of the slices' work before that pass and one stage in it, now 14.2, with the fp32 kernel 13.7; finite steps are
   // as fast as without the look.
   constexpr bool LEAVES = leaves_early<BLoader>::value;
   __shared__ unsigned lost[4];
@@ -488,6 +488,7 @@ __global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : BN == 128 ? 3 : 
     if (flag != 0u) {  // uniform over the workgroup
       constexpr int PASS = BK * (LDA + LDB);  // floats of a stage: [k][m], then [k][n]
       constexpr bool TWO = LEAVES;            // stages in LDS: one is multiplied while the next one is on its way
+      constexpr int UNROLL = TWO ? 4 : 1;
       static_assert(2 * (PA::BYTES + PB::BYTES) >= (TWO ? 2 : 1) * PASS * 4, "the fp32 pass reuses the planes");
       float *const planes = reinterpret_cast<float *>(lds);
       auto fetch = [&](int k0) {
@@ -527,9 +528,10 @@ __global__ __launch_bounds__(THREADS, BM *BN == 128 * 128 ? 2 : BN == 128 ? 3 : 
               for (int v = 0; v < 16; ++v) low[i][j][v] = 0.f;
         }
         auto &sum = TWO ? acc : low;
-        const float *const fa = planes + at + m_wave + lcol, *const fb = planes + at + BK * LDA + n_wave + lcol;
-#pragma unroll(TWO ? 4 : 1)
-        for (int k = lhalf; k < BK; k += 2)
+        const float *const fa = planes + at + lhalf * LDA + m_wave + lcol;
+        const float *const fb = planes + at + BK * LDA + lhalf * LDB + n_wave + lcol;
+#pragma unroll UNROLL
+        for (int k = 0; k < BK; k += 2)
 #pragma unroll
           for (int i = 0; i < TM; ++i)
 #pragma unroll
