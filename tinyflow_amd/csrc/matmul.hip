@@ -14,6 +14,8 @@
 #include "gemm_split.h"
 #include "internal.h"
 
+#include <algorithm>
+
 using namespace tf;
 using namespace tf::gemm;
 
@@ -62,9 +64,8 @@ __global__ __launch_bounds__(256) void split_sum_vec_kernel(const f32x4 *__restr
 }
 
 // Any other output: one lane per element adds the splits in index order.  Bound by the loads' latency: that lane has
-// kOrderedDepth of them in flight.  More splits of fewer elements than fill the CUs go through LDS: a workgroup fetches 512 splits of four
-// elements at a time, each lane eight values, while four lanes add the ones before.  The 150 filter words of a 1 -> 6 channel 5x5 layer:
-// 1 021 splits by one lane, thirty-two loads at a time, 28 us, this way 10.6; 392 splits 10.9 and 5.6.
+// kOrderedDepth of them in flight.  Many splits of few elements go through LDS (sum_through_lds): a workgroup fetches 512 splits of four
+// elements at a time, each lane eight values, while four lanes add the ones before.
 constexpr int kOrderedDepth = 32;
 __global__ __launch_bounds__(64) void split_sum_ordered_kernel(const float *__restrict__ partial,
                                                               float *__restrict__ out, int64_t count, int splits) {
@@ -82,6 +83,13 @@ __global__ __launch_bounds__(64) void split_sum_ordered_kernel(const float *__re
 #pragma unroll 4
   for (; k < splits; ++k) s += __builtin_nontemporal_load(partial + (int64_t)k * count + i);
   out[i] = s;
+}
+
+// Whether LDS is the better way.  us, one lane an element / through LDS: 150 values in 392 pieces 6.0 / 4.6, 1 021 17.9 / 9.5; 601 in 129
+// 3.9 / 3.6; 1 350 in 257 7.3 / 6.5; 2 402 in 513 13.2 / 12.9.  Past the line: 601 in 65 2.8 / 3.4, 1 350 in 129 4.4 / 4.7, 2 402 in 257
+// 7.5 / 7.7, 4 801 in 513 13.3 / 18.1 (a wave reads 16 bytes of a line), 65 533 in 33 3.7 / 21.4 and in 1 021 62 / 334.
+bool sum_through_lds(int64_t count, int splits) {
+  return splits > 4 * kOrderedDepth && count <= std::min(2048, 5 * splits);
 }
 
 __global__ __launch_bounds__(256) void split_sum_tiles_kernel(const float *__restrict__ partial, float *__restrict__ out,
@@ -213,12 +221,11 @@ int launch_split_sum(const float *partial, float *out, int64_t count, int splits
     else if (sg == 4) hipLaunchKernelGGL(split_sum_vec_kernel<4>, dim3(blocks), dim3(256), 0, s, p4, o4, count4, splits);
     else hipLaunchKernelGGL(split_sum_vec_kernel<16>, dim3(blocks), dim3(256), 0, s, p4, o4, count4, splits);
   } else {
-    // a wide output has lanes enough to be bound by the bytes
-    if (splits <= kOrderedDepth || count >= 65536)
-      hipLaunchKernelGGL(split_sum_ordered_kernel, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, s, partial, out, count,
+    if (sum_through_lds(count, splits))
+      hipLaunchKernelGGL(split_sum_tiles_kernel, dim3((unsigned)((count + 3) / 4)), dim3(256), 0, s, partial, out, count,
                          splits);
     else
-      hipLaunchKernelGGL(split_sum_tiles_kernel, dim3((unsigned)((count + 3) / 4)), dim3(256), 0, s, partial, out, count,
+      hipLaunchKernelGGL(split_sum_ordered_kernel, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, s, partial, out, count,
                          splits);
   }
   return 0;
