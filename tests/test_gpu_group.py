@@ -58,6 +58,16 @@ def test_group_writes_the_bytes_of_the_separate_calls(rt, shape, per_channel):
         assert [g == w for g, w in zip(got, want)] == [True] * len(want)
 
 
+def _alias(start, like):
+    """What looks like an array of the shape of `like` at the address of `start`, for calls that refuse it before anything is read."""
+    import ctypes
+    from types import SimpleNamespace
+    from tinyflow_amd.ndarray import DLArray
+    view = DLArray.from_buffer_copy(like.handle.contents)
+    view.data = start.handle.contents.data
+    return SimpleNamespace(handle=ctypes.pointer(view))
+
+
 def _steps(G, rows, per_channel=False):
     steps = (G.GroupStep * len(rows))()
     for step, (kind, value, a, b, out) in zip(steps, rows):
@@ -74,8 +84,12 @@ def test_group_refuses_what_it_cannot_order(rt):
     from tinyflow_amd import gpu_op as G, ndarray
     a, b, c = (ndarray.array(np.full((4, 8), v, np.float32), rt.ctx) for v in (1, 2, 3))
     short = ndarray.array(np.ones((4, 4), np.float32), rt.ctx)
+    one = ndarray.array(np.ones(1, np.float32), rt.ctx)
+    long_at_one = _alias(one, a)   # longer than the step's result at the same address
     add = G.GROUP_ADD_CONST
-    for rows in ([(add, 1.0, a, None, b), (add, 1.0, c, None, b)],          # written twice
+    for rows in ([(G.GROUP_SET, 1.0, None, None, one), (add, 1.0, a, None, b), (add, 1.0, long_at_one, None, c)],
+                 [(add, 1.0, a, None, b), (G.GROUP_SET, 1.0, None, None, one), (G.GROUP_MUL, 0.0, a, long_at_one, c)],
+                 [(add, 1.0, a, None, b), (add, 1.0, c, None, b)],          # written twice
                  [(add, 1.0, a, None, b), (add, 1.0, c, None, a)],          # a later step writes what an earlier one read
                  [(add, 1.0, a, None, a)],                                  # in place
                  [(add, 1.0, a, None, b), (add, 1.0, short, None, c)],      # lengths

@@ -156,9 +156,9 @@ extern "C" int DLGpuElementwiseGroup(const DLGroupStep *steps, int n_steps, int 
       for (int j = 0; j < k; ++j) TF_REQUIRE(g.s[j].out != s.a, "an operand that is spread cannot come from the group");
     } else {
       TF_REQUIRE((!has_a || numel(in.a) == m) && (!has_b || numel(in.b) == m), "shape mismatch");
-      for (int j = 0; j < k; ++j) {
-        if (has_a && g.s[j].out == s.a) s.from_a = j;
-        if (has_b && g.s[j].out == s.b) s.from_b = j;
+      for (int j = 0; j < k; ++j) {  // the whole of what a step makes: lanes have no more of it
+        if (has_a && g.s[j].out == s.a && g.s[j].n == m) s.from_a = j;
+        if (has_b && g.s[j].out == s.b && g.s[j].n == m) s.from_b = j;
       }
       if (has_a && s.from_a < 0) fits(in.a);
       if (has_b && s.from_b < 0) fits(in.b);
