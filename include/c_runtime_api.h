@@ -299,7 +299,7 @@ int DLGpuKeptByproductCounts(long long *kept_blocks, long long *taken_blocks, in
 
 /* No counterpart in the reference.  Up to six elementwise calls as one launch: each step writes its output as the
  * call that it stands for does, and a step may read what an earlier one wrote.  The outputs have one length, or a single
- * element; nothing that a step reads from outside may be written by the group.
+ * element, and the operands of a step its output's shape; nothing that a step reads from outside may be written by the group.
  *   kGroupSet out = value; kGroupAdd / kGroupMul out = a + b, a * b; kGroupAddConst / kGroupMulConst with value;
  *   kGroupRelu out = a < 0 ? 0 : a; kGroupReluGradient out = a > 0 ? b : 0;
  *   kGroupBroadcast out = a along the trailing dims, or with per_channel along dim 1.

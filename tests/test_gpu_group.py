@@ -84,6 +84,7 @@ def test_group_refuses_what_it_cannot_order(rt):
     from tinyflow_amd import gpu_op as G, ndarray
     a, b, c = (ndarray.array(np.full((4, 8), v, np.float32), rt.ctx) for v in (1, 2, 3))
     short = ndarray.array(np.ones((4, 4), np.float32), rt.ctx)
+    turned, four = ndarray.array(np.ones((8, 4), np.float32), rt.ctx), ndarray.array(np.ones(4, np.float32), rt.ctx)
     one = ndarray.array(np.ones(1, np.float32), rt.ctx)
     long_at_one = _alias(one, a)   # longer than the step's result at the same address
     add = G.GROUP_ADD_CONST
@@ -93,6 +94,8 @@ def test_group_refuses_what_it_cannot_order(rt):
                  [(add, 1.0, a, None, b), (add, 1.0, c, None, a)],          # a later step writes what an earlier one read
                  [(add, 1.0, a, None, a)],                                  # in place
                  [(add, 1.0, a, None, b), (add, 1.0, short, None, c)],      # lengths
+                 [(add, 1.0, turned, None, b)], [(G.GROUP_RELU_GRADIENT, 0.0, a, turned, b)],   # shapes of one length
+                 [(G.GROUP_BROADCAST, 0.0, four, None, b)], [(G.GROUP_BROADCAST, 0.0, short, None, b)],   # not the trailing dims
                  [(99, 1.0, a, None, b)], [(G.GROUP_ADD, 0.0, a, None, b)],
                  [(add, 1.0, a, None, b)] * 7):
         with pytest.raises(RuntimeError):
@@ -152,3 +155,19 @@ def test_which_nodes_form_a_group():
     assert find_groups(order, shapes, fed, {s: ("skip",), r: ("add_relu", s, [x, spread])}, {}) == {back2: [back2, shifted]}
     shapes.update({n: (2 ** 12, 2 ** 12) for n in (spread, s, r, back2, shifted)})
     assert find_groups(order, shapes, fed, {}, {}) == {}   # too long
+
+
+def test_nodes_of_unequal_shapes_are_left_to_their_own_calls():
+    """An adjoint of as many elements in another shape: ``ReluGradient`` refuses it, the activation's backward pass takes it."""
+    from tinyflow_amd import autodiff as ad
+    from tinyflow_amd.TrainExecute import find_groups
+    x, dy = ad.Placeholder("x"), ad.Placeholder("dy")
+    for gradient in (lambda: ad.relu_gradient_op(x, dy), lambda: ad.activation_backward_op(x, dy, x, "relu", [None])):
+        g = gradient()
+        shifted = g + 2.0
+        doubled = shifted * 2.0
+        order = [x, dy, g, shifted, doubled]
+        for shape, expected in (((8, 12), {g: [g, shifted, doubled]}), ((12, 8), {shifted: [shifted, doubled]})):
+            shapes = {n: (8, 12) for n in order}
+            shapes[dy] = shape
+            assert find_groups(order, shapes, {x, dy}, {}, {}) == expected

@@ -446,7 +446,15 @@ MAX_GROUP_ELEMENTS = 1 << 23
 
 
 def _group_step(node, shapes):
-    """How one step of ``elementwise_group`` computes ``node``: (kind, constant, operands), or None."""
+    """How one step of ``elementwise_group`` computes ``node``: (kind, constant, operands), or None.  Operands of another shape are
+    left to the node's own call, which takes or refuses them."""
+    step = _step_of(node, shapes)
+    if step is not None and step[0] != gpu_op.GROUP_BROADCAST and any(shapes[i] != shapes[node] for i in step[2]):
+        return None
+    return step
+
+
+def _step_of(node, shapes):
     op, inputs = node.op, node.inputs
     if isinstance(op, (ad.AddOp, ad.MulOp)) and len(inputs) == 2:
         which = _added_zeros_operand(node, shapes)
@@ -464,7 +472,7 @@ def _group_step(node, shapes):
     elif isinstance(op, (ad.OnesLikeOp, ad.ZerosLikeOp)):
         return gpu_op.GROUP_SET, 1.0 if isinstance(op, ad.OnesLikeOp) else 0.0, []
     elif isinstance(op, ad.BroadcastToOp):
-        # (1,) spreads over anything; else the operand is the channels, or the trailing dims
+        # a bias: one value for each channel, or for each column
         if node.type == "NCHW" or len(shapes[inputs[0]]) == 1 and shapes[node][-1:] == shapes[inputs[0]]:
             return gpu_op.GROUP_BROADCAST, 0.0, [inputs[0]]
     elif isinstance(op, ad.ReluOp):

@@ -145,17 +145,24 @@ extern "C" int DLGpuElementwiseGroup(const DLGroupStep *steps, int n_steps, int 
     TF_REQUIRE(m == n || m == 1, "the steps of a group have one length");
     fits(in.out);
     if (in.kind == kGroupBroadcast) {
+      // what DLGpuBroadcastTo0 and 1 take
       int64_t inner = 1;
       for (int i = 2; in.per_channel && i < in.out->ndim; ++i) inner *= in.out->shape[i];
       const int64_t channels = numel(in.a);
-      if (in.per_channel)
+      if (in.per_channel) {
         TF_REQUIRE(in.a->ndim == 1 && in.out->ndim >= 2 && channels == in.out->shape[1], "input must be (C,) and output (N, C, ...)");
-      TF_REQUIRE(channels > 0 && inner > 0 && m % (channels * inner) == 0, "the operand does not fill the output");
+      } else if (!(in.a->ndim == 1 && channels == 1)) {
+        TF_REQUIRE(in.a->ndim <= in.out->ndim, "input has more dims than output");
+        for (int i = 0; i < in.a->ndim; ++i)
+          TF_REQUIRE(in.a->shape[in.a->ndim - 1 - i] == in.out->shape[in.out->ndim - 1 - i],
+                     "input must match the trailing dims of the output");
+      }
+      TF_REQUIRE(channels > 0 && inner > 0, "empty operand");
       s.inner = FastDiv((uint32_t)inner);
       s.channels = FastDiv((uint32_t)channels);
       for (int j = 0; j < k; ++j) TF_REQUIRE(g.s[j].out != s.a, "an operand that is spread cannot come from the group");
     } else {
-      TF_REQUIRE((!has_a || numel(in.a) == m) && (!has_b || numel(in.b) == m), "shape mismatch");
+      TF_REQUIRE((!has_a || same_shape(in.a, in.out)) && (!has_b || same_shape(in.b, in.out)), "shape mismatch");
       for (int j = 0; j < k; ++j) {  // the whole of what a step makes: lanes have no more of it
         if (has_a && g.s[j].out == s.a && g.s[j].n == m) s.from_a = j;
         if (has_b && g.s[j].out == s.b && g.s[j].n == m) s.from_b = j;
