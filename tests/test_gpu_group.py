@@ -171,3 +171,27 @@ def test_nodes_of_unequal_shapes_are_left_to_their_own_calls():
             shapes = {n: (8, 12) for n in order}
             shapes[dy] = shape
             assert find_groups(order, shapes, {x, dy}, {}, {}) == expected
+
+
+@pytest.mark.gpu
+def test_a_steps_constants_are_those_of_their_nodes_now(rt):
+    """A program may set ``const_attr`` between two steps, as it may where the node has a launch of its own."""
+    from tinyflow_amd import autodiff as ad, gpu_op
+    from tinyflow_amd.TrainExecute import TrainExecutor, find_groups
+    x, w, y_ = ad.Placeholder("x"), ad.Variable("w"), ad.Placeholder("y_")
+    h = ad.matmul_op(x, w)
+    scaled = h * 2.0
+    shifted = scaled + 0.5
+    rng = np.random.RandomState(5)
+    X, W = rng.normal(0, 1, (6, 5)).astype(np.float32), rng.normal(0, 1, (5, 4)).astype(np.float32)
+    Y = np.eye(4, dtype=np.float32)[rng.randint(0, 4, 6)]
+    executor = TrainExecutor(ad.softmaxcrossentropy_op(shifted, y_), 0.0)
+    executor.init_Variable({w: W})
+    for factor, term in ((2.0, 0.5), (-3.0, 0.25)):
+        scaled.const_attr, shifted.const_attr = factor, term
+        executor.run({x: X, y_: Y})
+        groups = find_groups(executor.topo_order, executor.node_to_shape_map, {x, w, y_}, {}, {})
+        assert any(scaled in g and shifted in g for g in groups.values())
+        got = executor.value_of(h).asnumpy()
+        assert (executor.value_of(shifted).asnumpy() == got * np.float32(factor) + np.float32(term)).all()
+    executor.close()

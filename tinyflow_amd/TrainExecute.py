@@ -545,10 +545,14 @@ def _group_compute(members, shapes, arrays):
         entry.out = arrays[n].handle
         for field, operand in zip(("a", "b"), operands):
             setattr(entry, field, arrays[operand].handle)
+    # a constant is the node's at the time of the step
+    constants = [(entry, n) for entry, n in zip(steps, members) if isinstance(n.op, (ad.AddByConstOp, ad.MulByConstOp))]
     # the calls without a stream argument in the reference are ordered against every stream
     ordered = int(any(isinstance(n.op, (ad.ReluOp, ad.ReluGradientOp)) for n in members))
 
     def compute(node, input_vals, output_val, cudnnHandle, cublasHandle, cudaStream):
+        for entry, n in constants:
+            entry.value = n.const_attr
         gpu_op.elementwise_group(steps, ordered, cudaStream)
         return 0
     return compute
