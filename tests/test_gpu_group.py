@@ -195,3 +195,25 @@ def test_a_steps_constants_are_those_of_their_nodes_now(rt):
         got = executor.value_of(h).asnumpy()
         assert (executor.value_of(shifted).asnumpy() == got * np.float32(factor) + np.float32(term)).all()
     executor.close()
+
+
+def test_a_groups_call_keeps_its_arrays():
+    """They live as long as the plan, whatever becomes of the executor's map of them, as those of other plan entries do."""
+    import weakref
+    from types import SimpleNamespace
+    from tinyflow_amd import autodiff as ad, ndarray
+    from tinyflow_amd.TrainExecute import _group_compute
+
+    class Array(SimpleNamespace):
+        pass
+    x = ad.Placeholder("x")
+    shifted = x + 1.0
+    doubled = shifted * 2.0
+    shapes = {n: (3, 4) for n in (x, shifted, doubled)}
+    arrays = {n: Array(handle=ndarray.DLArrayHandle(ndarray.DLArray())) for n in shapes}
+    alive = [weakref.ref(a) for a in arrays.values()]
+    compute = _group_compute([shifted, doubled], shapes, arrays)
+    arrays.clear()
+    assert all(a() is not None for a in alive)
+    del compute
+    assert all(a() is None for a in alive)

@@ -539,8 +539,10 @@ def find_groups(topo_order, shapes, unavailable, roles, joins):
 def _group_compute(members, shapes, arrays):
     """Plan entry (same signature as ``Op.compute``) of a group."""
     steps = (gpu_op.GroupStep * len(members))()
+    held = []   # a handle alone does not keep its storage
     for entry, n in zip(steps, members):
         entry.kind, entry.value, operands = _group_step(n, shapes)
+        held += [arrays[i] for i in [n] + operands]
         entry.per_channel = isinstance(n.op, ad.BroadcastToOp) and n.type == "NCHW"
         entry.out = arrays[n].handle
         for field, operand in zip(("a", "b"), operands):
@@ -555,6 +557,7 @@ def _group_compute(members, shapes, arrays):
             entry.value = n.const_attr
         gpu_op.elementwise_group(steps, ordered, cudaStream)
         return 0
+    compute.arrays = held
     return compute
 
 
