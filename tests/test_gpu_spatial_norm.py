@@ -4,11 +4,13 @@ import pytest
 
 
 # one to four register slots a lane; one to sixteen chunks; images left over in the last chunk; one lane and one full slot;
-# 16-byte and single accesses; and the first sizes past the limit, which two passes take
+# 16-byte and single accesses; and the first sizes past the limit, which two passes take; short rows of many images on both sides of
+# the number of images, the size and the length from which on two passes take them
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(1, 3, 1, 1), (1, 2, 32, 32), (3, 1100, 5, 5), (5, 300, 9, 9), (8, 256, 10, 10),
                                    (4, 256, 56, 56), (8, 128, 20, 20), (2, 90, 31, 33), (7, 600, 16, 16), (16, 16, 8, 8),
-                                   (17, 64, 6, 6), (16, 64, 32, 32), (16, 64, 32, 36), (4, 300, 15, 17), (4, 300, 16, 17)],
+                                   (17, 64, 6, 6), (16, 64, 32, 32), (16, 64, 32, 36), (4, 300, 15, 17), (4, 300, 16, 17),
+                                   (31, 8500, 1, 3), (32, 8500, 1, 3), (32, 8191, 1, 3), (32, 2000, 4, 4)],
                          ids=str)
 def test_against_float64_and_its_joint_form(rt, shape):
     """A lane adds at most 16 values (64 past the limit) in float32 before float64 takes over, which bounds each sum by that
@@ -61,3 +63,21 @@ def test_against_float64_and_its_joint_form(rt, shape):
         bound = istd * (8 * u * (np.abs(masked) + np.abs(s1) / m + np.abs(xhat * s2) / m) +
                         (e1 + np.abs(xhat) * e2 + e_xhat * np.abs(s2)) / m) + rel_istd * np.abs(ref)
         assert np.all(np.abs(result.asnumpy() - ref) <= bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,launches", [((32, 8500, 1, 3), 2), ((512, 2048, 1, 1), 2), ((31, 8500, 1, 3), 1), ((32, 8191, 1, 3), 1),
+                                            ((32, 2000, 4, 4), 1), ((8, 256, 10, 10), 1)], ids=str)
+def test_which_channels_take_one_launch(rt, shape, launches):
+    """Two launches keep partial sums, which a forward call that finds no room reports beside the statistics."""
+    from tinyflow_amd import gpu_op, ndarray
+    gx = ndarray.array(np.ones(shape, np.float32), rt.ctx)
+    gy = ndarray.empty(shape, rt.ctx)
+    mean_p, var_p, lst = gpu_op.bn_get_cudnnlist(shape, "NCHW", "spatial")
+    gpu_op.set_device_memory_limit(max(1, gpu_op.device_memory_stats()[1]))   # nothing more can be allocated
+    try:
+        wanted = gpu_op.bn_forward(gx, gy, "spatial", 0, mean_p, var_p, lst, rt.cudnn, rt.stream)
+    finally:
+        gpu_op.set_device_memory_limit(0)
+    statistics = 2 * 4 * shape[1]
+    assert wanted >= statistics and (wanted >= statistics + shape[1] * (2 * 8 + 4)) == (launches == 2), wanted

@@ -591,7 +591,7 @@ __global__ __launch_bounds__(kThreads) void bn_sp_apply_kernel(const float *__re
 // chain of loads stays short, and what is larger has workgroups enough in two passes.  With the host's 4 us a call, two passes /
 // here, forward then backward: 8 images of 256 channels of 10 x 10 9.3 / 6.7 and 9.4 / 6.3 us, of 64 of 40 x 40 10.0 / 9.0 and
 // 10.1 / 8.4, of 256 of 40 x 40 14.9 / 10.7 and 16.1 / 10.4; 2 of 4096 of 40 x 40 35.7 / 24.6 and 49.7 / 32.2; 16 of 64 of
-// 32 x 32 (sixteen chunks, four slots: the most that is taken) 10.9 / 10.5 and 10.8 / 9.8.  None measured was slower.
+// 32 x 32 (sixteen chunks, four slots: the most that is taken) 10.9 / 10.5 and 10.8 / 9.8.  Short rows: see sp_one.
 // ResNet-50 on 8 images of 160 x 160: 212 launches of batch norm and 66 of their ReLUs become 110, 3.92 ms a step 3.44.
 // JOIN: forward also max(y, 0) to `second`; backward masks dy with bn(x) > 0 first and writes that to `second`.
 constexpr int kOneSlots = 4, kOneGroups = 4;
@@ -741,6 +741,14 @@ bool fold_in_apply(int chunks, int units_per_row, uint32_t units) {
   return lane_rows * (chunks + 8) * (4 + per_cu) <= 384;
 }
 
+// A channel's workgroup writes its rows in pieces of a line where they are short, the second of two passes whole lines; from 3 MB on the
+// pieces of 32 images and more cost more than the second launch.  us of both directions, two passes / one: 512 images of 8192 channels of
+// one pixel 82 / 139; 128 of 8192 of 1 x 3 66 / 90; 64 of 4096 of 2 x 2 28.6 / 34.3.  Not past the line: 16 of 4096 of 3 x 3 19.3 / 13.3, 64
+// of 1024 of 4 x 4 (64 bytes a row) 14.8 / 7.7, 64 of 2048 of 2 x 2 (2 MB) 19.8 / 17.1.  Of 714 shapes of up to 36 pixels and 32 MB
+// four stay slower in one launch, by up to 7 %; the 714 together take 0.70 of two passes' time.
+constexpr int kShortRow = 16, kManyRows = 32;
+constexpr int64_t kShortRowElements = 3 << 18;
+
 // Whether bn_sp_one_kernel takes the tensor, and how: `slots` 0 where it does not.
 struct SpOne {
   bool vec;
@@ -756,6 +764,7 @@ SpOne sp_one(const BNDesc *d, uintptr_t addresses) {
   const int64_t units = (int64_t)o.images_per_chunk * (o.vec ? d->HW / 4 : d->HW);
   const int64_t slots = (units + kThreads - 1) / kThreads * cdiv(o.chunks, o.groups);
   if (slots > kOneSlots) return o;
+  if (d->HW < kShortRow && d->N >= kManyRows && (int64_t)d->N * d->C * d->HW > kShortRowElements) return o;
   o.lane_units = (int)((units + kThreads - 1) / kThreads);
   o.slots = (int)slots;
   return o;
