@@ -81,3 +81,54 @@ def test_which_channels_take_one_launch(rt, shape, launches):
         gpu_op.set_device_memory_limit(0)
     statistics = 2 * 4 * shape[1]
     assert wanted >= statistics and (wanted >= statistics + shape[1] * (2 * 8 + 4)) == (launches == 2), wanted
+
+
+def _results(rt, x, dy, offset):
+    """y, both statistics, dx and the joint calls' outputs, of arrays that start `offset` elements into an allocation."""
+    import ctypes
+    from types import SimpleNamespace
+    from tinyflow_amd import gpu_op, ndarray
+    shape, keep = x.shape, []
+
+    def array(values=None):
+        room = ndarray.array(np.full(x.size + offset, 7.0, np.float32), rt.ctx)
+        like = ndarray.empty(shape, rt.ctx) if values is None else ndarray.array(values, rt.ctx)
+        view = ndarray.DLArray.from_buffer_copy(like.handle.contents)
+        view.data = room.handle.contents.data + 4 * offset
+        keep.extend((room, like, view))
+        inner = ndarray.NDArray(ctypes.pointer(view))
+        inner.is_freed = True   # its storage is the room's
+        if values is not None:
+            gpu_op.matrix_elementwise_add_by_const(like, 0.0, inner, rt.stream)
+        return inner
+    mean_p, var_p, lst = gpu_op.bn_get_cudnnlist(shape, "NCHW", "spatial")
+    act = gpu_op.activation_get_cudnnlist(shape, "NCHW", "relu")
+    gx, gdy = array(x), array(dy)
+    y, dx, y2, relu, drelu, dx2 = (array() for _ in range(6))
+    assert gpu_op.bn_forward(gx, y, "spatial", 0, mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+    statistics = []
+    for cell in (mean_p, var_p):
+        view = ndarray.DLArray(ctypes.cast(cell, ctypes.POINTER(ctypes.c_void_p))[0], rt.ctx, 1, (ctypes.c_int64 * 1)(shape[1]))
+        array_of = ndarray.NDArray(ctypes.pointer(view))
+        array_of.is_freed = True
+        statistics.append(array_of.asnumpy())
+    assert gpu_op.bn_backward(gx, gdy, dx, "spatial", mean_p, var_p, lst, rt.cudnn, rt.stream) == 0
+    assert gpu_op.bn_and_relu_forward(gx, y2, relu, "spatial", 0, mean_p, var_p, lst, act, rt.cudnn, rt.stream) == 0
+    assert gpu_op.bn_and_relu_backward(gx, y2, relu, gdy, drelu, dx2, "spatial", mean_p, var_p, lst, act, rt.cudnn, rt.stream) == 0
+    return [a.asnumpy() for a in (y, dx, y2, relu, drelu, dx2)] + statistics
+
+
+# slots of a lane's chunk and rounds of chunks: 1 in one to four rounds, 2 in one and two, 3, 4; the last chunk short; rows by
+# 16 bytes, by elements, and by elements because of where they lie
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(8, 256, 10, 10), (16, 16, 8, 8), (17, 64, 6, 6), (16, 64, 32, 32), (8, 64, 40, 40), (2, 90, 31, 33),
+                                   (3, 1100, 28, 28), (3, 1100, 15, 17), (4, 256, 45, 40), (4, 256, 56, 56), (5, 300, 9, 9), (1, 3, 1, 1)], ids=str)
+@pytest.mark.parametrize("offset", [0, 1])
+def test_one_launch_has_the_bytes_of_two_passes(rt, monkeypatch, shape, offset):
+    rng = np.random.default_rng(shape[1] + offset)
+    x = (rng.standard_normal(shape) * 3 - 1).astype(np.float32)
+    dy = rng.standard_normal(shape, dtype=np.float32)
+    got = _results(rt, x, dy, offset)
+    monkeypatch.setenv("TINYFLOW_SPATIAL_ONE_LAUNCH", "0")
+    want = _results(rt, x, dy, offset)
+    assert [a.tobytes() == b.tobytes() for a, b in zip(got, want)] == [True] * len(want)

@@ -178,6 +178,7 @@ struct BNDesc {
   // statistics published by the last forward and not yet consumed by a backward
   float *saved_mean, *saved_istd;
   hipStream_t saved_on;  // stream of that forward
+  bool two_passes;       // spatial mode: no one-launch form
 };
 
 struct ReduceDesc {
