@@ -69,12 +69,12 @@ def test_join_in_place_and_with_foreign_bits(rt):
         assert out.asnumpy().tobytes() == O.relu(c + d).tobytes()
 
 
-# the register kernels of 32, 64 and 128 rows, full and not; rows past the last of them and the spatial mode take the two
-# calls; columns that do not fill a workgroup
+# per activation: the register kernels of 32, 64 and 128 rows, full and not, and rows past the last of them, which take the two
+# calls; columns that do not fill a workgroup.  Spatial: channels that one workgroup holds, and the last one, which it does not
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["pre_activation", "spatial"])
 @pytest.mark.parametrize("shape", [(1, 3, 5, 7), (31, 4, 9, 9), (32, 16, 16, 16), (33, 5, 11, 3), (64, 3, 17, 5),
-                                   (65, 2, 8, 8), (128, 3, 6, 7), (129, 3, 6, 7)], ids=str)
+                                   (65, 2, 8, 8), (128, 3, 6, 7), (129, 3, 6, 7), (130, 2, 33, 35)], ids=str)
 def test_batch_norm_with_relu_writes_the_bytes_of_the_separate_calls(rt, shape, mode):
     from tinyflow_amd import gpu_op, ndarray
     ctx, cudnn, stream = rt.ctx, rt.cudnn, rt.stream
@@ -132,8 +132,8 @@ def test_which_sums_join():
 
 
 def test_which_batch_norms_join():
-    """A per-activation batch norm joins its ReLU, the ReLU's gradient that batch norm's gradient; spatial ones do not, nor
-    a gradient of another batch norm."""
+    """A batch norm of either mode joins its ReLU, the ReLU's gradient that batch norm's gradient, and not the gradient of
+    another batch norm."""
     from tinyflow_amd import autodiff as ad
     from tinyflow_amd.TrainExecute import find_joins
     x, y, dr = ad.Placeholder("x"), ad.Placeholder("y"), ad.Placeholder("dr")
@@ -144,7 +144,7 @@ def test_which_batch_norms_join():
         d = ad.bn_backward_op(x, a, mode, b.Save_p, b.cudnnlist)
         b2 = ad.bn_forward_op(y, "NCHW", mode)
         d2 = ad.bn_backward_op(y, a, mode, b2.Save_p, b2.cudnnlist)
-        joins = {b: r, a: d} if mode == "pre_activation" else {}
+        joins = {b: r, a: d}
         order = [x, y, dr, b, b2, r, a, d, d2]
         shapes = {n: (2, 3, 4, 4) for n in order}
         assert find_joins(order, shapes, set(), {}) == joins

@@ -105,9 +105,7 @@ class TrainExecutor(object):
         for role in fused.values():   # a fused call reads its sources as arrays
             if len(role) == 3:
                 unread_zeros -= set(role[2])
-        # spatial norms too: their calls do both in one launch where a channel fits a workgroup, else what the two did
-        joined = find_joins(self.topo_order, self.node_to_shape_map, set(feed_dict) | unread_zeros, fused,
-                            ("pre_activation", "spatial"))
+        joined = find_joins(self.topo_order, self.node_to_shape_map, set(feed_dict) | unread_zeros, fused)
         groups = find_groups(self.topo_order, self.node_to_shape_map, set(feed_dict) | unread_zeros, fused, joined)
         in_group = {n for members in groups.values() for n in members}
         joined = {n: r for n, r in joined.items() if n not in in_group}
@@ -366,11 +364,11 @@ def find_add_relu_pairs(topo_order, outputs, shapes):
     return roles
 
 
-def find_joins(topo_order, shapes, unavailable, roles, norm_modes=("pre_activation",)):
+def find_joins(topo_order, shapes, unavailable, roles):
     """Nodes S that are computed together with a reader: one pass that writes both, where the second of two passes would
     read S again (64 images of 256 channels of 56 x 56, sum and ReLU: 20 bytes per element become 16).  S is
 
-    - an elementwise sum or a batch norm of one of ``norm_modes``, its reader a ReLU;
+    - an elementwise sum or a batch norm, its reader a ReLU (a batch norm that no one pass takes with it keeps its two calls);
     - an elementwise sum, its reader a ReLU backward whose upstream gradient it is;
     - the ReLU backward behind such a batch norm, its reader that batch norm's backward.
 
@@ -385,7 +383,7 @@ def find_joins(topo_order, shapes, unavailable, roles, norm_modes=("pre_activati
                 and shapes[s.inputs[0]] == shapes[s.inputs[1]] == shapes[s])
 
     def is_norm(s):
-        return isinstance(s.op, ad.BNForwardOp) and s.batchNormMode in norm_modes
+        return isinstance(s.op, ad.BNForwardOp)
 
     for r in topo_order:
         if r in taken:
@@ -397,7 +395,7 @@ def find_joins(topo_order, shapes, unavailable, roles, norm_modes=("pre_activati
             s, others = r.inputs[1], roles[r][2] if r in roles else r.inputs
             others = [n for n in others if n is not s]
             fits = is_sum(s)
-        elif isinstance(r.op, ad.BNBackwardOp) and r.batchNormMode in norm_modes:
+        elif isinstance(r.op, ad.BNBackwardOp):
             s, others = r.inputs[1], r.inputs[:1]
             fits = (isinstance(s.op, ad.ActivationBackwardOp) and s.activationMode == "relu" and s not in roles
                     and is_norm(s.inputs[0]) and s.inputs[0].Save_p is r.Save_p and s.inputs[0].inputs[0] is r.inputs[0])
