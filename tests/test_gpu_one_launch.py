@@ -55,3 +55,26 @@ def test_softmax_cross_entropy_against_float64(rt, rows, cols):
     x[-1, 0] = np.nan
     gpu_op.softmax_cross_entropy(ndarray.array(x, rt.ctx), ndarray.array(t, rt.ctx), out, rt.stream)
     assert np.isnan(out.asnumpy()[0])
+
+
+# as many rows as one launch takes, and columns that leave a wave's lanes idle, beside the same with a column of no weight, which two
+# launches take
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [17, 63, 64, 65, 130, 255, 256])
+@pytest.mark.parametrize("cols", [1, 3, 10, 16])
+def test_softmax_cross_entropy_of_one_launch_has_the_bytes_of_two(rt, rows, cols):
+    """Logits of -1e30 add the exponential zero and, with labels of zero, nothing to the loss.  Seventeen columns still fall to one lane
+    each, so the sums are the same ones."""
+    from tinyflow_amd import gpu_op, ndarray
+    rng = np.random.default_rng(rows * 17 + cols)
+    x = (rng.standard_normal((rows, cols)) * 4).astype(np.float32)
+    t = rng.random((rows, cols), dtype=np.float32)
+    wide_x, wide_t = np.full((rows, 17), -1e30, np.float32), np.zeros((rows, 17), np.float32)
+    wide_x[:, :cols], wide_t[:, :cols] = x, t
+    results = []
+    for logits, labels in ((x, t), (wide_x, wide_t)):
+        out = ndarray.empty((1,), rt.ctx)
+        gpu_op.array_set(out, 7.0, rt.stream)
+        gpu_op.softmax_cross_entropy(ndarray.array(logits, rt.ctx), ndarray.array(labels, rt.ctx), out, rt.stream)
+        results.append(out.asnumpy().tobytes())
+    assert results[0] == results[1]
