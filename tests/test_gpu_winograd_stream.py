@@ -6,14 +6,17 @@ import parity
 from test_gpu_conv import _check_conv_case, _gpu
 
 
-# 36 values a tile, 256 channels and 2 940 tiles are 108 MB, and twice that with grad-filter's form: rows of whole and of half vectors
-# and of neither, on the side of the input and of the output gradient
+# 36 values a tile, 256 channels and 3 136 tiles are 116 MB, and twice that with grad-filter's form: rows of whole and of half vectors
+# and of neither, on the side of the input and of the output gradient; 2 940 tiles, whose planes' rows start inside a line, go past
+# the caches for products on slices alone
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", [(15, 256, 56, 56, 16), (15, 16, 56, 56, 256), (15, 256, 55, 54, 16), (15, 16, 55, 54, 256),
-                                  (15, 256, 54, 55, 16), (15, 16, 54, 55, 256)], ids=str)
-def test_large_transformed_inputs(rt, monkeypatch, case):
+@pytest.mark.parametrize("engine", ["0", "1"])
+@pytest.mark.parametrize("case", [(16, 256, 56, 56, 16), (16, 16, 56, 56, 256), (16, 256, 55, 54, 16), (16, 16, 55, 54, 256),
+                                  (16, 256, 54, 55, 16), (16, 16, 54, 55, 256), (15, 256, 56, 56, 16), (15, 16, 54, 55, 256)], ids=str)
+def test_large_transformed_inputs(rt, monkeypatch, case, engine):
     from tinyflow_amd import gpu_op, ndarray
     monkeypatch.setenv("TINYFLOW_WINOGRAD", "4")
+    monkeypatch.setenv("TINYFLOW_SPLIT", engine)
     N, C, H, W, K = case
     _check_conv_case(rt, (N, C, H, W, K, 3, 3, "SAME", 1, 1))
     # the later steps of a descriptor share the passes over x and dy: the bytes of the first

@@ -1875,14 +1875,19 @@ ConvPlan plan_wgrad(const ConvDesc *d) {
 // a wave writes 256 bytes to each of 36 or 72 planes, and lines that are not to stay make room for each other sooner.
 // One line, dy's pass of 72 planes, us before / after: 512 channels 28 x 28, 32 images, 231 MB 70 / 50 (4.0 -> 5.7 TB/s); 256
 // of 56 x 56, 463 MB 139 / 124; 64 of 224 x 224, 1.85 GB 510 / 491; V alone, 64 of 56 x 56, 64 images, 115 MB 35 / 28.  Of 58 MB
-// it is 16.0 / 14.9 and 24.4 / 25.8 for twice that with dM, and the products read them back slower.  VGG-16, batch 32, a step with lines
-// at none / 300 / 200 / 100 / 50 / 0 MB: 12.63, 12.28, 12.18, 12.16, 12.16, 12.17 ms; ResNet-50, batch 64: 15.91, 15.94, 15.88,
-// 15.84, 15.86, 15.88.  Between 100 and 200 MB: 64 channels of 55 x 55, 32 images, 116 MB with dM, three calls 206.0 us at 100 and 208.3 at
-// 200 (runs differ by 0.3 %); fused ResNet-50, batch 32, whose largest are 116 MB, 8.94 and 8.91 ms (0.7 %).
+// it is 16.0 / 14.9 and 24.4 / 25.8 for twice that with dM, and the products read them back slower.  Steps in ms with lines at none / 800 /
+// 400 / 200 / 100 MB, in turn in one process: VGG-16, batch 32, 12.22, 12.01, 11.84, 11.73, 11.71; batch 64, 128 x 128, 8.09, 7.99, 7.85,
+// 7.75, 7.70; ResNet-50, batch 64, 15.44, 15.42, 15.42, 15.39, 15.34; fused, batch 32, whose largest are 116 MB, 8.68 with any.
+// Planes whose rows start inside a line (numbers of tiles that are no multiple of 32) are written past the caches in parts of lines, which
+// products on slices outweigh and the fp32 ones, which read them back in longer stages, do not.  Steps in ms, never / always / by this rule:
+// VGG-16 on slices, 31 images, 12.39 / 12.11 / 12.11; 28 images 11.19 / 10.87 / 10.87; fused ResNet-50, fp32, 33 images 9.274 / 9.337 /
+// 9.267; ResNet-50, 61 images, 15.25 / 15.31 / 15.23; a layer of it by itself, 63 images, 230 / 249 us in both gradients.
 constexpr double kStreamTransforms = 100e6;
+constexpr int kLineFloats = 32;
 
+// `sliced`: the products that read V run on slices.
 void launch_wino_input(int tile, const float *in, float *V, float *dM, int images, int Cr, int H, int W, int pad_h,
-                       int pad_w, const FastDiv &div_tiles, const FastDiv &div_tw, int T, int Tp, hipStream_t s) {
+                       int pad_w, const FastDiv &div_tiles, const FastDiv &div_tw, int T, int Tp, bool sliced, hipStream_t s) {
   const dim3 grid(cdiv(Tp, 256), Cr), block(256);
   const uint32_t in_bytes = (uint32_t)((size_t)images * Cr * H * W * sizeof(float));  // under 4 GiB: smaller than V
   if (tile == 2) {
@@ -1892,7 +1897,7 @@ void launch_wino_input(int tile, const float *in, float *V, float *dM, int image
   }
   const bool row16 = pad_w == 1 && W % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
   const bool halves = !row16 && pad_w == 1 && W % 2 == 0 && (reinterpret_cast<uintptr_t>(in) & 7u) == 0;
-  const bool stream = (dM ? 2.0 : 1.0) * 36 * Cr * Tp * sizeof(float) > kStreamTransforms;
+  const bool stream = (dM ? 2.0 : 1.0) * 36 * Cr * Tp * sizeof(float) > kStreamTransforms && (sliced || Tp % kLineFloats == 0);
   auto by_form = [&](auto with_dm, auto stream_c) {
     constexpr bool DM = decltype(with_dm)::value, STREAM = decltype(stream_c)::value;
     auto go = [&](auto kernel) {
@@ -1971,7 +1976,7 @@ int run_winograd(ConvDesc *d, bool dgrad, const ConvPlan &plan, const float *in,
   }
   if (!V_kept)
     launch_wino_input(w.tile, in, V, dM_for_wgrad, d->N, w.Cr, w.in_h, w.in_w, w.pad_h, w.pad_w, div_tiles, div_tw, w.T, w.Tp,
-                      s);
+                      plan.split, s);
   with_tile(plan.bm, plan.bn, [&](auto bm_c, auto bn_c, auto bk_c) {
     constexpr int BM = decltype(bm_c)::value, BN = decltype(bn_c)::value, BK = decltype(bk_c)::value;
     const Geometry g = make_geometry(w.Mo, w.Tp, w.Cr, BM, BN, 1, BK);
@@ -2061,12 +2066,12 @@ int run_winograd_wgrad(ConvDesc *d, const ConvPlan &plan, const float *x, const 
   const bool rows_vec = d->Q % w.tile == 0 && (reinterpret_cast<uintptr_t>(dy) & (uintptr_t)(4 * w.tile - 1)) == 0;
   const dim3 block(256);
   if (!kept_V)
-    launch_wino_input(w.tile, x, V, nullptr, d->N, d->C, d->H, d->W, d->pad_h, d->pad_w, div_tiles, div_tw, w.T, w.Tp, s);
+    launch_wino_input(w.tile, x, V, nullptr, d->N, d->C, d->H, d->W, d->pad_h, d->pad_w, div_tiles, div_tw, w.T, w.Tp, plan.split, s);
   if (dM_kept)
     ;  // dM is grad-data's by-product
   else if (V_for_dgrad)  // one pass over dy writes grad-data's V (kept) and dM
     launch_wino_input(4, dy, V_for_dgrad, dM, d->N, d->K, d->P, d->Q, 2 - d->pad_h, 2 - d->pad_w, div_tiles, div_tw, w.T, w.Tp,
-                      s);
+                      plan.split, s);
   else if (w.tile == 2)
     hipLaunchKernelGGL(wino_dy_kernel<2>, dim3(cdiv(w.Tp, 256), d->K), block, 0, s, dy, dM, d->K, d->P, d->Q, div_tiles,
                        div_tw, w.T, w.Tp, rows_vec);
