@@ -1879,7 +1879,7 @@ ConvPlan plan_wgrad(const ConvDesc *d) {
 // 400 / 200 / 100 MB, in turn in one process: VGG-16, batch 32, 12.22, 12.01, 11.84, 11.73, 11.71; batch 64, 128 x 128, 8.09, 7.99, 7.85,
 // 7.75, 7.70; ResNet-50, batch 64, 15.44, 15.42, 15.42, 15.39, 15.34; fused, batch 32, whose largest are 116 MB, 8.68 with any.
 // Planes whose rows start inside a line (numbers of tiles that are no multiple of 32) are written past the caches in parts of lines, which
-// products on slices outweigh and the fp32 ones, which read them back in longer stages, do not.  Steps in ms, never / always / by this rule:
+// steps whose products run on slices gain from and those with fp32 products do not.  Steps in ms, never / always / by this rule:
 // VGG-16 on slices, 31 images, 12.39 / 12.11 / 12.11; 28 images 11.19 / 10.87 / 10.87; fused ResNet-50, fp32, 33 images 9.274 / 9.337 /
 // 9.267; ResNet-50, 61 images, 15.25 / 15.31 / 15.23; a layer of it by itself, 63 images, 230 / 249 us in both gradients.
 constexpr double kStreamTransforms = 100e6;
